@@ -155,6 +155,20 @@ qj_status ensure_partials(qj_workspace* ws, int64_t n, hipStream_t s) {
   return QJ_OK;
 }
 
+qj_status ensure_pinned(qj_workspace* ws, int64_t n, hipStream_t s) {
+  if (n <= ws->pinned_cap) return QJ_OK;
+  const int64_t want = n + n / 2 + 256;
+  if (ws->h_pinned) {
+    QJ_HIP(hipStreamSynchronize(s));
+    QJ_HIP(hipHostFree(ws->h_pinned));
+    ws->h_pinned = nullptr;
+    ws->pinned_cap = 0;
+  }
+  QJ_HIP(hipHostMalloc((void**)&ws->h_pinned, sizeof(double) * (size_t)want, hipHostMallocDefault));
+  ws->pinned_cap = want;
+  return QJ_OK;
+}
+
 void timing_mark(qj_workspace* ws, hipStream_t s) {
   if (!ws->timing) return;
   hipEvent_t e;
@@ -361,6 +375,7 @@ qj_status qj_workspace_destroy(qj_workspace* ws) {
   hipFree(ws->d_list);
   hipFree(ws->d_list_count);
   hipFree(ws->d_partials);
+  hipHostFree(ws->h_pinned);
   delete ws;
   return QJ_OK;
 }

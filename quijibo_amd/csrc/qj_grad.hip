@@ -1,18 +1,22 @@
 // Gradient kernels.
 //
-// k_ap_grads: the one-iteration AP score and exponent gradients of the
-//   optimizer (OPTIMIZE_3D.cpp computeScoreAP :3563, computeExpGradientAP
+// k_ap_fast, k_ap_grads: the one-iteration AP score and exponent gradients of
+//   the optimizer (OPTIMIZE_3D.cpp computeScoreAP :3563, computeExpGradientAP
 //   :3589-3625, computeTopGradientAP :8905-9106, computeBottomGradientAP
-//   :10012, computeTop/BottomBulkScalarGradientAP :9250/:10360). One lane per
-//   cell; every root's term is reduced over the block (wave shuffles + LDS)
-//   into per-block partials, summed in a fixed order by k_sum_partials, so the
-//   result is deterministic. The reference keeps per-cell prefix/suffix caches
-//   (POLYNOMIAL_CACHE); here nothing is stored per cell: a forward sweep forms
-//   T and B, and a backward sweep re-forms each term, carries the suffix
-//   product S and recovers the prefix as T * S^-1 (quaternion products are
-//   conformal, so this costs no accuracy).
-//   Cells that overflow FP64 are redone with a shared binary exponent per
-//   quaternion (the reference redoes them in long double, :9011-9103).
+//   :10012, computeTop/BottomBulkScalarGradientAP :9250/:10360).
+//   With one iteration only magnitudes matter. |T| = prod |b_i|^e_i, so F is a
+//   sum of logarithms. Each gradient term is dSdF Re(R^-1 R'): with R = L P S B^-1
+//   and R' = L (s P log b) S B^-1 every factor but log b cancels in the real part
+//   (Re(x y x^-1) = Re y), which leaves s log|b_i|; the bottom formula
+//   R' = T (-L (P / s) (log b)^-1 S)^-1 leaves -s log|b_j| in the same way.
+//   k_ap_fast computes just that, one logarithm per cell and root. A cell whose
+//   products could leave FP64's range (sum of e |log|b|| beyond kApRange, a cell
+//   on a root) is left to k_ap_grads, which forms the products of the formulas
+//   as they stand and redoes overflowed cells with a shared binary exponent per
+//   quaternion (the reference redoes them in long double, :9011-9103); so is
+//   every cell when some exponent is negative (QUATERNION::pow then drops the
+//   imaginary part, and |b^e| is not |b|^e).
+//   Sums are over fixed trees, so results do not depend on scheduling.
 //
 // k_adjoint: reverse mode through max_iter iterations of the map at points,
 //   recomputing every iteration's products instead of storing trajectories.
@@ -28,6 +32,7 @@
 
 #include "qj_geom.h"
 #include "qj_internal.h"
+#include "qj_math64.h"
 #include "qj_quat.h"
 
 namespace qj {
@@ -132,6 +137,8 @@ struct APArgs {
   MapArgs a;
   GridGeom wg;
   double alpha, thr;
+  double log_c;          // log(exp_scaling)
+  FastDiv div_x, div_xy;  // of the map's grid, for fewer than 2^32 cells
 };
 
 // slot layout of the partial sums
@@ -253,83 +260,117 @@ __device__ __forceinline__ Q poly_fwd(const RootRec64* __restrict__ r, int n, co
   return res;
 }
 
+// One cell outside the iteration: the origin (field left as it is) and cells
+// that start beyond the escape radius. Returns whether the cell iterates.
+__device__ __forceinline__ bool ap_cell(const APArgs& g, const double* __restrict__ weight,
+                                        double* __restrict__ field, int64_t idx, q64& q0, double& w, double& F) {
+  const MapArgs& a = g.a;
+  const int64_t X = a.res[0], XY = X * a.res[1];
+  int x, y, z;
+  if (XY * a.res[2] <= (int64_t)0xffffffffll) {
+    const uint32_t p = (uint32_t)idx, r = p - fast_div(p, g.div_xy) * (uint32_t)XY;
+    z = (int)fast_div(p, g.div_xy);
+    y = (int)fast_div(r, g.div_x);
+    x = (int)(r - (uint32_t)y * (uint32_t)X);
+  } else {
+    z = (int)(idx / XY), y = (int)((idx - z * XY) / X), x = (int)(idx - z * XY - (int64_t)y * X);
+  }
+  double c[3];
+  cell_center(a, x, y, z, c);
+  w = field_lookup(g.wg, weight, c);
+  q0 = q64{c[0], c[1], c[2], a.slice};
+  const double mag0 = qmag(q0);
+  if (mag0 < 1e-8) {
+    F = field[idx];  // unwritten cell: score terms read the existing value
+    return false;
+  }
+  if (!(mag0 < a.escape) || a.max_iter < 1) {
+    F = log(mag0);
+    field[idx] = F;
+    return false;
+  }
+  return true;
+}
+
+// the formulas as they stand, for the cells of `left` (one bit per cell, 64
+// cells a word), or for every cell when left is null. Each block takes a
+// contiguous run of groups of 256 cells and writes one row of partial sums.
 __global__ __launch_bounds__(kGBlock) void k_ap_grads(APArgs g, const RootRec64* __restrict__ roots,
                                                       const double* __restrict__ weight, double* __restrict__ field,
+                                                      const unsigned long long* __restrict__ left, int64_t per,
                                                       double* __restrict__ partials, int K,
                                                       unsigned long long* __restrict__ n_adaptive) {
   extern __shared__ double acc[];  // (kGBlock/64) x K
   const MapArgs& a = g.a;
   for (int i = threadIdx.x; i < (kGBlock / 64) * K; i += kGBlock) acc[i] = 0.0;
   __syncthreads();
-  const int64_t X = a.res[0], XY = X * a.res[1], N = XY * a.res[2];
-  const int64_t idx = (int64_t)blockIdx.x * kGBlock + threadIdx.x;
-  bool active = idx < N;
-  double c[3] = {0, 0, 0};
-  double w = 0.0;
-  q64 q0{0, 0, 0, 0};
-  double Ffield = 0.0;
-  bool iterate = false;
-  if (active) {
-    const int z = (int)(idx / XY), y = (int)((idx - z * XY) / X), x = (int)(idx - z * XY - (int64_t)y * X);
-    cell_center(a, x, y, z, c);
-    w = field_lookup(g.wg, weight, c);
-    q0 = q64{c[0], c[1], c[2], a.slice};
-    const double mag0 = qmag(q0);
-    if (mag0 < 1e-8) {
-      Ffield = field[idx];  // unwritten cell: score terms read the existing value
-    } else if (!(mag0 < a.escape) || a.max_iter < 1) {
-      Ffield = log(mag0);
-      field[idx] = Ffield;
-    } else {
-      iterate = true;
+  const int64_t N = (int64_t)a.res[0] * a.res[1] * a.res[2];
+  const int64_t groups = (N + kGBlock - 1) / kGBlock, g1 = min((int64_t)(blockIdx.x + 1) * per, groups);
+  int64_t g0 = (int64_t)blockIdx.x * per;
+  if (left) {
+    // a run without a flagged cell is passed over with one load per thread
+    const int64_t nw = (N + 63) / 64, w1 = min(g1 * (kGBlock / 64), nw);
+    bool any = false;
+    for (int64_t i = g0 * (kGBlock / 64) + threadIdx.x; i < w1; i += kGBlock) any |= left[i] != 0ull;
+    if (!__syncthreads_or(any)) g0 = g1;
+  }
+  for (int64_t gi = g0; gi < g1; gi++) {
+    const int64_t idx = gi * kGBlock + threadIdx.x;
+    bool active = idx < N;
+    if (left) active = active && ((left[idx >> 6] >> (idx & 63)) & 1ull);
+    if (!__ballot(active)) continue;
+    double w = 0.0;
+    q64 q0{0, 0, 0, 0};
+    double Ffield = 0.0;
+    bool iterate = false;
+    if (active) iterate = ap_cell(g, weight, field, idx, q0, w, Ffield);
+    // forward sweep (computeRationalMapAP with one iteration)
+    q64 T{1, 0, 0, 0}, B{1, 0, 0, 0};
+    bool ovf = false;
+    if (iterate) {
+      T = poly_fwd<q64>(roots, a.nt, q0);
+      q64 qn;
+      if (a.nb > 0) {
+        B = poly_fwd<q64>(roots + a.nt, a.nb, q0);
+        qn = qdiv(T, B);
+        const double m2 = B.w * B.w + B.x * B.x + B.y * B.y + B.z * B.z;
+        ovf = !(ok(T) && ok(B) && isfinite(m2) && ok(qn));
+      } else {
+        qn = T;
+        ovf = !ok(T);
+      }
+      qn = qscale(qn, a.exp_scaling);
+      const double mag = qmag(qn);
+      ovf |= !isfinite(mag);
+      Ffield = log(mag);
     }
-  }
-  // forward sweep (computeRationalMapAP with one iteration)
-  q64 T{1, 0, 0, 0}, B{1, 0, 0, 0};
-  bool ovf = false;
-  if (iterate) {
-    T = poly_fwd<q64>(roots, a.nt, q0);
-    q64 qn;
-    if (a.nb > 0) {
-      B = poly_fwd<q64>(roots + a.nt, a.nb, q0);
-      qn = qdiv(T, B);
-      const double m2 = B.w * B.w + B.x * B.x + B.y * B.y + B.z * B.z;
-      ovf = !(ok(T) && ok(B) && isfinite(m2) && ok(qn));
-    } else {
-      qn = T;
-      ovf = !ok(T);
+    // gradients in FP64 for the cells that stayed finite
+    cell_terms<q64>(g, roots, q0, T, B, w, iterate && !ovf, acc, K);
+    // overflowed cells: the whole cell with explicit binary exponents
+    const bool redo = iterate && ovf;
+    if (__ballot(redo)) {
+      xq TX = xfrom(q64{1, 0, 0, 0}), BX = TX;
+      if (redo) {
+        TX = poly_fwd<xq>(roots, a.nt, q0);
+        if (a.nb > 0) BX = poly_fwd<xq>(roots + a.nt, a.nb, q0);
+        const xq R = scaled(mul(TX, inv(BX)), a.exp_scaling);
+        const double l = logmag(R);
+        Ffield = isnan(l) ? 0.0 : l;  // OPTIMIZE_3D.cpp:1557-1561
+      }
+      cell_terms<xq>(g, roots, q0, TX, BX, w, redo, acc, K);
     }
-    qn = qscale(qn, a.exp_scaling);
-    const double mag = qmag(qn);
-    ovf |= !isfinite(mag);
-    Ffield = log(mag);
-  }
-  // gradients in FP64 for the cells that stayed finite
-  cell_terms<q64>(g, roots, q0, T, B, w, iterate && !ovf, acc, K);
-  // overflowed cells: the whole cell with explicit binary exponents
-  const bool redo = iterate && ovf;
-  if (__ballot(redo)) {
-    xq TX = xfrom(q64{1, 0, 0, 0}), BX = TX;
-    if (redo) {
-      TX = poly_fwd<xq>(roots, a.nt, q0);
-      if (a.nb > 0) BX = poly_fwd<xq>(roots + a.nt, a.nb, q0);
-      const xq R = scaled(mul(TX, inv(BX)), a.exp_scaling);
-      const double l = logmag(R);
-      Ffield = isnan(l) ? 0.0 : l;  // OPTIMIZE_3D.cpp:1557-1561
+    if (iterate) field[idx] = Ffield;
+    double sc = 0.0, ge = 0.0;
+    if (active) {
+      sc = -tanh(g.alpha * Ffield) * w;
+      const double S = tanh(g.alpha * (Ffield - g.thr));
+      ge = -g.alpha * w * (1.0 - S * S);
     }
-    cell_terms<xq>(g, roots, q0, TX, BX, w, redo, acc, K);
+    wave_acc(acc, K, SL_SCORE, sc);
+    wave_acc(acc, K, SL_GEXP, ge);
+    const unsigned long long nr = __popcll(__ballot(redo));
+    if ((threadIdx.x & 63) == 0 && nr) atomicAdd(n_adaptive, nr);
   }
-  if (iterate) field[idx] = Ffield;
-  double sc = 0.0, ge = 0.0;
-  if (active) {
-    sc = -tanh(g.alpha * Ffield) * w;
-    const double S = tanh(g.alpha * (Ffield - g.thr));
-    ge = -g.alpha * w * (1.0 - S * S);
-  }
-  wave_acc(acc, K, SL_SCORE, sc);
-  wave_acc(acc, K, SL_GEXP, ge);
-  const unsigned long long nr = __popcll(__ballot(redo));
-  if ((threadIdx.x & 63) == 0 && nr) atomicAdd(n_adaptive, nr);
   __syncthreads();
   for (int k = threadIdx.x; k < K; k += kGBlock) {
     double s = 0.0;
@@ -338,14 +379,225 @@ __global__ __launch_bounds__(kGBlock) void k_ap_grads(APArgs g, const RootRec64*
   }
 }
 
+// Wave sum in lane 63: row shifts and broadcasts instead of LDS shuffles.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, kCtrl, kRows, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), kCtrl, kRows, 0xf, false);
+  return v + __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double wave_sum63(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+  v = dpp_add<0x112, 0xf>(v);  // row_shr:2
+  v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+  v = dpp_add<0x118, 0xf>(v);  // row_shr:8
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31
+  return v;
+}
+
+// Sum of e |log|b|| over both polynomials and |log c| up to which every
+// product, |B|^2, quotient and |q|^2 of a cell, prefixes included, stays well
+// inside FP64's range (2 x 340 < 1022 ln 2).
+constexpr double kApRange = 340.0;
+constexpr int kApWaves = 8, kApBlock = 64 * kApWaves;
+constexpr int kApFastRows = 2;  // score, grad_exp, then sum of dSdF log|b_i| per root
+
+// log(|q - r|^2) for a point (x, y, z, .) with (q.z - r.z)^2 given
+__device__ __forceinline__ double log_norm2(double x, double y, double z, const RootRec64& r, double dz2) {
+  const double dw = x - r.w, dx = y - r.x, dy = z - r.y;
+  return log64(__builtin_fma(dw, dw, __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz2))));
+}
+
+// The AP pass of the cells that stay in range: 64 M cells per block, lane l of
+// every wave holding cells l, l + 64, ... Each of the eight waves takes an eighth
+// of the roots for all of the block's cells: the logarithms and, through LDS,
+// each cell's sum of e log|b|; then, with dSdF known, the sum of dSdF log|b_i|
+// over the cells, one wave reduction per root and block. R > 0: a wave has at
+// most R roots and keeps their M R logarithms in registers between the two
+// steps (R roots unrolled, in groups of kGroup so that four logarithms are
+// always in flight; a group past the wave's last root is skipped, a root past
+// it inside a group weighs 0). R = 0: any number of roots, and the second step
+// computes the logarithms again for the cells whose dSdF is not exactly 0
+// (tanh saturates at |alpha F| > 19). FP64 VALU bound: 36 instructions per cell
+// and root. Figures beside ap_grads.
+template <int M, int R>
+__global__ __launch_bounds__(kApBlock) void k_ap_fast(APArgs g, const RootRec64* __restrict__ roots,
+                                                     const double* __restrict__ weight, double* __restrict__ field,
+                                                     unsigned long long* __restrict__ left,
+                                                     double* __restrict__ partials,
+                                                     unsigned long long* __restrict__ n_adaptive) {
+  constexpr int kCells = 64 * M, kWaves = kApWaves, kGroup = M >= 4 ? 1 : 4 / M;
+  static_assert(R % kGroup == 0, "whole groups of roots");
+  __shared__ double s_a[kWaves][kCells], s_b[kWaves][kCells];
+  __shared__ double s_q[3][kCells];
+  __shared__ double s_sum[2][kWaves];
+  __shared__ int s_n[kWaves];
+  const MapArgs& a = g.a;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t N = (int64_t)a.res[0] * a.res[1] * a.res[2];
+  const int64_t idx = (int64_t)blockIdx.x * kCells + tid;
+  if (blockIdx.x == 0 && tid == 0) *n_adaptive = 0ull;
+  const bool owner = tid < kCells && idx < N;
+  bool iterate = false;
+  double w = 0.0, F = 0.0;
+  q64 q0{1, 1, 1, 1};
+  if (owner) iterate = ap_cell(g, weight, field, idx, q0, w, F);
+  if (tid < kCells) {
+    s_q[0][tid] = q0.w;
+    s_q[1][tid] = q0.x;
+    s_q[2][tid] = q0.y;
+  }
+  __syncthreads();
+  const int nr = a.nt + a.nb, i0 = wave * nr / kWaves, i1 = (wave + 1) * nr / kWaves;
+  double x[M], y[M], z[M], f[M] = {}, s[M] = {}, lm[M] = {}, l[R > 0 ? R : 1][M];
+#pragma unroll
+  for (int u = 0; u < M; u++) {
+    x[u] = s_q[0][lane + 64 * u];
+    y[u] = s_q[1][lane + 64 * u];
+    z[u] = s_q[2][lane + 64 * u];
+  }
+  auto add = [&](const RootRec64& r, double h, bool top, double* lg) {
+    const double dz = a.slice - r.z, dz2 = dz * dz, sg = top ? h : -h;
+#pragma unroll
+    for (int u = 0; u < M; u++) {
+      lg[u] = log_norm2(x[u], y[u], z[u], r, dz2);
+      f[u] = __builtin_fma(sg, lg[u], f[u]);
+      s[u] = __builtin_fma(h, fabs(lg[u]), s[u]);
+      lm[u] = fabs(lg[u]) > lm[u] ? fabs(lg[u]) : lm[u];
+    }
+  };
+  if (R > 0) {
+#pragma unroll
+    for (int j = 0; j < R; j += kGroup) {
+      if (i0 + j < i1) {
+#pragma unroll
+        for (int k = j; k < j + kGroup; k++) {
+          const bool in = i0 + k < i1;
+          const int i = in ? i0 + k : i1 - 1;
+          const RootRec64 r = roots[i];
+          add(r, in ? 0.5 * r.e : 0.0, i < a.nt, l[k]);
+        }
+      }
+    }
+  } else {
+    for (int i = i0; i < i1; i++) {
+      const RootRec64 r = roots[i];
+      add(r, 0.5 * r.e, i < a.nt, l[0]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < M; u++) {
+    s_a[wave][lane + 64 * u] = f[u];
+    // |b|^2 zero, denormal or beyond the range shows as |log| > 700
+    s_b[wave][lane + 64 * u] = lm[u] < 600.0 ? s[u] : __builtin_inf();
+  }
+  __syncthreads();
+  bool act = false, flagged = false;
+  double d = 0.0, sc = 0.0, ge = 0.0;
+  if (owner) {
+    bool mine = true;
+    if (iterate) {
+      double fs = 0.0, ss = 0.0;
+      for (int v = 0; v < kWaves; v++) {
+        fs += s_a[v][tid];
+        ss += s_b[v][tid];
+      }
+      const double lc = g.log_c;
+      mine = ss + fabs(lc) < kApRange;
+      flagged = !mine;
+      if (mine) {
+        F = fs + lc;
+        field[idx] = F;
+      }
+    }
+    if (mine) {
+      const double t0 = tanh(g.alpha * F);
+      const double t1 = g.thr == 0.0 ? t0 : tanh(g.alpha * (F - g.thr));
+      sc = -t0 * w;
+      ge = -g.alpha * w * (1.0 - t1 * t1);
+      act = iterate && isfinite(ge) && ge != 0.0;  // a non-finite weight leaves the root terms out
+      d = act ? ge : 0.0;
+    }
+  }
+  const unsigned long long mf = __ballot(flagged), ma = __ballot(act);
+  sc = wave_sum63(sc);
+  ge = wave_sum63(ge);
+  if (lane == 63) {
+    s_sum[0][wave] = sc;
+    s_sum[1][wave] = ge;
+    s_n[wave] = (int)__popcll(ma);
+    if (tid < kCells && (idx & ~63ll) < N) left[idx >> 6] = mf;
+  }
+  __syncthreads();  // s_a and s_b have been read by their owners
+  const int K = kApFastRows + nr;
+  double* row = partials + (int64_t)blockIdx.x * K;
+  if (tid < 2) {
+    double t = 0.0;
+    for (int v = 0; v < kWaves; v++) t += s_sum[tid][v];
+    row[tid] = t;
+  }
+  double dd[M];
+  if (R > 0) {
+    // (log64 is finite for every argument, so a weight of 0 leaves a cell out)
+    if (tid < kCells) s_a[0][tid] = d;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < M; u++) dd[u] = s_a[0][lane + 64 * u];
+#pragma unroll
+    for (int k = 0; k < (R > 0 ? R : 1); k++) {
+      if (i0 + k < i1) {
+        double v = 0.0;
+#pragma unroll
+        for (int u = 0; u < M; u++) v = __builtin_fma(dd[u], l[k][u], v);
+        v = wave_sum63(v);
+        if (lane == 63) row[kApFastRows + i0 + k] = 0.5 * v;
+      }
+    }
+    return;
+  }
+  // R = 0: the cells with a dSdF, listed in cell order
+  int at = (int)__popcll(ma & ((1ull << lane) - 1ull)), nact = 0;
+  for (int v = 0; v < kWaves; v++) {
+    if (v < wave) at += s_n[v];
+    nact += s_n[v];
+  }
+  if (act) {
+    s_a[0][at] = q0.w;
+    s_a[1][at] = q0.x;
+    s_a[2][at] = q0.y;
+    s_a[3][at] = d;
+  }
+  __syncthreads();
+  const int nu = (nact + 63) >> 6;  // the same for the whole block
+#pragma unroll
+  for (int u = 0; u < M; u++) {
+    const int j = lane + 64 * u;
+    const bool in = j < nact;
+    x[u] = in ? s_a[0][j] : 0.0;
+    y[u] = in ? s_a[1][j] : 0.0;
+    z[u] = in ? s_a[2][j] : 0.0;
+    dd[u] = in ? s_a[3][j] : 0.0;
+  }
+  for (int i = i0; i < i1; i++) {
+    const RootRec64 r = roots[i];
+    const double dz = a.slice - r.z, dz2 = dz * dz;
+    double v = 0.0;
+#pragma unroll
+    for (int u = 0; u < M; u++)
+      if (u < nu) v = __builtin_fma(dd[u], log_norm2(x[u], y[u], z[u], r, dz2), v);
+    v = wave_sum63(v);
+    if (lane == 63) row[kApFastRows + i] = 0.5 * v;
+  }
+}
+
 // sums partials[b][k] over b: one block per k, each thread a strided run of
 // blocks in order, then a fixed tree over the threads (deterministic; a serial
 // sum over thousands of blocks per k took most of a millisecond)
 constexpr int kSumThreads = 256;
-__global__ __launch_bounds__(kSumThreads) void k_sum_partials(const double* __restrict__ partials, int64_t nb, int K,
-                                                              double* __restrict__ out) {
+__device__ __forceinline__ double column_sum(const double* __restrict__ partials, int64_t nb, int K, int k) {
   __shared__ double s_v[kSumThreads];
-  const int k = blockIdx.x;
   double v = 0.0;
   for (int64_t b = threadIdx.x; b < nb; b += kSumThreads) v += partials[b * K + k];
   s_v[threadIdx.x] = v;
@@ -354,47 +606,113 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_partials(const double* __re
     if ((int)threadIdx.x < w) s_v[threadIdx.x] += s_v[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[k] = s_v[0];
+  return s_v[0];
+}
+__global__ __launch_bounds__(kSumThreads) void k_sum_partials(const double* __restrict__ partials, int64_t nb, int K,
+                                                              double* __restrict__ out) {
+  const int k = blockIdx.x;
+  const double v = column_sum(partials, nb, K, k);
+  if (threadIdx.x == 0) out[k] = v;
+}
+__global__ void k_zero_count(unsigned long long* p) {
+  if (threadIdx.x == 0) *p = 0ull;
 }
 
+// k_sum_partials over two arrays at once: block (k, 0) sums column k of the
+// first, block (k, 1) of the second, and both results and the cell count go to
+// pinned host memory, which the caller reads after its one wait.
+__global__ __launch_bounds__(kSumThreads) void k_ap_finish(const double* __restrict__ p0, int64_t n0, int K0,
+                                                           const double* __restrict__ p1, int64_t n1, int K1,
+                                                           const unsigned long long* __restrict__ n_adaptive,
+                                                           double* __restrict__ h) {
+  const int k = blockIdx.x, second = blockIdx.y;
+  const int K = second ? K1 : K0;
+  if (k >= K) return;
+  const double v = column_sum(second ? p1 : p0, second ? n1 : n0, K, k);
+  if (threadIdx.x == 0) {
+    h[1 + (second ? K0 : 0) + k] = v;
+    if (k == 0 && second) h[0] = (double)*n_adaptive;  // exact below 2^53
+  }
+}
+
+// 256 cells a block keep four logarithms per lane in flight and share the block's
+// set-up; below 128 such blocks (half the CUs) 64 cells a block spread the work
+// further: 25^3 35.4 against 39.1 us a call, 40^3 43.5 against 39.8, 64^3 77.5
+// against 59.3 (64- against 256-cell blocks, 32+32 real exponents). A wave keeps up
+// to 8, 16 or 32 roots' logarithms in registers (128 to 192 VGPRs); beyond 256
+// roots they are computed twice (97^3 with 32+32 roots: 149 us that way, 128
+// kept). Against the product formulas for every cell: 97^3 2264 to 128 us a call,
+// 25^3 254 to 36 us; the kernel takes 113 us of the 128, its FP64 issue about 80.
 qj_status ap_grads(qj_workspace* ws, const MapArgs& a, const qj_rational* f, const qj_grid* wg, const double* d_weight,
                    double alpha, double thr, double* d_field, double* gt, double* gb, qj_ap_grads* out,
                    hipStream_t s) {
   const int64_t N = (int64_t)a.res[0] * a.res[1] * a.res[2];
-  const int K = SL_ROOTS + a.nt + a.nb;
-  const int64_t nblocks = (N + kGBlock - 1) / kGBlock;
+  const int nr = a.nt + a.nb, K = SL_ROOTS + nr, KF = kApFastRows + nr;
   const size_t lds = sizeof(double) * (kGBlock / 64) * K;
   if (lds > 64 * 1024) {
-    set_error("too many roots for the gradient kernel (%d)", a.nt + a.nb);
+    set_error("too many roots for the gradient kernel (%d)", nr);
     return QJ_ERR_CAPACITY;
   }
-  qj_status st = ensure_partials(ws, nblocks * K + K + 1, s);
+  bool fast = true;  // |b^e| = |b|^e needs exponents that are not negative
+  for (const RootRec64& r : f->h64) fast &= r.e >= 0.0 && r.e <= DBL_MAX;
+  const int64_t groups = (N + kGBlock - 1) / kGBlock;
+  const bool wide = groups >= 128;
+  const int per_wave = (nr + kApWaves - 1) / kApWaves;  // roots of the busiest wave
+  const int64_t cells = wide || per_wave > 32 ? 256 : 64;
+  const int64_t rows_f = fast ? (N + cells - 1) / cells : 0;
+  // rows of the general kernel: one per group when it does all the work
+  const int64_t per = fast ? (groups + 255) / 256 : 1, rows_g = (groups + per - 1) / per;
+  const int64_t nwords = (N + 63) / 64;
+  qj_status st = ensure_partials(ws, rows_f * KF + rows_g * K + nwords + 1, s);
   if (st) return st;
+  if ((st = ensure_pinned(ws, 1 + KF + K, s))) return st;
   APArgs g;
   g.a = a;
   make_geom(wg, &g.wg);
   g.alpha = alpha;
   g.thr = thr;
-  double* sums = ws->d_partials + nblocks * K;
-  unsigned long long* nad = (unsigned long long*)(sums + K);
-  QJ_HIP(hipMemsetAsync(nad, 0, sizeof(unsigned long long), s));
-  hipLaunchKernelGGL(k_ap_grads, dim3((unsigned)nblocks), dim3(kGBlock), lds, s, g, f->d64, d_weight, d_field,
-                     ws->d_partials, K, nad);
+  g.log_c = ::log(a.exp_scaling);
+  const uint64_t XY = (uint64_t)a.res[0] * (uint64_t)a.res[1];
+  g.div_x = make_fastdiv((uint32_t)a.res[0]);
+  g.div_xy = make_fastdiv(XY <= 0xffffffffull ? (uint32_t)XY : 1u);
+  double* pf = ws->d_partials;
+  double* pg = pf + rows_f * KF;
+  unsigned long long* left = (unsigned long long*)(pg + rows_g * K);
+  unsigned long long* nad = left + nwords;
+  if (fast) {
+    const auto k = cells == 64 ? (per_wave <= 8 ? k_ap_fast<1, 8> : k_ap_fast<1, 32>)
+                               : (per_wave <= 8 ? k_ap_fast<4, 8> : per_wave <= 16 ? k_ap_fast<4, 16> : k_ap_fast<4, 0>);
+    hipLaunchKernelGGL(k, dim3((unsigned)rows_f), dim3(kApBlock), 0, s, g, f->d64, d_weight, d_field, left, pf, nad);
+  } else {
+    hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(64), 0, s, nad);
+  }
   QJ_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_sum_partials, dim3(K), dim3(kSumThreads), 0, s, ws->d_partials, nblocks, K, sums);
+  hipLaunchKernelGGL(k_ap_grads, dim3((unsigned)rows_g), dim3(kGBlock), lds, s, g, f->d64, d_weight, d_field,
+                     fast ? (const unsigned long long*)left : (const unsigned long long*)nullptr, per, pg, K, nad);
   QJ_HIP(hipGetLastError());
-  std::vector<double> h(K + 1);
-  QJ_HIP(hipMemcpyAsync(h.data(), sums, sizeof(double) * (K + 1), hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_ap_finish, dim3(K, 2), dim3(kSumThreads), 0, s, (const double*)pf, rows_f, KF,
+                     (const double*)pg, rows_g, K, (const unsigned long long*)nad, ws->h_pinned);
+  QJ_HIP(hipGetLastError());
   QJ_HIP(hipStreamSynchronize(s));
-  out->score = h[SL_SCORE];
-  out->grad_exp = h[SL_GEXP];
-  out->grad_top_scalar = h[SL_GTS];
-  out->grad_bottom_scalar = h[SL_GBS];
-  unsigned long long na;
-  ::memcpy(&na, &h[K], sizeof(na));
-  out->adaptive_cells = (int64_t)na;
-  for (int i = 0; i < a.nt; i++) gt[i] = h[SL_ROOTS + i];
-  for (int i = 0; i < a.nb; i++) gb[i] = h[SL_ROOTS + a.nt + i];
+  const double* hf = ws->h_pinned + 1;        // fast cells
+  const double* hg = ws->h_pinned + 1 + KF;  // the others
+  out->score = hf[0] + hg[SL_SCORE];
+  out->grad_exp = hf[1] + hg[SL_GEXP];
+  out->adaptive_cells = (int64_t)ws->h_pinned[0];
+  double gts = hg[SL_GTS], gbs = hg[SL_GBS];
+  for (int i = 0; i < a.nt; i++) {
+    const double v = hf[kApFastRows + i];
+    gt[i] = a.sc_top * v + hg[SL_ROOTS + i];
+    gts += f->h64[i].p * v;
+  }
+  for (int i = a.nt; i < nr; i++) {
+    const double v = hf[kApFastRows + i], p = f->h64[i].p;
+    // OPTIMIZE_3D.cpp:10084 and :10404-10405
+    gb[i - a.nt] = (a.sc_bottom > 0.0 ? -a.sc_bottom * v : 0.0) + hg[SL_ROOTS + i];
+    if (!(p < 1e-8)) gbs -= p * v;
+  }
+  out->grad_top_scalar = gts;
+  out->grad_bottom_scalar = gbs;
   return QJ_OK;
 }
 

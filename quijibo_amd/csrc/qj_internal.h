@@ -72,6 +72,9 @@ struct qj_workspace {
   // gradient partials
   double* d_partials = nullptr;
   int64_t partials_cap = 0;
+  // pinned host memory that kernels write a call's scalar results into
+  double* h_pinned = nullptr;
+  int64_t pinned_cap = 0;
   // sampled FP64 cross-check of every field (qj_workspace_check); 0 = off
   int64_t check_samples = 0;
   // kernel timing (qj_workspace_timing)
@@ -98,6 +101,9 @@ double term_bits(const std::vector<RootRec64>& roots, double escape);
 double near_bits(const std::vector<RootRec64>& roots);
 qj_status ensure_list(qj_workspace* ws, int64_t n, bool adaptive, hipStream_t s);
 qj_status ensure_partials(qj_workspace* ws, int64_t n, hipStream_t s);
+// Room for n doubles in the workspace's pinned host memory. The callers wait
+// for the stream before they return, so nothing is in flight when it grows.
+qj_status ensure_pinned(qj_workspace* ws, int64_t n, hipStream_t s);
 // Records an event on s when timing is enabled (slot order: bulk0, bulk1, band0, band1).
 void timing_mark(qj_workspace* ws, hipStream_t s);
 

@@ -1,0 +1,136 @@
+// FP64 logarithm, angle, sine / cosine and reciprocal square root for the
+// polar powers, written for the arguments that occur there.
+//
+// The device library's log, acos, exp and sincos spend most of their
+// instructions on double-double carries, range reduction for huge arguments
+// and special values. The map's arguments are positive normal squared norms,
+// angles in [0, pi] and their products with an exponent, so a short reduction
+// and one polynomial do (coefficients: fit_math64.py): log 26 instead of about
+// 70 instructions, angle + sine + cosine about 65 instead of about 200.
+// Largest errors, measured on gfx950 over the ranges below against 80-bit
+// arithmetic (2^22 arguments each): quotient 0.5 ulp, log 0.9 ulp, angle 2.5
+// ulp (the library's acos of a rounded w / |q| loses far more near 0 and pi),
+// sine 1.2 ulp, cosine 1.2e-16, square root and its reciprocal 0.5 and 1.7 ulp.
+//
+// Callers keep arguments in range themselves (see the range tests beside each
+// use); outside it the results are finite garbage or NaN, never a trap.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace qj {
+
+// n / d for normal d and quotient: reciprocal estimate, one Newton step, one
+// residual correction.
+__device__ __forceinline__ double div64(double n, double d) {
+#pragma clang fp contract(off)
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+
+// log(x) for normal positive x. x = 2^k m with m in [sqrt(1/2), sqrt(2)),
+// f = m - 1 (exact), s = f / (2 + f): log m = 2 atanh(s) = 2 s + s R(s^2) =
+// f - s (f - R), since 2 s = f - s f. Zero, denormal, infinite and NaN x give
+// a finite result beyond +-700.
+__device__ __forceinline__ double log64(double x) {
+#pragma clang fp contract(off)
+  const uint64_t bits = __builtin_bit_cast(uint64_t, x);
+  const uint32_t hi = (uint32_t)(bits >> 32) + (0x3ff00000u - 0x3fe6a09eu);
+  const int k = (int)(hi >> 20) - 0x3ff;
+  const uint32_t mh = (hi & 0x000fffffu) + 0x3fe6a09eu;
+  const double m = __builtin_bit_cast(double, (uint64_t)mh << 32 | (uint32_t)bits);
+  const double f = m - 1.0;
+  const double s = div64(f, m + 1.0);
+  const double z = s * s;
+  double p = 0.14616449685043406;
+  p = __builtin_fma(p, z, 0.15331721600556042);
+  p = __builtin_fma(p, z, 0.18182889125261723);
+  p = __builtin_fma(p, z, 0.2222221113479508);
+  p = __builtin_fma(p, z, 0.28571428625975487);
+  p = __builtin_fma(p, z, 0.39999999999899505);
+  p = __builtin_fma(p, z, 0.666666666666667);
+  const double t = __builtin_fma(-p, z, f);  // f - R
+  const double dk = (double)k;
+  // ln 2 = 0x1.62e42fefa38p-1 (k times it is exact) + 0x1.ef35793c7673p-45
+  const double lo = __builtin_fma(-s, t, dk * 0x1.ef35793c7673p-45);
+  return __builtin_fma(dk, 0x1.62e42fefa38p-1, f + lo);
+}
+
+// sqrt(x) and 1 / sqrt(x) for normal x in [2^-900, 2^900] (Goldschmidt steps
+// from the estimate). x = 0 gives NaN for both.
+__device__ __forceinline__ void sqrt_rsqrt64(double x, double& root, double& inverse) {
+#pragma clang fp contract(off)
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double r = __builtin_fma(-g, h, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  r = __builtin_fma(-g, h, 0.5);
+  h = __builtin_fma(h, r, h);
+  root = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  inverse = 2.0 * h;
+}
+
+// The angle of w + i y for y >= 0, in [0, pi] (y and w finite, not both 0,
+// their larger one in [2^-450, 2^450]): octant reduction to mn / mx, beyond
+// tan(pi / 8) a rotation by pi / 4, then atan(u) = u + u z P(z).
+__device__ __forceinline__ double angle64(double y, double w) {
+#pragma clang fp contract(off)
+  const double aw = __builtin_fabs(w);
+  const bool steep = y > aw;
+  const double mx = steep ? y : aw, mn = steep ? aw : y;
+  const bool wide = mn > 0.41421356237309503 * mx;
+  const double n = wide ? mn - mx : mn, d = wide ? mn + mx : mx;
+  const double u = div64(n, d);
+  const double z = u * u;
+  double p = 0.016285756855221028;
+  p = __builtin_fma(p, z, -0.034570561981427744);
+  p = __builtin_fma(p, z, 0.04551593220626549);
+  p = __builtin_fma(p, z, -0.05230454270650244);
+  p = __builtin_fma(p, z, 0.05878928997834775);
+  p = __builtin_fma(p, z, -0.06666424885738255);
+  p = __builtin_fma(p, z, 0.07692296375032143);
+  p = __builtin_fma(p, z, -0.09090908753500877);
+  p = __builtin_fma(p, z, 0.11111111105155447);
+  p = __builtin_fma(p, z, -0.14285714285659828);
+  p = __builtin_fma(p, z, 0.19999999999999804);
+  p = __builtin_fma(p, z, -0.3333333333333333);
+  // +-(u + u z P) added to its multiple of pi / 4 in two parts: atan(t) = u or
+  // pi / 4 + u; y steep: pi / 2 - atan(t); w < 0: pi - that
+  double a = __builtin_fma(u * z, p, wide ? 0.78539816339744828 : 0.0);  // pi / 4 - 3.06e-17
+  a = (wide ? u + 3.061616997868383e-17 : u) + a;
+  if (steep) a = 1.5707963267948966 - (a - 6.123233995736766e-17);
+  return w < 0.0 ? 3.141592653589793 - (a - 1.2246467991473532e-16) : a;
+}
+
+// sin(x) and cos(x) for |x| <= 2^20: x - k pi / 2 in three parts of pi / 2,
+// then the two polynomials, swapped and signed by k.
+__device__ __forceinline__ void sincos64(double x, double& sn, double& cs) {
+#pragma clang fp contract(off)
+  const double dk = __builtin_rint(x * 0.63661977236758138);
+  double r = __builtin_fma(-dk, 1.5707963267948966, x);
+  r = __builtin_fma(-dk, 6.123233995736766e-17, r);
+  const int k = (int)dk;
+  const double z = r * r;
+  double p = 1.5918129294866608e-10;
+  p = __builtin_fma(p, z, -2.5051131845003624e-08);
+  p = __builtin_fma(p, z, 2.755731610255244e-06);
+  p = __builtin_fma(p, z, -0.00019841269836758574);
+  p = __builtin_fma(p, z, 0.008333333333330948);
+  p = __builtin_fma(p, z, -0.16666666666666666);
+  const double s = __builtin_fma(r * z, p, r);
+  double c = -1.1382632425521717e-11;
+  c = __builtin_fma(c, z, 2.08761462684032e-09);
+  c = __builtin_fma(c, z, -2.7557317271729793e-07);
+  c = __builtin_fma(c, z, 2.480158729876569e-05);
+  c = __builtin_fma(c, z, -0.0013888888888887398);
+  c = __builtin_fma(c, z, 0.041666666666666664);
+  c = __builtin_fma(z, __builtin_fma(z, c, -0.5), 1.0);
+  const double a = (k & 1) ? c : s, b = (k & 1) ? s : c;
+  sn = (k & 2) ? -a : a;
+  cs = ((k + 1) & 2) ? -b : b;
+}
+
+}  // namespace qj
