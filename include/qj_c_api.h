@@ -99,15 +99,15 @@ typedef struct qj_map_params {
 #define QJ_PRESET_AP_ESCAPE 20.0             /* computeRationalMapAP, flags = SKIP_ORIGIN|ADAPTIVE */
 
 typedef enum qj_precision {
-  QJ_FP64 = 0,       /* every voxel in FP64, reference expression order */
+  QJ_FP64 = 0,       /* every voxel in FP64: the reference's factor order, exponents exactly 1 and 2 as b
+                        and b*b, other powers polar (the reference's values to a few ulps per term, with
+                        its special cases); the last iteration, of which only |q| is used, from norms */
   QJ_FP32_BAND = 1,  /* FP32 bulk; FP64 re-evaluation of the band |F| < band, of
                         non-finite results and of voxels whose escape or black-hole
                         test was within FP32's error of its threshold */
-  QJ_FP64_EXACT = 2  /* every voxel in FP64, exponents exactly 1 and 2 as the exact
-                        products b and b*b (a few ulps from the polar form, with its
-                        special cases), other exponents polar; the FP32 path's band
-                        arithmetic. qj_field_eval, qj_field_eval_noalloc and
-                        qj_points_eval; not with QJ_MAP_LAGRANGE */
+  QJ_FP64_EXACT = 2  /* the FP32 path's band arithmetic for every voxel: the same evaluation as
+                        QJ_FP64. qj_field_eval, qj_field_eval_noalloc and qj_points_eval; not with
+                        QJ_MAP_LAGRANGE */
 } qj_precision;
 
 /* Counters accumulated by the evaluation calls on a workspace since the last
@@ -120,7 +120,7 @@ typedef struct qj_eval_stats {
   int64_t adaptive_voxels;   /* cells flagged as overflowed (QJ_MAP_ADAPTIVE) */
   int64_t nonfinite;         /* non-finite results written */
   /* the sampled FP64 cross-check (qj_workspace_check), summed over fields */
-  int64_t checked;           /* cells re-evaluated with the reference method in FP64 */
+  int64_t checked;           /* cells re-evaluated in FP64 */
   int64_t check_sign_flips;  /* of those, cells where (float)F > 0 differs from FP64's */
   int64_t check_class_mismatch; /* cells whose class (finite, NaN, +inf, -inf) differs */
   double check_max_abs_dF;   /* largest |F - F_fp64| over checked cells finite in both */
@@ -154,11 +154,11 @@ qj_status qj_workspace_reset_stats(qj_workspace* ws, void* stream);
 /* The error statement of every field (no counterpart in the reference, which
  * has one precision): with samples > 0, each qj_field_eval on ws re-evaluates
  * `samples` evenly spaced cells (cell (2i+1) N / (2 samples), i < samples)
- * with the reference method in FP64 (polar powers, reference expression
- * order; the extended-range re-pass for cells QJ_MAP_ADAPTIVE flags) after
+ * in FP64 as QJ_FP64 does (the extended-range re-pass for cells
+ * QJ_MAP_ADAPTIVE flags) after
  * the field is written, and adds the comparison to the workspace statistics
  * (qj_eval_stats.checked ...). One extra kernel per field, about the latency
- * of one FP64 evaluation per cell (0.5 ms for 32+32 roots, maxIter 4).
+ * of one FP64 evaluation per cell.
  * 0 (the default) turns it off; at most 2^24. */
 qj_status qj_workspace_check(qj_workspace* ws, int64_t samples);
 
@@ -424,7 +424,7 @@ typedef struct qj_server_config {
                                  footprint or more wait behind it) and takes up to a quarter of each
                                  launch (0 = 0.25) */
   int32_t check_samples;      /* per-result error statement: cells of every finished field re-evaluated with
-                                 the reference method in FP64 and compared (qj_completion.checked ...; 0 = off) */
+                                 FP64 and compared (qj_completion.checked ...; 0 = off) */
   double escalate_abs_dF;     /* FP32_BAND servers with check_samples: a result whose sample shows a sign flip,
                                  a class mismatch or max |F - F_fp64| above this is computed again with every
                                  voxel in FP64 (exact integer powers) before it completes; its completion says

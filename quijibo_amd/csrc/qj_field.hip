@@ -17,7 +17,7 @@
 //                   into a compacted list (wave ballot + one atomic per block).
 //   k_points32      the same for a list of points.
 //   k_list64        FP64 re-evaluation of a compacted list (band or points);
-//                   k_list64<.., true> runs eval64x, FP64 with an explicit
+//                   k_list64<.., kRepass> runs eval64x, FP64 with an explicit
 //                   binary exponent (extended range) for cells that
 //                   overflowed: the reference's long double re-pass.
 //   k_batch32, k_batch64_list, k_batch64
@@ -105,12 +105,14 @@ __device__ __forceinline__ Res64 eval64x(const MapArgs& a, const RootRec64* __re
 // ---------------------------------------------------------------- kernels
 
 
-// kLagrange: the map may be in Lagrange order (QJ_MAP_LAGRANGE); the
-// factored-order instance carries no Lagrange code and needs fewer registers.
-// kPow: kPolar is the reference method (QJ_FP64); kExactOnly / kExactInt take
-// exponents 1 and 2 as exact products (QJ_FP64_EXACT). kExt: the
-// extended-range evaluator (QJ_MAP_EXTENDED_RANGE).
-template <bool kLagrange, int kPow = kPolar, bool kExt = false>
+// kPow: kExactOnly / kExactInt for QJ_FP64 and QJ_FP64_EXACT, kPolar for the
+// Lagrange order (QJ_MAP_LAGRANGE). kExt: the extended-range evaluator
+// (QJ_MAP_EXTENDED_RANGE). FP64 VALU bound: 32+32 roots with exponents 1 and 2,
+// 256^3, 4 iterations 43.7 to 3.4 ms, 64^3 with 8 roots 78 to 14 us against the
+// device library's polar form for every power; with real exponents, 50^3 and one
+// iteration, 267 to 36 us. The extended range's band list of a 256^3 torus tile
+// (128+128 roots) 1.69 to 0.64 ms, the request loop's 1.40 to 0.80 ms a launch.
+template <int kPow, bool kExt = false>
 __global__ __launch_bounds__(kBlock) void k_grid64(MapArgs a, const RootRec64* __restrict__ roots,
                                                    double* __restrict__ out, unsigned long long* __restrict__ cnt,
                                                    uint32_t* __restrict__ alist, uint32_t* __restrict__ acount,
@@ -124,7 +126,9 @@ __global__ __launch_bounds__(kBlock) void k_grid64(MapArgs a, const RootRec64* _
     double c[3];
     cell_center(a, x, y, z + a.zoff, c);
     const q64 q0{c[0], c[1], c[2], a.slice};
-    const Res64 r = kExt ? eval64e<kPow>(a, roots, q0) : eval64<kPow, const RootRec64*, kLagrange>(a, roots, q0);
+    Res64 r;
+    if constexpr (kExt) r = eval64e<kPow>(a, roots, q0);
+    else r = eval64<kPow>(a, roots, q0);
     if (r.written) {
       out[idx] = r.F;
       nonfinite = !isfinite(r.F);
@@ -181,7 +185,8 @@ __global__ __launch_bounds__(kBlock) void k_points32(MapArgs a, Consts32 k, cons
 // FP64 over a compacted list (count read on the device, at most cap entries
 // held), or over all n indices when list == nullptr. kPow: the PowMode
 // (kExactInt / kExactOnly for the FP32 path's band and range re-evaluation).
-template <class Src, bool kExtended, int kPow = kPolar>
+enum EvalKind { kPlainRange = 0, kExtRange = 1, kRepass = 2 };
+template <class Src, int kEval, int kPow = kPolar>
 __global__ __launch_bounds__(kBlock) void k_list64(MapArgs a, const RootRec64* __restrict__ roots,
                                                    const double* __restrict__ pts,
                                                    const uint32_t* __restrict__ list,
@@ -199,14 +204,17 @@ __global__ __launch_bounds__(kBlock) void k_list64(MapArgs a, const RootRec64* _
     if (i < n) {
       idx = list ? list[i] : (uint32_t)i;
       const q64 q0 = Src::start(a, pts, idx);
-      const Res64 r = kExtended ? eval64x(a, roots, q0) : eval64_any<kPow>(a, roots, q0);
+      Res64 r;
+      if constexpr (kEval == kRepass) r = eval64x(a, roots, q0);
+      else if constexpr (kEval == kExtRange) r = eval64e<kPow>(a, roots, q0);
+      else r = eval64<kPow>(a, roots, q0);
       if (r.written) out[idx] = r.F;
       else if (pts) out[idx] = __builtin_nan("");
       vox++;
       iters += r.iters;
       ovf = r.overflow;
     }
-    if (!kExtended && (a.flags & QJ_MAP_ADAPTIVE)) block_append(ovf, idx, alist, acount, acap);
+    if (kEval != kRepass && (a.flags & QJ_MAP_ADAPTIVE)) block_append(ovf, idx, alist, acount, acap);
   }
   block_count(vox, cnt, slot_vox);
   block_count(iters, cnt, slot_iter);
@@ -215,7 +223,7 @@ __global__ __launch_bounds__(kBlock) void k_list64(MapArgs a, const RootRec64* _
 // The cells (or points) that the FP32 pass found in need of FP64 after the
 // band list had filled up (they hold kBandMark), evaluated as k_list64
 // evaluates the listed ones. Returns at once when the list held them all.
-template <class Src, int kPow>
+template <class Src, int kEval, int kPow>
 __global__ __launch_bounds__(kBlock) void k_band_sweep(MapArgs a, const RootRec64* __restrict__ roots,
                                                        const double* __restrict__ pts,
                                                        const uint32_t* __restrict__ count, int64_t cap,
@@ -231,7 +239,9 @@ __global__ __launch_bounds__(kBlock) void k_band_sweep(MapArgs a, const RootRec6
     bool ovf = false;
     if (i < n_all && ((const unsigned long long*)out)[i] == kBandMark) {
       const q64 q0 = Src::start(a, pts, (uint32_t)i);
-      const Res64 r = eval64_any<kPow>(a, roots, q0);
+      Res64 r;
+      if constexpr (kEval == kExtRange) r = eval64e<kPow>(a, roots, q0);
+      else r = eval64<kPow>(a, roots, q0);
       if (r.written) out[i] = r.F;
       else if (pts) out[i] = __builtin_nan("");
       vox++;
@@ -268,15 +278,14 @@ __device__ __forceinline__ void block_max(double v, unsigned long long* cnt, int
 }
 
 // The error statement of a finished field: at `samples` evenly spaced cells
-// the reference method is evaluated again in FP64 (polar powers, reference
-// expression order; the extended-range re-pass where QJ_MAP_ADAPTIVE flags an
-// overflow) and compared with the value written: counts of checked cells,
+// the map is evaluated again as QJ_FP64 does (the extended-range re-pass where
+// QJ_MAP_ADAPTIVE flags an overflow) and compared with the value written: counts of checked cells,
 // sign disagreements of (float)F > 0 (the mesher's predicate) and class
 // disagreements (finite / NaN / +-inf), and the largest absolute and relative
 // (to max(1, |F64|)) differences over cells finite in both.
 // kSpread: copies per counter slot (a workspace's counters), or 1 for the
 // request loop's per-result block of CNT_N counters.
-template <int kSpread = kCounterSpread>
+template <int kPow, int kSpread = kCounterSpread>
 __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* __restrict__ roots,
                                                     const double* __restrict__ field, int64_t nvox, int64_t samples,
                                                     unsigned long long* __restrict__ cnt) {
@@ -286,8 +295,7 @@ __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* 
   if (i < samples) {
     const int64_t idx = ((2 * i + 1) * nvox) / (2 * samples);
     const q64 q0 = GridSource::start(a, nullptr, idx);
-    Res64 r = (a.flags & QJ_MAP_EXTENDED_RANGE) ? eval64e<kPolar>(a, roots, q0)
-                                                : eval64<kPolar, const RootRec64*, true>(a, roots, q0);
+    Res64 r = eval64_any<kPow>(a, roots, q0);
     if ((a.flags & QJ_MAP_ADAPTIVE) && r.overflow) r = eval64x(a, roots, q0);
     if (r.written) {
       const double F = field[idx];
@@ -309,6 +317,13 @@ __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* 
   block_max<kSpread>(drel, cnt, CNT_CHECK_MAXREL);
 }
 
+template <int kSpread>
+static auto check_kernel(const MapArgs& a) {
+  return (a.flags & QJ_MAP_LAGRANGE) ? k_check64<kPolar, kSpread>
+         : a.gen                     ? k_check64<kExactInt, kSpread>
+                                     : k_check64<kExactOnly, kSpread>;
+}
+
 __global__ void k_zero_u64(unsigned long long* p, int n) {
   if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
 }
@@ -320,8 +335,8 @@ qj_status launch_check_one(const MapArgs& a, const RootRec64* roots, const doubl
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, d_out, (int)CNT_N);
   QJ_HIP(hipGetLastError());
   if (m <= 0) return QJ_OK;
-  hipLaunchKernelGGL(k_check64<1>, dim3((unsigned)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, a, roots, field,
-                     nvox, m, d_out);
+  hipLaunchKernelGGL(check_kernel<1>(a), dim3((unsigned)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, a, roots,
+                     field, nvox, m, d_out);
   QJ_HIP(hipGetLastError());
   return QJ_OK;
 }
@@ -467,7 +482,7 @@ __global__ __launch_bounds__(kBlock) void k_batch64_list(const ChunkDesc* __rest
   }
 }
 
-// FP64 (the reference method) for every voxel of every chunk, work-queue tiles
+// FP64 for every voxel of every chunk, work-queue tiles
 __global__ __launch_bounds__(kBlock) void k_batch64(const ChunkDesc* __restrict__ descs, int blocks_per_chunk,
                                                     uint32_t* __restrict__ counters) {
   const int tiles = descs[0].total * blocks_per_chunk;
@@ -477,7 +492,8 @@ __global__ __launch_bounds__(kBlock) void k_batch64(const ChunkDesc* __restrict_
     const ChunkDesc& d = descs[c];
     if (local < d.count) {
       const int64_t idx = d.start + local;
-      const Res64 r = eval64_any(d.a, d.r64, chunk_start(d.a, idx));
+      const Res64 r = (d.a.flags & QJ_MAP_LAGRANGE) ? eval64<kPolar>(d.a, d.r64, chunk_start(d.a, idx))
+                                                    : eval64_any<kExactInt>(d.a, d.r64, chunk_start(d.a, idx));
       if (r.written) d.out[idx] = r.F;
     }
   }
@@ -611,15 +627,22 @@ static FieldBufs ws_bufs(qj_workspace* ws) {
 template <class Src>
 static qj_status launch_sweep(const FieldBufs& fb, const MapArgs& a, const qj_rational* f, const double* pts,
                               int64_t n, double* d_out, hipStream_t s) {
-  const dim3 g(list_grid(n / 16)), b(kBlock);
-  if (a.gen)
-    hipLaunchKernelGGL((k_band_sweep<Src, kExactInt>), g, b, 0, s, a, f->d64, pts, fb.list_count, fb.list_cap, n,
-                       d_out, fb.counters, fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
-  else
-    hipLaunchKernelGGL((k_band_sweep<Src, kExactOnly>), g, b, 0, s, a, f->d64, pts, fb.list_count, fb.list_cap, n,
-                       d_out, fb.counters, fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
+  const bool ext = (a.flags & QJ_MAP_EXTENDED_RANGE) != 0;
+  const auto k = a.gen ? (ext ? k_band_sweep<Src, kExtRange, kExactInt> : k_band_sweep<Src, kPlainRange, kExactInt>)
+                       : (ext ? k_band_sweep<Src, kExtRange, kExactOnly> : k_band_sweep<Src, kPlainRange, kExactOnly>);
+  hipLaunchKernelGGL(k, dim3(list_grid(n / 16)), dim3(kBlock), 0, s, a, f->d64, pts, fb.list_count, fb.list_cap, n,
+                     d_out, fb.counters, fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
   QJ_HIP(hipGetLastError());
   return QJ_OK;
+}
+
+// The FP64 list kernel of the map's power mode and range.
+template <class Src>
+static auto list_kernel(const MapArgs& a) {
+  if (a.flags & QJ_MAP_LAGRANGE) return k_list64<Src, kPlainRange, kPolar>;
+  if (a.flags & QJ_MAP_EXTENDED_RANGE)
+    return a.gen ? k_list64<Src, kExtRange, kExactInt> : k_list64<Src, kExtRange, kExactOnly>;
+  return a.gen ? k_list64<Src, kPlainRange, kExactInt> : k_list64<Src, kPlainRange, kExactOnly>;
 }
 
 static void mark(const FieldBufs& b, hipStream_t s) {
@@ -630,11 +653,11 @@ static qj_status run_adaptive(const FieldBufs& fb, const MapArgs& a, const qj_ra
                               int64_t n, double* d_out, hipStream_t s) {
   if (!(a.flags & QJ_MAP_ADAPTIVE)) return QJ_OK;
   if (pts)
-    hipLaunchKernelGGL((k_list64<PointSource, true>), dim3(list_grid(n / 64 + 1)), dim3(kBlock), 0, s, a, f->d64,
+    hipLaunchKernelGGL((k_list64<PointSource, kRepass>), dim3(list_grid(n / 64 + 1)), dim3(kBlock), 0, s, a, f->d64,
                        pts, fb.alist, fb.list_count + 1, fb.alist_cap, (int64_t)0, d_out, fb.counters,
                        (int)CNT_BAND_VOXELS, (int)CNT_BAND_ITERS, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u);
   else
-    hipLaunchKernelGGL((k_list64<GridSource, true>), dim3(list_grid(n / 64 + 1)), dim3(kBlock), 0, s, a, f->d64,
+    hipLaunchKernelGGL((k_list64<GridSource, kRepass>), dim3(list_grid(n / 64 + 1)), dim3(kBlock), 0, s, a, f->d64,
                        pts, fb.alist, fb.list_count + 1, fb.alist_cap, (int64_t)0, d_out, fb.counters,
                        (int)CNT_BAND_VOXELS, (int)CNT_BAND_ITERS, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u);
   QJ_HIP(hipGetLastError());
@@ -657,35 +680,17 @@ static qj_status launch_field_bufs(const FieldBufs& fb, const MapArgs& a, const 
   mark(fb, s);
   const bool ext = (a.flags & QJ_MAP_EXTENDED_RANGE) != 0;
   const dim3 g64((unsigned)nblocks), b64(kBlock);
-  if (prec == QJ_FP64_EXACT) {
-    if (a.gen && ext)
-      hipLaunchKernelGGL((k_grid64<false, kExactInt, true>), g64, b64, 0, s, a, f->d64, d_out, fb.counters, fb.alist,
-                         fb.list_count + 1, (uint32_t)fb.alist_cap);
-    else if (a.gen)
-      hipLaunchKernelGGL((k_grid64<false, kExactInt>), g64, b64, 0, s, a, f->d64, d_out, fb.counters, fb.alist,
-                         fb.list_count + 1, (uint32_t)fb.alist_cap);
-    else if (ext)
-      hipLaunchKernelGGL((k_grid64<false, kExactOnly, true>), g64, b64, 0, s, a, f->d64, d_out, fb.counters,
-                         fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
-    else
-      hipLaunchKernelGGL((k_grid64<false, kExactOnly>), g64, b64, 0, s, a, f->d64, d_out, fb.counters, fb.alist,
-                         fb.list_count + 1, (uint32_t)fb.alist_cap);
+  if (a.flags & QJ_MAP_LAGRANGE) {
+    hipLaunchKernelGGL(k_grid64<kPolar>, g64, b64, 0, s, a, f->d64, d_out, fb.counters, fb.alist, fb.list_count + 1,
+                       (uint32_t)fb.alist_cap);
     QJ_HIP(hipGetLastError());
     mark(fb, s);
     mark(fb, s);
-  } else if (prec == QJ_FP64 && ext) {
-    hipLaunchKernelGGL((k_grid64<false, kPolar, true>), g64, b64, 0, s, a, f->d64, d_out, fb.counters, fb.alist,
-                       fb.list_count + 1, (uint32_t)fb.alist_cap);
-    QJ_HIP(hipGetLastError());
-    mark(fb, s);
-    mark(fb, s);
-  } else if (prec == QJ_FP64) {
-    if (a.flags & QJ_MAP_LAGRANGE)
-      hipLaunchKernelGGL(k_grid64<true>, dim3((unsigned)nblocks), dim3(kBlock), 0, s, a, f->d64, d_out,
-                         fb.counters, fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
-    else
-      hipLaunchKernelGGL(k_grid64<false>, dim3((unsigned)nblocks), dim3(kBlock), 0, s, a, f->d64, d_out,
-                         fb.counters, fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
+  } else if (prec == QJ_FP64 || prec == QJ_FP64_EXACT) {
+    const auto k = a.gen ? (ext ? k_grid64<kExactInt, true> : k_grid64<kExactInt>)
+                         : (ext ? k_grid64<kExactOnly, true> : k_grid64<kExactOnly>);
+    hipLaunchKernelGGL(k, g64, b64, 0, s, a, f->d64, d_out, fb.counters, fb.alist, fb.list_count + 1,
+                       (uint32_t)fb.alist_cap);
     QJ_HIP(hipGetLastError());
     mark(fb, s);
     mark(fb, s);
@@ -707,16 +712,9 @@ static qj_status launch_field_bufs(const FieldBufs& fb, const MapArgs& a, const 
     QJ_HIP(hipGetLastError());
     mark(fb, s);
     mark(fb, s);
-    if (a.gen)
-      hipLaunchKernelGGL((k_list64<GridSource, false, kExactInt>), dim3(list_grid(nvox / 16)), dim3(kBlock), 0, s, a,
-                         f->d64, (const double*)nullptr, fb.list, fb.list_count, fb.list_cap, (int64_t)0, d_out,
-                         fb.counters, (int)CNT_BAND_VOXELS, (int)CNT_BAND_ITERS, fb.alist, fb.list_count + 1,
-                         (uint32_t)fb.alist_cap);
-    else
-      hipLaunchKernelGGL((k_list64<GridSource, false, kExactOnly>), dim3(list_grid(nvox / 16)), dim3(kBlock), 0, s,
-                         a, f->d64, (const double*)nullptr, fb.list, fb.list_count, fb.list_cap, (int64_t)0, d_out,
-                         fb.counters, (int)CNT_BAND_VOXELS, (int)CNT_BAND_ITERS, fb.alist, fb.list_count + 1,
-                         (uint32_t)fb.alist_cap);
+    hipLaunchKernelGGL(list_kernel<GridSource>(a), dim3(list_grid(nvox / 16)), dim3(kBlock), 0, s, a, f->d64,
+                       (const double*)nullptr, fb.list, fb.list_count, fb.list_cap, (int64_t)0, d_out, fb.counters,
+                       (int)CNT_BAND_VOXELS, (int)CNT_BAND_ITERS, fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
     QJ_HIP(hipGetLastError());
     qj_status st = launch_sweep<GridSource>(fb, a, f, nullptr, nvox, d_out, s);
     if (st) return st;
@@ -738,7 +736,7 @@ qj_status launch_field(qj_workspace* ws, const MapArgs& a, const qj_rational* f,
   if ((st = launch_field_bufs(ws_bufs(ws), a, f, prec, band, d_out, s))) return st;
   if (ws->check_samples > 0) {
     const int64_t m = ws->check_samples < nvox ? ws->check_samples : nvox;
-    hipLaunchKernelGGL(k_check64<>, dim3((unsigned)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, a, f->d64,
+    hipLaunchKernelGGL(check_kernel<kCounterSpread>(a), dim3((unsigned)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, a, f->d64,
                        (const double*)d_out, nvox, m, ws->d_counters);
     QJ_HIP(hipGetLastError());
   }
@@ -755,22 +753,10 @@ qj_status launch_points(qj_workspace* ws, const MapArgs& a, const qj_rational* f
   // list counters cleared by a kernel, not a memset node, so the call can be captured in a graph
   hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, fb.list_count, 2);
   QJ_HIP(hipGetLastError());
-  if (prec == QJ_FP64) {
-    hipLaunchKernelGGL((k_list64<PointSource, false>), dim3(list_grid(n)), dim3(kBlock), 0, s, a, f->d64, d_pts,
-                       (const uint32_t*)nullptr, (const uint32_t*)nullptr, (int64_t)0, n, d_out, fb.counters,
-                       (int)CNT_VOXELS, (int)CNT_ITERS, fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
-    QJ_HIP(hipGetLastError());
-  } else if (prec == QJ_FP64_EXACT) {
-    if (a.gen)
-      hipLaunchKernelGGL((k_list64<PointSource, false, kExactInt>), dim3(list_grid(n)), dim3(kBlock), 0, s, a,
-                         f->d64, d_pts, (const uint32_t*)nullptr, (const uint32_t*)nullptr, (int64_t)0, n, d_out,
-                         fb.counters, (int)CNT_VOXELS, (int)CNT_ITERS, fb.alist, fb.list_count + 1,
-                         (uint32_t)fb.alist_cap);
-    else
-      hipLaunchKernelGGL((k_list64<PointSource, false, kExactOnly>), dim3(list_grid(n)), dim3(kBlock), 0, s, a,
-                         f->d64, d_pts, (const uint32_t*)nullptr, (const uint32_t*)nullptr, (int64_t)0, n, d_out,
-                         fb.counters, (int)CNT_VOXELS, (int)CNT_ITERS, fb.alist, fb.list_count + 1,
-                         (uint32_t)fb.alist_cap);
+  if (prec == QJ_FP64 || prec == QJ_FP64_EXACT) {
+    hipLaunchKernelGGL(list_kernel<PointSource>(a), dim3(list_grid(n)), dim3(kBlock), 0, s, a, f->d64, d_pts, (const uint32_t*)nullptr,
+                       (const uint32_t*)nullptr, (int64_t)0, n, d_out, fb.counters, (int)CNT_VOXELS, (int)CNT_ITERS,
+                       fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
     QJ_HIP(hipGetLastError());
   } else {
     const int64_t nb = (n + kBlock - 1) / kBlock;
@@ -789,16 +775,9 @@ qj_status launch_points(qj_workspace* ws, const MapArgs& a, const qj_rational* f
       hipLaunchKernelGGL((k_points32<PointSource, 2, false>), g, b, 0, s, a, k, (const F4*)f->d32, d_pts, n, d_out,
                          fb.counters, fb.list, fb.list_count, (uint32_t)fb.list_cap);
     QJ_HIP(hipGetLastError());
-    if (a.gen)
-      hipLaunchKernelGGL((k_list64<PointSource, false, kExactInt>), dim3(list_grid(n / 16)), dim3(kBlock), 0, s, a,
-                         f->d64, d_pts, fb.list, fb.list_count, fb.list_cap, (int64_t)0, d_out, fb.counters,
-                         (int)CNT_BAND_VOXELS, (int)CNT_BAND_ITERS, fb.alist, fb.list_count + 1,
-                         (uint32_t)fb.alist_cap);
-    else
-      hipLaunchKernelGGL((k_list64<PointSource, false, kExactOnly>), dim3(list_grid(n / 16)), dim3(kBlock), 0, s, a,
-                         f->d64, d_pts, fb.list, fb.list_count, fb.list_cap, (int64_t)0, d_out, fb.counters,
-                         (int)CNT_BAND_VOXELS, (int)CNT_BAND_ITERS, fb.alist, fb.list_count + 1,
-                         (uint32_t)fb.alist_cap);
+    hipLaunchKernelGGL(list_kernel<PointSource>(a), dim3(list_grid(n / 16)), dim3(kBlock), 0, s, a, f->d64, d_pts,
+                       fb.list, fb.list_count, fb.list_cap, (int64_t)0, d_out, fb.counters, (int)CNT_BAND_VOXELS,
+                       (int)CNT_BAND_ITERS, fb.alist, fb.list_count + 1, (uint32_t)fb.alist_cap);
     QJ_HIP(hipGetLastError());
     if ((st = launch_sweep<PointSource>(fb, a, f, d_pts, n, d_out, s))) return st;
   }

@@ -10,7 +10,8 @@
 // Largest errors, measured on gfx950 over the ranges below against 80-bit
 // arithmetic (2^22 arguments each): quotient 0.5 ulp, log 0.9 ulp, angle 2.5
 // ulp (the library's acos of a rounded w / |q| loses far more near 0 and pi),
-// sine 1.2 ulp, cosine 1.2e-16, square root and its reciprocal 0.5 and 1.7 ulp.
+// sine 1.2 ulp, cosine 1.2e-16, square root and its reciprocal 0.5 and 1.7 ulp,
+// exponential 1.0 ulp.
 //
 // Callers keep arguments in range themselves (see the range tests beside each
 // use); outside it the results are finite garbage or NaN, never a trap.
@@ -19,6 +20,17 @@
 #include <stdint.h>
 
 namespace qj {
+
+// kInLoop: every constant is set in a scalar register pair where it is used. The
+// compiler otherwise keeps a polar power's constants in registers across the
+// root loop (178 instead of 101 VGPRs in k_grid64); two scalar moves per use
+// issue beside other waves' vector work. Code that runs once per point leaves
+// the constants to the compiler.
+template <bool kInLoop>
+__device__ __forceinline__ double k64(double c) {
+  if constexpr (kInLoop) asm volatile("" : "+s"(c));
+  return c;
+}
 
 // n / d for normal d and quotient: reciprocal estimate, one Newton step, one
 // residual correction.
@@ -34,6 +46,7 @@ __device__ __forceinline__ double div64(double n, double d) {
 // f = m - 1 (exact), s = f / (2 + f): log m = 2 atanh(s) = 2 s + s R(s^2) =
 // f - s (f - R), since 2 s = f - s f. Zero, denormal, infinite and NaN x give
 // a finite result beyond +-700.
+template <bool kInLoop = false>
 __device__ __forceinline__ double log64(double x) {
 #pragma clang fp contract(off)
   const uint64_t bits = __builtin_bit_cast(uint64_t, x);
@@ -44,18 +57,18 @@ __device__ __forceinline__ double log64(double x) {
   const double f = m - 1.0;
   const double s = div64(f, m + 1.0);
   const double z = s * s;
-  double p = 0.14616449685043406;
-  p = __builtin_fma(p, z, 0.15331721600556042);
-  p = __builtin_fma(p, z, 0.18182889125261723);
-  p = __builtin_fma(p, z, 0.2222221113479508);
-  p = __builtin_fma(p, z, 0.28571428625975487);
-  p = __builtin_fma(p, z, 0.39999999999899505);
-  p = __builtin_fma(p, z, 0.666666666666667);
+  double p = k64<kInLoop>(0.14616449685043406);
+  p = __builtin_fma(p, z, k64<kInLoop>(0.15331721600556042));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.18182889125261723));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.2222221113479508));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.28571428625975487));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.39999999999899505));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.666666666666667));
   const double t = __builtin_fma(-p, z, f);  // f - R
   const double dk = (double)k;
   // ln 2 = 0x1.62e42fefa38p-1 (k times it is exact) + 0x1.ef35793c7673p-45
-  const double lo = __builtin_fma(-s, t, dk * 0x1.ef35793c7673p-45);
-  return __builtin_fma(dk, 0x1.62e42fefa38p-1, f + lo);
+  const double lo = __builtin_fma(-s, t, dk * k64<kInLoop>(0x1.ef35793c7673p-45));
+  return __builtin_fma(dk, k64<kInLoop>(0x1.62e42fefa38p-1), f + lo);
 }
 
 // sqrt(x) and 1 / sqrt(x) for normal x in [2^-900, 2^900] (Goldschmidt steps
@@ -76,27 +89,28 @@ __device__ __forceinline__ void sqrt_rsqrt64(double x, double& root, double& inv
 // The angle of w + i y for y >= 0, in [0, pi] (y and w finite, not both 0,
 // their larger one in [2^-450, 2^450]): octant reduction to mn / mx, beyond
 // tan(pi / 8) a rotation by pi / 4, then atan(u) = u + u z P(z).
+template <bool kInLoop = false>
 __device__ __forceinline__ double angle64(double y, double w) {
 #pragma clang fp contract(off)
   const double aw = __builtin_fabs(w);
   const bool steep = y > aw;
   const double mx = steep ? y : aw, mn = steep ? aw : y;
-  const bool wide = mn > 0.41421356237309503 * mx;
+  const bool wide = mn > k64<kInLoop>(0.41421356237309503) * mx;
   const double n = wide ? mn - mx : mn, d = wide ? mn + mx : mx;
   const double u = div64(n, d);
   const double z = u * u;
-  double p = 0.016285756855221028;
-  p = __builtin_fma(p, z, -0.034570561981427744);
-  p = __builtin_fma(p, z, 0.04551593220626549);
-  p = __builtin_fma(p, z, -0.05230454270650244);
-  p = __builtin_fma(p, z, 0.05878928997834775);
-  p = __builtin_fma(p, z, -0.06666424885738255);
-  p = __builtin_fma(p, z, 0.07692296375032143);
-  p = __builtin_fma(p, z, -0.09090908753500877);
-  p = __builtin_fma(p, z, 0.11111111105155447);
-  p = __builtin_fma(p, z, -0.14285714285659828);
-  p = __builtin_fma(p, z, 0.19999999999999804);
-  p = __builtin_fma(p, z, -0.3333333333333333);
+  double p = k64<kInLoop>(0.016285756855221028);
+  p = __builtin_fma(p, z, k64<kInLoop>(-0.034570561981427744));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.04551593220626549));
+  p = __builtin_fma(p, z, k64<kInLoop>(-0.05230454270650244));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.05878928997834775));
+  p = __builtin_fma(p, z, k64<kInLoop>(-0.06666424885738255));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.07692296375032143));
+  p = __builtin_fma(p, z, k64<kInLoop>(-0.09090908753500877));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.11111111105155447));
+  p = __builtin_fma(p, z, k64<kInLoop>(-0.14285714285659828));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.19999999999999804));
+  p = __builtin_fma(p, z, k64<kInLoop>(-0.3333333333333333));
   // +-(u + u z P) added to its multiple of pi / 4 in two parts: atan(t) = u or
   // pi / 4 + u; y steep: pi / 2 - atan(t); w < 0: pi - that
   double a = __builtin_fma(u * z, p, wide ? 0.78539816339744828 : 0.0);  // pi / 4 - 3.06e-17
@@ -105,28 +119,52 @@ __device__ __forceinline__ double angle64(double y, double w) {
   return w < 0.0 ? 3.141592653589793 - (a - 1.2246467991473532e-16) : a;
 }
 
-// sin(x) and cos(x) for |x| <= 2^20: x - k pi / 2 in three parts of pi / 2,
+// exp(x) for finite x: 2^k exp(r), |r| <= ln 2 / 2. Overflow gives inf,
+// underflow a denormal or 0, as the scaling by 2^k rounds them.
+template <bool kInLoop = false>
+__device__ __forceinline__ double exp64(double x) {
+#pragma clang fp contract(off)
+  const double dk = __builtin_rint(x * k64<kInLoop>(1.4426950408889634));
+  double r = __builtin_fma(-dk, k64<kInLoop>(0x1.62e42fefa39efp-1), x);
+  r = __builtin_fma(-dk, k64<kInLoop>(0x1.abc9e3b39803fp-56), r);
+  double p = k64<kInLoop>(2.0914679376583935e-09);
+  p = __builtin_fma(p, r, k64<kInLoop>(2.510520637395701e-08));
+  p = __builtin_fma(p, r, k64<kInLoop>(2.7557273661348637e-07));
+  p = __builtin_fma(p, r, k64<kInLoop>(2.7557255425746435e-06));
+  p = __builtin_fma(p, r, k64<kInLoop>(2.4801587325533363e-05));
+  p = __builtin_fma(p, r, k64<kInLoop>(0.00019841269874800493));
+  p = __builtin_fma(p, r, k64<kInLoop>(0.0013888888888883752));
+  p = __builtin_fma(p, r, k64<kInLoop>(0.008333333333326141));
+  p = __builtin_fma(p, r, k64<kInLoop>(0.04166666666666667));
+  p = __builtin_fma(p, r, k64<kInLoop>(0.1666666666666667));
+  p = __builtin_fma(p, r, k64<kInLoop>(0.5));
+  const double k = __builtin_fmin(__builtin_fmax(dk, -4000.0), 4000.0);
+  return __builtin_amdgcn_ldexp(1.0 + __builtin_fma(r * r, p, r), (int)k);
+}
+
+// sin(x) and cos(x) for |x| <= 2^30: x - k pi / 2 with pi / 2 in two parts,
 // then the two polynomials, swapped and signed by k.
+template <bool kInLoop = false>
 __device__ __forceinline__ void sincos64(double x, double& sn, double& cs) {
 #pragma clang fp contract(off)
-  const double dk = __builtin_rint(x * 0.63661977236758138);
-  double r = __builtin_fma(-dk, 1.5707963267948966, x);
-  r = __builtin_fma(-dk, 6.123233995736766e-17, r);
+  const double dk = __builtin_rint(x * k64<kInLoop>(0.63661977236758138));
+  double r = __builtin_fma(-dk, k64<kInLoop>(1.5707963267948966), x);
+  r = __builtin_fma(-dk, k64<kInLoop>(6.123233995736766e-17), r);
   const int k = (int)dk;
   const double z = r * r;
-  double p = 1.5918129294866608e-10;
-  p = __builtin_fma(p, z, -2.5051131845003624e-08);
-  p = __builtin_fma(p, z, 2.755731610255244e-06);
-  p = __builtin_fma(p, z, -0.00019841269836758574);
-  p = __builtin_fma(p, z, 0.008333333333330948);
-  p = __builtin_fma(p, z, -0.16666666666666666);
+  double p = k64<kInLoop>(1.5918129294866608e-10);
+  p = __builtin_fma(p, z, k64<kInLoop>(-2.5051131845003624e-08));
+  p = __builtin_fma(p, z, k64<kInLoop>(2.755731610255244e-06));
+  p = __builtin_fma(p, z, k64<kInLoop>(-0.00019841269836758574));
+  p = __builtin_fma(p, z, k64<kInLoop>(0.008333333333330948));
+  p = __builtin_fma(p, z, k64<kInLoop>(-0.16666666666666666));
   const double s = __builtin_fma(r * z, p, r);
-  double c = -1.1382632425521717e-11;
-  c = __builtin_fma(c, z, 2.08761462684032e-09);
-  c = __builtin_fma(c, z, -2.7557317271729793e-07);
-  c = __builtin_fma(c, z, 2.480158729876569e-05);
-  c = __builtin_fma(c, z, -0.0013888888888887398);
-  c = __builtin_fma(c, z, 0.041666666666666664);
+  double c = k64<kInLoop>(-1.1382632425521717e-11);
+  c = __builtin_fma(c, z, k64<kInLoop>(2.08761462684032e-09));
+  c = __builtin_fma(c, z, k64<kInLoop>(-2.7557317271729793e-07));
+  c = __builtin_fma(c, z, k64<kInLoop>(2.480158729876569e-05));
+  c = __builtin_fma(c, z, k64<kInLoop>(-0.0013888888888887398));
+  c = __builtin_fma(c, z, k64<kInLoop>(0.041666666666666664));
   c = __builtin_fma(z, __builtin_fma(z, c, -0.5), 1.0);
   const double a = (k & 1) ? c : s, b = (k & 1) ? s : c;
   sn = (k & 2) ? -a : a;

@@ -1039,11 +1039,13 @@ void mc_free(qj_workspace* ws) {
 
 // kPow: kExactOnly when every exponent is 1 or 2 (no polar code, far fewer
 // registers), kExactInt otherwise; both give the same values for exponents 1
-// and 2. kLag: the map in Lagrange order (QJ_MAP_LAGRANGE).
-template <int kPow, bool kLag>
+// and 2. kMap: the map in Lagrange order (QJ_MAP_LAGRANGE), in the extended
+// range (QJ_MAP_EXTENDED_RANGE) or neither.
+enum NlMap { kNlPlain = 0, kNlExt = 1, kNlLag = 2 };
+template <int kPow, int kMap>
 __device__ __forceinline__ double nonlinear_value(const MapArgs& a, const RootRec64* __restrict__ roots,
                                                   const double* p, double iso) {
-  if (kLag) {
+  if (kMap == kNlLag) {
     // lagrangeNonlinearValue (TRIANGLE_MESH.cpp:1684-1730): an infinite |q|
     // restores the previous iterate and stops. Before the first iteration the
     // reference's previous magnitude is uninitialised; here it is |q0|.
@@ -1065,7 +1067,8 @@ __device__ __forceinline__ double nonlinear_value(const MapArgs& a, const RootRe
     const double v = log(magnitude) - iso;
     return isinf(v) ? (double)FLT_MAX : v;
   }
-  const Res64 r = eval64_any<kPow>(a, roots, q64{p[0], p[1], p[2], a.slice});
+  const q64 q0{p[0], p[1], p[2], a.slice};
+  const Res64 r = kMap == kNlExt ? eval64e<kPow>(a, roots, q0) : eval64<kPow>(a, roots, q0);
   return r.F - iso;
 }
 
@@ -1122,48 +1125,71 @@ __global__ __launch_bounds__(kMcBlock) void k_nl_edges(const uint8_t* __restrict
 
 // One vertex by bisection between grid points (x, y, z) and its +axis
 // neighbour (computeNonlinearEdgeInterpolationsHuge :2034-2123 with
-// midpointSearch :2232-2271). va: value at (x, y, z). Counts edges whose end
-// values do not straddle the surface in *bad (the reference exits there).
-// fb: the field value at the +axis neighbour when the caller has it (the value
-// minus iso is the neighbour's end value), else null and it is evaluated.
-template <int kPow, bool kLag>
+// midpointSearch :2232-2271). fa, fb: the field values at the two ends when the
+// caller has them (the values minus iso are the end values), else null and they
+// are evaluated. Counts edges whose end values do not straddle the surface in
+// *bad (the reference exits there). Ends and midpoints go through one
+// evaluation in one loop, so the map's code is there once (three inlined copies
+// took 51 KB of instructions and 172 VGPRs for exponents 1 and 2).
+template <int kPow, int kMap>
 __device__ __forceinline__ void place_vertex(const MapArgs& a, const RootRec64* __restrict__ roots, double iso,
-                                             int x, int y, int z, int axis, const double* pa, double va,
-                                             const double* fb, double* __restrict__ out,
-                                             unsigned int* __restrict__ bad) {
+                                             int x, int y, int z, int axis, const double* fa, const double* fb,
+                                             double* __restrict__ out, unsigned int* __restrict__ bad) {
 #pragma clang fp contract(off)
-  double pb[3];
-  cell_center(a, x + (axis == 0), y + (axis == 1), z + (axis == 2), pb);
-  const double vb = fb ? *fb - iso : nonlinear_value<kPow, kLag>(a, roots, pb, iso);
-  // first = lower endpoint; the positive end is the first unless firstValue < 0
-  double pp[3], pn[3], vp, vn;
-  if (va < 0) {
-    pp[0] = pb[0]; pp[1] = pb[1]; pp[2] = pb[2]; vp = vb;
-    pn[0] = pa[0]; pn[1] = pa[1]; pn[2] = pa[2]; vn = va;
-  } else {
-    pp[0] = pa[0]; pp[1] = pa[1]; pp[2] = pa[2]; vp = va;
-    pn[0] = pb[0]; pn[1] = pb[1]; pn[2] = pb[2]; vn = vb;
+  double pp[3], pn[3], m[3], vp = 0.0, vn = 0.0;
+  cell_center(a, x, y, z, pp);
+  cell_center(a, x + (axis == 0), y + (axis == 1), z + (axis == 2), pn);
+  if (fa) {
+    vp = *fa - iso;
+    vn = *fb - iso;
   }
-  if (va * vb >= 0.0) atomicAdd(bad, 1u);  // the reference exits here (:2082-2097)
-  double m[3];
-  for (int rec = 0;; rec++) {
-    m[0] = pp[0] + pn[0];
-    m[1] = pp[1] + pn[1];
-    m[2] = pp[2] + pn[2];
-    m[0] *= 0.5;
-    m[1] *= 0.5;
-    m[2] *= 0.5;
-    if (vp * vn >= 0.0) {
-      if (rec > 0) atomicAdd(bad, 1u);
-      break;
-    }
-    if (rec >= 6) break;
-    const double vm = nonlinear_value<kPow, kLag>(a, roots, m, iso);
-    if (fabs(vm) < 1e-8) break;
-    if (vm < 0) {
-      pn[0] = m[0]; pn[1] = m[1]; pn[2] = m[2]; vn = vm;
+  // steps -2 and -1 evaluate the lower and the upper end, then up to 6 midpoints
+  for (int step = fa ? 0 : -2;; step++) {
+    if (step < 0) {
+      m[0] = step == -2 ? pp[0] : pn[0];
+      m[1] = step == -2 ? pp[1] : pn[1];
+      m[2] = step == -2 ? pp[2] : pn[2];
     } else {
-      pp[0] = m[0]; pp[1] = m[1]; pp[2] = m[2]; vp = vm;
+      if (step == 0) {
+        // the positive end is the first (the lower endpoint) unless its value is negative
+        if (vp * vn >= 0.0) atomicAdd(bad, 1u);  // the reference exits here (:2082-2097)
+        if (vp < 0) {
+          for (int i = 0; i < 3; i++) {
+            const double t = pp[i];
+            pp[i] = pn[i];
+            pn[i] = t;
+          }
+          const double t = vp;
+          vp = vn;
+          vn = t;
+        }
+      }
+      m[0] = pp[0] + pn[0];
+      m[1] = pp[1] + pn[1];
+      m[2] = pp[2] + pn[2];
+      m[0] *= 0.5;
+      m[1] *= 0.5;
+      m[2] *= 0.5;
+      if (vp * vn >= 0.0) {
+        if (step > 0) atomicAdd(bad, 1u);
+        break;
+      }
+      if (step >= 6) break;
+    }
+    const double v = nonlinear_value<kPow, kMap>(a, roots, m, iso);
+    if (step == -2) {
+      vp = v;
+    } else if (step == -1) {
+      vn = v;
+    } else {
+      if (fabs(v) < 1e-8) break;
+      const bool neg = v < 0;
+      for (int i = 0; i < 3; i++) {
+        pn[i] = neg ? m[i] : pn[i];
+        pp[i] = neg ? pp[i] : m[i];
+      }
+      vn = neg ? v : vn;
+      vp = neg ? vp : v;
     }
   }
   out[0] = m[0];
@@ -1202,7 +1228,7 @@ __global__ __launch_bounds__(kMcBlock) void k_nl_vlist(const uint8_t* __restrict
 // the point relative to their range's first point. ends_a / ends_b: null, or
 // the slab's values from the range's first point on, when they are the end
 // values' own (see slab_holds_end_values); the midpoints are always evaluated.
-template <int kPow, bool kLag>
+template <int kPow, int kMap>
 __global__ __launch_bounds__(kMcBlock) void k_nl_vertices(MapArgs a, const RootRec64* __restrict__ roots,
                                                           double iso, int64_t p0a, const double* __restrict__ ends_a,
                                                           const uint32_t* __restrict__ off_a,
@@ -1233,11 +1259,9 @@ __global__ __launch_bounds__(kMcBlock) void k_nl_vertices(MapArgs a, const RootR
   const int axis = vax[t];
   const int64_t lz = q / XY, r = q - lz * XY;
   const int y = (int)(r / X), x = (int)(r - (int64_t)y * X), z = (int)(p0 + lz);
-  double pa[3];
-  cell_center(a, x, y, z, pa);
-  const double va = ends ? ends[q] - iso : nonlinear_value<kPow, kLag>(a, roots, pa, iso);
+  const double* fa = ends ? ends + q : nullptr;
   const double* fb = ends ? ends + q + (axis == 0 ? 1 : axis == 1 ? X : XY) : nullptr;
-  place_vertex<kPow, kLag>(a, roots, iso, x, y, z, axis, pa, va, fb, verts + 3 * k, bad);
+  place_vertex<kPow, kMap>(a, roots, iso, x, y, z, axis, fa, fb, verts + 3 * k, bad);
   edges[4 * k + 0] = x;
   edges[4 * k + 1] = y;
   edges[4 * k + 2] = z;
@@ -1248,11 +1272,14 @@ __global__ __launch_bounds__(kMcBlock) void k_nl_vertices(MapArgs a, const RootR
 // order (see nonlinear_value).
 template <class... Args>
 static void launch_nl_vertices(const MapArgs& a, dim3 grid, hipStream_t s, Args... args) {
-  const bool lag = (a.flags & QJ_MAP_LAGRANGE) != 0;
-  if (a.gen && lag) hipLaunchKernelGGL((k_nl_vertices<kExactInt, true>), grid, dim3(kMcBlock), 0, s, a, args...);
-  else if (a.gen) hipLaunchKernelGGL((k_nl_vertices<kExactInt, false>), grid, dim3(kMcBlock), 0, s, a, args...);
-  else if (lag) hipLaunchKernelGGL((k_nl_vertices<kExactOnly, true>), grid, dim3(kMcBlock), 0, s, a, args...);
-  else hipLaunchKernelGGL((k_nl_vertices<kExactOnly, false>), grid, dim3(kMcBlock), 0, s, a, args...);
+  const int map = (a.flags & QJ_MAP_LAGRANGE) ? kNlLag : (a.flags & QJ_MAP_EXTENDED_RANGE) ? kNlExt : kNlPlain;
+  const auto k = a.gen ? (map == kNlLag   ? k_nl_vertices<kExactInt, kNlLag>
+                          : map == kNlExt ? k_nl_vertices<kExactInt, kNlExt>
+                                          : k_nl_vertices<kExactInt, kNlPlain>)
+                       : (map == kNlLag   ? k_nl_vertices<kExactOnly, kNlLag>
+                          : map == kNlExt ? k_nl_vertices<kExactOnly, kNlExt>
+                                          : k_nl_vertices<kExactOnly, kNlPlain>);
+  hipLaunchKernelGGL(k, grid, dim3(kMcBlock), 0, s, a, args...);
 }
 // (x, y, z, flag) of the chunk's active cells, appended in cell order
 __global__ __launch_bounds__(kMcBlock) void k_nl_cells(const uint32_t* __restrict__ active, int64_t na,
@@ -1634,7 +1661,7 @@ qj_status nlmc_cache(qj_workspace* ws, int64_t* n_edges, int32_t* edges, int64_t
   return QJ_OK;
 }
 
-template <int kPow, bool kLag>
+template <int kPow, int kMap>
 __global__ __launch_bounds__(kMcBlock) void k_cache_vertices(MapArgs a, const RootRec64* __restrict__ roots,
                                                              double iso, const int32_t* __restrict__ edges, int64_t ne,
                                                              double* __restrict__ verts,
@@ -1642,19 +1669,19 @@ __global__ __launch_bounds__(kMcBlock) void k_cache_vertices(MapArgs a, const Ro
   const int64_t i = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
   if (i >= ne) return;
   const int x = edges[4 * i], y = edges[4 * i + 1], z = edges[4 * i + 2], axis = edges[4 * i + 3];
-  double pa[3];
-  cell_center(a, x, y, z, pa);
-  const double va = nonlinear_value<kPow, kLag>(a, roots, pa, iso);
-  place_vertex<kPow, kLag>(a, roots, iso, x, y, z, axis, pa, va, nullptr, verts + 3 * i, bad);
+  place_vertex<kPow, kMap>(a, roots, iso, x, y, z, axis, nullptr, nullptr, verts + 3 * i, bad);
 }
 
 template <class... Args>
 static void launch_cache_vertices(const MapArgs& a, dim3 grid, hipStream_t s, Args... args) {
-  const bool lag = (a.flags & QJ_MAP_LAGRANGE) != 0;
-  if (a.gen && lag) hipLaunchKernelGGL((k_cache_vertices<kExactInt, true>), grid, dim3(kMcBlock), 0, s, a, args...);
-  else if (a.gen) hipLaunchKernelGGL((k_cache_vertices<kExactInt, false>), grid, dim3(kMcBlock), 0, s, a, args...);
-  else if (lag) hipLaunchKernelGGL((k_cache_vertices<kExactOnly, true>), grid, dim3(kMcBlock), 0, s, a, args...);
-  else hipLaunchKernelGGL((k_cache_vertices<kExactOnly, false>), grid, dim3(kMcBlock), 0, s, a, args...);
+  const int map = (a.flags & QJ_MAP_LAGRANGE) ? kNlLag : (a.flags & QJ_MAP_EXTENDED_RANGE) ? kNlExt : kNlPlain;
+  const auto k = a.gen ? (map == kNlLag   ? k_cache_vertices<kExactInt, kNlLag>
+                          : map == kNlExt ? k_cache_vertices<kExactInt, kNlExt>
+                                          : k_cache_vertices<kExactInt, kNlPlain>)
+                       : (map == kNlLag   ? k_cache_vertices<kExactOnly, kNlLag>
+                          : map == kNlExt ? k_cache_vertices<kExactOnly, kNlExt>
+                                          : k_cache_vertices<kExactOnly, kNlPlain>);
+  hipLaunchKernelGGL(k, grid, dim3(kMcBlock), 0, s, a, args...);
 }
 
 __global__ __launch_bounds__(kMcBlock) void k_cache_tricount(const int32_t* __restrict__ cells, int64_t nc,

@@ -17,15 +17,16 @@ import fit_math64  # noqa: E402
 @pytest.mark.parametrize("name, begins, ends", [
     ("log", "const double z = s * s;", "// f - R"),
     ("atan", "const double z = u * u;", "// +-(u + u z P)"),
-    ("sin", "double p = 1.59", "const double s = "),
-    ("cos", "double c = ", "c = __builtin_fma(z, "),
+    ("sin", "double p = k64<kInLoop>(1.59", "const double s = "),
+    ("cos", "double c = k64<kInLoop>(", "c = __builtin_fma(z, "),
+    ("exp", "double p = k64<kInLoop>(2.09", "const double k = "),
 ])
 def test_constants_are_the_fit(name, begins, ends):
     src = open(os.path.join(CSRC, "qj_math64.h")).read()
     body = src[src.index(begins):]
     body = body[:body.index(ends)]
-    first = re.search(r"double [pc] = ([-0-9.e]+);", body).group(1)
-    rest = re.findall(r"__builtin_fma\([pc], z, ([-0-9.e]+)\)", body)
+    first = re.search(r"double [pc] = k64<kInLoop>\(([-0-9.e]+)\);", body).group(1)
+    rest = re.findall(r"__builtin_fma\([pc], [zr], k64<kInLoop>\(([-0-9.e]+)\)\)", body)
     got = [float(v) for v in [first] + rest][::-1]
     assert got == fit_math64.coefficients(name)
     assert fit_math64.max_error(name, 100) < 2.0 ** -53 * 1.1
