@@ -18,18 +18,19 @@
 //   imaginary part, and |b^e| is not |b|^e).
 //   Sums are over fixed trees, so results do not depend on scheduling.
 //
-// k_adjoint: reverse mode through max_iter iterations of the map at points,
-//   recomputing every iteration's products instead of storing trajectories.
-//   Each point is a group of 8 lanes, each lane taking a share of the roots;
-//   the ordered product of the shares is a prefix/suffix scan of quaternion
-//   products over the group, and each root's gradient is summed over the
-//   wave's points by shuffles before one lane adds it to the block's LDS.
+// k_adjoint: reverse mode through max_iter iterations of the map at points.
+//   Each point is a group of 4 to 32 lanes, each lane taking a share of the
+//   roots; the ordered product of the shares is a suffix scan of quaternion
+//   products over the group, and each root's gradient is summed over the wave's
+//   points by row swaps before one lane adds it to the block's LDS.
 #include <float.h>
 
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 
+#include "qj_fp32.h"
 #include "qj_geom.h"
 #include "qj_internal.h"
 #include "qj_math64.h"
@@ -608,17 +609,11 @@ __device__ __forceinline__ double column_sum(const double* __restrict__ partials
   }
   return s_v[0];
 }
-__global__ __launch_bounds__(kSumThreads) void k_sum_partials(const double* __restrict__ partials, int64_t nb, int K,
-                                                              double* __restrict__ out) {
-  const int k = blockIdx.x;
-  const double v = column_sum(partials, nb, K, k);
-  if (threadIdx.x == 0) out[k] = v;
-}
 __global__ void k_zero_count(unsigned long long* p) {
   if (threadIdx.x == 0) *p = 0ull;
 }
 
-// k_sum_partials over two arrays at once: block (k, 0) sums column k of the
+// Column sums over two arrays at once: block (k, 0) sums column k of the
 // first, block (k, 1) of the second, and both results and the cell count go to
 // pinned host memory, which the caller reads after its one wait.
 __global__ __launch_bounds__(kSumThreads) void k_ap_finish(const double* __restrict__ p0, int64_t n0, int K0,
@@ -743,259 +738,395 @@ __device__ __forceinline__ Q4<T> unit(const Q4<T>& a) {
   return n > T(0) ? sc(a, T(1) / n) : a;
 }
 
-// One polar power term in unit form: t = |b|^e * that, with that = (cos m, sin m v/|v|),
-// m = e * atan2(|v|, w) (QUATERNION::pow, QUATERNION.cpp:375-393, for e > 0).
-__device__ __forceinline__ void sincos_t(double m, double* s, double* c) { sincos(m, s, c); }
-__device__ __forceinline__ void sincos_t(float m, float* s, float* c) { sincosf(m, s, c); }
+// The elementary functions of the adjoint's backward sweep in its two precisions.
+template <class T>
+struct Fn;
+template <>
+struct Fn<double> {
+  __device__ __forceinline__ static void root(double x, double& r, double& inv) { sqrt_rsqrt64(x, r, inv); }
+  __device__ __forceinline__ static double recip(double x) { return div64(1.0, x); }
+  __device__ __forceinline__ static double log(double x) { return log64<true>(x); }
+  __device__ __forceinline__ static double exp(double x) { return exp64<true>(x); }
+  __device__ __forceinline__ static double angle(double y, double w) { return angle64<true>(y, w); }
+  __device__ __forceinline__ static void sincos(double m, double& s, double& c) { sincos64<true>(m, s, c); }
+};
+template <>
+struct Fn<float> {
+  __device__ __forceinline__ static void root(float x, float& r, float& inv) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    inv = __builtin_fmaf(0.5f * y, __builtin_fmaf(-x * y, y, 1.0f), y);
+    r = x * inv;
+  }
+  __device__ __forceinline__ static float recip(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+  }
+  __device__ __forceinline__ static float log(float x) { return logf(x); }
+  __device__ __forceinline__ static float exp(float x) { return expf(x); }
+  __device__ __forceinline__ static float angle(float y, float w) { return angle_upper(y, w); }
+  __device__ __forceinline__ static void sincos(float m, float& s, float& c) { sincosf(m, &s, &c); }
+};
 
+// One root; the block's copy of them is in LDS, where a lane's read takes about
+// 100 cycles instead of the 500 of a scattered load.
+struct AdjRoot {
+  double w, x, y, z, e;
+};
+
+// One power term t = (q - r)^e (QUATERNION::pow, QUATERNION.cpp:375-393, for
+// e > 0). Exponents 1 and 2 are p = b and b b, |p| = |b|^e; others (kGen) the
+// unit polar p = (A, C v) with A = cos m, C = sin m / |v|, m = e angle(|v|, w).
+// b is taken in FP64 also where the rest is FP32: q - r next to a root.
 template <class T>
 struct Term {
-  Q4<T> b;
-  Q4<T> that;
-  T r, rho, th, lb;  // |b|, |v|, angle, log|b|
-  T A, C;            // that = (A, C v)
+  Q4<T> b, p;
+  T n2, part;  // |b|^2, |v|^2
+  T e, A, C;
+  bool two, gen;
 };
-template <class T>
-__device__ __forceinline__ Term<T> make_term(const Q4<T>& q, const RootRec64& rr, T e) {
+template <class T, bool kGen>
+__device__ __forceinline__ Term<T> make_term(const Q4<double>& q, const AdjRoot& rr) {
   Term<T> t;
-  t.b = Q4<T>{q.w - T(rr.w), q.x - T(rr.x), q.y - T(rr.y), q.z - T(rr.z)};
-  const T p = t.b.x * t.b.x + t.b.y * t.b.y + t.b.z * t.b.z;
-  t.rho = sqrt(p);
-  t.r = sqrt(p + t.b.w * t.b.w);
-  t.th = atan2(t.rho, t.b.w);
-  t.lb = log(t.r);
-  const T m = e * t.th;
-  T s, c;
-  sincos_t(m, &s, &c);
-  t.A = c;
-  t.C = t.rho > T(0) ? s / t.rho : e / t.b.w;  // limit v -> 0 (w > 0)
-  t.that = Q4<T>{t.A, t.C * t.b.x, t.C * t.b.y, t.C * t.b.z};
+  t.e = T(rr.e);
+  t.two = rr.e == 2.0;
+  t.gen = kGen && rr.e != 1.0 && !t.two;
+  t.b = Q4<T>{T(q.w - rr.w), T(q.x - rr.x), T(q.y - rr.y), T(q.z - rr.z)};
+  t.part = t.b.x * t.b.x + t.b.y * t.b.y + t.b.z * t.b.z;
+  t.n2 = t.part + t.b.w * t.b.w;
+  t.p = t.b;
+  if (t.two) {
+    const T w2 = T(2) * t.b.w;
+    t.p = Q4<T>{t.b.w * t.b.w - t.part, w2 * t.b.x, w2 * t.b.y, w2 * t.b.z};
+  }
+  if (t.gen) {
+    T rho, vi, s, c;
+    Fn<T>::root(t.part, rho, vi);
+    const bool v0 = !(t.part > T(0));
+    Fn<T>::sincos(t.e * (v0 ? (t.b.w < T(0) ? T(3.141592653589793) : T(0)) : Fn<T>::angle(rho, t.b.w)), s, c);
+    t.A = c;
+    t.C = v0 ? t.e / t.b.w : s * vi;  // limit v -> 0 (w > 0)
+    t.p = Q4<T>{t.A, t.C * t.b.x, t.C * t.b.y, t.C * t.b.z};
+  }
   return t;
 }
-// b_bar = J'^T tbar' for the unit-form power (J = |b|^e J')
+// b's adjoint from p = |t| / |Q| times the polar term's, in unit form
 template <class T>
-__device__ __forceinline__ Q4<T> pow_vjp(const Term<T>& t, const Q4<T>& tb, T e) {
-  const T r = t.r, rho = t.rho, w = t.b.w;
-  const T gA = tb.w;
-  const T gC = tb.x * t.b.x + tb.y * t.b.y + tb.z * t.b.z;
-  const T Gr = (gA * e * t.A + gC * e * t.C) / r;
-  if (!(rho > T(0))) {
+__device__ __forceinline__ Q4<T> polar_vjp(const Term<T>& t, const Q4<T>& p) {
+  T r, ri;
+  Fn<T>::root(t.n2, r, ri);
+  const T w = t.b.w, e = t.e;
+  const T gA = p.w;
+  const T gC = p.x * t.b.x + p.y * t.b.y + p.z * t.b.z;
+  const T Gr = (gA * e * t.A + gC * e * t.C) * ri;
+  if (!(t.part > T(0))) {
     // purely real base: d/db of (w^e, e w^(e-1) v) / w^e
-    return Q4<T>{Gr, t.C * tb.x, t.C * tb.y, t.C * tb.z};
+    return Q4<T>{Gr, t.C * p.x, t.C * p.y, t.C * p.z};
   }
-  const T Gth = -gA * e * t.C * rho + gC * e * t.A / rho;
-  const T Grho = -gC * t.C / rho;
-  const T r2 = r * r;
-  const T coef = Gr / r + Gth * w / (r2 * rho) + Grho / rho;
-  return Q4<T>{Gr * (w / r) - Gth * (rho / r2), coef * t.b.x + t.C * tb.x, coef * t.b.y + t.C * tb.y,
-               coef * t.b.z + t.C * tb.z};
+  T rho, vi;
+  Fn<T>::root(t.part, rho, vi);
+  const T Gth = -gA * e * t.C * rho + gC * e * t.A * vi;
+  const T ri2 = ri * ri;
+  const T coef = Gr * ri + Gth * w * (ri2 * vi) - gC * t.C * (vi * vi);
+  return Q4<T>{Gr * (w * ri) - Gth * (rho * ri2), coef * t.b.x + t.C * p.x, coef * t.b.y + t.C * p.y,
+               coef * t.b.z + t.C * p.z};
+}
+// One step of the backward sweep: b's adjoint from W = R M conj(R) (see
+// k_adjoint), and W turned past the term, u W conj(u) with u = p / |p|. The
+// exponents 1 and 2 take 1 / |b|^2 and no square root.
+template <class T>
+__device__ __forceinline__ Q4<T> sweep_step(const Term<T>& t, Q4<T>& W) {
+  if (t.gen) {
+    const Q4<T> tb = mul(t.p, W);
+    W = mul(tb, conj(t.p));
+    return polar_vjp(t, tb);
+  }
+  const T s = Fn<T>::recip(t.n2);
+  const Q4<T> tb = sc(mul(t.p, W), s);
+  if (!t.two) {
+    W = mul(tb, conj(t.b));
+    return tb;
+  }
+  // t = b^2: (p conj(b) + conj(b) p) / |b|^2
+  W = sc(mul(tb, conj(t.p)), s);
+  const T f = T(2) * s;
+  return Q4<T>{f * (tb.w * t.b.w + (tb.x * t.b.x + tb.y * t.b.y + tb.z * t.b.z)), f * (t.b.w * tb.x - tb.w * t.b.x),
+               f * (t.b.w * tb.y - tb.w * t.b.y), f * (t.b.w * tb.z - tb.w * t.b.z)};
 }
 
 constexpr int kAdjBlock = 128;
 constexpr int kMaxAdjIter = 16;
-// lanes per point: each lane of a group takes a contiguous share of the top
-// roots and of the bottom roots, so 40k points keep every SIMD busy
-template <class T>
-constexpr int adj_lanes() {
-  return sizeof(T) == 4 ? 16 : 8;  // FP64: 8 (twice the registers per value, 16 measured slower)
-}
+// iterations whose group products are kept for the backward sweep (private
+// memory: 17 values each); later ones are formed again
+constexpr int kAdjKeep = 3;
 
-template <class T>
-__device__ __forceinline__ Q4<T> shfl_up_q(const Q4<T>& a, int d) {
-  return {__shfl_up(a.w, d, adj_lanes<T>()), __shfl_up(a.x, d, adj_lanes<T>()), __shfl_up(a.y, d, adj_lanes<T>()),
-          __shfl_up(a.z, d, adj_lanes<T>())};
+template <int kCtrl>
+__device__ __forceinline__ float dpp_mov(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, false));
 }
-template <class T>
-__device__ __forceinline__ Q4<T> shfl_down_q(const Q4<T>& a, int d) {
-  return {__shfl_down(a.w, d, adj_lanes<T>()), __shfl_down(a.x, d, adj_lanes<T>()), __shfl_down(a.y, d, adj_lanes<T>()),
-          __shfl_down(a.z, d, adj_lanes<T>())};
+template <int kCtrl>
+__device__ __forceinline__ double dpp_mov(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, kCtrl, 0xf, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), kCtrl, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
-template <class T>
-__device__ __forceinline__ Q4<T> shfl_q(const Q4<T>& a, int src) {
-  return {__shfl(a.w, src, adj_lanes<T>()), __shfl(a.x, src, adj_lanes<T>()), __shfl(a.y, src, adj_lanes<T>()),
-          __shfl(a.z, src, adj_lanes<T>())};
-}
-// sum over the lanes of a group
-template <class T>
-__device__ __forceinline__ T group_sum(T v) {
-  for (int o = adj_lanes<T>() / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-template <class T>
-__device__ __forceinline__ Q4<T> group_sum_q(const Q4<T>& a) {
-  return {group_sum(a.w), group_sum(a.x), group_sum(a.y), group_sum(a.z)};
+// v + the value 16 (32) lanes across: the row swaps of v with itself
+template <int kRows>
+__device__ __forceinline__ double swap_add(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)b, hi = (uint32_t)(b >> 32);
+  if constexpr (kRows == 16) {
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __builtin_bit_cast(double, (uint64_t)h[0] << 32 | l[0]) + __builtin_bit_cast(double, (uint64_t)h[1] << 32 | l[1]);
+  } else {
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return __builtin_bit_cast(double, (uint64_t)h[0] << 32 | l[0]) + __builtin_bit_cast(double, (uint64_t)h[1] << 32 | l[1]);
+  }
 }
 // sum over the groups of a wave, lane by lane (the lanes that hold the same roots)
-template <class T>
+template <int L>
 __device__ __forceinline__ double across_groups(double v) {
-  for (int o = adj_lanes<T>(); o < 64; o <<= 1) v += __shfl_xor(v, o);
+  if constexpr (L <= 4) v += dpp_mov<0x124>(v);  // row_ror:4
+  if constexpr (L <= 8) v += dpp_mov<0x128>(v);  // row_ror:8
+  if constexpr (L <= 16) v = swap_add<16>(v);
+  if constexpr (L <= 32) v = swap_add<32>(v);
   return v;
 }
+// the value d lanes up inside a group (lanes past its end: anything)
+template <int L, int d, class T>
+__device__ __forceinline__ Q4<T> lanes_up(const Q4<T>& a) {
+  if constexpr (L <= 16) {
+    constexpr int c = 0x100 + d;  // row_shl
+    return {dpp_mov<c>(a.w), dpp_mov<c>(a.x), dpp_mov<c>(a.y), dpp_mov<c>(a.z)};
+  } else {
+    return {__shfl_down(a.w, d, L), __shfl_down(a.x, d, L), __shfl_down(a.y, d, L), __shfl_down(a.z, d, L)};
+  }
+}
+template <int L, class T>
+__device__ __forceinline__ T group_sum(T v) {
+  for (int o = L / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+template <int L, class T>
+__device__ __forceinline__ Q4<T> group_sum_q(const Q4<T>& a) {
+  return {group_sum<L>(a.w), group_sum<L>(a.x), group_sum<L>(a.y), group_sum<L>(a.z)};
+}
 
-// The unit product of polynomial roots [lo, hi) in order, its log magnitude,
-// and over the group: the whole polynomial's unit product and log magnitude,
-// and the unit product of the roots after this lane's share.
+// Over a group: a polynomial's unit product, and the unit product of the roots
+// after this lane's share.
 template <class T>
 struct Share {
   Q4<T> all, after;
-  T L;
 };
-template <class T>
-__device__ __forceinline__ Share<T> group_product(const RootRec64* __restrict__ roots, int lo, int hi, const Q4<T>& q,
-                                                  int sub) {
-  Q4<T> p{1, 0, 0, 0};
-  T l = 0;
-  for (int i = lo; i < hi; i++) {
-    const RootRec64 rr = roots[i];
-    const Term<T> t = make_term(q, rr, T(rr.e));
-    p = mul(p, t.that);
-    l += T(rr.e) * t.lb;
-    if (((i - lo) & 7) == 7) p = unit(p);
+template <int L, int d, class T>
+__device__ __forceinline__ void suffix_step(Q4<T>& suf, int sub) {
+  if constexpr (d < L) {
+    const Q4<T> z = mul(suf, lanes_up<L, d>(suf));
+    if (sub + d < L) suf = z;
+    suffix_step<L, 2 * d>(suf, sub);
   }
-  p = unit(p);
-  // ordered inclusive prefix and suffix products over the group (Hillis-Steele)
-  Q4<T> pre = p, suf = p;
-  for (int d = 1; d < adj_lanes<T>(); d <<= 1) {
-    const Q4<T> y = shfl_up_q(pre, d);
-    const Q4<T> z = shfl_down_q(suf, d);
-    if (sub >= d) pre = mul(y, pre);
-    if (sub + d < adj_lanes<T>()) suf = mul(suf, z);
+}
+// c: root steps of every lane (uniform); the lane's roots are [lo, hi). Always in
+// FP64; ln: the polynomial's log magnitude.
+template <int L, bool kGen>
+__device__ __forceinline__ Share<double> group_product(const AdjRoot* roots, int lo, int hi, int c,
+                                                       const Q4<double>& q, int sub, double& ln) {
+  // exponents 1 and 2 as they are, brought to a norm in [0.7, 1.5) by a power
+  // of two each (2^+-60 over a share of 100 roots)
+  Q4<double> p{1, 0, 0, 0};
+  double lg = 0;
+  int E = 0;
+  for (int j = 0; j < c; j++) {
+    if (lo + j < hi) {
+      const Term<double> t = make_term<double, kGen>(q, roots[lo + j]);
+      if (kGen && t.gen) {
+        p = mul(p, t.p);
+        lg += t.e * log64<true>(t.n2);
+      } else {
+        // half the norm's exponent
+        int k = ((int)(__builtin_bit_cast(uint64_t, t.n2) >> 52) - 1022) >> 1;
+        if (t.two) k *= 2;
+        E += k;
+        p = mul(p, sc(t.p, __builtin_bit_cast(double, (uint64_t)(1023 - k) << 52)));
+      }
+    }
   }
-  Share<T> s;
-  s.all = unit(shfl_q(pre, adj_lanes<T>() - 1));
-  const Q4<T> nxt = shfl_down_q(suf, 1);
-  s.after = sub + 1 < adj_lanes<T>() ? unit(nxt) : Q4<T>{1, 0, 0, 0};
-  s.L = group_sum(l);
+  double n2 = dot(p, p), r, ri;
+  sqrt_rsqrt64(n2, r, ri);
+  p = sc(p, ri);
+  ln = group_sum<L>(0.5 * (lg + log64<true>(n2)) + E * 0.6931471805599453);
+  // ordered inclusive suffix products over the group (Hillis-Steele)
+  suffix_step<L, 1>(p, sub);
+  Share<double> s;
+  s.all = unit(Q4<double>{__shfl(p.w, 0, L), __shfl(p.x, 0, L), __shfl(p.y, 0, L), __shfl(p.z, 0, L)});
+  const Q4<double> nxt = lanes_up<L, 1>(p);
+  s.after = sub + 1 < L ? unit(nxt) : Q4<double>{1, 0, 0, 0};
   return s;
+}
+template <class T>
+__device__ __forceinline__ Q4<T> as(const Q4<double>& a) {
+  return {T(a.w), T(a.x), T(a.y), T(a.z)};
 }
 
 // slot layout per root i (top then bottom): 5 i + {0..3} = d/d root component, 5 i + 4 = d/d e_i
-// One group of adj_lanes<T>() lanes per point; lane `sub` of a group takes top
-// roots [sub ct, sub ct + ct) and bottom roots [sub cb, sub cb + cb). Control
-// flow is uniform over the wave (every group runs max_iter steps and ct / cb
-// root steps, masked), so the shuffles always see active partners.
-template <class T>
-__global__ __launch_bounds__(kAdjBlock) void k_adjoint(MapArgs a, const RootRec64* __restrict__ roots,
+//
+// Reverse mode through max_iter iterations of the map. One group of L lanes
+// per point; lane `sub` takes top roots [sub ct, sub ct + ct) and bottom roots
+// [sub cb, sub cb + cb). Control flow is uniform over the wave (every group
+// runs the same iterations and root steps, masked), so lane exchanges always
+// see active partners. Forward, in FP64 for both precisions (an FP32 iterate is
+// off by its rounding times the map's growth, 10 to 30 per iteration): the
+// iterates up to the last one's start, with each iteration's group products.
+// Backward, in T:
+//   * a point's last iteration needs no product: F = log c + sum e log|b| over
+//     the top roots - the same over the bottom ones, so b's adjoint is
+//     +-g e b / |b|^2 and e's is +-g log|b|;
+//   * before that, with q' = c T B^-1, M = |Q| conj(T) (Q' B) in unit parts and
+//     R the product of the roots after root i, the term's adjoint is
+//     u_i W_i, u_i its unit part and W_i = R M conj(R) (-M for the bottom
+//     roots), which the sweep turns from one root to the next: W <- u W conj(u).
+//     e's adjoint is W . log b.
+// FP64 / FP32 VALU bound, long dependent chains. Figures beside points_adjoint.
+template <class T, int L, bool kGen>
+__global__ __launch_bounds__(kAdjBlock, 4) void k_adjoint(MapArgs a, const RootRec64* __restrict__ g_roots,
                                                        const double* __restrict__ pts, int64_t n,
                                                        const double* __restrict__ dJdF,
                                                        double* __restrict__ partials, int K) {
-  extern __shared__ double acc[];  // (kAdjBlock/64) x K
+  extern __shared__ double acc[];  // (kAdjBlock/64) x K, then the roots
+  AdjRoot* const roots = (AdjRoot*)(acc + (kAdjBlock / 64) * K);
   for (int i = threadIdx.x; i < (kAdjBlock / 64) * K; i += kAdjBlock) acc[i] = 0.0;
+  for (int i = threadIdx.x; i < a.nt + a.nb; i += kAdjBlock)
+    roots[i] = AdjRoot{g_roots[i].w, g_roots[i].x, g_roots[i].y, g_roots[i].z, g_roots[i].e};
   __syncthreads();
-  constexpr int kL = adj_lanes<T>();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sub = lane & (kL - 1);
-  const int64_t pid = ((int64_t)blockIdx.x * kAdjBlock + threadIdx.x) / kL;
-  const bool active = pid < n;
-  const int ct = (a.nt + kL - 1) / kL, cb = (a.nb + kL - 1) / kL;
-  const int t0 = sub * ct, t1 = min(a.nt, t0 + ct);
-  const int b0 = sub * cb, b1 = min(a.nb, b0 + cb);
-  Q4<T> qs[kMaxAdjIter + 1];
-  int Kx = 0;
-  T gF = 0;
-  qs[0] = active ? Q4<T>{T(pts[3 * pid]), T(pts[3 * pid + 1]), T(pts[3 * pid + 2]), T(a.slice)}
-                 : Q4<T>{1, 0, 0, 0};
-  if (active) gF = T(dJdF[pid]);
-  bool running = active && sqrt(dot(qs[0], qs[0])) < T(a.escape) && a.max_iter > 0;
-  for (int k = 0; k < a.max_iter; k++) {
-    const Q4<T> q = running ? qs[k] : Q4<T>{1, 0, 0, 0};
-    const Share<T> tp = group_product(roots, t0, t1, q, sub);
-    const Share<T> bt = group_product(roots + a.nt, b0, b1, q, sub);
-    if (running) {
-      const Q4<T> Qh = a.nb > 0 ? mul(tp.all, conj(bt.all)) : tp.all;
-      const T scale = T(a.exp_scaling) * exp(tp.L - (a.nb > 0 ? bt.L : T(0)));
-      qs[k + 1] = sc(Qh, scale);
-      Kx = k + 1;
-      const T mag = sqrt(dot(qs[k + 1], qs[k + 1]));
-      if (!(mag < T(a.escape)) || ((a.flags & QJ_MAP_BLACK_HOLE) && mag < T(10.0 * (double)FLT_MIN)))
-        running = false;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = lane & (L - 1);
+  const int c[2] = {(a.nt + L - 1) / L, (a.nb + L - 1) / L};
+  const int first[2] = {0, a.nt}, count[2] = {a.nt, a.nb};
+  double* const mine = acc + wave * K;
+  // one root's gradient, summed over the wave's points
+  auto add = [&](int i, bool in, const Q4<T>& bb, T ge) {
+    const double g0 = across_groups<L>(-(double)bb.w), g1 = across_groups<L>(-(double)bb.x),
+                 g2 = across_groups<L>(-(double)bb.y), g3 = across_groups<L>(-(double)bb.z),
+                 g4 = across_groups<L>((double)ge);
+    if (lane < L && in) {
+      // LDS adds without a return: the slots are this wave's own, so they land in program order
+      double* r = mine + 5 * i;
+      unsafeAtomicAdd(r, g0);
+      unsafeAtomicAdd(r + 1, g1);
+      unsafeAtomicAdd(r + 2, g2);
+      unsafeAtomicAdd(r + 3, g3);
+      unsafeAtomicAdd(r + 4, g4);
     }
-  }
-  // dJ/dq_K for F = log|q_K|
-  Q4<T> qbar{0, 0, 0, 0};
-  if (active && gF != T(0)) {
-    const Q4<T> qk = qs[Kx];
-    qbar = sc(qk, gF / dot(qk, qk));
-  }
-  for (int k = a.max_iter - 1; k >= 0; k--) {
-    const bool live = active && k < Kx;
-    const Q4<T> q = live ? qs[k] : Q4<T>{1, 0, 0, 0};
-    const Share<T> tp = group_product(roots, t0, t1, q, sub);
-    const Share<T> bt = group_product(roots + a.nt, b0, b1, q, sub);
-    const Q4<T> Th = tp.all;
-    const Q4<T> Bh = a.nb > 0 ? bt.all : Q4<T>{1, 0, 0, 0};
-    const T Qmag = exp(tp.L - (a.nb > 0 ? bt.L : T(0)));
-    const Q4<T> Qbar = sc(qbar, T(a.exp_scaling));  // q_{k+1} = c Q
-    Q4<T> qnew{0, 0, 0, 0};
-    // top terms: tbar' = conj(Phat) Qbar Bhat conj(Shat_{i+1})
-    {
-      const Q4<T> QB = mul(Qbar, Bh);
-      Q4<T> S = tp.after;
-      for (int j = 0; j < ct; j++) {
-        const int i = t0 + ct - 1 - j;
-        double g0 = 0, g1 = 0, g2 = 0, g3 = 0, g4 = 0;
-        if (live && i < t1) {
-          const RootRec64 rr = roots[i];
-          const Term<T> t = make_term(q, rr, T(rr.e));
-          const Q4<T> right = S;
-          S = mul(t.that, S);
-          const Q4<T> P = (i > 0) ? mul(Th, conj(S)) : Q4<T>{1, 0, 0, 0};
-          const Q4<T> tb = mul(mul(conj(P), QB), conj(right));
-          const Q4<T> bb = sc(pow_vjp(t, tb, T(rr.e)), Qmag);
-          // d t / d e = t log(b); log(b) = (log|b|, th v/|v|)
-          const T lv = t.rho > T(0) ? t.th / t.rho : T(0);
-          const Q4<T> lg{t.lb, lv * t.b.x, lv * t.b.y, lv * t.b.z};
-          const T ge = Qmag * dot(tb, mul(t.that, lg));
-          qnew = Q4<T>{qnew.w + bb.w, qnew.x + bb.x, qnew.y + bb.y, qnew.z + bb.z};
-          g0 = -(double)bb.w; g1 = -(double)bb.x; g2 = -(double)bb.y; g3 = -(double)bb.z; g4 = (double)ge;
-          if ((j & 7) == 7) S = unit(S);
-        }
-        g0 = across_groups<T>(g0);
-        g1 = across_groups<T>(g1);
-        g2 = across_groups<T>(g2);
-        g3 = across_groups<T>(g3);
-        g4 = across_groups<T>(g4);
-        if (lane < kL && i < t1) {
-          double* r = acc + wave * K + 5 * i;
-          r[0] += g0; r[1] += g1; r[2] += g2; r[3] += g3; r[4] += g4;
-        }
+  };
+  constexpr int kPoints = kAdjBlock / L;
+  for (int64_t base = (int64_t)blockIdx.x * kPoints; base < n; base += (int64_t)gridDim.x * kPoints) {
+    const int64_t pid = base + threadIdx.x / L;
+    const bool active = pid < n;
+    Q4<double> qs[kMaxAdjIter];
+    Share<T> kept[kAdjKeep][2];
+    T kept_mag[kAdjKeep];
+    qs[0] = active ? Q4<double>{pts[3 * pid], pts[3 * pid + 1], pts[3 * pid + 2], a.slice} : Q4<double>{1, 0, 0, 0};
+    const T gF = active ? T(dJdF[pid]) : T(0);
+    // one iteration's group products; Qmag = |q'|
+    auto products = [&](const Q4<double>& q, Share<T>* s, Q4<double>& Qh, T& Qmag) {
+      double lt, lb;
+      const Share<double> t =
+          group_product<L, kGen>(roots, sub * c[0], min(count[0], sub * c[0] + c[0]), c[0], q, sub, lt);
+      Share<double> b{{1, 0, 0, 0}, {1, 0, 0, 0}};
+      lb = 0.0;
+      if (a.nb > 0)
+        b = group_product<L, kGen>(roots + a.nt, sub * c[1], min(count[1], sub * c[1] + c[1]), c[1], q, sub, lb);
+      const double m = a.exp_scaling * exp64<true>(lt - lb);
+      s[0] = Share<T>{as<T>(t.all), as<T>(t.after)};
+      s[1] = Share<T>{as<T>(b.all), as<T>(b.after)};
+      Qh = sc(mul(t.all, conj(b.all)), m);
+      Qmag = T(m);
+    };
+    // Kx: iterations the point runs; a point without a gradient runs none
+    int Kx = 0;
+    bool running = active && gF != T(0) && sqrt(dot(qs[0], qs[0])) < a.escape && a.max_iter > 0;
+    for (int k = 0; __ballot(running); k++) {
+      if (running) Kx = k + 1;
+      if (k + 1 >= a.max_iter) break;
+      const Q4<double> q = running ? qs[k] : Q4<double>{1, 0, 0, 0};
+      Share<T> s[2];
+      Q4<double> Qh;
+      T Qmag;
+      products(q, s, Qh, Qmag);
+      if (k < kAdjKeep) {
+        kept[k][0] = s[0];
+        kept[k][1] = s[1];
+        kept_mag[k] = Qmag;
+      }
+      if (running) {
+        qs[k + 1] = Qh;
+        const double mag = sqrt(dot(Qh, Qh));
+        if (!(mag < a.escape) || ((a.flags & QJ_MAP_BLACK_HOLE) && mag < 10.0 * (double)FLT_MIN)) running = false;
       }
     }
-    // bottom terms: ubar' = -conj(PBhat) Bhat conj(That) Qbar Bhat conj(SBhat_{j+1})
-    if (a.nb > 0) {
-      const Q4<T> M = mul(mul(Bh, conj(Th)), mul(Qbar, Bh));
-      Q4<T> S = bt.after;
-      for (int jj = 0; jj < cb; jj++) {
-        const int j = b0 + cb - 1 - jj;
-        double g0 = 0, g1 = 0, g2 = 0, g3 = 0, g4 = 0;
-        if (live && j < b1) {
-          const RootRec64 rr = roots[a.nt + j];
-          const Term<T> t = make_term(q, rr, T(rr.e));
-          const Q4<T> right = S;
-          S = mul(t.that, S);
-          const Q4<T> P = (j > 0) ? mul(Bh, conj(S)) : Q4<T>{1, 0, 0, 0};
-          const Q4<T> ub = sc(mul(mul(conj(P), M), conj(right)), T(-1));
-          const Q4<T> bb = sc(pow_vjp(t, ub, T(rr.e)), Qmag);
-          const T lv = t.rho > T(0) ? t.th / t.rho : T(0);
-          const Q4<T> lg{t.lb, lv * t.b.x, lv * t.b.y, lv * t.b.z};
-          const T ge = Qmag * dot(ub, mul(t.that, lg));
-          qnew = Q4<T>{qnew.w + bb.w, qnew.x + bb.x, qnew.y + bb.y, qnew.z + bb.z};
-          g0 = -(double)bb.w; g1 = -(double)bb.x; g2 = -(double)bb.y; g3 = -(double)bb.z; g4 = (double)ge;
-          if ((jj & 7) == 7) S = unit(S);
-        }
-        g0 = across_groups<T>(g0);
-        g1 = across_groups<T>(g1);
-        g2 = across_groups<T>(g2);
-        g3 = across_groups<T>(g3);
-        g4 = across_groups<T>(g4);
-        if (lane < kL && j < b1) {
-          double* r = acc + wave * K + 5 * (a.nt + j);
-          r[0] += g0; r[1] += g1; r[2] += g2; r[3] += g3; r[4] += g4;
+    Q4<T> qbar{0, 0, 0, 0};
+    for (int k = a.max_iter - 1; k >= 0; k--) {
+      const bool last = k + 1 == Kx, inner = k + 1 < Kx;
+      if (!__ballot(last || inner)) continue;
+      const Q4<double> q = (last || inner) ? qs[k] : Q4<double>{1, 0, 0, 0};
+      Q4<T> qnew{0, 0, 0, 0};
+      if (__ballot(last)) {
+        for (int p = 0; p < 2; p++) {
+          const T g = p ? -gF : gF;
+          const int lo = sub * c[p], hi = min(count[p], lo + c[p]);
+          for (int j = 0; j < c[p]; j++) {
+            const int i = first[p] + lo + j;
+            Q4<T> bb{0, 0, 0, 0};
+            T ge = 0;
+            if (last && lo + j < hi) {
+              const AdjRoot rr = roots[i];
+              const Q4<T> b{T(q.w - rr.w), T(q.x - rr.x), T(q.y - rr.y), T(q.z - rr.z)};
+              const T n2 = dot(b, b);
+              bb = sc(b, g * T(rr.e) * Fn<T>::recip(n2));
+              ge = g * T(0.5) * Fn<T>::log(n2);
+              qnew = Q4<T>{qnew.w + bb.w, qnew.x + bb.x, qnew.y + bb.y, qnew.z + bb.z};
+            }
+            add(i, lo + j < hi, bb, ge);
+          }
         }
       }
+      if (__ballot(inner)) {
+        Share<T> s[2];
+        T Qmag;
+        if (k < kAdjKeep) {
+          s[0] = kept[k][0];
+          s[1] = kept[k][1];
+          Qmag = kept_mag[k];
+        } else {
+          Q4<double> Qh;
+          products(q, s, Qh, Qmag);
+        }
+        const Q4<T> M = sc(mul(conj(s[0].all), mul(qbar, s[1].all)), Qmag);
+        for (int p = 0; p < 2; p++) {
+          const int lo = sub * c[p], hi = min(count[p], lo + c[p]);
+          Q4<T> W = mul(mul(s[p].after, p ? sc(M, T(-1)) : M), conj(s[p].after));
+          for (int j = c[p] - 1; j >= 0; j--) {
+            const int i = first[p] + lo + j;
+            Q4<T> bb{0, 0, 0, 0};
+            T ge = 0;
+            if (inner && lo + j < hi) {
+              const Term<T> t = make_term<T, kGen>(q, roots[i]);
+              // d t / d e = t log(b); log(b) = (log|b|, angle v / |v|)
+              T rho, vi;
+              Fn<T>::root(t.part, rho, vi);
+              const T lv = t.part > T(0) ? Fn<T>::angle(rho, t.b.w) * vi : T(0);
+              ge = W.w * (T(0.5) * Fn<T>::log(t.n2)) + lv * (W.x * t.b.x + W.y * t.b.y + W.z * t.b.z);
+              bb = sweep_step(t, W);
+              qnew = Q4<T>{qnew.w + bb.w, qnew.x + bb.x, qnew.y + bb.y, qnew.z + bb.z};
+            }
+            add(i, lo + j < hi, bb, ge);
+          }
+        }
+      }
+      qnew = group_sum_q<L>(qnew);
+      if (last || inner) qbar = qnew;
     }
-    qnew = group_sum_q(qnew);
-    if (live) qbar = qnew;
   }
   __syncthreads();
   for (int k = threadIdx.x; k < K; k += kAdjBlock) {
@@ -1005,17 +1136,44 @@ __global__ __launch_bounds__(kAdjBlock) void k_adjoint(MapArgs a, const RootRec6
   }
 }
 
-// sums the per-block partials and scatters: roots (n x 4) and powers (dJ/dp = s dJ/de)
-__global__ void k_adjoint_finish(const double* __restrict__ partials, int64_t nb, int nt, int nr, double sc_top,
-                                 double sc_bottom, double* __restrict__ grad_roots, double* __restrict__ grad_powers) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  const int K = 5 * nr;
-  if (k >= K) return;
-  double s = 0.0;
-  for (int64_t b = 0; b < nb; b++) s += partials[b * K + k];
+// Block k: the sum of slot k's partials over the rows (rows = 0: no points),
+// written to the root gradients (n x 4) or the powers' (dJ/dp = s dJ/de).
+__global__ __launch_bounds__(kSumThreads) void k_adjoint_finish(const double* __restrict__ partials, int64_t rows,
+                                                                int nt, int nr, double sc_top, double sc_bottom,
+                                                                double* __restrict__ grad_roots,
+                                                                double* __restrict__ grad_powers) {
+  const int k = blockIdx.x;
+  const double s = column_sum(partials, rows, 5 * nr, k);
+  if (threadIdx.x != 0) return;
   const int i = k / 5, c = k - 5 * i;
   if (c < 4) grad_roots[4 * i + c] = s;
   else grad_powers[i] = s * (i < nt ? sc_top : sc_bottom);
+}
+
+// Blocks beyond kAdjRows loop over points, so at most that many rows are summed.
+// Lanes per point by the roots a lane would have (gradient in us with 4 / 8 / 16 /
+// 32 lanes, FP64): 40k points with 8+8 roots 42 / 57 / 96 / 184, with 64+64 200 /
+// 186 / 186 / 245 (exponents 1) and 339 / 294 / 274 / 329 (real), 12k with 32+32
+// 117 / 73 / 75 / 82; few points take twice the lanes to fill the chip: 3001 with
+// 64+64 89 / 53 / 48 / 40, 300 with 16+16 31 / 22 / 20 / 20. FP32 has its minima at
+// the same places (40k 64+64: 157 / 148 / 143 / 187). Against polar terms formed
+// three times per iteration and every group product twice: 40k points with 64+64
+// roots 917 to 186 us in FP64 and 354 to 143 in FP32, whose error against FP64 went
+// from 3e-5 to 6e-8 with the FP64 iterates.
+constexpr int64_t kAdjRows = 2048;
+static int adj_lanes(const MapArgs& a, int64_t n) {
+  const int m = a.nt > a.nb ? a.nt : a.nb;
+  const int L = m <= 12 ? 4 : m < 32 ? 8 : 16;
+  return n <= 8192 ? 2 * L : L;
+}
+template <class T, bool kGen>
+static auto adjoint_kernel_of(int L) {
+  return L == 4 ? k_adjoint<T, 4, kGen> : L == 8 ? k_adjoint<T, 8, kGen> : L == 16 ? k_adjoint<T, 16, kGen>
+                                                                                 : k_adjoint<T, 32, kGen>;
+}
+static auto adjoint_kernel(qj_precision prec, int L, bool gen) {
+  return prec == QJ_FP64 ? (gen ? adjoint_kernel_of<double, true>(L) : adjoint_kernel_of<double, false>(L))
+                         : (gen ? adjoint_kernel_of<float, true>(L) : adjoint_kernel_of<float, false>(L));
 }
 
 qj_status points_adjoint(qj_workspace* ws, const MapArgs& a, const qj_rational* f, qj_precision prec,
@@ -1032,30 +1190,23 @@ qj_status points_adjoint(qj_workspace* ws, const MapArgs& a, const qj_rational* 
       set_error("the adjoint needs positive exponents (power_scalar * power > 0)");
       return QJ_ERR_INVALID;
     }
-  const size_t lds = sizeof(double) * (kAdjBlock / 64) * K;
-  if (lds > 64 * 1024) {
+  if (sizeof(double) * (kAdjBlock / 64) * K > 64 * 1024) {
     set_error("too many roots for the adjoint kernel (%d)", nr);
     return QJ_ERR_CAPACITY;
   }
-  const int64_t per_block = kAdjBlock / (prec == QJ_FP64 ? adj_lanes<double>() : adj_lanes<float>());  // points
-  const int64_t nblocks = n > 0 ? (n + per_block - 1) / per_block : 1;
-  qj_status st = ensure_partials(ws, nblocks * K + K, s);
+  // the sums and the roots: at most 64 + 32 KiB
+  const size_t lds = sizeof(double) * (kAdjBlock / 64) * K + sizeof(AdjRoot) * (size_t)nr;
+  const int L = adj_lanes(a, n);
+  const int64_t per_block = kAdjBlock / L;  // points
+  const int64_t rows = std::min<int64_t>((n + per_block - 1) / per_block, kAdjRows);
+  qj_status st = ensure_partials(ws, rows * K, s);
   if (st) return st;
-  double* sums = ws->d_partials + nblocks * K;
   if (n > 0) {
-    if (prec == QJ_FP64)
-      hipLaunchKernelGGL(k_adjoint<double>, dim3((unsigned)nblocks), dim3(kAdjBlock), lds, s, a, f->d64, d_pts, n,
-                         d_dJdF, ws->d_partials, K);
-    else
-      hipLaunchKernelGGL(k_adjoint<float>, dim3((unsigned)nblocks), dim3(kAdjBlock), lds, s, a, f->d64, d_pts, n,
-                         d_dJdF, ws->d_partials, K);
+    hipLaunchKernelGGL(adjoint_kernel(prec, L, a.gen != 0), dim3((unsigned)rows), dim3(kAdjBlock), lds, s, a, f->d64,
+                       d_pts, n, d_dJdF, ws->d_partials, K);
     QJ_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_sum_partials, dim3(K), dim3(kSumThreads), 0, s, ws->d_partials, nblocks, K, sums);
-    QJ_HIP(hipGetLastError());
-  } else {
-    QJ_HIP(hipMemsetAsync(sums, 0, sizeof(double) * K, s));
   }
-  hipLaunchKernelGGL(k_adjoint_finish, dim3((K + 127) / 128), dim3(128), 0, s, sums, (int64_t)1, a.nt, nr,
+  hipLaunchKernelGGL(k_adjoint_finish, dim3(K), dim3(kSumThreads), 0, s, (const double*)ws->d_partials, rows, a.nt, nr,
                      a.sc_top, a.sc_bottom, d_gr, d_gp);
   QJ_HIP(hipGetLastError());
   return QJ_OK;
