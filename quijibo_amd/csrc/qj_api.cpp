@@ -234,6 +234,18 @@ void pack_roots32(const RootRec32* rec, int nt, int nb, std::vector<uint8_t>& bl
   }
 }
 
+// The device block of a rational function as it is copied: the FP64 records
+// (48 bytes each, so the block after them stays 16-byte aligned), then the
+// FP32 root block.
+static void stage_roots(qj_rational* f) {
+  std::vector<uint8_t> blk;
+  pack_roots32(f->h32.data(), f->nt, f->nb, blk);
+  const size_t n64 = sizeof(RootRec64) * f->h64.size();
+  f->stage.resize(n64 + blk.size());
+  memcpy(f->stage.data(), f->h64.data(), n64);
+  memcpy(f->stage.data() + n64, blk.data(), blk.size());
+}
+
 }  // namespace qj
 
 using namespace qj;
@@ -286,19 +298,17 @@ qj_status qj_rational_create(const qj_poly* top, const qj_poly* bottom, qj_ratio
   f->sc_bottom = bottom->power_scalar;
   fill_records(top, f->h64, f->h32);
   fill_records(bottom, f->h64, f->h32);
-  pack_roots32(f->h32.data(), f->nt, f->nb, f->blk32);
+  stage_roots(f);
   hipGetDevice(&f->device);
-  const size_t n = f->h64.size();
-  hipError_t e = hipMalloc(&f->d64, sizeof(RootRec64) * n);
-  if (e == hipSuccess) e = hipMalloc(&f->d32, f->blk32.size());
-  if (e == hipSuccess) e = hipMemcpy(f->d64, f->h64.data(), sizeof(RootRec64) * n, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(f->d32, f->blk32.data(), f->blk32.size(), hipMemcpyHostToDevice);
+  // one block: the FP64 records, then the FP32 roots
+  hipError_t e = hipMalloc((void**)&f->d64, f->stage.size());
+  if (e == hipSuccess) e = hipMemcpy(f->d64, f->stage.data(), f->stage.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     hipFree(f->d64);
-    hipFree(f->d32);
     delete f;
     return hip_fail(e, "qj_rational_create");
   }
+  f->d32 = f->d64 + f->h64.size();
   *out = f;
   return QJ_OK;
 }
@@ -325,10 +335,8 @@ qj_status qj_rational_update(qj_rational* f, const qj_poly* top, const qj_poly* 
   f->sc_bottom = bottom->power_scalar;
   fill_records(top, f->h64, f->h32);
   fill_records(bottom, f->h64, f->h32);
-  pack_roots32(f->h32.data(), f->nt, f->nb, f->blk32);
-  const size_t n = f->h64.size();
-  QJ_HIP(hipMemcpyAsync(f->d64, f->h64.data(), sizeof(RootRec64) * n, hipMemcpyHostToDevice, s));
-  QJ_HIP(hipMemcpyAsync(f->d32, f->blk32.data(), f->blk32.size(), hipMemcpyHostToDevice, s));
+  stage_roots(f);
+  QJ_HIP(hipMemcpyAsync(f->d64, f->stage.data(), f->stage.size(), hipMemcpyHostToDevice, s));
   return QJ_OK;
 }
 
@@ -342,7 +350,6 @@ qj_status qj_rational_counts(const qj_rational* f, int32_t* n_top, int32_t* n_bo
 qj_status qj_rational_destroy(qj_rational* f) {
   if (!f) return QJ_OK;
   hipFree(f->d64);
-  hipFree(f->d32);
   delete f;
   return QJ_OK;
 }

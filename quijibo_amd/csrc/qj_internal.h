@@ -52,11 +52,11 @@ struct GridGeom {
 struct qj_rational {
   int32_t nt = 0, nb = 0;
   double sc_top = 1, sc_bottom = 1;
-  qj::RootRec64* d64 = nullptr;
-  void* d32 = nullptr;  // FP32 root block (roots32_view)
+  qj::RootRec64* d64 = nullptr;  // the device block: FP64 records, then the FP32 root block
+  void* d32 = nullptr;           // FP32 root block (roots32_view), inside d64's
   std::vector<qj::RootRec64> h64;
   std::vector<qj::RootRec32> h32;
-  std::vector<uint8_t> blk32;
+  std::vector<uint8_t> stage;  // the device block's host copy
   int device = 0;
 };
 

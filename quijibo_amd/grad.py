@@ -40,9 +40,13 @@ class JuliaField(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gF):
         (points,) = ctx.saved_tensors
-        g = torch.where(torch.isfinite(gF), gF, torch.zeros_like(gF))
+        g = torch.nan_to_num(gF, nan=0.0, posinf=0.0, neginf=0.0)
         gr, gp = api.points_adjoint(points, ctx.rational, ctx.params, g, ctx.precision)
         nt = ctx.nt
+        if gr.is_cuda and all(d.type == "cpu" for d in ctx.devices):
+            # one copy to the host (each waits for the stream) instead of one per gradient
+            both = torch.cat([gr.view(-1), gp]).cpu()
+            gr, gp = both[:gr.numel()].view(-1, 4), both[gr.numel():]
         outs = [gr[:nt], gp[:nt], gr[nt:], gp[nt:]]
         outs = [o.to(device=d, dtype=t) for o, d, t in zip(outs, ctx.devices, ctx.dtypes)]
         return (None, outs[0], outs[1], outs[2], outs[3], None, None, None, None, None)

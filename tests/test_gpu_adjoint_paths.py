@@ -67,6 +67,7 @@ def _reference(pts, tr, tp, br, bp, g, iters, c, escape):
     (8200, 5, 4, "real", 2),    # 4 lanes
     (8200, 17, 3, "int", 1),    # 8 lanes, one iteration
     (8200, 33, 32, "ones", 2),  # 16 lanes
+    (9, 410, 409, "ones", 1),   # the most roots: 96 KiB of LDS
 ])
 def test_adjoint_against_autograd(gpu, n, nt, nb, powers, iters):
     rng = np.random.default_rng(7 * n + nt)
