@@ -25,10 +25,11 @@
 // them into the mean, and the replacement.
 #include <math.h>
 
-#include <vector>
+#include <algorithm>
 
 #include "qj_geom.h"
 #include "qj_internal.h"
+#include "qj_math64.h"
 
 namespace qj {
 
@@ -107,6 +108,31 @@ __device__ Acc block_reduce(Acc a) {
   return Acc{{s_hi[0], s_lo[0]}, s_sp[0], s_ct[0]};
 }
 
+__device__ __forceinline__ void store_part(double* __restrict__ part, int64_t at, const Acc& a) {
+  double* p = part + 4 * at;
+  p[0] = a.s.hi;
+  p[1] = a.s.lo;
+  p[2] = a.special;
+  p[3] = a.count;
+}
+// the partials of one sum combined by one block, in a fixed order
+__device__ Acc combine(const double* __restrict__ part, int nparts) {
+  Acc a{{0.0, 0.0}, 0.0, 0.0};
+  for (int i = threadIdx.x; i < nparts; i += kOpsBlock) {
+    const double* p = part + 4 * (int64_t)i;
+    a = acc_add(a, Acc{{p[0], p[1]}, p[2], p[3]});
+  }
+  return block_reduce(a);
+}
+__device__ __forceinline__ double total_of(const Acc& a) {
+  return isfinite(a.special) ? a.s.hi + a.s.lo : a.special;
+}
+__device__ __forceinline__ void acc_value(Acc& a, double v) {
+  a.count += 1.0;
+  if (isfinite(v)) a.s = dd_add1(a.s, v);
+  else a.special += v;
+}
+
 template <bool kNan>
 __global__ __launch_bounds__(kOpsBlock) void k_mean_partials(const double* __restrict__ f, int64_t n,
                                                             double* __restrict__ part) {
@@ -114,35 +140,23 @@ __global__ __launch_bounds__(kOpsBlock) void k_mean_partials(const double* __res
   const int64_t stride = (int64_t)gridDim.x * kOpsBlock;
   for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
     const double v = f[i];
-    if (summed<kNan>(v)) {
-      a.count += 1.0;
-      if (isfinite(v)) a.s = dd_add1(a.s, v);
-      else a.special += v;
-    }
+    if (summed<kNan>(v)) acc_value(a, v);
   }
   a = block_reduce(a);
-  if (threadIdx.x == 0) {
-    double* p = part + 4 * (int64_t)blockIdx.x;
-    p[0] = a.s.hi;
-    p[1] = a.s.lo;
-    p[2] = a.special;
-    p[3] = a.count;
-  }
+  if (threadIdx.x == 0) store_part(part, blockIdx.x, a);
 }
 
-// one block: combine the partials, write [mean, count] after them
-__global__ __launch_bounds__(kOpsBlock) void k_mean_final(double* __restrict__ part, int nparts) {
-  Acc a{{0.0, 0.0}, 0.0, 0.0};
-  for (int i = threadIdx.x; i < nparts; i += kOpsBlock) {
-    const double* p = part + 4 * (int64_t)i;
-    a = acc_add(a, Acc{{p[0], p[1]}, p[2], p[3]});
-  }
-  a = block_reduce(a);
+// one block: combine the partials, write [mean, count] after them (and the
+// mean to pinned host memory when the caller reads it)
+__global__ __launch_bounds__(kOpsBlock) void k_mean_final(double* __restrict__ part, int nparts,
+                                                          double* __restrict__ h_mean) {
+  const Acc a = combine(part, nparts);
   if (threadIdx.x == 0) {
     // Real mean = sum / nonInfsSeen: 0 / 0 is NaN when no cell is summed
-    const double total = isfinite(a.special) ? a.s.hi + a.s.lo : a.special;
-    part[4 * (int64_t)nparts] = total / a.count;
+    const double mean = total_of(a) / a.count;
+    part[4 * (int64_t)nparts] = mean;
     part[4 * (int64_t)nparts + 1] = a.count;
+    if (h_mean) *h_mean = mean;
   }
 }
 
@@ -189,13 +203,11 @@ __global__ __launch_bounds__(kOpsBlock) void k_set_borders(double* __restrict__ 
 
 // ---------------------------------------------------------------- scoring fields of the shape optimizer
 
-// outerShell + innerShell (FIELD_3D.cpp:5070-5145): 1 where the cell has a
+// outerShell + innerShell (FIELD_3D.cpp:5070-5145): whether the cell has a
 // 26-neighbour of the other sign (cells at 0 have none)
-__global__ __launch_bounds__(kOpsBlock) void k_shells(const double* __restrict__ d, int64_t X, int64_t Y, int64_t Z,
-                                                      double* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x, XY = X * Y;
-  if (i >= XY * Z) return;
-  const int64_t z = i / XY, r = i - z * XY, y = r / X, x = r - y * X;
+__device__ __forceinline__ bool shell_cell(const double* __restrict__ d, int64_t i, int64_t x, int64_t y, int64_t z,
+                                           int64_t X, int64_t Y, int64_t Z) {
+  const int64_t XY = X * Y;
   const double c = d[i];
   bool flip = false;
   for (int k = -1; k <= 1; k++)
@@ -206,132 +218,259 @@ __global__ __launch_bounds__(kOpsBlock) void k_shells(const double* __restrict__
         if (xn < 0 || xn > X - 1 || yn < 0 || yn > Y - 1 || zn < 0 || zn > Z - 1) continue;
         if (d[xn + yn * X + zn * XY] * c < 0) flip = true;
       }
-  out[i] = flip ? 1.0 : 0.0;
+  return flip;
 }
 
-// One sweep of invertedDistance's layer numbering (FIELD_3D.cpp:5248-5283):
-// every cell at or below 1e-5 in `in` takes 1 + its smallest 6-neighbour
-// above 1e-5, written to `out` (the sweep reads only the previous one, so the
-// result does not depend on the order of the cells). cnt[0] counts the cells
-// still at or below 1e-5 before the sweep, cnt[1] those the sweep numbered.
-__global__ __launch_bounds__(kOpsBlock) void k_relax(const double* __restrict__ in, int64_t X, int64_t Y, int64_t Z,
-                                                     double* __restrict__ out, unsigned long long* __restrict__ cnt) {
-  __shared__ unsigned s_zero[kOpsBlock / 64], s_upd[kOpsBlock / 64];
-  const int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x, XY = X * Y, n = XY * Z;
-  bool zero = false, upd = false;
-  if (i < n) {
-    const double v = in[i];
-    double w = v;
-    if (!(v > 1e-5)) {
-      zero = true;
-      const int64_t z = i / XY, r = i - z * XY, y = r / X, x = r - y * X;
-      double nb[6];
-      nb[0] = (x != 0) ? in[i - 1] : 0;
-      nb[1] = (x != X - 1) ? in[i + 1] : 0;
-      nb[2] = (y != 0) ? in[i - X] : 0;
-      nb[3] = (y != Y - 1) ? in[i + X] : 0;
-      nb[4] = (z != 0) ? in[i - XY] : 0;
-      nb[5] = (z != Z - 1) ? in[i + XY] : 0;
-      double biggest = (double)n + 1;
-      for (int k = 0; k < 6; k++)
-        if (nb[k] > 1e-5 && nb[k] < biggest) biggest = nb[k];
-      if (biggest < (double)n) {
-        w = biggest + 1;
-        upd = true;
+// The layer numbers of invertedDistance (FIELD_3D.cpp:5248-5283: shell cells 1,
+// then sweep after sweep every unnumbered cell 1 + its smallest 6-neighbour)
+// are 1 + the taxicab distance to the nearest shell cell, and that distance is
+// separable: one pass per axis, each the minimum over the line of value +
+// distance along it. (The sweeps took one launch, one counter read-back and
+// one wait each, about half the grid's edge of them: 50^3 25 sweeps, 1.5 ms.)
+// A block takes kLines lines of one axis; the minimum over a line of n cells by
+// doubling, v[i] = min(v[i], v[i - d] + d, v[i + d] + d) for d = 1, 2, 4, ... < n,
+// between two LDS copies. Lines of neighbouring x are taken together along y and
+// z, so that loads stay in runs of 64 B. The x pass starts from the shells; the
+// z pass writes the inverted, signed value (FIELD_3D.cpp:5286-5296: 1 / number,
+// negated inside and quartered outside) and the partial sums of its absolute
+// value; part's last entry counts the cells no shell reaches. Latency bound:
+// 50^3, 157 blocks a pass: 21.5 us along x (26 neighbours per cell for the
+// shells), 7.4 along y, 9.1 along z.
+constexpr int kLines = 16, kMaxLine = 512;
+constexpr uint32_t kFar = 0x3fffffffu;  // no shell cell on the lines so far
+enum LineAxis { kAxisX = 0, kAxisY = 1, kAxisZ = 2 };
+
+__device__ __forceinline__ double inverted_value(uint32_t layers, double dist) {
+  double x = 1.0 / ((double)layers + 1.0);
+  if (dist < 0) x *= -1;
+  else x *= 0.25;
+  return x;
+}
+
+template <int kAxis>
+__global__ __launch_bounds__(kOpsBlock) void k_layers(const double* __restrict__ d, int64_t X, int64_t Y, int64_t Z,
+                                                      uint32_t* __restrict__ lay, double* __restrict__ out,
+                                                      double* __restrict__ part) {
+  extern __shared__ uint32_t s_v[];  // 2 x n x kLines
+  const int64_t XY = X * Y;
+  const int n = (int)(kAxis == kAxisX ? X : kAxis == kAxisY ? Y : Z);
+  // the block's lines: consecutive rows (x), consecutive x of one z (y), consecutive x + y X (z)
+  const int64_t per = kAxis == kAxisX ? Y * Z : kAxis == kAxisY ? X : XY;
+  const int64_t groups = (per + kLines - 1) / kLines;
+  const int64_t outer = blockIdx.x / groups, l0 = (blockIdx.x - outer * groups) * kLines;
+  const int lines = (int)(per - l0 < kLines ? per - l0 : kLines);
+  uint32_t *cur = s_v, *nxt = s_v + n * kLines;
+  const int total = n * kLines;
+  // element e: line e / n of a row block (x: memory order), else position e / kLines of line e % kLines
+  auto place = [&](int e, int& line, int& pos, int64_t& at) {
+    if (kAxis == kAxisX) {
+      line = e / n;
+      pos = e - line * n;
+      at = (l0 + line) * X + pos;
+    } else {
+      line = e % kLines;
+      pos = e / kLines;
+      at = kAxis == kAxisY ? outer * XY + pos * X + l0 + line : pos * XY + l0 + line;
+    }
+  };
+  for (int e = threadIdx.x; e < total; e += kOpsBlock) {
+    int line, pos;
+    int64_t at;
+    place(e, line, pos, at);
+    uint32_t v = kFar;
+    if (line < lines) {
+      if (kAxis == kAxisX) {
+        const int64_t row = l0 + line, z = row / Y;
+        v = shell_cell(d, at, pos, row - z * Y, z, X, Y, Z) ? 0u : kFar;
+      } else {
+        v = lay[at];
       }
     }
-    out[i] = w;
-  }
-  const unsigned long long mz = __ballot(zero), mu = __ballot(upd);
-  if ((threadIdx.x & 63) == 0) {
-    s_zero[threadIdx.x >> 6] = (unsigned)__popcll(mz);
-    s_upd[threadIdx.x >> 6] = (unsigned)__popcll(mu);
+    cur[pos * kLines + line] = v;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long a = 0, b = 0;
-    for (int k = 0; k < kOpsBlock / 64; k++) {
-      a += s_zero[k];
-      b += s_upd[k];
+  for (int step = 1; step < n; step *= 2) {
+    for (int e = threadIdx.x; e < total; e += kOpsBlock) {
+      const int pos = e / kLines;
+      uint32_t v = cur[e];
+      if (pos >= step) v = min(v, cur[e - step * kLines] + step);
+      if (pos + step < n) v = min(v, cur[e + step * kLines] + step);
+      nxt[e] = v;
     }
-    if (a) atomicAdd(&cnt[0], a);
-    if (b) atomicAdd(&cnt[1], b);
+    __syncthreads();
+    uint32_t* t = cur;
+    cur = nxt;
+    nxt = t;
+  }
+  Acc a{{0.0, 0.0}, 0.0, 0.0};
+  unsigned far = 0;
+  for (int e = threadIdx.x; e < total; e += kOpsBlock) {
+    int line, pos;
+    int64_t at;
+    place(e, line, pos, at);
+    if (line >= lines) continue;
+    const uint32_t v = cur[pos * kLines + line];
+    if (kAxis != kAxisZ) {
+      lay[at] = v < kFar ? v : kFar;
+    } else {
+      far += v >= kFar;
+      const double x = inverted_value(v, d[at]);
+      out[at] = x;
+      acc_value(a, fabs(x));
+    }
+  }
+  if (kAxis == kAxisZ) {
+    a.count = (double)far;  // what the partial carries here: the cells without a number
+    a = block_reduce(a);
+    if (threadIdx.x == 0) store_part(part, blockIdx.x, a);
   }
 }
 
-// 1 / value, negated inside (distance < 0) and quartered outside (FIELD_3D.cpp:5286-5296)
-__global__ __launch_bounds__(kOpsBlock) void k_invert_signed(double* __restrict__ v, const double* __restrict__ d,
-                                                             int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x;
-  if (i >= n) return;
-  double x = 1.0 / v[i];
-  if (d[i] < 0) x *= -1;
-  else x *= 0.25;
-  v[i] = x;
+// The same passes for lines beyond kMaxLine cells (their two LDS copies would
+// not fit): one line per thread, forward and back.
+template <int kAxis>
+__global__ __launch_bounds__(kOpsBlock) void k_layers_long(const double* __restrict__ d, int64_t X, int64_t Y,
+                                                           int64_t Z, uint32_t* __restrict__ lay,
+                                                           double* __restrict__ out, double* __restrict__ part) {
+  const int64_t XY = X * Y, n = kAxis == kAxisX ? X : kAxis == kAxisY ? Y : Z;
+  const int64_t stride = kAxis == kAxisX ? 1 : kAxis == kAxisY ? X : XY;
+  const int64_t count = XY * Z / n, l = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x;
+  Acc a{{0.0, 0.0}, 0.0, 0.0};
+  if (l < count) {
+    const int64_t first = kAxis == kAxisX ? l * X : kAxis == kAxisY ? (l / X) * XY + l % X : l;
+    uint32_t v = kFar;
+    for (int64_t p = 0; p < n; p++) {
+      const int64_t at = first + p * stride;
+      const uint32_t own = kAxis == kAxisX ? (shell_cell(d, at, p, l % Y, l / Y, X, Y, Z) ? 0u : kFar) : lay[at];
+      v = min(own, v < kFar ? v + 1 : kFar);
+      lay[at] = v;
+    }
+    double far = 0.0;
+    for (int64_t p = n - 1; p >= 0; p--) {
+      const int64_t at = first + p * stride;
+      v = min(lay[at], v < kFar ? v + 1 : kFar);
+      if (kAxis != kAxisZ) {
+        lay[at] = v;
+      } else {
+        far += v >= kFar;
+        const double x = inverted_value(v, d[at]);
+        out[at] = x;
+        acc_value(a, fabs(x));
+      }
+    }
+    a.count = far;
+  }
+  if (kAxis == kAxisZ) {
+    a = block_reduce(a);
+    if (threadIdx.x == 0) store_part(part, blockIdx.x, a);
+  }
 }
 
-// partial sums (double-double) of |v| (mode 0), of v where d < 0 (mode 1),
-// of v where d >= 0 (mode 2)
-__global__ __launch_bounds__(kOpsBlock) void k_masked_sum(const double* __restrict__ v, const double* __restrict__ d,
-                                                          int64_t n, int mode, double* __restrict__ part) {
-  Acc a{{0.0, 0.0}, 0.0, 0.0};
+// invertedDistanceNormalized's passes (FIELD_3D.cpp:5316-5352), each with the
+// sums the next one needs: kStage 0 scales by 1 / the absolute sum and sums the
+// inside and the outside (two partials per block), 1 scales those to absolute
+// sum 0.5 each and sums absolute values. scal: what k_fold_sums left.
+template <int kStage>
+__global__ __launch_bounds__(kOpsBlock) void k_normalize(double* __restrict__ v, const double* __restrict__ d,
+                                                         int64_t n, const double* __restrict__ scal,
+                                                         double* __restrict__ part) {
+  Acc a{{0.0, 0.0}, 0.0, 0.0}, b = a;
+  const double s_in = kStage == 0 ? 1.0 / scal[0] : 0.5 / fabs(scal[0]);
+  const double s_out = kStage == 0 ? s_in : 0.5 / fabs(scal[1]);
   const int64_t stride = (int64_t)gridDim.x * kOpsBlock;
   for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
-    const double x = v[i];
-    if (mode == 1 && !(d[i] < 0)) continue;
-    if (mode == 2 && (d[i] < 0)) continue;
-    const double y = mode == 0 ? fabs(x) : x;
-    a.count += 1.0;
-    if (isfinite(y)) a.s = dd_add1(a.s, y);
-    else a.special += y;
+    const bool inside = d[i] < 0;
+    const double x = v[i] * (inside ? s_in : s_out);
+    v[i] = x;
+    if (kStage == 0) acc_value(inside ? a : b, x);
+    else acc_value(a, fabs(x));
   }
   a = block_reduce(a);
-  if (threadIdx.x == 0) {
-    double* p = part + 4 * (int64_t)blockIdx.x;
-    p[0] = a.s.hi;
-    p[1] = a.s.lo;
-    p[2] = a.special;
-    p[3] = a.count;
+  if (threadIdx.x == 0) store_part(part, blockIdx.x, a);
+  if (kStage == 0) {
+    __syncthreads();
+    b = block_reduce(b);
+    if (threadIdx.x == 0) store_part(part, (int64_t)gridDim.x + blockIdx.x, b);
   }
 }
 
-// v *= inside-scale where d < 0, outside-scale elsewhere
-__global__ __launch_bounds__(kOpsBlock) void k_scale_by_sign(double* __restrict__ v, const double* __restrict__ d,
-                                                             int64_t n, double s_in, double s_out) {
-  const int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x;
-  if (i >= n) return;
-  v[i] *= (d[i] < 0) ? s_in : s_out;
+// Block b: the total of partials [b nparts, (b + 1) nparts) to d_out[b] and,
+// with h_out, to pinned host memory; count0: the first one's count there too.
+__global__ __launch_bounds__(kOpsBlock) void k_fold_sums(const double* __restrict__ part, int nparts,
+                                                         double* __restrict__ d_out, double* __restrict__ h_out,
+                                                         double* __restrict__ h_count) {
+  const Acc a = combine(part + 4 * (int64_t)blockIdx.x * nparts, nparts);
+  if (threadIdx.x == 0) {
+    const double t = total_of(a);
+    if (d_out) d_out[blockIdx.x] = t;
+    if (h_out) h_out[blockIdx.x] = t;
+    if (h_count && blockIdx.x == 0) *h_count = a.count;
+  }
 }
 
-// weightScore / inverseDistanceScore (OPTIMIZE_3D.cpp:4502-4563) for threshold
-// blockIdx.y: -tanh(alpha (F - threshold)) w(cell centre); the block for the
-// last threshold slot also sums |w| (computeMaximumScaledPowerRationalScore,
-// :4484-4498). w is the trilinear lookup of the weight field.
-__global__ __launch_bounds__(kOpsBlock) void k_weight_score(const double* __restrict__ f, GridGeom g, GridGeom wg,
-                                                            const double* __restrict__ w,
-                                                            const double* __restrict__ thresholds, int nthr,
-                                                            double alpha, double* __restrict__ part) {
+// The weight at every cell centre (the trilinear lookup) and the partial sums of
+// its absolute value: once per call, where the score kernel repeated both for
+// every threshold.
+__global__ __launch_bounds__(kOpsBlock) void k_cell_weights(GridGeom g, GridGeom wg, const double* __restrict__ w,
+                                                            double* __restrict__ out, double* __restrict__ part) {
   const int64_t n = (int64_t)g.res[0] * g.res[1] * g.res[2], X = g.res[0], XY = X * g.res[1];
-  const int t = blockIdx.y;
+  const bool small = n <= (int64_t)0xffffffffll;
   Acc a{{0.0, 0.0}, 0.0, 0.0};
   const int64_t stride = (int64_t)gridDim.x * kOpsBlock;
   for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
-    const int64_t z = i / XY, r = i - z * XY, y = r / X, x = r - y * X;
+    int64_t x, y, z;
+    if (small) {
+      const uint32_t p = (uint32_t)i, zu = fast_div(p, g.div_xy), r = p - zu * (uint32_t)XY;
+      const uint32_t yu = fast_div(r, g.div_x);
+      z = zu;
+      y = yu;
+      x = r - yu * (uint32_t)X;
+    } else {
+      z = i / XY;
+      const int64_t r = i - z * XY;
+      y = r / X;
+      x = r - y * X;
+    }
     double c[3];
     cell_center(g, (int)x, (int)y, (int)z, c);
     const double wt = field_lookup(wg, w, c);
-    const double v = t < nthr ? -tanh(alpha * (f[i] - thresholds[t])) * wt : fabs(wt);
-    a.count += 1.0;
-    if (isfinite(v)) a.s = dd_add1(a.s, v);
-    else a.special += v;
+    out[i] = wt;
+    acc_value(a, fabs(wt));
   }
   a = block_reduce(a);
-  if (threadIdx.x == 0) {
-    double* p = part + 4 * ((int64_t)t * gridDim.x + blockIdx.x);
-    p[0] = a.s.hi;
-    p[1] = a.s.lo;
-    p[2] = a.special;
-    p[3] = a.count;
+  if (threadIdx.x == 0) store_part(part, blockIdx.x, a);
+}
+
+// weightScore / inverseDistanceScore (OPTIMIZE_3D.cpp:4502-4563) for kScores
+// thresholds from blockIdx.y kScores on: the partial sums of
+// -tanh(alpha (F - threshold)) w(cell centre). FP64 VALU bound (the tanh); the
+// field and the cells' weights are read once per kScores thresholds. 50^3, 100
+// thresholds: 41 us; one threshold per block with the lookup and the library's
+// tanh 169 us, this split with the library's tanh 67 us.
+constexpr int kScores = 4;
+__global__ __launch_bounds__(kOpsBlock) void k_weight_score(const double* __restrict__ f,
+                                                            const double* __restrict__ cw, int64_t n,
+                                                            const double* __restrict__ thresholds, int nthr,
+                                                            double alpha, double* __restrict__ part) {
+  const int t0 = blockIdx.y * kScores;
+  Acc a[kScores];
+  double thr[kScores];
+#pragma unroll
+  for (int k = 0; k < kScores; k++) {
+    a[k] = Acc{{0.0, 0.0}, 0.0, 0.0};
+    thr[k] = thresholds[t0 + k < nthr ? t0 + k : nthr - 1];
+  }
+  const int64_t stride = (int64_t)gridDim.x * kOpsBlock;
+  for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
+    const double F = f[i], w = cw[i];
+#pragma unroll
+    for (int k = 0; k < kScores; k++) acc_value(a[k], -tanh64(alpha * (F - thr[k])) * w);
+  }
+#pragma unroll
+  for (int k = 0; k < kScores; k++) {
+    const Acc s = block_reduce(a[k]);
+    if (threadIdx.x == 0 && t0 + k < nthr) store_part(part, (int64_t)(t0 + k) * gridDim.x + blockIdx.x, s);
+    __syncthreads();
   }
 }
 
@@ -355,18 +494,8 @@ __device__ __forceinline__ VI vi_max(VI a, VI b) {
   return (b.v > a.v || (b.v == a.v && b.i < a.i)) ? b : a;
 }
 
-__global__ __launch_bounds__(kOpsBlock) void k_min_max(const double* __restrict__ f, int64_t n,
-                                                       double* __restrict__ part) {
-  __shared__ double s_v[2][kOpsBlock];
-  __shared__ int64_t s_i[2][kOpsBlock];
-  VI mn{0.0, -1}, mx{0.0, -1};
-  const int64_t stride = (int64_t)gridDim.x * kOpsBlock;
-  for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
-    const double v = f[i];
-    if (isnan(v)) continue;
-    mn = vi_min(mn, VI{v, i});
-    mx = vi_max(mx, VI{v, i});
-  }
+// the block's extrema in thread 0's mn and mx
+__device__ void extrema_reduce(VI& mn, VI& mx, double (*s_v)[kOpsBlock], int64_t (*s_i)[kOpsBlock]) {
   const int t = threadIdx.x;
   s_v[0][t] = mn.v;
   s_i[0][t] = mn.i;
@@ -384,27 +513,50 @@ __global__ __launch_bounds__(kOpsBlock) void k_min_max(const double* __restrict_
     }
     __syncthreads();
   }
-  if (t == 0) {
+  mn = VI{s_v[0][0], s_i[0][0]};
+  mx = VI{s_v[1][0], s_i[1][0]};
+}
+
+__global__ __launch_bounds__(kOpsBlock) void k_min_max(const double* __restrict__ f, int64_t n,
+                                                       double* __restrict__ part) {
+  __shared__ double s_v[2][kOpsBlock];
+  __shared__ int64_t s_i[2][kOpsBlock];
+  VI mn{0.0, -1}, mx{0.0, -1};
+  const int64_t stride = (int64_t)gridDim.x * kOpsBlock;
+  for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
+    const double v = f[i];
+    if (isnan(v)) continue;
+    mn = vi_min(mn, VI{v, i});
+    mx = vi_max(mx, VI{v, i});
+  }
+  extrema_reduce(mn, mx, s_v, s_i);
+  if (threadIdx.x == 0) {
     double* p = part + 4 * (int64_t)blockIdx.x;
-    p[0] = s_v[0][0];
-    p[1] = (double)s_i[0][0];  // exact: indexes stay below 2^53
-    p[2] = s_v[1][0];
-    p[3] = (double)s_i[1][0];
+    p[0] = mn.v;
+    p[1] = (double)mn.i;  // exact: indexes stay below 2^53
+    p[2] = mx.v;
+    p[3] = (double)mx.i;
   }
 }
 
-// host: the sum of nparts partials (4 doubles each) read back
-static double host_sum(const std::vector<double>& p, int64_t first, int64_t nparts) {
-  double hi = 0, lo = 0, special = 0;
-  for (int64_t k = first; k < first + nparts; k++) {
-    // two-sum on the host too, so the total stays the correctly rounded sum
-    const double a = p[4 * k], b = p[4 * k + 1];
-    double s = hi + a, bb = s - hi, e = (hi - (s - bb)) + (a - bb);
-    lo += e + b;
-    hi = s;
-    special += p[4 * k + 2];
+// one block: the extrema of the blocks' extrema, to pinned host memory. A NaN
+// in cell 0 makes both NaN (nothing compares against a NaN start).
+__global__ __launch_bounds__(kOpsBlock) void k_min_max_final(const double* __restrict__ part, int nparts,
+                                                             const double* __restrict__ f, double* __restrict__ h) {
+  __shared__ double s_v[2][kOpsBlock];
+  __shared__ int64_t s_i[2][kOpsBlock];
+  VI mn{0.0, -1}, mx{0.0, -1};
+  for (int i = threadIdx.x; i < nparts; i += kOpsBlock) {
+    const double* p = part + 4 * (int64_t)i;
+    mn = vi_min(mn, VI{p[0], (int64_t)p[1]});
+    mx = vi_max(mx, VI{p[2], (int64_t)p[3]});
   }
-  return isfinite(special) ? hi + lo : special;
+  extrema_reduce(mn, mx, s_v, s_i);
+  if (threadIdx.x == 0) {
+    const bool nan = isnan(f[0]);
+    h[0] = nan ? f[0] : mn.v;
+    h[1] = nan ? f[0] : mx.v;
+  }
 }
 
 }  // namespace
@@ -422,15 +574,17 @@ qj_status field_clamp_to_mean(qj_workspace* ws, double* d_field, int64_t n, bool
   if (nans) hipLaunchKernelGGL(k_mean_partials<true>, dim3(grid), dim3(kOpsBlock), 0, s, d_field, n, ws->d_partials);
   else hipLaunchKernelGGL(k_mean_partials<false>, dim3(grid), dim3(kOpsBlock), 0, s, d_field, n, ws->d_partials);
   QJ_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_mean_final, dim3(1), dim3(kOpsBlock), 0, s, ws->d_partials, grid);
+  if (mean_out && (st = ensure_pinned(ws, 1, s))) return st;
+  hipLaunchKernelGGL(k_mean_final, dim3(1), dim3(kOpsBlock), 0, s, ws->d_partials, grid,
+                     mean_out ? ws->h_pinned : (double*)nullptr);
   QJ_HIP(hipGetLastError());
   const double* mean_at = ws->d_partials + 4 * (int64_t)grid;
   if (nans) hipLaunchKernelGGL(k_replace<true>, dim3(grid), dim3(kOpsBlock), 0, s, d_field, n, mean_at);
   else hipLaunchKernelGGL(k_replace<false>, dim3(grid), dim3(kOpsBlock), 0, s, d_field, n, mean_at);
   QJ_HIP(hipGetLastError());
   if (mean_out) {
-    QJ_HIP(hipMemcpyAsync(mean_out, mean_at, sizeof(double), hipMemcpyDeviceToHost, s));
     QJ_HIP(hipStreamSynchronize(s));
+    *mean_out = ws->h_pinned[0];
   }
   return QJ_OK;
 }
@@ -449,74 +603,90 @@ qj_status field_set_borders(const int32_t* res, double value, double* d_field, h
 
 namespace qj {
 
+// Per-cell scratch of a call: kept in the workspace up to kKeepCells cells
+// (128 MiB), a temporary of the call beyond, so that one call on a huge grid
+// does not hold its memory.
+constexpr int64_t kKeepCells = int64_t(1) << 24;
+struct CellScratch {
+  void* p = nullptr;
+  bool own = false;
+  ~CellScratch() {
+    if (own) (void)hipFree(p);
+  }
+};
+
+template <int kAxis>
+static qj_status launch_layers(const double* d, int64_t X, int64_t Y, int64_t Z, uint32_t* lay, double* out,
+                               double* part, int64_t* blocks, hipStream_t s) {
+  const int64_t n = kAxis == kAxisX ? X : kAxis == kAxisY ? Y : Z, lines = X * Y * Z / n;
+  if (n <= kMaxLine) {
+    const int64_t per = kAxis == kAxisY ? X : lines, outer = kAxis == kAxisY ? Z : 1;
+    *blocks = outer * ((per + kLines - 1) / kLines);
+    if (*blocks > INT32_MAX) return QJ_ERR_CAPACITY;
+    hipLaunchKernelGGL(k_layers<kAxis>, dim3((unsigned)*blocks), dim3(kOpsBlock),
+                       2 * sizeof(uint32_t) * kLines * (size_t)n, s, d, X, Y, Z, lay, out, part);
+  } else {
+    *blocks = (lines + kOpsBlock - 1) / kOpsBlock;
+    if (*blocks > INT32_MAX) return QJ_ERR_CAPACITY;
+    hipLaunchKernelGGL(k_layers_long<kAxis>, dim3((unsigned)*blocks), dim3(kOpsBlock), 0, s, d, X, Y, Z, lay, out,
+                       part);
+  }
+  QJ_HIP(hipGetLastError());
+  return QJ_OK;
+}
+
+// Three layer passes, then (normalized) two scaling passes, every sum folded on
+// the device: one wait at the end.
 qj_status field_inverted_distance(qj_workspace* ws, const double* d_dist, const qj_grid* grid, bool normalized,
                                   double* d_out, double* abs_sum, hipStream_t s) {
   const int64_t X = grid->res[0], Y = grid->res[1], Z = grid->res[2], n = X * Y * Z;
   if (n <= 0) return QJ_OK;
-  const unsigned nb = (unsigned)((n + kOpsBlock - 1) / kOpsBlock);
-  double* tmp = nullptr;
-  unsigned long long* cnt = nullptr;
-  QJ_HIP(hipMalloc(&tmp, sizeof(double) * (size_t)n));
-  struct Free {
-    void* a;
-    void* b;
-    ~Free() {
-      (void)hipFree(a);
-      (void)hipFree(b);
-    }
-  } guard{tmp, nullptr};
-  QJ_HIP(hipMalloc(&cnt, 2 * sizeof(unsigned long long)));
-  guard.b = cnt;
-  hipLaunchKernelGGL(k_shells, dim3(nb), dim3(kOpsBlock), 0, s, d_dist, X, Y, Z, d_out);
-  QJ_HIP(hipGetLastError());
-  // sweeps until no cell is left at or below 1e-5; a sweep that numbers no
-  // cell while some remain would repeat forever in the reference
-  double* cur = d_out;
-  double* nxt = tmp;
-  for (;;) {
-    unsigned long long h[2] = {0, 0};
-    QJ_HIP(hipMemsetAsync(cnt, 0, 2 * sizeof(unsigned long long), s));
-    hipLaunchKernelGGL(k_relax, dim3(nb), dim3(kOpsBlock), 0, s, (const double*)cur, X, Y, Z, nxt, cnt);
-    QJ_HIP(hipGetLastError());
-    QJ_HIP(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, s));
-    QJ_HIP(hipStreamSynchronize(s));
-    std::swap(cur, nxt);
-    if (h[0] == 0) break;
-    if (h[1] == 0) {
-      set_error("inverted distance: %llu cells can never be numbered (no surface reaches them)", h[0]);
-      return QJ_ERR_NUMERIC;
-    }
-  }
-  if (cur != d_out) QJ_HIP(hipMemcpyAsync(d_out, cur, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, s));
-  hipLaunchKernelGGL(k_invert_signed, dim3(nb), dim3(kOpsBlock), 0, s, d_out, d_dist, n);
-  QJ_HIP(hipGetLastError());
-  if (!normalized && !abs_sum) return QJ_OK;
-  qj_status st = ensure_partials(ws, 4 * (int64_t)kOpsGrid, s);
+  const int64_t zlines = X * Y;
+  const int64_t zblocks = Z <= kMaxLine ? (zlines + kLines - 1) / kLines : (zlines + kOpsBlock - 1) / kOpsBlock;
+  const int64_t want = (n + kOpsBlock - 1) / kOpsBlock;
+  const int grid_sum = (int)(want < kOpsGrid ? want : kOpsGrid);
+  const int64_t nparts = std::max<int64_t>(zblocks, 2 * (int64_t)grid_sum);
+  const bool keep = n <= kKeepCells;
+  qj_status st = ensure_partials(ws, 4 * nparts + 2 + (keep ? (n + 1) / 2 : 0), s);
   if (st) return st;
-  const int grid_sum = (int)(nb < (unsigned)kOpsGrid ? nb : kOpsGrid);
-  std::vector<double> part(4 * (size_t)grid_sum);
-  auto sum = [&](int mode, double* out) -> qj_status {
-    hipLaunchKernelGGL(k_masked_sum, dim3(grid_sum), dim3(kOpsBlock), 0, s, (const double*)d_out, d_dist, n, mode,
-                       ws->d_partials);
-    QJ_HIP(hipGetLastError());
-    QJ_HIP(hipMemcpyAsync(part.data(), ws->d_partials, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s));
-    QJ_HIP(hipStreamSynchronize(s));
-    *out = host_sum(part, 0, grid_sum);
-    return QJ_OK;
-  };
+  if ((st = ensure_pinned(ws, 2, s))) return st;
+  double* part = ws->d_partials;
+  double* scal = part + 4 * nparts;
+  CellScratch cells;
+  if (keep) cells.p = scal + 2;
+  else QJ_HIP(hipMalloc(&cells.p, sizeof(uint32_t) * (size_t)n));
+  cells.own = !keep;
+  uint32_t* lay = (uint32_t*)cells.p;
+  int64_t nb = 0;
+  if ((st = launch_layers<kAxisX>(d_dist, X, Y, Z, lay, d_out, part, &nb, s)) ||
+      (st = launch_layers<kAxisY>(d_dist, X, Y, Z, lay, d_out, part, &nb, s)) ||
+      (st = launch_layers<kAxisZ>(d_dist, X, Y, Z, lay, d_out, part, &nb, s)))
+    return st;
+  // h_pinned: [0] the absolute sum of the result, [1] the cells without a number
+  double* h = ws->h_pinned;
+  hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kOpsBlock), 0, s, (const double*)part, (int)nb, scal, h, h + 1);
+  QJ_HIP(hipGetLastError());
   if (normalized) {
-    // invertedDistanceNormalized (FIELD_3D.cpp:5316-5352)
-    double total = 0, inside = 0, outside = 0;
-    if ((st = sum(0, &total))) return st;
-    const double scale = 1.0 / total;
-    hipLaunchKernelGGL(k_scale_by_sign, dim3(nb), dim3(kOpsBlock), 0, s, d_out, d_dist, n, scale, scale);
+    hipLaunchKernelGGL(k_normalize<0>, dim3(grid_sum), dim3(kOpsBlock), 0, s, d_out, d_dist, n, (const double*)scal,
+                       part);
     QJ_HIP(hipGetLastError());
-    if ((st = sum(1, &inside)) || (st = sum(2, &outside))) return st;
-    hipLaunchKernelGGL(k_scale_by_sign, dim3(nb), dim3(kOpsBlock), 0, s, d_out, d_dist, n, 0.5 / fabs(inside),
-                       0.5 / fabs(outside));
+    hipLaunchKernelGGL(k_fold_sums, dim3(2), dim3(kOpsBlock), 0, s, (const double*)part, grid_sum, scal,
+                       (double*)nullptr, (double*)nullptr);
+    QJ_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_normalize<1>, dim3(grid_sum), dim3(kOpsBlock), 0, s, d_out, d_dist, n, (const double*)scal,
+                       part);
+    QJ_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kOpsBlock), 0, s, (const double*)part, grid_sum, (double*)nullptr, h,
+                       (double*)nullptr);
     QJ_HIP(hipGetLastError());
   }
-  if (abs_sum && (st = sum(0, abs_sum))) return st;
+  QJ_HIP(hipStreamSynchronize(s));
+  if (h[1] > 0.0) {
+    // a cell that no shell cell reaches: the reference's sweeps never end
+    set_error("inverted distance: %.0f cells can never be numbered (no surface reaches them)", h[1]);
+    return QJ_ERR_NUMERIC;
+  }
+  if (abs_sum) *abs_sum = h[0];
   return QJ_OK;
 }
 
@@ -526,33 +696,15 @@ qj_status field_min_max(qj_workspace* ws, const double* d_field, int64_t n, doub
   const int grid = (int)(want < kOpsGrid ? want : kOpsGrid);
   qj_status st = ensure_partials(ws, 4 * (int64_t)grid, s);
   if (st) return st;
+  if ((st = ensure_pinned(ws, 2, s))) return st;
   hipLaunchKernelGGL(k_min_max, dim3(grid), dim3(kOpsBlock), 0, s, d_field, n, ws->d_partials);
   QJ_HIP(hipGetLastError());
-  std::vector<double> part(4 * (size_t)grid);
-  double first = 0;
-  QJ_HIP(hipMemcpyAsync(part.data(), ws->d_partials, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s));
-  QJ_HIP(hipMemcpyAsync(&first, d_field, sizeof(double), hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_min_max_final, dim3(1), dim3(kOpsBlock), 0, s, (const double*)ws->d_partials, grid, d_field,
+                     ws->h_pinned);
+  QJ_HIP(hipGetLastError());
   QJ_HIP(hipStreamSynchronize(s));
-  if (isnan(first)) {  // nothing compares against a NaN start
-    *mn = *mx = first;
-    return QJ_OK;
-  }
-  double bv = 0, tv = 0;
-  int64_t bi = -1, ti = -1;
-  for (int b = 0; b < grid; b++) {
-    const int64_t i0 = (int64_t)part[4 * b + 1], i1 = (int64_t)part[4 * b + 3];
-    const double v0 = part[4 * b], v1 = part[4 * b + 2];
-    if (i0 >= 0 && (bi < 0 || v0 < bv || (v0 == bv && i0 < bi))) {
-      bv = v0;
-      bi = i0;
-    }
-    if (i1 >= 0 && (ti < 0 || v1 > tv || (v1 == tv && i1 < ti))) {
-      tv = v1;
-      ti = i1;
-    }
-  }
-  *mn = bv;
-  *mx = tv;
+  *mn = ws->h_pinned[0];
+  *mx = ws->h_pinned[1];
   return QJ_OK;
 }
 
@@ -567,18 +719,35 @@ qj_status weight_scores(qj_workspace* ws, const double* d_field, const qj_grid* 
   const int64_t want = (n + kOpsBlock - 1) / kOpsBlock;
   const int gx = (int)(want < 256 ? want : 256);
   const int slots = nthr + 1;
-  qj_status st = ensure_partials(ws, 4 * (int64_t)gx * slots + (int64_t)slots, s);
+  // the partials (the last slot's: the weights' absolute sum), the thresholds, the cells' weights
+  const bool keep = n <= kKeepCells;
+  qj_status st = ensure_partials(ws, 4 * (int64_t)gx * slots + (int64_t)slots + (keep ? n : 0), s);
   if (st) return st;
-  double* d_thr = ws->d_partials + 4 * (int64_t)gx * slots;
-  if (nthr) QJ_HIP(hipMemcpyAsync(d_thr, thresholds, sizeof(double) * (size_t)nthr, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_weight_score, dim3(gx, slots), dim3(kOpsBlock), 0, s, d_field, g, wg, d_weight,
-                     (const double*)d_thr, nthr, alpha, ws->d_partials);
+  if ((st = ensure_pinned(ws, 2 * (int64_t)slots, s))) return st;
+  double* part = ws->d_partials;
+  double* d_thr = part + 4 * (int64_t)gx * slots;
+  CellScratch cells;
+  if (keep) cells.p = d_thr + slots;
+  else QJ_HIP(hipMalloc(&cells.p, sizeof(double) * (size_t)n));
+  cells.own = !keep;
+  double* cw = (double*)cells.p;
+  hipLaunchKernelGGL(k_cell_weights, dim3(gx), dim3(kOpsBlock), 0, s, g, wg, d_weight, cw,
+                     part + 4 * (int64_t)gx * nthr);
   QJ_HIP(hipGetLastError());
-  std::vector<double> part(4 * (size_t)gx * slots);
-  QJ_HIP(hipMemcpyAsync(part.data(), ws->d_partials, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s));
+  if (nthr) {
+    double* h_thr = ws->h_pinned + slots;
+    for (int t = 0; t < nthr; t++) h_thr[t] = thresholds[t];
+    QJ_HIP(hipMemcpyAsync(d_thr, h_thr, sizeof(double) * (size_t)nthr, hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_weight_score, dim3(gx, (nthr + kScores - 1) / kScores), dim3(kOpsBlock), 0, s, d_field,
+                       (const double*)cw, n, (const double*)d_thr, nthr, alpha, part);
+    QJ_HIP(hipGetLastError());
+  }
+  hipLaunchKernelGGL(k_fold_sums, dim3(slots), dim3(kOpsBlock), 0, s, (const double*)part, gx, (double*)nullptr,
+                     ws->h_pinned, (double*)nullptr);
+  QJ_HIP(hipGetLastError());
   QJ_HIP(hipStreamSynchronize(s));
-  for (int t = 0; t < nthr; t++) scores[t] = host_sum(part, (int64_t)t * gx, gx);
-  if (max_score) *max_score = host_sum(part, (int64_t)nthr * gx, gx);
+  for (int t = 0; t < nthr; t++) scores[t] = ws->h_pinned[t];
+  if (max_score) *max_score = ws->h_pinned[nthr];
   return QJ_OK;
 }
 

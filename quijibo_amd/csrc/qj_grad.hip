@@ -514,8 +514,8 @@ __global__ __launch_bounds__(kApBlock) void k_ap_fast(APArgs g, const RootRec64*
       }
     }
     if (mine) {
-      const double t0 = tanh(g.alpha * F);
-      const double t1 = g.thr == 0.0 ? t0 : tanh(g.alpha * (F - g.thr));
+      const double t0 = tanh64(g.alpha * F);
+      const double t1 = g.thr == 0.0 ? t0 : tanh64(g.alpha * (F - g.thr));
       sc = -t0 * w;
       ge = -g.alpha * w * (1.0 - t1 * t1);
       act = iterate && isfinite(ge) && ge != 0.0;  // a non-finite weight leaves the root terms out

@@ -119,14 +119,10 @@ __device__ __forceinline__ double angle64(double y, double w) {
   return w < 0.0 ? 3.141592653589793 - (a - 1.2246467991473532e-16) : a;
 }
 
-// exp(x) for finite x: 2^k exp(r), |r| <= ln 2 / 2. Overflow gives inf,
-// underflow a denormal or 0, as the scaling by 2^k rounds them.
-template <bool kInLoop = false>
-__device__ __forceinline__ double exp64(double x) {
+// (e^r - 1 - r) / r^2 for |r| <= ln 2 / 2
+template <bool kInLoop>
+__device__ __forceinline__ double exp_poly(double r) {
 #pragma clang fp contract(off)
-  const double dk = __builtin_rint(x * k64<kInLoop>(1.4426950408889634));
-  double r = __builtin_fma(-dk, k64<kInLoop>(0x1.62e42fefa39efp-1), x);
-  r = __builtin_fma(-dk, k64<kInLoop>(0x1.abc9e3b39803fp-56), r);
   double p = k64<kInLoop>(2.0914679376583935e-09);
   p = __builtin_fma(p, r, k64<kInLoop>(2.510520637395701e-08));
   p = __builtin_fma(p, r, k64<kInLoop>(2.7557273661348637e-07));
@@ -138,8 +134,37 @@ __device__ __forceinline__ double exp64(double x) {
   p = __builtin_fma(p, r, k64<kInLoop>(0.04166666666666667));
   p = __builtin_fma(p, r, k64<kInLoop>(0.1666666666666667));
   p = __builtin_fma(p, r, k64<kInLoop>(0.5));
+  return p;
+}
+
+// exp(x) for finite x: 2^k exp(r), |r| <= ln 2 / 2. Overflow gives inf,
+// underflow a denormal or 0, as the scaling by 2^k rounds them.
+template <bool kInLoop = false>
+__device__ __forceinline__ double exp64(double x) {
+#pragma clang fp contract(off)
+  const double dk = __builtin_rint(x * k64<kInLoop>(1.4426950408889634));
+  double r = __builtin_fma(-dk, k64<kInLoop>(0x1.62e42fefa39efp-1), x);
+  r = __builtin_fma(-dk, k64<kInLoop>(0x1.abc9e3b39803fp-56), r);
+  const double p = exp_poly<kInLoop>(r);
   const double k = __builtin_fmin(__builtin_fmax(dk, -4000.0), 4000.0);
   return __builtin_amdgcn_ldexp(1.0 + __builtin_fma(r * r, p, r), (int)k);
+}
+
+// tanh(x) for every x: E / (E + 2) with E = e^(2 |x|) - 1 = (2^k - 1) + 2^k p,
+// p = e^r - 1 as in exp64, which keeps small arguments' relative precision.
+// Beyond |x| = 20 the quotient rounds to 1.
+template <bool kInLoop = false>
+__device__ __forceinline__ double tanh64(double x) {
+#pragma clang fp contract(off)
+  const double y = 2.0 * __builtin_fmin(__builtin_fabs(x), 20.0);
+  const double dk = __builtin_rint(y * k64<kInLoop>(1.4426950408889634));
+  double r = __builtin_fma(-dk, k64<kInLoop>(0x1.62e42fefa39efp-1), y);
+  r = __builtin_fma(-dk, k64<kInLoop>(0x1.abc9e3b39803fp-56), r);
+  const double p = __builtin_fma(r * r, exp_poly<kInLoop>(r), r);
+  const double t = __builtin_amdgcn_ldexp(1.0, (int)dk);
+  const double e = __builtin_fma(t, p, t - 1.0);
+  const double q = __builtin_copysign(div64(e, e + 2.0), x);
+  return x != x ? x : (x == 0.0 ? x : q);
 }
 
 // sin(x) and cos(x) for |x| <= 2^30: x - k pi / 2 with pi / 2 in two parts,

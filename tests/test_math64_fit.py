@@ -19,7 +19,7 @@ import fit_math64  # noqa: E402
     ("atan", "const double z = u * u;", "// +-(u + u z P)"),
     ("sin", "double p = k64<kInLoop>(1.59", "const double s = "),
     ("cos", "double c = k64<kInLoop>(", "c = __builtin_fma(z, "),
-    ("exp", "double p = k64<kInLoop>(2.09", "const double k = "),
+    ("exp", "double p = k64<kInLoop>(2.09", "return p;"),
 ])
 def test_constants_are_the_fit(name, begins, ends):
     src = open(os.path.join(CSRC, "qj_math64.h")).read()
