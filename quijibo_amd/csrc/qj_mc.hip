@@ -3,29 +3,22 @@
 // CPU mesher: same flags, same vertex set and numbering, same vertex
 // arithmetic, same triangle order, same degenerate filter.
 //
-// Pipeline per field (one lane per grid point / cell, point blocks dealt to
-// the XCDs in contiguous runs; no host synchronisation between fields, see
-// mc_run_tiles):
-//   k_mc_cells      cell case from the float sign test (the 8 corners read
-//                   once), and which of the case row's triangles survive the
-//                   degenerate filter (edge < 1e-7 dropped): an FP32 estimate
-//                   of where each vertex sits on its edge clears every
-//                   triangle with fewer than two vertices near an edge end,
-//                   the other cells go to a list; per block of cells:
-//                   kept-triangle count
-//   k_mc_measure    the listed cells' triangles measured with the FP64
-//                   vertices, one cell per lane
-//   k_mc_edges      per grid point: which of its +x,+y,+z edges some adjacent
-//                   cell's case row references (the edge-use masks of the four
-//                   cell rows around a block staged in LDS), packed with the
-//                   point's first vertex id within its block; per block of
-//                   points: vertex count
-//   scan            block vertex counts -> first vertex id per block (the
+// Pipeline per field (no host synchronisation between fields, see
+// mc_run_tiles). The sign test is kept as one bit per grid point, so that the
+// edges, cases and triangle counts of 64 points are a few operations on
+// 64-bit words, and only vertices and triangles themselves take a lane each:
+//   k_mc_signs      one bit per point: the float sign test
+//   k_mc_edges      the +x, +y, +z edges that carry a vertex, and the vertices
+//                   before every 8 points within a group of 16384 points
+//   k_mc_scan       groups' vertex counts -> first vertex id per group (the
 //                   reference numbers vertices by std::map<pair<int,int>> order
 //                   = lower endpoint, then x<y<z)
-//   k_mc_vertices   ids within the block, p0 + d0/(d0-d1) (p1-p0) at cell
-//                   centres, no contraction
-//   scan            block triangle counts -> first triangle per block
+//   k_mc_vertices   p0 + d0/(d0-d1) (p1-p0) at cell centres, no contraction,
+//                   and a bit per edge whose vertex lies near an end (an FP32
+//                   estimate)
+//   k_mc_cells      triangle counts, and the degenerate filter (edge < 1e-7
+//                   dropped) on the cells with two or more near vertices
+//   k_mc_scan       groups' triangle counts -> first triangle per group
 //   k_mc_tris       each kept triangle written once, in cell then table order
 #include <float.h>
 #include <math.h>
@@ -57,13 +50,13 @@ struct McTables {
   signed char tri[256][16];
   unsigned char ntri[256];
   unsigned short emask[256];
-  // edge mask | triangle count << 12
-  unsigned short emn[256];
-  // per case row and triangle: the bit mask of its 3 edges, and its 3 corners
-  // in table order, 5 bits each: dx | (dy + 2 dz) << 1 | axis << 3 (the row
-  // of owner points and the axis the triangle kernel looks up)
+  // per case row and triangle: the bit mask of its 3 edges, and its 3 edges in
+  // table order, 4 bits each
   unsigned short tmask[256][5];
-  unsigned short tcorner[256][5];
+  unsigned short tedge[256][5];
+  // the pairs of its edges that meet at a corner: bit 3 k + (xy, xz, yz) for
+  // corner k = 4 dx + 2 dy + dz
+  unsigned tpair[256][5];
 };
 
 constexpr McTables make_tables() {
@@ -77,23 +70,26 @@ constexpr McTables make_tables() {
     }
     t.ntri[c] = (unsigned char)(n / 3);
     t.emask[c] = (unsigned short)m;
-    t.emn[c] = (unsigned short)(m | (unsigned)(n / 3) << 12);
     for (int q = 0; q < n / 3; q++) {
       unsigned tm = 0, tc = 0;
       for (int j = 0; j < 3; j++) {
         const int e = t.tri[c][3 * q + j];
-        int dx = 0, dy = 0, dz = 0, axis = 0;
-        edge_parts(e, dx, dy, dz, axis);
         tm |= 1u << e;
-        tc |= (unsigned)(dx | (dy + 2 * dz) << 1 | axis << 3) << (5 * j);
+        tc |= (unsigned)e << (4 * j);
       }
       t.tmask[c][q] = (unsigned short)tm;
-      t.tcorner[c][q] = (unsigned short)tc;
+      t.tedge[c][q] = (unsigned short)tc;
+      for (int k = 0; k < 8; k++) {
+        const int dx = k >> 2, dy = (k >> 1) & 1, dz = k & 1;
+        const bool x = tm >> (dy + 2 * dz) & 1, y = tm >> (4 + dx + 2 * dz) & 1, z = tm >> (8 + dx + 2 * dy) & 1;
+        t.tpair[c][q] |= (unsigned)((x && y) | (x && z) << 1 | (y && z) << 2) << (3 * k);
+      }
     }
   }
   return t;
 }
 
+constexpr McTables kMcHost = make_tables();
 __constant__ McTables kMc = make_tables();
 
 // Case tables staged in LDS for the kernels that look them up per lane: with
@@ -122,13 +118,6 @@ __device__ __forceinline__ void edge_geom(int e, int& dx, int& dy, int& dz, int&
   edge_parts(e, dx, dy, dz, axis);
 }
 
-// per-triangle tables (5 per case row) staged in LDS as 640 words
-__device__ __forceinline__ void stage_tri5(unsigned short* dst, const unsigned short (*src)[5]) {
-  const uint32_t* s32 = (const uint32_t*)&src[0][0];
-  uint32_t* d32 = (uint32_t*)dst;
-  for (int i = threadIdx.x; i < 640; i += kMcBlock) d32[i] = s32[i];
-}
-
 __device__ __forceinline__ double sq3(double e0, double e1, double e2) {
 #pragma clang fp contract(off)
   return e0 * e0 + e1 * e1 + e2 * e2;
@@ -140,16 +129,15 @@ struct McState {
   uint8_t* flags = nullptr;
   uint8_t* emask = nullptr;
   uint32_t* cnt = nullptr;     // per point edge count -> vertex base (scanned in place; non-linear mesher)
-  uint16_t* pk16 = nullptr;    // linear mesher, per point: first vertex id within its block << 3 | edge mask
-  uint8_t* kmask = nullptr;    // per cell: bit t set when triangle t of its case row is kept
-  int64_t cap_kmask = 0;
-  uint32_t* mlist = nullptr;   // cells that await the degenerate measurement
-  int64_t cap_mlist = 0;
-  uint32_t* d_mcount = nullptr;
-  uint32_t* blkt = nullptr;    // per block of cells triangle count -> first triangle of the block
-  int64_t cap_blkt = 0;
-  uint32_t* blkv = nullptr;    // per block vertex count -> first vertex id of the block
-  int64_t cap_pk16 = 0, cap_blkv = 0;
+  // linear mesher: bit words of 64 points each (kMcArrays arrays of one
+  // length), vertex ranks per 8 points, kept triangles of the cells that lost
+  // some, first triangle per word, counts per group of 16384 points
+  uint64_t* words = nullptr;
+  uint2* ranks = nullptr;
+  uint8_t* kmask = nullptr;
+  uint32_t* tword = nullptr;
+  uint32_t* groups = nullptr;
+  int64_t cap_words = 0, cap_ranks = 0, cap_kmask = 0, cap_tword = 0, cap_groups = 0;
   uint32_t* blk = nullptr;     // per block active count -> offset
   uint32_t* active = nullptr;  // active cells
   uint32_t* tri_off = nullptr; // per active cell triangle count -> offset
@@ -180,11 +168,9 @@ struct McState {
   int32_t* c_cells = nullptr;
   int64_t cap_ce = 0, cap_cc = 0, ncells = 0;
   bool cache_valid = false;
-  // linear mesher over several fields: running vertex / triangle totals and
-  // per-field counts on the device
+  // linear mesher over several fields: the vertices and triangles before each
   uint64_t* d_base = nullptr;
-  int64_t* d_counts = nullptr;
-  int64_t cap_counts = 0;
+  int64_t cap_base = 0;
 };
 
 __device__ __forceinline__ int cell_flag(const double* __restrict__ f, int64_t i, int64_t X, int64_t XY, double iso) {
@@ -216,142 +202,6 @@ __device__ __forceinline__ void point_xyz(const GridGeom& g, int64_t p, int64_t&
 __device__ __forceinline__ int64_t xcd_block(int64_t nb) {
   const int64_t b = blockIdx.x, x = b & 7, k = b >> 3, per = nb >> 3, rem = nb & 7;
   return x * per + (x < rem ? x : rem) + k;
-}
-
-// Block-wide exclusive prefix and total of a small per-thread count given as
-// three bit flags of weights W0, W1, W2 (edge bits 1,1,1; a triangle count
-// 0..5 in binary 1,2,4): three ballots and masked popcounts, no shuffles.
-struct BlockPrefix {
-  uint32_t excl;
-  uint32_t total;
-};
-template <int W0, int W1, int W2>
-__device__ __forceinline__ BlockPrefix mc_block_prefix3(unsigned v) {
-  __shared__ uint32_t s_w[kMcBlock / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const unsigned long long lt = (1ull << lane) - 1ull;
-  const unsigned long long b0 = __ballot(v & 1u), b1 = __ballot(v & 2u), b2 = __ballot(v & 4u);
-  const uint32_t within = W0 * __popcll(b0 & lt) + W1 * __popcll(b1 & lt) + W2 * __popcll(b2 & lt);
-  if (lane == 0) s_w[wave] = W0 * __popcll(b0) + W1 * __popcll(b1) + W2 * __popcll(b2);
-  __syncthreads();
-  uint32_t before = 0, total = 0;
-  for (int i = 0; i < kMcBlock / 64; i++) {
-    const uint32_t c = s_w[i];
-    if (i < wave) before += c;
-    total += c;
-  }
-  return BlockPrefix{before + within, total};
-}
-
-// ---- linear mesher: one wave per block of 256 points (the unit of the
-// vertex and triangle numbering), four blocks per workgroup. Lane l of a wave
-// takes points l, l + 64, l + 128 and l + 192 of its block: every load
-// instruction is contiguous over the wave, each lane has four independent
-// points in flight, and prefixes in point order are wave ballots with no
-// barrier.
-constexpr int kMcWaves = 4;              // blocks per workgroup
-constexpr int kMcGroup = 64 * kMcWaves;  // threads per workgroup
-static_assert(kMcGroup == kMcBlock, "the table stagings use one thread per case");
-
-struct WavePrefix {
-  uint32_t excl;
-  uint32_t total;
-};
-// exclusive prefix over the wave's lanes and wave total of a count 0..7 given
-// as three bits of weights W0, W1, W2
-template <int W0, int W1, int W2>
-__device__ __forceinline__ WavePrefix wave_prefix3(unsigned v) {
-  const int lane = threadIdx.x & 63;
-  const unsigned long long lt = (1ull << lane) - 1ull;
-  const unsigned long long b0 = __ballot(v & 1u), b1 = __ballot(v & 2u), b2 = __ballot(v & 4u);
-  return WavePrefix{(uint32_t)(W0 * __popcll(b0 & lt) + W1 * __popcll(b1 & lt) + W2 * __popcll(b2 & lt)),
-                    (uint32_t)(W0 * __popcll(b0) + W1 * __popcll(b1) + W2 * __popcll(b2))};
-}
-
-// this wave's block of points (blocks of a workgroup are consecutive), or -1
-// past the last block
-__device__ __forceinline__ int64_t wave_block(int64_t nb) {
-  const int64_t B = xcd_block((nb + kMcWaves - 1) / kMcWaves) * kMcWaves + (threadIdx.x >> 6);
-  return B < nb ? B : -1;
-}
-
-// Edge masks (bit axis set when the +axis edge from the point carries a
-// vertex) and each point's first vertex id within its block, packed as
-// pk16[p] = id << 3 | mask (ids within a block stay below 3 x 256), and each
-// block's vertex count. The edges of point p are referenced by the cells
-// p - a X - b XY (x edge), p - a - b XY (y edge) and p - a - b X (z edge),
-// a, b in {0, 1}: entries -1..255 of the four cell rows that start at
-// p0 - a X - b XY. Each wave stages those rows' edge-use masks (the case
-// table's emask of each cell's flag) in LDS, so a point's 12 tests are LDS
-// reads and each flag is looked up once.
-__global__ __launch_bounds__(kMcGroup) void k_mc_edges(const uint8_t* __restrict__ flags, GridGeom g,
-                                                       uint16_t* __restrict__ pk16, uint32_t* __restrict__ blkv) {
-  __shared__ unsigned short s_em[256];
-  __shared__ unsigned short s_ce[kMcWaves][4][kMcBlock + 1];
-  s_em[threadIdx.x] = kMc.emask[threadIdx.x];
-  __syncthreads();
-  const int64_t X = g.res[0], Y = g.res[1], Z = g.res[2], XY = X * Y, N = XY * Z;
-  const int64_t B = wave_block((N + kMcBlock - 1) / kMcBlock);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (B >= 0) {
-    // all 20 loads issued before the first table lookup (case 0 uses no edge)
-    const int64_t p0 = B * kMcBlock;
-    unsigned f[4][5];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int64_t c0 = p0 - (r & 1) * X - (r >> 1) * XY - 1;
-#pragma unroll
-      for (int k = 0; k < 5; k++) {
-        const int64_t c = c0 + lane + 64 * k;
-        f[r][k] = ((k < 4 || lane == 0) && c >= 0 && c < N) ? (unsigned)flags[c] : 0u;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-#pragma unroll
-      for (int k = 0; k < 5; k++)
-        if (k < 4 || lane == 0) s_ce[w][r][lane + 64 * k] = s_em[f[r][k]];
-  }
-  __syncthreads();
-  if (B < 0) return;
-  uint32_t base = 0;
-  for (int sub = 0; sub < 4; sub++) {
-    const int j = sub * 64 + lane;
-    const int64_t p = B * kMcBlock + j;
-    unsigned bits = 0;
-    if (p < N) {
-      int64_t x, y, z;
-      point_xyz(g, p, x, y, z);
-      // x-edge (p, p+1): cells p - (0,a,b), row a + 2b, local edge a + 2b
-      if (x < X - 1) {
-        unsigned ref = 0;
-        for (int b = 0; b < 2; b++)
-          for (int a = 0; a < 2; a++)
-            if (y >= a && z >= b) ref |= (s_ce[w][a + 2 * b][j + 1] >> (a + 2 * b)) & 1u;
-        bits |= ref;
-      }
-      // y-edge (p, p+X): cells p - (a,0,b), row 2b, local edge 4 + a + 2b
-      if (y < Y - 1) {
-        unsigned ref = 0;
-        for (int b = 0; b < 2; b++)
-          for (int a = 0; a < 2; a++)
-            if (x >= a && z >= b) ref |= (s_ce[w][2 * b][j + 1 - a] >> (4 + a + 2 * b)) & 1u;
-        bits |= ref << 1;
-      }
-      // z-edge (p, p+XY): cells p - (a,b,0), row b, local edge 8 + a + 2b
-      if (z < Z - 1) {
-        unsigned ref = 0;
-        for (int b = 0; b < 2; b++)
-          for (int a = 0; a < 2; a++)
-            if (x >= a && y >= b) ref |= (s_ce[w][b][j + 1 - a] >> (8 + a + 2 * b)) & 1u;
-        bits |= ref << 2;
-      }
-    }
-    const WavePrefix vp = wave_prefix3<1, 1, 1>(bits);
-    if (p < N) pk16[p] = (uint16_t)((base + vp.excl) << 3 | bits);
-    base += vp.total;
-  }
-  if (lane == 0) blkv[B] = base;
 }
 
 // One vertex of computeEdgeInterpolations (TRIANGLE_MESH.cpp:2373-2425): the
@@ -386,7 +236,7 @@ __device__ __forceinline__ double edge_len(const double* a, const double* b) {
 // two edges meeting at a corner c the vertices satisfy |v1 - v2| >=
 // max |vi - c| (the edges are perpendicular). So with h >= kPrefilterSpacing
 // a triangle with at most one vertex within 2e-7 of an end of its edge has
-// every side longer than 1e-7. k_mc_cells marks a vertex "near" from an FP32
+// every side longer than 1e-7. k_mc_vertices marks a vertex "near" from an FP32
 // estimate t' of its place t on the edge: near unless t' h >= kNearLimit and
 // (1 - t') h >= kNearLimit. |t' - t| stays below 2.5e-7 (corner values
 // rounded to float, one division and one subtraction), so with
@@ -396,23 +246,35 @@ __device__ __forceinline__ double edge_len(const double* a, const double* b) {
 constexpr float kNearLimit = 1e-6f;
 constexpr double kPrefilterSpacing = 1e-6;
 constexpr double kPrefilterMaxSpacing = 3.0;
+// On two edges that meet at a corner the vertices are sqrt(d0^2 + d1^2) apart
+// for distances d0, d1 from it. FP32 estimates of those (relative error below
+// 1e-6) decide all but a band of 1 % around 1e-7, as long as rounding of the
+// FP64 coordinates (1e-11 up to kSureExtent) stays far inside the band; the rest is
+// measured. kMeasureNear: coordinates beyond that. kMeasureAll: no prefilter.
+constexpr float kSureShort = 0.99e-7f * 0.99e-7f, kSureLong = 1.01e-7f * 1.01e-7f;
+constexpr double kSureExtent = 1e4;
+enum McPrefilter { kMeasureAll = 0, kMeasureNear = 1, kMeasureUnsure = 2 };
 
-// The 12-bit mask of a cell's edges whose vertex may lie within 2e-7 of an
-// end of its edge, from the float corner values (corner k = 4 dx + 2 dy + dz):
-// near unless |v0| h >= 1e-6 |v0 - v1| and |v1| h >= 1e-6 |v0 - v1| (a vertex
-// at place t has t = |v0| / |v0 - v1| and 1 - t = |v1| / |v0 - v1|, so no
-// division); NaN and infinite corners make it near. prefilter = 0: all 12.
+// Whether the vertex of an edge with end values v0, v1 and grid spacing h may
+// lie within 2e-7 of an end: near unless |v0| h >= 1e-6 |v0 - v1| and
+// |v1| h >= 1e-6 |v0 - v1| (a vertex at place t has t = |v0| / |v0 - v1| and
+// 1 - t = |v1| / |v0 - v1|, so no division); NaN and infinite ends make it near.
+__device__ __forceinline__ bool mc_near(float v0, float v1, float h) {
+  const float lim = kNearLimit * fabsf(v0 - v1);
+  return !(fabsf(v0) * h >= lim && fabsf(v1) * h >= lim);
+}
+
+// The 12-bit mask of a cell's near edges from its float corner values (corner
+// k = 4 dx + 2 dy + dz). prefilter = 0: all 12.
 __device__ __forceinline__ unsigned mc_near_edges(const float* v, const GridGeom& g, int prefilter) {
   if (!prefilter) return 0xfffu;
-  const float h[3] = {fabsf((float)g.dx[0]), fabsf((float)g.dx[1]), fabsf((float)g.dx[2])};
   unsigned near = 0;
 #pragma unroll
   for (int e = 0; e < 12; e++) {
     int dx = 0, dy = 0, dz = 0, axis = 0;
     edge_parts(e, dx, dy, dz, axis);
     const int k0 = 4 * dx + 2 * dy + dz, k1 = k0 + (axis == 0 ? 4 : (axis == 1 ? 2 : 1));
-    const float a0 = fabsf(v[k0]), a1 = fabsf(v[k1]), lim = kNearLimit * fabsf(v[k0] - v[k1]);
-    near |= (a0 * h[axis] >= lim && a1 * h[axis] >= lim) ? 0u : (1u << e);
+    near |= mc_near(v[k0], v[k1], fabsf((float)g.dx[axis])) ? (1u << e) : 0u;
   }
   return near;
 }
@@ -432,347 +294,653 @@ __device__ __forceinline__ int mc_corners(const double* __restrict__ field, int6
   return flag;
 }
 
-// Bit 7 of kmask: the cell awaits measurement and did not fit the list.
-constexpr unsigned kMeasureMark = 0x80u;
-// The measure list is split in kMeasureLists sub-lists of equal capacity, one
-// counter each (block lb appends to sub-list lb % kMeasureLists): one counter
-// for all blocks serialised the appends (65536 atomics on one address per
-// 256^3 field). Counter kMeasureLists is set when a cell did not fit.
-constexpr int kMeasureLists = 251;
+// ---- linear mesher: one bit per grid point, 64 points (one word) at a time
 
-// Cell case and provisional kept triangles of every cell. flags[p] is the
-// case of the cell with lowest corner p (0 on the last layer of each axis),
-// kmask[p] bit t is set when triangle t of that case row is kept, blkt[block]
-// counts the block's kept triangles. A cell with two or more near vertices
-// may hold a degenerate triangle: it keeps all its triangles here and goes to
-// the measure list (mlist: kMeasureLists sub-lists of mcap entries; beyond
-// that its kmask gets kMeasureMark), which k_mc_measure works through with
-// full waves. The FP64 measurement is rare but long, and one lane of a wave
-// taking it held up the whole wave here (the borders of a field set by
-// setBorders put such cells in every row). One cell per thread, a block of
-// 256 cells per block of the numbering.
-__global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict__ field, GridGeom g, double iso,
-                                                       int prefilter, uint8_t* __restrict__ flags,
-                                                       uint8_t* __restrict__ kmask, uint32_t* __restrict__ blkt,
-                                                       uint32_t* __restrict__ mlist, uint32_t* __restrict__ mcount,
-                                                       uint32_t mcap) {
-  __shared__ unsigned short s_emn[256];
-  __shared__ uint32_t s_w[kMcBlock / 64], s_m[kMcBlock / 64];
-  __shared__ uint32_t s_mbase;
-  s_emn[threadIdx.x] = kMc.emn[threadIdx.x];
-  __syncthreads();
-  const int64_t X = g.res[0], Y = g.res[1], Z = g.res[2], XY = X * Y, N = XY * Z;
-  const int64_t lb = xcd_block((N + kMcBlock - 1) / kMcBlock);
-  const int64_t p = lb * kMcBlock + threadIdx.x;
-  int flag = 0;
-  unsigned keep = 0;
-  bool measure = false;
-  if (p < N) {
-    int64_t x, y, z;
-    point_xyz(g, p, x, y, z);
-    if (x < X - 1 && y < Y - 1 && z < Z - 1) {
-      float v[8];
-      flag = mc_corners(field, p, X, XY, iso, v);
-      const unsigned emn = s_emn[flag];
-      const int n = (int)(emn >> 12);
-      if (n) {
-        keep = (1u << n) - 1u;
-        measure = __popc(mc_near_edges(v, g, prefilter) & emn & 0xfffu) >= 2;
-      }
-    }
-  }
-  // kept-triangle count of the block and this block's share of the measure list
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const unsigned cnt = (unsigned)__popc(keep);
-  const unsigned long long b0 = __ballot(cnt & 1u), b1 = __ballot(cnt & 2u), b2 = __ballot(cnt & 4u);
-  const unsigned long long bm = __ballot(measure);
-  if (lane == 0) {
-    s_w[wave] = (uint32_t)(__popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2));
-    s_m[wave] = (uint32_t)__popcll(bm);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t t = 0, m = 0;
-    for (int i = 0; i < kMcBlock / 64; i++) {
-      t += s_w[i];
-      const uint32_t c = s_m[i];
-      s_m[i] = m;
-      m += c;
-    }
-    blkt[lb] = t;
-    const int sub = (int)(lb % kMeasureLists);
-    const uint32_t base = m ? atomicAdd(&mcount[sub], m) : 0u;
-    s_mbase = base;
-    if (m && base + m > mcap) mcount[kMeasureLists] = 1u;  // some cells did not fit
-  }
-  __syncthreads();
-  if (p < N) {
-    const uint32_t slot = s_mbase + s_m[wave] + (uint32_t)__popcll(bm & ((1ull << lane) - 1ull));
-    const bool listed = measure && slot < mcap;
-    if (listed) mlist[(int64_t)(lb % kMeasureLists) * mcap + slot] = (uint32_t)p;
-    flags[p] = (uint8_t)flag;
-    kmask[p] = (uint8_t)(keep | (measure && !listed ? kMeasureMark : 0u));
-  }
+constexpr int kMcWaves = kMcBlock / 64;        // waves per workgroup
+constexpr int kMcGroupWords = kMcBlock;        // words per group: the unit of the two scans, one word per thread
+constexpr int kMcGroupPoints = 64 * kMcGroupWords;
+constexpr int kSignPoints = 8;                 // points per thread of k_mc_signs
+constexpr int kVertWords = 8;                  // words per wave of k_mc_vertices
+constexpr int kTriBlocks = 4;                  // blocks of 256 cells per wave of k_mc_tris, at most
+constexpr int kTriWaves = 256 * 16;            // waves that fill the chip before one takes a second block
+constexpr int kScanBlock = 1024;
+
+// Words whose bit i is point (or cell with lowest corner) 64 w + i; each array
+// is wmax words long: those of the field's points, then at least
+// mc_pad_words(g) that reads of a word's shifted rows may reach. Their bits
+// and those of points past the last one are read but masked.
+struct McGrid {
+  GridGeom g;
+  double iso;
+  int prefilter;
+  int64_t N, XY, nw;  // points, points per slice, words
+  uint64_t* sgn;      // field value above the isovalue
+  uint64_t* edge[3];  // the point's +x, +y, +z edge carries a vertex
+  uint64_t* near[3];  // ... that may lie near an end of the edge
+  uint64_t* drop;     // some of the cell's triangles were dropped: kmask holds the kept ones
+};
+constexpr int kMcArrays = 8;
+
+static int64_t mc_pad_words(const GridGeom& g) {
+  return ((int64_t)g.res[0] * g.res[1] + g.res[0] + 1) / 64 + 16;
 }
 
-// The degenerate filter (TRIANGLE_MESH.cpp:1088-1102) for one listed cell:
-// triangles with two or three near vertices are measured with the FP64
-// vertices (the function the vertex kernel uses, so both see the same bits).
-// Only a side between two near vertices can be short: a vertex that is not
-// near is at least 2e-7 from both ends of its edge, so at least that far from
-// a vertex on an edge through either end, and a grid spacing from vertices on
-// the other edges. Dropped triangles leave kmask and the block's count.
-__device__ __forceinline__ void mc_measure_cell(const double* __restrict__ field, const GridGeom& g, double iso,
-                                                int prefilter, int64_t p, uint8_t* __restrict__ kmask,
-                                                uint32_t* __restrict__ blkt) {
-  const int64_t X = g.res[0], XY = X * g.res[1];
-  int64_t x, y, z;
-  point_xyz(g, p, x, y, z);
-  float v[8];
-  const int flag = mc_corners(field, p, X, XY, iso, v);
-  const unsigned near = mc_near_edges(v, g, prefilter) & kMc.emask[flag];
-  const int n = kMc.ntri[flag];
-  unsigned keep = kmask[p] & 0x1fu, dropped = 0;
-  for (int t = 0; t < n; t++) {
-    const unsigned nm = near & kMc.tmask[flag][t];
-    const int m = __popc(nm);
-    if (m < 2) continue;
-    double w[3][3] = {};
-    unsigned r = nm;
+static McGrid make_mc_grid(const McState& m, const GridGeom& g, int64_t wmax, double iso, int prefilter) {
+  McGrid a;
+  a.g = g;
+  a.iso = iso;
+  a.prefilter = prefilter;
+  a.XY = (int64_t)g.res[0] * g.res[1];
+  a.N = a.XY * g.res[2];
+  a.nw = (a.N + 63) / 64;
+  uint64_t* p[kMcArrays];
+  for (int i = 0; i < kMcArrays; i++) p[i] = m.words + i * wmax;
+  a.sgn = p[0];
+  for (int i = 0; i < 3; i++) {
+    a.edge[i] = p[1 + i];
+    a.near[i] = p[4 + i];
+  }
+  a.drop = p[7];
+  return a;
+}
+
+// A case row's triangles use exactly the edges whose corners differ in sign,
+// except row 158, which leaves out kRow158Missing: the x edge at corner (0,0,0)
+// and the y and z edges at (1,0,0). k_mc_edges builds on this.
+constexpr int kRow158 = 158;
+constexpr unsigned kRow158Missing = 1u << 0 | 1u << 5 | 1u << 9;
+constexpr bool rows_use_crossing_edges() {
+  for (int c = 0; c < 256; c++) {
+    unsigned m = 0;
+    for (int e = 0; e < 12; e++) {
+      int dx = 0, dy = 0, dz = 0, axis = 0;
+      edge_parts(e, dx, dy, dz, axis);
+      const int k0 = 4 * dx + 2 * dy + dz, k1 = k0 + (axis == 0 ? 4 : (axis == 1 ? 2 : 1));
+      if (((c >> k0) ^ (c >> k1)) & 1) m |= 1u << e;
+    }
+    if (kMcHost.emask[c] != (c == kRow158 ? m & ~kRow158Missing : m)) return false;
+  }
+  return true;
+}
+static_assert(rows_use_crossing_edges(), "the edges of the case rows");
+
+// Bit B of the triangle count of 64 cells from the words of their corners (k =
+// 4 dx + 2 dy + dz): the count's decision diagram over corners K-1..0 for the
+// cases that agree with BASE above; equal halves need no test, and the compiler
+// merges equal subtrees.
+template <int B, int K, int BASE>
+struct CountBits {
+  static constexpr bool halves_equal() {
+    for (int i = 0; i < (1 << (K - 1)); i++)
+      if (((kMcHost.ntri[BASE + i] ^ kMcHost.ntri[BASE + (1 << (K - 1)) + i]) >> B) & 1) return false;
+    return true;
+  }
+  static __device__ __forceinline__ uint64_t eval(const uint64_t* c) {
+    const uint64_t lo = CountBits<B, K - 1, BASE>::eval(c);
+    if constexpr (halves_equal()) {
+      return lo;
+    } else {
+      const uint64_t hi = CountBits<B, K - 1, BASE + (1 << (K - 1))>::eval(c);
+      return (c[K - 1] & hi) | (~c[K - 1] & lo);
+    }
+  }
+};
+template <int B, int BASE>
+struct CountBits<B, 0, BASE> {
+  static __device__ __forceinline__ uint64_t eval(const uint64_t*) {
+    return (kMcHost.ntri[BASE] >> B) & 1 ? ~0ull : 0ull;
+  }
+};
+
+// bits b.. of a word (b any integer)
+__device__ __forceinline__ uint64_t bits_from(int64_t b) { return b <= 0 ? ~0ull : (b >= 64 ? 0ull : ~0ull << b); }
+
+// word w of the array shifted down by `off` bits
+__device__ __forceinline__ uint64_t shifted_word(const uint64_t* __restrict__ a, int64_t w, int64_t off) {
+  const int64_t i = w + (off >> 6);
+  const int sh = (int)(off & 63);
+  const uint64_t lo = a[i], hi = a[i + 1];
+  return (lo >> sh) | ((hi << 1) << (63 - sh));
+}
+
+// the points of word w that are last along x, along y, along z (or past the field's last)
+struct EndMasks {
+  uint64_t x, y, z;
+};
+__device__ __forceinline__ EndMasks end_masks(const McGrid& a, int64_t w) {
+  EndMasks m{0, 0, bits_from(a.N - a.XY - 64 * w)};
+  const int64_t X = a.g.res[0];
+  const uint32_t p0 = (uint32_t)(64 * w);
+  const uint32_t r0 = p0 - fast_div(p0, a.g.div_xy) * (uint32_t)a.XY;
+  const uint32_t x0 = r0 - fast_div(r0, a.g.div_x) * (uint32_t)X;
+  for (int64_t b = X - 1 - (int64_t)x0; b < 64; b += X) m.x |= 1ull << b;
+  for (int64_t b = a.XY - X - (int64_t)r0; b < 64; b += a.XY) m.y |= bits_from(b) & ~bits_from(b + X);
+  return m;
+}
+
+// inclusive prefix sum over the wave's lanes (DPP row shifts and broadcasts)
+__device__ __forceinline__ uint32_t wave_inclusive(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_last(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
+
+// exclusive prefix over the block's threads; *total: the block's sum. Every thread of the block takes part.
+template <int kThreads>
+__device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* total) {
+  __shared__ uint32_t s_w[kThreads / 64];
+  const uint32_t incl = wave_inclusive(v);
+  if ((threadIdx.x & 63) == 63) s_w[threadIdx.x >> 6] = incl;
+  __syncthreads();
+  uint32_t before = 0, sum = 0;
+  for (int i = 0; i < kThreads / 64; i++) {
+    const uint32_t c = s_w[i];
+    before += i < (int)(threadIdx.x >> 6) ? c : 0u;
+    sum += c;
+  }
+  __syncthreads();
+  *total = sum;
+  return before + incl - v;
+}
+
+// this workgroup's wave number, workgroups in contiguous runs per XCD
+__device__ __forceinline__ int64_t wave_index() {
+  return (int64_t)__builtin_amdgcn_readfirstlane((int)(xcd_block(gridDim.x) * kMcWaves + (threadIdx.x >> 6)));
+}
+
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The float sign test of every point (CUBE corners are floats,
+// TRIANGLE_MESH.h:283-288; test at TRIANGLE_MESH.cpp:1037-1039). HBM-bound: one
+// read of the field; a wave takes 512 consecutive points, eight loads in
+// flight per lane. 256^3: 29.6 us, 4.5 TB/s (the 8 corners read per cell and a
+// case byte written per cell, before: 109 us).
+__global__ __launch_bounds__(kMcBlock) void k_mc_signs(const double* __restrict__ field, int64_t N, double iso,
+                                                       uint64_t* __restrict__ sgn) {
+  const int lane = threadIdx.x & 63;
+  const int64_t p0 = ((int64_t)blockIdx.x * kMcWaves + (threadIdx.x >> 6)) * 64 * kSignPoints;
+  if (p0 >= N) return;
+  double v[kSignPoints];
 #pragma unroll
-    for (int j = 0; j < 3; j++) {
-      if (j < m) {  // constant indices into w keep it in registers
-        const int e = __ffs(r) - 1;
-        r &= r - 1;
-        int dx, dy, dz, axis;
-        edge_geom(e, dx, dy, dz, axis);
-        const int64_t q0 = p + dx + dy * X + dz * XY;
-        const int64_t q1 = q0 + (axis == 0 ? 1 : (axis == 1 ? X : XY));
-        mc_vertex(g, (int)x + dx, (int)y + dy, (int)z + dz, axis, field[q0], field[q1], iso, w[j]);
+  for (int i = 0; i < kSignPoints; i++) {
+    const int64_t p = p0 + 64 * i + lane;
+    v[i] = field[p < N ? p : N - 1];
+  }
+  uint64_t mine = 0;
+#pragma unroll
+  for (int i = 0; i < kSignPoints; i++) {
+    const uint64_t word = __ballot((float)(v[i] - iso) > 0.0f);
+    mine = lane == i ? word : mine;
+  }
+  if (lane < kSignPoints && p0 + 64 * lane < N) sgn[p0 / 64 + lane] = mine;
+}
+
+// every third bit of 24 from 8
+__device__ __forceinline__ uint32_t spread8(uint32_t x) {
+  x = (x | x << 8) & 0x00f00fu;
+  x = (x | x << 4) & 0x0c30c3u;
+  return (x | x << 2) & 0x249249u;
+}
+
+// The edges that carry a vertex, one word of points per thread: those with
+// ends of different sign, except where the only cells around an edge are of
+// case 158 and leave it out (on three border lines of the grid). ranks[8 w + j]
+// serves the triangle kernel's lookups: for points 64 w + 8 j.. the vertices
+// before them in the group and the 24 edge bits in id order (point, then axis),
+// so that a vertex's id is one masked bit count away. groups[]: vertices per
+// group. Latency-bound: 256^3, 1024 blocks, 10.7 us (from the case bytes of the
+// 12 cells around a point: 54 us).
+__global__ __launch_bounds__(kMcBlock) void k_mc_edges(McGrid a, uint2* __restrict__ ranks,
+                                                       uint32_t* __restrict__ groups) {
+  const int64_t w = (int64_t)blockIdx.x * kMcGroupWords + threadIdx.x;
+  const int64_t X = a.g.res[0];
+  uint64_t e[3] = {0, 0, 0};
+  if (w < a.nw) {
+    const uint64_t s0 = a.sgn[w];
+    const EndMasks end = end_masks(a, w);
+    const uint64_t in = ~bits_from(a.N - 64 * w);
+    e[0] = (s0 ^ shifted_word(a.sgn, w, 1)) & ~end.x & in;
+    e[1] = (s0 ^ shifted_word(a.sgn, w, X)) & ~end.y & in;
+    e[2] = (s0 ^ shifted_word(a.sgn, w, a.XY)) & ~end.z;
+    const uint64_t z0 = ~bits_from(a.XY - 64 * w);                                // z = 0
+    const uint64_t y0z0 = ~bits_from(X - 64 * w);                                 // and y = 0
+    const uint32_t p0 = (uint32_t)(64 * w), slice = fast_div(p0, a.g.div_xy);
+    uint64_t y0 = y0z0;                                                           // y = 0
+    for (int64_t b = (int64_t)(slice + (slice > 0 ? 0 : 1)) * a.XY - (int64_t)p0; b < 64; b += a.XY)
+      y0 |= bits_from(b) & ~bits_from(b + X);
+    const uint64_t line[3] = {y0z0, z0 & end.x, y0 & end.x};
+#pragma unroll
+    for (int axis = 0; axis < 3; axis++)
+      for (uint64_t m = e[axis] & line[axis]; m; m &= m - 1) {
+        const int b = __ffsll((unsigned long long)m) - 1;
+        const int64_t c = 64 * w + b - (axis ? 1 : 0);  // the cell that may leave the edge out, alone around it
+        int flag = 0;
+        for (int k = 0; k < 8; k++) {
+          const int64_t q = c + (k >> 2) + ((k >> 1) & 1) * X + (k & 1) * a.XY;
+          flag |= (int)((a.sgn[q >> 6] >> (q & 63)) & 1u) << k;
+        }
+        if (flag == kRow158) e[axis] &= ~(1ull << b);
       }
-    }
-    const double eps = 1e-7;
-    bool degenerate = edge_len(w[0], w[1]) < eps;
-    if (m == 3) degenerate = degenerate || edge_len(w[0], w[2]) < eps || edge_len(w[1], w[2]) < eps;
-    if (degenerate) {
-      keep &= ~(1u << t);
-      dropped++;
-    }
+    for (int axis = 0; axis < 3; axis++) a.edge[axis][w] = e[axis];
   }
-  kmask[p] = (uint8_t)keep;
-  if (dropped) atomicSub(&blkt[p / kMcBlock], dropped);
+  uint32_t total;
+  uint32_t run = block_prefix<kMcBlock>((uint32_t)(__popcll(e[0]) + __popcll(e[1]) + __popcll(e[2])), &total);
+  if (threadIdx.x == 0) groups[blockIdx.x] = total;
+  if (w >= a.nw) return;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const uint32_t bits = spread8((uint32_t)(e[0] >> (8 * j)) & 0xffu) | spread8((uint32_t)(e[1] >> (8 * j)) & 0xffu) << 1 |
+                          spread8((uint32_t)(e[2] >> (8 * j)) & 0xffu) << 2;
+    ranks[8 * w + j] = uint2{run, bits};
+    run += (uint32_t)__popc(bits);
+  }
 }
 
-// The listed cells, one per thread; then, if the list overflowed, every cell
-// that carries kMeasureMark.
-__global__ __launch_bounds__(kMcBlock) void k_mc_measure(const double* __restrict__ field, GridGeom g, double iso,
-                                                         int prefilter, const uint32_t* __restrict__ mlist,
-                                                         const uint32_t* __restrict__ mcount, uint32_t mcap,
-                                                         uint8_t* __restrict__ kmask, uint32_t* __restrict__ blkt) {
-  const int64_t stride = (int64_t)gridDim.x * kMcBlock;
-  const int64_t total = (int64_t)kMeasureLists * mcap;
-  for (int64_t i = (int64_t)blockIdx.x * kMcBlock + threadIdx.x; i < total; i += stride) {
-    const int64_t sub = i / mcap, j = i - sub * mcap;
-    if (j < (int64_t)mcount[sub]) mc_measure_cell(field, g, iso, prefilter, (int64_t)mlist[i], kmask, blkt);
+// One block: the groups' counts to exclusive offsets in place, and the running
+// total after this tile: base[2 tile + which] is what came before it.
+__global__ __launch_bounds__(kScanBlock) void k_mc_scan(uint32_t* __restrict__ groups, int64_t n,
+                                                        uint64_t* __restrict__ base, int tile, int which) {
+  const int64_t per = (n + kScanBlock - 1) / kScanBlock, b = (int64_t)threadIdx.x * per;
+  uint32_t v = 0;
+  for (int64_t i = b; i < b + per && i < n; i++) v += groups[i];
+  uint32_t total;
+  uint32_t run = block_prefix<kScanBlock>(v, &total);
+  for (int64_t i = b; i < b + per && i < n; i++) {
+    const uint32_t c = groups[i];
+    groups[i] = run;
+    run += c;
   }
-  if (!mcount[kMeasureLists]) return;  // the same for every thread
-  const int64_t N = (int64_t)g.res[0] * g.res[1] * g.res[2];
-  for (int64_t p = (int64_t)blockIdx.x * kMcBlock + threadIdx.x; p < N; p += stride)
-    if (kmask[p] & kMeasureMark) mc_measure_cell(field, g, iso, prefilter, p, kmask, blkt);
+  if (threadIdx.x == 0) {
+    if (tile == 0) base[which] = 0;
+    base[2 * (tile + 1) + which] = (tile == 0 ? 0 : base[2 * tile + which]) + total;
+  }
 }
 
-// computeEdgeInterpolations (TRIANGLE_MESH.cpp:2373-2425). Vertex ids follow
-// the point order: the block's first id from blk_off, then pk16 >> 3. The tile's
-// vertices go to verts from the running vertex total base[0] (several tiles
-// share the buffer); ids at or beyond cap are not written (the host sees the
-// overflow in the totals and meshes again).
-__global__ __launch_bounds__(kMcGroup) void k_mc_vertices(const double* __restrict__ field, GridGeom g, double iso,
-                                                          const uint16_t* __restrict__ pk16,
-                                                          const uint32_t* __restrict__ blk_off,
+// computeEdgeInterpolations (TRIANGLE_MESH.cpp:2373-2425). A wave lists the
+// vertices of its 512 points (at most 3 per point) in LDS in id order and
+// computes them one per lane, so that the FP64 work is not spread over mostly
+// idle lanes; the tile's vertices go to verts from base[0] on (several tiles
+// share the buffer). Ids at or beyond cap are not written (the host sees the
+// overflow in the totals). Also marks the vertices near an end of their edge.
+// Bound by the field's second read and the vertices' writes: a 256^3 torus tile
+// (4.5 million vertices, 109 MB) 69 us, 3.5 TB/s; neither two vertices per lane
+// in flight, nor stores made contiguous through LDS, nor leaving out the rotation
+// made it faster.
+__global__ __launch_bounds__(kMcBlock) void k_mc_vertices(const double* __restrict__ field, McGrid a,
+                                                          const uint2* __restrict__ ranks,
+                                                          const uint32_t* __restrict__ groups,
                                                           const uint64_t* __restrict__ base, int64_t cap,
                                                           double* __restrict__ verts) {
-  // each wave lists its block's vertices (at most 3 per point) in LDS in id
-  // order and computes them one per lane, so the FP64 work is not spread
-  // over mostly idle lanes
-  __shared__ uint8_t s_pt[kMcWaves][3 * kMcBlock];
-  __shared__ uint8_t s_ax[kMcWaves][3 * kMcBlock];
-  const int64_t X = g.res[0], XY = X * g.res[1], N = XY * g.res[2];
-  const int64_t B = wave_block((N + kMcBlock - 1) / kMcBlock);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ uint16_t s_v[kMcWaves][3 * 64 * kVertWords];
+  __shared__ uint32_t s_near[kMcWaves][3][2 * kVertWords];
+  const int64_t X = a.g.res[0], w0 = wave_index() * kVertWords;
+  if (w0 >= a.nw) return;
+  const int lane = threadIdx.x & 63;
+  uint16_t* const list = s_v[threadIdx.x >> 6];
+  uint32_t(*near)[2 * kVertWords] = s_near[threadIdx.x >> 6];
+  if (lane < 3 * 2 * kVertWords) (&near[0][0])[lane] = 0u;
+  const uint64_t *const ex = a.edge[0], *const ey = a.edge[1], *const ez = a.edge[2];
   uint32_t total = 0;
-  if (B >= 0) {
-    unsigned pks[4];
 #pragma unroll
-    for (int sub = 0; sub < 4; sub++) {
-      const int64_t p = B * kMcBlock + sub * 64 + lane;
-      pks[sub] = p < N ? (unsigned)pk16[p] : 0u;
+  for (int i = 0; i < kVertWords; i++) {
+    uint64_t e[3] = {0, 0, 0};
+    if (w0 + i < a.nw) {
+      e[0] = ex[w0 + i];
+      e[1] = ey[w0 + i];
+      e[2] = ez[w0 + i];
     }
+    uint32_t k = total;
 #pragma unroll
-    for (int sub = 0; sub < 4; sub++) {
-      const int64_t p = B * kMcBlock + sub * 64 + lane;
-      unsigned bits = 0;
-      if (p < N) {
-        const unsigned pk = pks[sub];
-        bits = pk & 7u;
-        uint32_t k = pk >> 3;
-        for (int axis = 0; axis < 3; axis++)
-          if (bits & (1u << axis)) {
-            s_pt[w][k] = (uint8_t)(sub * 64 + lane);
-            s_ax[w][k] = (uint8_t)axis;
-            k++;
-          }
+    for (int axis = 0; axis < 3; axis++)
+      k = __builtin_amdgcn_mbcnt_hi((uint32_t)(e[axis] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)e[axis], k));
+#pragma unroll
+    for (int axis = 0; axis < 3; axis++)
+      if (__builtin_amdgcn_inverse_ballot_w64(e[axis])) list[k++] = (uint16_t)(i * 64 + lane | axis << 10);
+    total += (uint32_t)(__popcll(e[0]) + __popcll(e[1]) + __popcll(e[2]));
+  }
+  wave_sync();
+  if (total) {
+    const int64_t first = (int64_t)(base[0] + groups[w0 / kMcGroupWords] + ranks[8 * w0].x);
+    for (uint32_t j = lane; j < total; j += 64) {
+      const unsigned en = list[j];
+      const int axis = (int)(en >> 10), pt = (int)(en & 1023u);
+      const int64_t q = 64 * w0 + pt;
+      int64_t x, y, z;
+      point_xyz(a.g, q, x, y, z);
+      const double f0 = field[q], f1 = field[q + (axis == 0 ? 1 : (axis == 1 ? X : a.XY))];
+      const float h = fabsf((float)(axis == 0 ? a.g.dx[0] : (axis == 1 ? a.g.dx[1] : a.g.dx[2])));
+      if (!a.prefilter || mc_near((float)(f0 - a.iso), (float)(f1 - a.iso), h))
+        atomicOr(&near[axis][pt >> 5], 1u << (pt & 31));
+      double v[3];
+      mc_vertex(a.g, (int)x, (int)y, (int)z, axis, f0, f1, a.iso, v);
+      const int64_t id = first + j;
+      if (id < cap) {
+        verts[3 * id + 0] = v[0];
+        verts[3 * id + 1] = v[1];
+        verts[3 * id + 2] = v[2];
       }
-      total += wave_prefix3<1, 1, 1>(bits).total;
     }
   }
-  __syncthreads();
-  if (B < 0) return;
-  const int64_t first = (int64_t)base[0] + blk_off[B];
-  for (uint32_t j = lane; j < total; j += 64) {
-    const int64_t id = first + j;
-    if (id >= cap) break;
-    const int64_t q = B * kMcBlock + s_pt[w][j];
-    const int axis = s_ax[w][j];
-    int64_t x64, y64, z64;
-    point_xyz(g, q, x64, y64, z64);
-    double v[3];
-    mc_vertex(g, (int)x64, (int)y64, (int)z64, axis, field[q], field[q + (axis == 0 ? 1 : (axis == 1 ? X : XY))], iso,
-              v);
-    verts[3 * id + 0] = v[0];
-    verts[3 * id + 1] = v[1];
-    verts[3 * id + 2] = v[2];
+  wave_sync();
+  const int i = lane & (kVertWords - 1), axis = lane / kVertWords;
+  if (axis < 3 && w0 + i < a.nw)
+    (axis == 0 ? a.near[0] : (axis == 1 ? a.near[1] : a.near[2]))[w0 + i] =
+        (uint64_t)near[axis][2 * i + 1] << 32 | near[axis][2 * i];
+}
+
+// The degenerate filter (TRIANGLE_MESH.cpp:1088-1102) for one cell with two or
+// more near vertices: its triangles with two or three are measured with the
+// FP64 vertices (the function the vertex kernel uses, so both see the same
+// bits). Only a side between two near vertices can be short: a vertex that is
+// not near is at least 2e-7 from both ends of its edge, so at least that far
+// from a vertex on an edge through either end, and a grid spacing from vertices
+// on the other edges. Estimates come first (kSureShort): a border of one value
+// puts every vertex along it near, 1e-9 to 1e-6 from its corner. Returns the
+// dropped triangles' bits; *row: all of the row's.
+__device__ __forceinline__ unsigned mc_measure_cell(const double* __restrict__ field, const McGrid& a, int64_t p,
+                                                    unsigned* row) {
+  const int64_t X = a.g.res[0], XY = a.XY;
+  int64_t x, y, z;
+  point_xyz(a.g, p, x, y, z);
+  float v[8];
+  const int flag = mc_corners(field, p, X, XY, a.iso, v);
+  const int n = kMc.ntri[flag];
+  // per corner and pair of its edges (xy, xz, yz), bit 3 k + pair: surely short; not surely long
+  unsigned brief = 0, unsure = 0xffffffu;
+  if (a.prefilter == kMeasureUnsure) {
+    unsure = 0;
+    float d2[8][3];  // per corner and axis: the squared distance of the edge's vertex
+#pragma unroll
+    for (int e = 0; e < 12; e++) {
+      int dx = 0, dy = 0, dz = 0, axis = 0;
+      edge_parts(e, dx, dy, dz, axis);
+      const int k0 = 4 * dx + 2 * dy + dz, k1 = k0 + (axis == 0 ? 4 : (axis == 1 ? 2 : 1));
+      const float d = fabsf(v[k0] - v[k1]);
+      const float scale = d >= 1e-30f && d <= 1e30f ? fabsf((float)a.g.dx[axis]) * __builtin_amdgcn_rcpf(d)
+                                                    : __builtin_nanf("");
+      d2[k0][axis] = (v[k0] * scale) * (v[k0] * scale);
+      d2[k1][axis] = (v[k1] * scale) * (v[k1] * scale);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        const float d = d2[k][q == 2 ? 1 : 0] + d2[k][q == 0 ? 1 : 2];
+        brief |= d < kSureShort ? 1u << (3 * k + q) : 0u;
+        unsure |= d > kSureLong ? 0u : 1u << (3 * k + q);
+      }
+  }
+  unsigned dropped = 0;
+#pragma clang loop unroll(disable)
+  for (int t = 0; t < n; t++) {
+    const unsigned pairs = kMc.tpair[flag][t];
+    if (pairs & brief) dropped |= 1u << t;
+    if (a.prefilter && ((pairs & brief) || !(pairs & unsure))) continue;
+    const unsigned nm = mc_near_edges(v, a.g, a.prefilter) & kMc.tmask[flag][t];
+    const int m = __popc(nm);
+    if (m < 2) continue;
+    // the near vertices in turn against the one before and the first (one
+    // inlined vertex: instruction fetches weigh on a kernel this short)
+    const double eps = 1e-7;
+    double first[3] = {}, before[3] = {};
+    bool degenerate = false;
+    unsigned r = nm;
+#pragma clang loop unroll(disable)
+    for (int j = 0; j < m; j++) {
+      const int e = __ffs(r) - 1;
+      r &= r - 1;
+      int dx, dy, dz, axis;
+      edge_geom(e, dx, dy, dz, axis);
+      const int64_t q0 = p + dx + dy * X + dz * XY;
+      const int64_t q1 = q0 + (axis == 0 ? 1 : (axis == 1 ? X : XY));
+      double v1[3];
+      mc_vertex(a.g, (int)x + dx, (int)y + dy, (int)z + dz, axis, field[q0], field[q1], a.iso, v1);
+      if (j > 0) degenerate |= edge_len(before, v1) < eps;
+      if (j == 2) degenerate |= edge_len(first, v1) < eps;
+      for (int i = 0; i < 3; i++) {
+        first[i] = j == 0 ? v1[i] : first[i];
+        before[i] = v1[i];
+      }
+    }
+    if (degenerate) dropped |= 1u << t;
+  }
+  *row = (1u << n) - 1u;
+  return dropped;
+}
+
+// The cases of 8 cells from bit b on, one byte each: byte k of m holds corner
+// k's bits, transposed in three exchanges of blocks.
+__device__ __forceinline__ uint64_t cases8(const uint64_t* c, int b) {
+  uint64_t m = 0;
+#pragma unroll
+  for (int k = 0; k < 8; k++) m |= ((c[k] >> b) & 0xffull) << (8 * k);
+  uint64_t t = (m ^ (m >> 7)) & 0x00aa00aa00aa00aaull;
+  m ^= t ^ (t << 7);
+  t = (m ^ (m >> 14)) & 0x0000cccc0000ccccull;
+  m ^= t ^ (t << 14);
+  t = (m ^ (m >> 28)) & 0x00000000f0f0f0f0ull;
+  return m ^ t ^ (t << 28);
+}
+
+// Triangle counts, one word of cells per thread: the counts' three bits as
+// word operations on the corners' words. The degenerate filter measures the
+// cells with near vertices on two edges that meet at a corner, found the same
+// way (a border set by setBorders puts near vertices in every cell along it,
+// but on parallel edges), listed per wave and measured one per lane.
+// flags: the case of every cell that has
+// triangles, else 0. Latency-bound: 256^3, 1024 blocks, 21 us, of which the
+// measurement's longest chain is 9. tword: the triangles before word w in its group; groups:
+// per group.
+__global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict__ field, McGrid a,
+                                                       uint8_t* __restrict__ flags, uint8_t* __restrict__ kmask,
+                                                       uint32_t* __restrict__ tword,
+                                                       uint32_t* __restrict__ groups) {
+  __shared__ uint16_t s_list[kMcWaves][64 * 64];
+  __shared__ uint32_t s_drop[2 * kMcGroupWords], s_lost[kMcGroupWords];
+  const int64_t w = (int64_t)blockIdx.x * kMcGroupWords + threadIdx.x;
+  const int64_t X = a.g.res[0], XY = a.XY;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint64_t act = 0, candidates = 0;
+  uint32_t count = 0;
+  if (w < a.nw) {
+    const EndMasks end = end_masks(a, w);
+    const uint64_t valid = ~(end.x | end.y | end.z);
+    uint64_t c[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      c[k] = shifted_word(a.sgn, w, (k >> 2) + ((k >> 1) & 1) * X + (k & 1) * XY);
+    const uint64_t n0 = CountBits<0, 8, 0>::eval(c) & valid, n1 = CountBits<1, 8, 0>::eval(c) & valid,
+                   n2 = CountBits<2, 8, 0>::eval(c) & valid;
+    act = n0 | n1 | n2;
+    if (act) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) c[k] &= act;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; k++) c[k] = 0;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const uint64_t f0 = cases8(c, 16 * j), f1 = cases8(c, 16 * j + 8);
+      ((uint4*)flags)[4 * w + j] = uint4{(uint32_t)f0, (uint32_t)(f0 >> 32), (uint32_t)f1, (uint32_t)(f1 >> 32)};
+    }
+    count = (uint32_t)(__popcll(n0) + 2 * __popcll(n1) + 4 * __popcll(n2));
+    if (act && a.prefilter) {
+      uint64_t near[12];
+#pragma unroll
+      for (int e = 0; e < 12; e++) {
+        int dx = 0, dy = 0, dz = 0, axis = 0;
+        edge_parts(e, dx, dy, dz, axis);
+        near[e] = shifted_word(a.near[axis], w, dx + dy * X + dz * XY);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int dx = k >> 2, dy = (k >> 1) & 1, dz = k & 1;
+        const uint64_t nx = near[dy + 2 * dz], ny = near[4 + dx + 2 * dz], nz = near[8 + dx + 2 * dy];
+        candidates |= (nx & (ny | nz)) | (ny & nz);
+      }
+    } else {
+      candidates = ~0ull;
+    }
+    candidates &= act;
+  }
+  s_drop[2 * threadIdx.x] = s_drop[2 * threadIdx.x + 1] = 0u;
+  s_lost[threadIdx.x] = 0u;
+  const uint32_t mine = (uint32_t)__popcll(candidates), incl = wave_inclusive(mine), cells = wave_last(incl);
+  if (cells) {
+    uint32_t k = incl - mine;
+    for (uint64_t m = candidates; m; m &= m - 1)
+      s_list[wave][k++] = (uint16_t)(lane << 6 | (__ffsll((unsigned long long)m) - 1));
+    wave_sync();
+    const int64_t p0 = 64 * (w - lane);
+    for (uint32_t j = lane; j < cells; j += 64) {
+      const unsigned i = s_list[wave][j];
+      unsigned row;
+      const unsigned d = mc_measure_cell(field, a, p0 + i, &row);
+      if (d) {
+        kmask[p0 + i] = (uint8_t)(row & ~d);
+        atomicOr(&s_drop[2 * 64 * wave + (i >> 5)], 1u << (i & 31u));
+        atomicAdd(&s_lost[64 * wave + (i >> 6)], (uint32_t)__popc(d));
+      }
+    }
+    wave_sync();
+  }
+  count -= s_lost[threadIdx.x];
+  uint32_t total;
+  const uint32_t before = block_prefix<kMcBlock>(count, &total);
+  if (threadIdx.x == 0) groups[blockIdx.x] = total;
+  if (w < a.nw) {
+    a.drop[w] = (uint64_t)s_drop[2 * threadIdx.x + 1] << 32 | s_drop[2 * threadIdx.x];
+    tword[w] = before;
   }
 }
 
-// The vertex ids of the points that own the edges of a block's cells: the
-// owner of an edge of cell p is p + dx + dy*X + dz*XY, so they lie in 4 rows
-// of 257 points from the block's first point (this row, +y, +z, +y+z). Per
-// owner its pk16 word (first vertex id within its block << 3 | edge mask);
-// per row the first ids of the (at most two) blocks it spans and the entry
-// where the second begins.
-struct OwnerRows {
-  uint16_t pk[4][kMcBlock + 1];
-  uint32_t bo[4][2];
-  int32_t jb[4];
-};
-
-// The block's kept triangles in id order, (cell << 3) | triangle of the case
-// row, and the cells' cases.
-struct TriList {
-  uint16_t e[5 * kMcBlock];
-  uint8_t flag[kMcBlock];
-};
-
-// addVertexPairTriangle (TRIANGLE_MESH.cpp:2490-2503) in cell order then
-// table order, degenerate triangles dropped (kmask from k_mc_cells): the
-// block's kept triangles go to the running triangle total base[1] + the
-// block's first triangle. Each wave lists its block's kept triangles in LDS
-// and then writes them one per lane, so consecutive lanes write consecutive
-// triangles. Ids at or beyond tcap are not written.
-__global__ __launch_bounds__(kMcGroup) void k_mc_tris(const uint8_t* __restrict__ flags,
-                                                      const uint8_t* __restrict__ kmask, GridGeom g,
-                                                      const uint16_t* __restrict__ pk16,
-                                                      const uint32_t* __restrict__ blk_off,
-                                                      const uint64_t* __restrict__ base,
-                                                      const uint32_t* __restrict__ blk_toff, int64_t tcap,
+// addVertexPairTriangle (TRIANGLE_MESH.cpp:2490-2503) in cell order then table
+// order. A wave takes blocks of 256 cells, four consecutive ones per lane: it
+// lists a block's kept triangles (case row and triangle << 8 | cell) in LDS and
+// writes them one per lane, so that consecutive lanes write consecutive
+// triangles. The owner of an edge of cell p is p + dx + dy X + dz XY: four rows
+// of points, whose ranks are staged in LDS with the groups' offsets added, so
+// that a corner's vertex id is one LDS read and a masked bit count. Ids at or
+// beyond tcap are not written. Bound by vector instructions and LDS latency: a
+// 256^3 torus tile (9.1 million triangles, 109 MB) 62 us, 76 with a 16-bit rank
+// per point and case and kept bytes of every cell. `blocks` per wave: the
+// tables' staging is shared by up to kTriBlocks of them once the chip is full
+// (97 x 101 x 89, one block per wave: 6.5 us, four: 20.7).
+constexpr int kRankRow = 34;  // 8-point ranks per row: 257 points from any phase
+__global__ __launch_bounds__(kMcBlock) void k_mc_tris(McGrid a, int blocks, const uint8_t* __restrict__ flags,
+                                                      const uint64_t* __restrict__ drop,
+                                                      const uint8_t* __restrict__ kmask,
+                                                      const uint2* __restrict__ ranks,
+                                                      const uint32_t* __restrict__ vgroups,
+                                                      const uint32_t* __restrict__ tword,
+                                                      const uint32_t* __restrict__ tgroups,
+                                                      const uint64_t* __restrict__ base, int64_t tcap,
                                                       int32_t* __restrict__ tris) {
-  __shared__ uint32_t s_tc32[256 * 5 / 2];
-  __shared__ OwnerRows s_own[kMcWaves];
-  __shared__ TriList s_tl[kMcWaves];
-  unsigned short* s_tc = (unsigned short*)s_tc32;
-  stage_tri5(s_tc, kMc.tcorner);
-  const int64_t X = g.res[0], XY = X * g.res[1], N = XY * g.res[2];
-  const int64_t nb = (N + kMcBlock - 1) / kMcBlock;
-  const int64_t B = wave_block(nb);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  OwnerRows& own = s_own[w];
-  TriList& tl = s_tl[w];
-  uint32_t total = 0;
-  if (B >= 0) {
-    // every load of the staging issued before the first LDS write
-    const int64_t p0 = B * kMcBlock;
-    unsigned v[4][5], fl[4], km[4], bo[4][2] = {{0u, 0u}, {0u, 0u}, {0u, 0u}, {0u, 0u}};
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int64_t row = p0 + (r & 1) * X + (r >> 1) * XY;
-#pragma unroll
-      for (int k = 0; k < 5; k++) {
-        const int64_t q = row + lane + 64 * k;
-        v[r][k] = ((k < 4 || lane == 0) && q < N) ? (unsigned)pk16[q] : 0u;
-      }
-      const int64_t b0 = row / kMcBlock;
-      if (lane == 0) {
-        bo[r][0] = b0 < nb ? blk_off[b0] : 0u;
-        bo[r][1] = b0 + 1 < nb ? blk_off[b0 + 1] : 0u;
-      }
-    }
-#pragma unroll
-    for (int sub = 0; sub < 4; sub++) {
-      const int64_t p = p0 + sub * 64 + lane;
-      fl[sub] = p < N ? (unsigned)flags[p] : 0u;
-      km[sub] = p < N ? (unsigned)kmask[p] : 0u;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int64_t row = p0 + (r & 1) * X + (r >> 1) * XY;
-#pragma unroll
-      for (int k = 0; k < 5; k++)
-        if (k < 4 || lane == 0) own.pk[r][lane + 64 * k] = (uint16_t)v[r][k];
-      if (lane == 0) {
-        own.bo[r][0] = bo[r][0];
-        own.bo[r][1] = bo[r][1];
-        own.jb[r] = (int32_t)(kMcBlock - (row - (row / kMcBlock) * kMcBlock));
-      }
-    }
-#pragma unroll
-    for (int sub = 0; sub < 4; sub++) {
-      const int c = sub * 64 + lane;
-      const unsigned flag = fl[sub];
-      const unsigned keep = km[sub];
-      tl.flag[c] = (uint8_t)flag;
-      const WavePrefix tp = wave_prefix3<1, 2, 4>((unsigned)__popc(keep));
-      uint32_t k = total + tp.excl;
-      for (unsigned m = keep; m; m &= m - 1) tl.e[k++] = (uint16_t)(c << 3 | (__ffs(m) - 1));
-      total += tp.total;
-    }
+  __shared__ uint32_t s_te32[256 * 5 / 2];
+  __shared__ uint8_t s_n[256];
+  __shared__ uint32_t s_edge[12];
+  __shared__ uint32_t s_list[kMcWaves][5 * 256];
+  __shared__ uint2 s_rank[kMcWaves][4 * kRankRow];
+  const unsigned short* s_te = (const unsigned short*)s_te32;
+  const int64_t X = a.g.res[0], XY = a.XY;
+  for (int i = threadIdx.x; i < 640; i += kMcBlock) s_te32[i] = ((const uint32_t*)&kMc.tedge[0][0])[i];
+  s_n[threadIdx.x] = kMc.ntri[threadIdx.x];
+  if (threadIdx.x < 12) {
+    // per edge: its owner's place from the cell's in the staged rows << 2 | axis
+    int dx, dy, dz, axis;
+    edge_geom((int)threadIdx.x, dx, dy, dz, axis);
+    const int phase = (int)((dy * X + dz * XY) & 7);
+    s_edge[threadIdx.x] = (uint32_t)((dx + phase + 8 * kRankRow * (dy + 2 * dz)) << 2 | axis);
   }
   __syncthreads();
-  if (B < 0) return;
-  const int64_t o = (int64_t)base[1] + blk_toff[B];
-  for (uint32_t j = lane; j < total; j += 64) {
-    const int64_t t_id = o + j;
-    if (t_id >= tcap) break;
-    const unsigned e = tl.e[j];
-    const int c = (int)(e >> 3);
-    const unsigned tc = s_tc[tl.flag[c] * 5 + (e & 7u)];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t* const list = s_list[wave];
+  uint2* const rank = s_rank[wave];
+  const int64_t last_group = (a.nw - 1) / kMcGroupWords;
+  const int64_t B0 = wave_index() * blocks;
+  // the next block's cases are fetched while this one is written; words past the field's last hold no cells
+  uint32_t next = 4 * B0 + (lane >> 4) < a.nw ? ((const uint32_t*)flags)[64 * B0 + lane] : 0u;
+  for (int it = 0; it < blocks; it++) {
+    const int64_t w0 = 4 * (B0 + it);
+    const bool in = w0 + (lane >> 4) < a.nw;
+    const uint32_t f4 = next;
+    if (it + 1 < blocks) next = w0 + 4 + (lane >> 4) < a.nw ? ((const uint32_t*)flags)[16 * (w0 + 4) + lane] : 0u;
+    if (!__ballot(f4 != 0u)) continue;
+    // the four rows' ranks
+    uint2 rv[4];
+    uint32_t gv[4];
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const unsigned d = (tc >> (5 * k)) & 31u;
-      const int dx = d & 1, r = (d >> 1) & 3, axis = d >> 3;
-      const int jj = c + dx;
-      const unsigned pk = own.pk[r][jj];
-      tris[3 * t_id + k] = (int32_t)(own.bo[r][jj >= own.jb[r]] + (pk >> 3) + __popc(pk & ((1u << axis) - 1u)));
+    for (int r = 0; r < 4; r++) {
+      if (lane >= kRankRow) continue;
+      const int64_t q = 8 * w0 + (((r & 1) * X + (r >> 1) * XY) >> 3) + lane;
+      const int64_t gr = q / (kMcGroupPoints / 8);
+      rv[r] = ranks[q];
+      gv[r] = vgroups[gr < last_group ? gr : last_group];
     }
+    const uint64_t lost = in ? drop[w0 + (lane >> 4)] : 0;
+    unsigned keep = 0, lost4 = (unsigned)(lost >> (4 * (lane & 15))) & 15u;  // keep: 5 bits per cell
+    unsigned n[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) n[i] = s_n[(f4 >> (8 * i)) & 0xffu];
+    const bool some_lost = __ballot(lost4 != 0u) != 0;
+    if (some_lost) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        unsigned m = (1u << n[i]) - 1u;
+        if (lost4 >> i & 1u) m = kmask[64 * w0 + 4 * lane + i];
+        keep |= m << (5 * i);
+        n[i] = (unsigned)__popc(m);
+      }
+    }
+    const uint32_t mine = n[0] + n[1] + n[2] + n[3], incl = wave_inclusive(mine), total = wave_last(incl);
+    uint32_t at = incl - mine;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t e0 = (((f4 >> (8 * i)) & 0xffu) * 5u) << 8 | (uint32_t)(4 * lane + i);
+      if (some_lost) {
+        uint32_t k = at;
+        for (unsigned m = keep >> (5 * i) & 31u; m; m &= m - 1) list[k++] = e0 + ((uint32_t)(__ffs(m) - 1) << 8);
+      } else {
+#pragma unroll
+        for (uint32_t t = 0; t < 5; t++)
+          if (t < n[i]) list[at + t] = e0 + (t << 8);
+      }
+      at += n[i];
+    }
+    if (lane < kRankRow) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) rank[kRankRow * r + lane] = uint2{rv[r].x + gv[r], rv[r].y};
+    }
+    wave_sync();
+    const int64_t o = (int64_t)(base[1] + tgroups[w0 / kMcGroupWords] + tword[w0]);
+    for (uint32_t j = lane; j < total; j += 64) {
+      const uint32_t e = list[j];
+      const uint32_t te = s_te[e >> 8], c = e & 255u;
+      int32_t id[3];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const uint32_t ed = s_edge[(te >> (4 * k)) & 15u], q = c + (ed >> 2);
+        const uint2 rk = rank[q >> 3];
+        id[k] = (int32_t)(rk.x + (uint32_t)__popc(rk.y & ((1u << (3u * (q & 7u) + (ed & 3u))) - 1u)));
+      }
+      if (o + j < tcap) {
+        int32_t* const out = tris + 3 * (o + j);
+        out[0] = id[0];
+        out[1] = id[1];
+        out[2] = id[2];
+      }
+    }
+    wave_sync();
   }
-}
-
-// After a tile: its vertex and triangle counts (the scans' totals) recorded
-// and added to the running totals.
-// (Both also clear the measure-list counters for the next field.)
-__global__ void k_mc_advance(const uint32_t* __restrict__ totals, uint64_t* __restrict__ base, int tile,
-                             int64_t* __restrict__ counts, uint32_t* __restrict__ mcount) {
-  for (int i = threadIdx.x; i <= kMeasureLists; i += blockDim.x) mcount[i] = 0u;
-  if (threadIdx.x != 0) return;
-  const uint64_t nv = totals[1], nt = totals[2];
-  counts[2 * tile + 0] = (int64_t)nv;
-  counts[2 * tile + 1] = (int64_t)nt;
-  base[0] += nv;
-  base[1] += nt;
-}
-
-__global__ void k_mc_reset(uint64_t* __restrict__ base, uint32_t* __restrict__ mcount) {
-  for (int i = threadIdx.x; i <= kMeasureLists; i += blockDim.x) mcount[i] = 0u;
-  if (threadIdx.x < 2) base[threadIdx.x] = 0;
 }
 
 // koff is the exclusive scan of the keep flags: triangle i is kept when its
@@ -810,11 +978,6 @@ static qj_status grow(T*& p, int64_t& cap, int64_t n, hipStream_t s) {
 
 static unsigned nblocks(int64_t n) { return (unsigned)((n + kMcBlock - 1) / kMcBlock); }
 
-__global__ void k_mc_zero_totals(uint32_t* __restrict__ totals) {
-  if (threadIdx.x < 4) totals[threadIdx.x] = 0u;
-}
-
-
 // Meshes n fields one after another on the stream without waiting on the
 // host: every count stays on the device (running vertex and triangle totals,
 // per-tile counts) and is read back once at the end. The vertex and triangle
@@ -833,8 +996,8 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
   m.cache_valid = false;
   if (n <= 0) return QJ_OK;
   std::vector<GridGeom> geo((size_t)n);
-  std::vector<bool> prefilter((size_t)n);
-  int64_t nmax = 0, total_pts = 0;
+  std::vector<int> prefilter((size_t)n);
+  int64_t nmax = 0, total_pts = 0, pad_max = 0;
   for (int k = 0; k < n; k++) {
     GridGeom& g = geo[(size_t)k];
     make_geom(&grids[k], &g);
@@ -847,6 +1010,7 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
     }
     nmax = N > nmax ? N : nmax;
     total_pts += N;
+    pad_max = std::max(pad_max, mc_pad_words(g));
     // the degenerate-test prefilter holds when the cell-centre map is a
     // rotation (edges meeting at a corner stay perpendicular) and every grid
     // spacing lies in [kPrefilterSpacing, kPrefilterMaxSpacing]
@@ -858,76 +1022,74 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
         pf &= fabs(d - (i == j ? 1.0 : 0.0)) < 1e-9;
       }
     }
-    prefilter[(size_t)k] = pf;
+    double extent = 0.0;
+    for (int i = 0; i < 3; i++) extent += fabs(g.center[i]) + fabs(g.lengths[i]);
+    prefilter[(size_t)k] = !pf ? kMeasureAll : (extent <= kSureExtent ? kMeasureUnsure : kMeasureNear);
   }
   qj_status st;
-  const int64_t nbmax = nblocks(nmax);
-  if ((st = grow(m.flags, m.cap_flags, nmax, s)) || (st = grow(m.kmask, m.cap_kmask, nmax, s)) ||
-      (st = grow(m.pk16, m.cap_pk16, nmax, s)) || (st = grow(m.blkv, m.cap_blkv, nbmax, s)) ||
-      (st = grow(m.mlist, m.cap_mlist, std::max(nmax / 16, (int64_t)kMeasureLists * 256), s)) ||
-      (st = grow(m.blkt, m.cap_blkt, nbmax, s)) || (st = grow(m.d_counts, m.cap_counts, 2 * (int64_t)n, s)))
+  // words of 64 points, plus what the reads of a word's +y and +z rows run past the end
+  const int64_t wmax = (nmax + 63) / 64 + pad_max;
+  const int64_t gmax = (nmax + kMcGroupPoints - 1) / kMcGroupPoints;
+  if ((st = grow(m.words, m.cap_words, kMcArrays * wmax, s)) || (st = grow(m.ranks, m.cap_ranks, 8 * wmax, s)) ||
+      (st = grow(m.flags, m.cap_flags, 64 * ((nmax + 63) / 64), s)) || (st = grow(m.kmask, m.cap_kmask, nmax, s)) || (st = grow(m.tword, m.cap_tword, wmax, s)) ||
+      (st = grow(m.groups, m.cap_groups, 2 * gmax, s)) || (st = grow(m.d_base, m.cap_base, 2 * ((int64_t)n + 1), s)))
     return st;
-  const size_t need_tmp = scan_tmp_bytes(nbmax > 4096 ? nbmax : 4096);
-  if (need_tmp > m.tmp_bytes) {
-    if (m.tmp) {
-      QJ_HIP(hipStreamSynchronize(s));
-      QJ_HIP(hipFree(m.tmp));
-    }
-    m.tmp = nullptr;
-    m.tmp_bytes = 0;
-    QJ_HIP(hipMalloc(&m.tmp, need_tmp));
-    m.tmp_bytes = need_tmp;
-  }
-  if (!m.totals) QJ_HIP(hipMalloc(&m.totals, 4 * sizeof(uint32_t)));
-  if (!m.d_base) QJ_HIP(hipMalloc(&m.d_base, 2 * sizeof(uint64_t)));
-  if (!m.d_mcount) QJ_HIP(hipMalloc(&m.d_mcount, sizeof(uint32_t) * (kMeasureLists + 1)));
   // first sizes: a quarter of the points as vertices, half as triangles
   // (a 256^3 torus tile holds 0.42 and 0.73 of its points)
   if (!ext && m.cap_v == 0 && (st = grow(m.verts, m.cap_v, 3 * (total_pts / 4 + 1024), s))) return st;
   if (!ext && m.cap_t == 0 && (st = grow(m.tris, m.cap_t, 3 * (total_pts / 2 + 1024), s))) return st;
+  std::vector<uint64_t> base(2 * ((size_t)n + 1));
   std::vector<int64_t> counts(2 * (size_t)n);
   uint64_t totals[2] = {0, 0};
   for (int pass = 0; pass < 2; pass++) {
     const int64_t vcap = ext ? ext_vcap : m.cap_v / 3, tcap = ext ? ext_tcap : m.cap_t / 3;
     double* const verts = ext ? ext_v : m.verts;
     int32_t* const tris = ext ? ext_t : m.tris;
-    hipLaunchKernelGGL(k_mc_reset, dim3(1), dim3(64), 0, s, m.d_base, m.d_mcount);
-    QJ_HIP(hipGetLastError());
     for (int k = 0; k < n; k++) {
       const GridGeom& g = geo[(size_t)k];
       const int64_t N = (int64_t)g.res[0] * g.res[1] * g.res[2];
       const int64_t cells = (int64_t)(g.res[0] - 1) * (g.res[1] - 1) * (g.res[2] - 1);
-      const dim3 nb(nblocks(N));
-      if (cells <= 0) {
-        hipLaunchKernelGGL(k_mc_zero_totals, dim3(1), dim3(64), 0, s, m.totals);
+      const McGrid mg = make_mc_grid(m, g, wmax, iso, prefilter[(size_t)k]);
+      const int64_t ng = cells > 0 ? (N + kMcGroupPoints - 1) / kMcGroupPoints : 0;
+      uint32_t *gv = m.groups, *gt = m.groups + gmax;
+      const auto blocks_of = [](int64_t items, int64_t per) { return dim3((unsigned)((items + per - 1) / per)); };
+      if (ng) {
+        hipLaunchKernelGGL(k_mc_signs, blocks_of(N, kSignPoints * kMcBlock), dim3(kMcBlock), 0, s, fields[k], N, iso,
+                           mg.sgn);
         QJ_HIP(hipGetLastError());
-      } else {
-        const int pf = prefilter[(size_t)k] ? 1 : 0;
-        const dim3 nwg((nb.x + kMcWaves - 1) / kMcWaves);
-        const uint32_t mcap = (uint32_t)(m.cap_mlist / kMeasureLists);  // entries per sub-list
-        hipLaunchKernelGGL(k_mc_cells, nb, dim3(kMcBlock), 0, s, fields[k], g, iso, pf, m.flags, m.kmask, m.blkt,
-                           m.mlist, m.d_mcount, mcap);
-        QJ_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_mc_measure, dim3(std::min<unsigned>(nb.x, 1024u)), dim3(kMcBlock), 0, s, fields[k], g,
-                           iso, pf, (const uint32_t*)m.mlist, (const uint32_t*)m.d_mcount, mcap, m.kmask, m.blkt);
-        QJ_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_mc_edges, nwg, dim3(kMcGroup), 0, s, m.flags, g, m.pk16, m.blkv);
-        QJ_HIP(hipGetLastError());
-        if ((st = scan_u32(m.blkv, m.blkv, nb.x, m.totals + 1, m.tmp, m.tmp_bytes, s))) return st;
-        hipLaunchKernelGGL(k_mc_vertices, nwg, dim3(kMcGroup), 0, s, fields[k], g, iso, m.pk16, m.blkv,
-                           (const uint64_t*)m.d_base, vcap, verts);
-        QJ_HIP(hipGetLastError());
-        if ((st = scan_u32(m.blkt, m.blkt, nb.x, m.totals + 2, m.tmp, m.tmp_bytes, s))) return st;
-        hipLaunchKernelGGL(k_mc_tris, nwg, dim3(kMcGroup), 0, s, m.flags, m.kmask, g, m.pk16, m.blkv,
-                           (const uint64_t*)m.d_base, m.blkt, tcap, tris);
+        hipLaunchKernelGGL(k_mc_edges, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.ranks, gv);
         QJ_HIP(hipGetLastError());
       }
-      hipLaunchKernelGGL(k_mc_advance, dim3(1), dim3(64), 0, s, m.totals, m.d_base, k, m.d_counts, m.d_mcount);
+      hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gv, ng, m.d_base, k, 0);
       QJ_HIP(hipGetLastError());
+      if (ng) {
+        hipLaunchKernelGGL(k_mc_vertices, blocks_of(mg.nw, kVertWords * kMcWaves), dim3(kMcBlock), 0, s, fields[k], mg,
+                           (const uint2*)m.ranks, (const uint32_t*)gv, (const uint64_t*)(m.d_base + 2 * k), vcap,
+                           verts);
+        QJ_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_mc_cells, dim3((unsigned)ng), dim3(kMcBlock), 0, s, fields[k], mg, m.flags, m.kmask,
+                           m.tword, gt);
+        QJ_HIP(hipGetLastError());
+      }
+      hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gt, ng, m.d_base, k, 1);
+      QJ_HIP(hipGetLastError());
+      if (ng) {
+        const int64_t nb = (mg.nw + 3) / 4;
+        const int per = (int)std::min<int64_t>(kTriBlocks, std::max<int64_t>(1, nb / kTriWaves));
+        hipLaunchKernelGGL(k_mc_tris, blocks_of(nb, per * kMcWaves), dim3(kMcBlock), 0, s, mg, per,
+                           (const uint8_t*)m.flags, (const uint64_t*)mg.drop, (const uint8_t*)m.kmask,
+                           (const uint2*)m.ranks, (const uint32_t*)gv, (const uint32_t*)m.tword, (const uint32_t*)gt,
+                           (const uint64_t*)(m.d_base + 2 * k), tcap, tris);
+        QJ_HIP(hipGetLastError());
+      }
     }
-    QJ_HIP(hipMemcpyAsync(counts.data(), m.d_counts, sizeof(int64_t) * 2 * (size_t)n, hipMemcpyDeviceToHost, s));
-    QJ_HIP(hipMemcpyAsync(totals, m.d_base, sizeof(totals), hipMemcpyDeviceToHost, s));
+    QJ_HIP(hipMemcpyAsync(base.data(), m.d_base, sizeof(uint64_t) * base.size(), hipMemcpyDeviceToHost, s));
     QJ_HIP(hipStreamSynchronize(s));
+    for (int k = 0; k < n; k++)
+      for (int i = 0; i < 2; i++)
+        counts[2 * (size_t)k + i] = (int64_t)(base[2 * ((size_t)k + 1) + i] - base[2 * (size_t)k + i]);
+    totals[0] = base[2 * (size_t)n];
+    totals[1] = base[2 * (size_t)n + 1];
     if ((int64_t)totals[0] <= vcap && (int64_t)totals[1] <= tcap) break;
     if (ext) {
       // the caller's buffers are too small: report the sizes needed
@@ -986,12 +1148,11 @@ void mc_free(qj_workspace* ws) {
   hipFree(m->flags);
   hipFree(m->emask);
   hipFree(m->cnt);
-  hipFree(m->pk16);
-  hipFree(m->mlist);
-  hipFree(m->d_mcount);
+  hipFree(m->words);
+  hipFree(m->ranks);
   hipFree(m->kmask);
-  hipFree(m->blkt);
-  hipFree(m->blkv);
+  hipFree(m->tword);
+  hipFree(m->groups);
   hipFree(m->blk);
   hipFree(m->active);
   hipFree(m->tri_off);
@@ -1016,7 +1177,6 @@ void mc_free(qj_workspace* ws) {
   hipFree(m->c_edges);
   hipFree(m->c_cells);
   hipFree(m->d_base);
-  hipFree(m->d_counts);
   delete m;
   ws->mc = nullptr;
 }
