@@ -92,15 +92,10 @@ constexpr McTables make_tables() {
 constexpr McTables kMcHost = make_tables();
 __constant__ McTables kMc = make_tables();
 
-// Case tables staged in LDS for the kernels that look them up per lane: with
-// divergent indices, reads of __constant__ memory are scattered vector loads
-// (12 per grid point in the edge kernels); from LDS they are ds_reads.
+// The triangle table staged in LDS for the kernels that look it up per lane: with
+// divergent indices, reads of __constant__ memory are scattered vector loads;
+// from LDS they are ds_reads.
 static_assert(kMcBlock == 256, "one table entry per thread");
-
-__device__ __forceinline__ void stage_emask(unsigned short* s_em) {
-  s_em[threadIdx.x] = kMc.emask[threadIdx.x];
-  __syncthreads();
-}
 
 // s_tri: the 256 x 16 triangle table as 1024 words; s_ntri: triangles per case
 __device__ __forceinline__ void stage_tri(uint32_t* s_tri, uint8_t* s_ntri) {
@@ -124,11 +119,9 @@ __device__ __forceinline__ double sq3(double e0, double e1, double e2) {
 }
 
 struct McState {
-  int64_t cap_flags = 0, cap_emask = 0, cap_cnt = 0, cap_active = 0, cap_toff = 0, cap_blk = 0;
+  int64_t cap_flags = 0, cap_toff = 0;
   int64_t cap_v = 0, cap_tp = 0, cap_keep = 0, cap_t = 0;
   uint8_t* flags = nullptr;
-  uint8_t* emask = nullptr;
-  uint32_t* cnt = nullptr;     // per point edge count -> vertex base (scanned in place; non-linear mesher)
   // linear mesher: bit words of 64 points each (kMcArrays arrays of one
   // length), vertex ranks per 8 points, kept triangles of the cells that lost
   // some, first triangle per word, counts per group of 16384 points
@@ -138,8 +131,6 @@ struct McState {
   uint32_t* tword = nullptr;
   uint32_t* groups = nullptr;
   int64_t cap_words = 0, cap_ranks = 0, cap_kmask = 0, cap_tword = 0, cap_groups = 0;
-  uint32_t* blk = nullptr;     // per block active count -> offset
-  uint32_t* active = nullptr;  // active cells
   uint32_t* tri_off = nullptr; // per active cell triangle count -> offset
   double* verts = nullptr;
   int32_t* tris_pre = nullptr;
@@ -156,8 +147,8 @@ struct McState {
   int64_t cap_slab[2] = {0, 0};
   hipStream_t s2 = nullptr;
   hipEvent_t ev_start = nullptr, ev_field[2] = {nullptr, nullptr}, ev_free[2] = {nullptr, nullptr};
-  uint32_t* slice_off = nullptr;
-  int64_t cap_slice = 0;
+  uint32_t *aword = nullptr, *lost = nullptr;  // per word: active cells before it in its group; dropped triangles
+  int64_t cap_aword = 0, cap_lost = 0;
   uint32_t* vpt = nullptr;  // vertices of a range of points: owning point, edge axis
   uint8_t* vax = nullptr;
   int64_t cap_vpt = 0, cap_vax = 0;
@@ -172,18 +163,6 @@ struct McState {
   uint64_t* d_base = nullptr;
   int64_t cap_base = 0;
 };
-
-__device__ __forceinline__ int cell_flag(const double* __restrict__ f, int64_t i, int64_t X, int64_t XY, double iso) {
-  // CUBE corners are floats (TRIANGLE_MESH.h:283-288); test at TRIANGLE_MESH.cpp:1037-1039
-  int flag = 0;
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const int dx = k >> 2, dy = (k >> 1) & 1, dz = k & 1;
-    const float v = (float)(f[i + dx + dy * X + dz * XY] - iso);
-    flag |= (v > 0.0f) << k;
-  }
-  return flag;
-}
 
 // grid coordinates of a point index (the mesher runs on fields of < 2^32 points)
 __device__ __forceinline__ void point_xyz(const GridGeom& g, int64_t p, int64_t& x, int64_t& y, int64_t& z) {
@@ -253,6 +232,7 @@ constexpr double kPrefilterMaxSpacing = 3.0;
 // measured. kMeasureNear: coordinates beyond that. kMeasureAll: no prefilter.
 constexpr float kSureShort = 0.99e-7f * 0.99e-7f, kSureLong = 1.01e-7f * 1.01e-7f;
 constexpr double kSureExtent = 1e4;
+constexpr double kSureSpacing = 1e-4;
 enum McPrefilter { kMeasureAll = 0, kMeasureNear = 1, kMeasureUnsure = 2 };
 
 // Whether the vertex of an edge with end values v0, v1 and grid spacing h may
@@ -303,6 +283,7 @@ constexpr int kSignPoints = 8;                 // points per thread of k_mc_sign
 constexpr int kVertWords = 8;                  // words per wave of k_mc_vertices
 constexpr int kTriBlocks = 4;                  // blocks of 256 cells per wave of k_mc_tris, at most
 constexpr int kTriWaves = 256 * 16;            // waves that fill the chip before one takes a second block
+constexpr int kListWords = 4;                  // words per wave of k_nl_vlist
 constexpr int kScanBlock = 1024;
 
 // Words whose bit i is point (or cell with lowest corner) 64 w + i; each array
@@ -314,6 +295,9 @@ struct McGrid {
   double iso;
   int prefilter;
   int64_t N, XY, nw;  // points, points per slice, words
+  int64_t cells;      // cells with a lowest corner below this
+  int64_t owned;      // edges of points below this
+  bool floor;         // slice 0 is the grid's (not a slab's inside it)
   uint64_t* sgn;      // field value above the isovalue
   uint64_t* edge[3];  // the point's +x, +y, +z edge carries a vertex
   uint64_t* near[3];  // ... that may lie near an end of the edge
@@ -333,6 +317,9 @@ static McGrid make_mc_grid(const McState& m, const GridGeom& g, int64_t wmax, do
   a.XY = (int64_t)g.res[0] * g.res[1];
   a.N = a.XY * g.res[2];
   a.nw = (a.N + 63) / 64;
+  a.cells = a.N - a.XY;
+  a.owned = a.N;
+  a.floor = true;
   uint64_t* p[kMcArrays];
   for (int i = 0; i < kMcArrays; i++) p[i] = m.words + i * wmax;
   a.sgn = p[0];
@@ -506,17 +493,16 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_edges(McGrid a, uint2* __restri
   if (w < a.nw) {
     const uint64_t s0 = a.sgn[w];
     const EndMasks end = end_masks(a, w);
-    const uint64_t in = ~bits_from(a.N - 64 * w);
+    const uint64_t in = ~bits_from(a.owned - 64 * w);
     e[0] = (s0 ^ shifted_word(a.sgn, w, 1)) & ~end.x & in;
     e[1] = (s0 ^ shifted_word(a.sgn, w, X)) & ~end.y & in;
-    e[2] = (s0 ^ shifted_word(a.sgn, w, a.XY)) & ~end.z;
-    const uint64_t z0 = ~bits_from(a.XY - 64 * w);                                // z = 0
-    const uint64_t y0z0 = ~bits_from(X - 64 * w);                                 // and y = 0
-    const uint32_t p0 = (uint32_t)(64 * w), slice = fast_div(p0, a.g.div_xy);
-    uint64_t y0 = y0z0;                                                           // y = 0
-    for (int64_t b = (int64_t)(slice + (slice > 0 ? 0 : 1)) * a.XY - (int64_t)p0; b < 64; b += a.XY)
+    e[2] = (s0 ^ shifted_word(a.sgn, w, a.XY)) & ~end.z & in;
+    const uint64_t z0 = a.floor ? ~bits_from(a.XY - 64 * w) : 0;  // z = 0
+    const uint32_t p0 = (uint32_t)(64 * w);
+    uint64_t y0 = 0;  // y = 0
+    for (int64_t b = (int64_t)fast_div(p0, a.g.div_xy) * a.XY - (int64_t)p0; b < 64; b += a.XY)
       y0 |= bits_from(b) & ~bits_from(b + X);
-    const uint64_t line[3] = {y0z0, z0 & end.x, y0 & end.x};
+    const uint64_t line[3] = {y0 & z0, z0 & end.x, y0 & end.x};
 #pragma unroll
     for (int axis = 0; axis < 3; axis++)
       for (uint64_t m = e[axis] & line[axis]; m; m &= m - 1) {
@@ -730,6 +716,29 @@ __device__ __forceinline__ uint64_t cases8(const uint64_t* c, int b) {
   return m ^ t ^ (t << 28);
 }
 
+// Word w's cells: *count triangles, the cases of those that have any (else 0)
+// to flags; returns those cells' bits.
+__device__ __forceinline__ uint64_t word_cases(const McGrid& a, int64_t w, uint8_t* __restrict__ flags,
+                                               uint32_t* count) {
+  const EndMasks end = end_masks(a, w);
+  const uint64_t valid = ~(end.x | end.y | end.z | bits_from(a.cells - 64 * w));
+  uint64_t c[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++)
+    c[k] = shifted_word(a.sgn, w, (k >> 2) + ((k >> 1) & 1) * (int64_t)a.g.res[0] + (k & 1) * a.XY);
+  const uint64_t n0 = CountBits<0, 8, 0>::eval(c) & valid, n1 = CountBits<1, 8, 0>::eval(c) & valid,
+                 n2 = CountBits<2, 8, 0>::eval(c) & valid, act = n0 | n1 | n2;
+#pragma unroll
+  for (int k = 0; k < 8; k++) c[k] &= act;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const uint64_t f0 = cases8(c, 16 * j), f1 = cases8(c, 16 * j + 8);
+    ((uint4*)flags)[4 * w + j] = uint4{(uint32_t)f0, (uint32_t)(f0 >> 32), (uint32_t)f1, (uint32_t)(f1 >> 32)};
+  }
+  *count = (uint32_t)(__popcll(n0) + 2 * __popcll(n1) + 4 * __popcll(n2));
+  return act;
+}
+
 // Triangle counts, one word of cells per thread: the counts' three bits as
 // word operations on the corners' words. The degenerate filter measures the
 // cells with near vertices on two edges that meet at a corner, found the same
@@ -751,28 +760,7 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict_
   uint64_t act = 0, candidates = 0;
   uint32_t count = 0;
   if (w < a.nw) {
-    const EndMasks end = end_masks(a, w);
-    const uint64_t valid = ~(end.x | end.y | end.z);
-    uint64_t c[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-      c[k] = shifted_word(a.sgn, w, (k >> 2) + ((k >> 1) & 1) * X + (k & 1) * XY);
-    const uint64_t n0 = CountBits<0, 8, 0>::eval(c) & valid, n1 = CountBits<1, 8, 0>::eval(c) & valid,
-                   n2 = CountBits<2, 8, 0>::eval(c) & valid;
-    act = n0 | n1 | n2;
-    if (act) {
-#pragma unroll
-      for (int k = 0; k < 8; k++) c[k] &= act;
-    } else {
-#pragma unroll
-      for (int k = 0; k < 8; k++) c[k] = 0;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const uint64_t f0 = cases8(c, 16 * j), f1 = cases8(c, 16 * j + 8);
-      ((uint4*)flags)[4 * w + j] = uint4{(uint32_t)f0, (uint32_t)(f0 >> 32), (uint32_t)f1, (uint32_t)(f1 >> 32)};
-    }
-    count = (uint32_t)(__popcll(n0) + 2 * __popcll(n1) + 4 * __popcll(n2));
+    act = word_cases(a, w, flags, &count);
     if (act && a.prefilter) {
       uint64_t near[12];
 #pragma unroll
@@ -829,8 +817,9 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict_
 // writes them one per lane, so that consecutive lanes write consecutive
 // triangles. The owner of an edge of cell p is p + dx + dy X + dz XY: four rows
 // of points, whose ranks are staged in LDS with the groups' offsets added, so
-// that a corner's vertex id is one LDS read and a masked bit count. Ids at or
-// beyond tcap are not written. Bound by vector instructions and LDS latency: a
+// that a corner's vertex id is one LDS read and a masked bit count; ids count
+// from id0, triangles from base[1] (null: 0). Triangles at or beyond tcap are not
+// written. Bound by vector instructions and LDS latency: a
 // 256^3 torus tile (9.1 million triangles, 109 MB) 62 us, 76 with a 16-bit rank
 // per point and case and kept bytes of every cell. `blocks` per wave: the
 // tables' staging is shared by up to kTriBlocks of them once the chip is full
@@ -843,7 +832,7 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_tris(McGrid a, int blocks, cons
                                                       const uint32_t* __restrict__ vgroups,
                                                       const uint32_t* __restrict__ tword,
                                                       const uint32_t* __restrict__ tgroups,
-                                                      const uint64_t* __restrict__ base, int64_t tcap,
+                                                      const uint64_t* __restrict__ base, uint32_t id0, int64_t tcap,
                                                       int32_t* __restrict__ tris) {
   __shared__ uint32_t s_te32[256 * 5 / 2];
   __shared__ uint8_t s_n[256];
@@ -918,10 +907,10 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_tris(McGrid a, int blocks, cons
     }
     if (lane < kRankRow) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) rank[kRankRow * r + lane] = uint2{rv[r].x + gv[r], rv[r].y};
+      for (int r = 0; r < 4; r++) rank[kRankRow * r + lane] = uint2{rv[r].x + gv[r] + id0, rv[r].y};
     }
     wave_sync();
-    const int64_t o = (int64_t)(base[1] + tgroups[w0 / kMcGroupWords] + tword[w0]);
+    const int64_t o = (int64_t)((base ? base[1] : 0) + tgroups[w0 / kMcGroupWords] + tword[w0]);
     for (uint32_t j = lane; j < total; j += 64) {
       const uint32_t e = list[j];
       const uint32_t te = s_te[e >> 8], c = e & 255u;
@@ -978,6 +967,42 @@ static qj_status grow(T*& p, int64_t& cap, int64_t n, hipStream_t s) {
 
 static unsigned nblocks(int64_t n) { return (unsigned)((n + kMcBlock - 1) / kMcBlock); }
 
+// whether the cell-centre map is a rotation (edges meeting at a corner stay
+// perpendicular) and every grid spacing lies in [lo, hi]
+template <class G>
+static bool is_turned_grid(const G& g, double lo, double hi) {
+  bool ok = true;
+  for (int i = 0; i < 3; i++) {
+    ok &= fabs(g.dx[i]) >= lo && fabs(g.dx[i]) <= hi;
+    for (int j = 0; j < 3; j++) {
+      const double d = g.rot[i] * g.rot[j] + g.rot[3 + i] * g.rot[3 + j] + g.rot[6 + i] * g.rot[6 + j];
+      ok &= fabs(d - (i == j ? 1.0 : 0.0)) < 1e-9;
+    }
+  }
+  return ok;
+}
+
+// a bound on the coordinates' magnitudes
+template <class G>
+static double grid_extent(const G& g) {
+  double e = 0.0;
+  for (int i = 0; i < 3; i++) e += fabs(g.center[i]) + fabs(g.dx[i]) * g.res[i];
+  return e;
+}
+
+static dim3 blocks_of(int64_t items, int64_t per) { return dim3((unsigned)((items + per - 1) / per)); }
+
+static qj_status launch_tris(const McState& m, const McGrid& mg, const uint32_t* gv, const uint32_t* gt,
+                             const uint64_t* base, uint32_t id0, int64_t tcap, int32_t* tris, hipStream_t s) {
+  const int64_t nb = (mg.nw + 3) / 4;
+  const int per = (int)std::min<int64_t>(kTriBlocks, std::max<int64_t>(1, nb / kTriWaves));
+  hipLaunchKernelGGL(k_mc_tris, blocks_of(nb, per * kMcWaves), dim3(kMcBlock), 0, s, mg, per, (const uint8_t*)m.flags,
+                     (const uint64_t*)mg.drop, (const uint8_t*)m.kmask, (const uint2*)m.ranks, gv,
+                     (const uint32_t*)m.tword, gt, base, id0, tcap, tris);
+  QJ_HIP(hipGetLastError());
+  return QJ_OK;
+}
+
 // Meshes n fields one after another on the stream without waiting on the
 // host: every count stays on the device (running vertex and triangle totals,
 // per-tile counts) and is read back once at the end. The vertex and triangle
@@ -1011,20 +1036,9 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
     nmax = N > nmax ? N : nmax;
     total_pts += N;
     pad_max = std::max(pad_max, mc_pad_words(g));
-    // the degenerate-test prefilter holds when the cell-centre map is a
-    // rotation (edges meeting at a corner stay perpendicular) and every grid
-    // spacing lies in [kPrefilterSpacing, kPrefilterMaxSpacing]
-    bool pf = true;
-    for (int i = 0; i < 3; i++) {
-      pf &= fabs(g.dx[i]) >= kPrefilterSpacing && fabs(g.dx[i]) <= kPrefilterMaxSpacing;
-      for (int j = 0; j < 3; j++) {
-        const double d = g.rot[i] * g.rot[j] + g.rot[3 + i] * g.rot[3 + j] + g.rot[6 + i] * g.rot[6 + j];
-        pf &= fabs(d - (i == j ? 1.0 : 0.0)) < 1e-9;
-      }
-    }
-    double extent = 0.0;
-    for (int i = 0; i < 3; i++) extent += fabs(g.center[i]) + fabs(g.lengths[i]);
-    prefilter[(size_t)k] = !pf ? kMeasureAll : (extent <= kSureExtent ? kMeasureUnsure : kMeasureNear);
+    prefilter[(size_t)k] = !is_turned_grid(g, kPrefilterSpacing, kPrefilterMaxSpacing) ? kMeasureAll
+                           : grid_extent(g) <= kSureExtent                            ? kMeasureUnsure
+                                                                                      : kMeasureNear;
   }
   qj_status st;
   // words of 64 points, plus what the reads of a word's +y and +z rows run past the end
@@ -1052,7 +1066,6 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
       const McGrid mg = make_mc_grid(m, g, wmax, iso, prefilter[(size_t)k]);
       const int64_t ng = cells > 0 ? (N + kMcGroupPoints - 1) / kMcGroupPoints : 0;
       uint32_t *gv = m.groups, *gt = m.groups + gmax;
-      const auto blocks_of = [](int64_t items, int64_t per) { return dim3((unsigned)((items + per - 1) / per)); };
       if (ng) {
         hipLaunchKernelGGL(k_mc_signs, blocks_of(N, kSignPoints * kMcBlock), dim3(kMcBlock), 0, s, fields[k], N, iso,
                            mg.sgn);
@@ -1074,13 +1087,7 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
       hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gt, ng, m.d_base, k, 1);
       QJ_HIP(hipGetLastError());
       if (ng) {
-        const int64_t nb = (mg.nw + 3) / 4;
-        const int per = (int)std::min<int64_t>(kTriBlocks, std::max<int64_t>(1, nb / kTriWaves));
-        hipLaunchKernelGGL(k_mc_tris, blocks_of(nb, per * kMcWaves), dim3(kMcBlock), 0, s, mg, per,
-                           (const uint8_t*)m.flags, (const uint64_t*)mg.drop, (const uint8_t*)m.kmask,
-                           (const uint2*)m.ranks, (const uint32_t*)gv, (const uint32_t*)m.tword, (const uint32_t*)gt,
-                           (const uint64_t*)(m.d_base + 2 * k), tcap, tris);
-        QJ_HIP(hipGetLastError());
+        if ((st = launch_tris(m, mg, gv, gt, (const uint64_t*)(m.d_base + 2 * k), 0, tcap, tris, s))) return st;
       }
     }
     QJ_HIP(hipMemcpyAsync(base.data(), m.d_base, sizeof(uint64_t) * base.size(), hipMemcpyDeviceToHost, s));
@@ -1146,15 +1153,11 @@ void mc_free(qj_workspace* ws) {
   McState* m = (McState*)ws->mc;
   if (!m) return;
   hipFree(m->flags);
-  hipFree(m->emask);
-  hipFree(m->cnt);
   hipFree(m->words);
   hipFree(m->ranks);
   hipFree(m->kmask);
   hipFree(m->tword);
   hipFree(m->groups);
-  hipFree(m->blk);
-  hipFree(m->active);
   hipFree(m->tri_off);
   hipFree(m->verts);
   hipFree(m->tris_pre);
@@ -1170,7 +1173,8 @@ void mc_free(qj_workspace* ws) {
   }
   for (hipEvent_t e : {m->ev_start, m->ev_field[0], m->ev_field[1], m->ev_free[0], m->ev_free[1]})
     if (e) hipEventDestroy(e);
-  hipFree(m->slice_off);
+  hipFree(m->aword);
+  hipFree(m->lost);
   hipFree(m->vpt);
   hipFree(m->vax);
   hipFree(m->d_bad);
@@ -1186,9 +1190,10 @@ void mc_free(qj_workspace* ws) {
 
 // TRIANGLE_MESH::computeNonlinearMarchingCubesLowMemoryHuge (TRIANGLE_MESH.cpp:681-768)
 // streamed over z-chunks: for chunk [z0, z1) the map is evaluated on slices
-// [z0-1, z1+1] (one halo slice below for the edges at z0, two above for the
-// edges of the points at z1, whose ids belong to the next chunk), cases come
-// from the raw slab values log|q| (TRIANGLE_MESH.cpp:379), and every vertex is
+// [z0, z1 + 1] (two above for the edges of the points at z1, whose ids belong to
+// the next chunk; none below: an edge's ends say whether it carries a vertex),
+// cases come from the raw slab values log|q| (TRIANGLE_MESH.cpp:379) as sign
+// words, as in the linear mesher, and every vertex is
 // placed by bisection on re-evaluated values log|q| - iso (nonlinearValue
 // :1755-1795, midpointSearch :2232-2271, at most 6 halvings, early exit at
 // |value| < 1e-8). Vertex numbering, triangle order and the degenerate filter
@@ -1230,57 +1235,6 @@ __device__ __forceinline__ double nonlinear_value(const MapArgs& a, const RootRe
   const q64 q0{p[0], p[1], p[2], a.slice};
   const Res64 r = kMap == kNlExt ? eval64e<kPow>(a, roots, q0) : eval64<kPow>(a, roots, q0);
   return r.F - iso;
-}
-
-// cases of cells in slab slices [0, ns-1) (global z = s0 + local z)
-__global__ __launch_bounds__(kMcBlock) void k_nl_flags(const double* __restrict__ slab, int64_t X, int64_t Y,
-                                                       int64_t Z, int64_t s0, int64_t ns,
-                                                       uint8_t* __restrict__ flags) {
-  const int64_t XY = X * Y, N = XY * ns;
-  const int64_t p = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
-  if (p >= N) return;
-  const int64_t lz = p / XY, r = p - lz * XY, y = r / X, x = r - y * X;
-  int flag = 0;
-  if (x < X - 1 && y < Y - 1 && s0 + lz < Z - 1 && lz + 1 < ns) flag = cell_flag(slab, p, X, XY, 0.0);
-  flags[p] = (uint8_t)flag;
-}
-
-// edge masks of points in global slices [p0, p0 + np); flags are slab-local with slab start s0
-__global__ __launch_bounds__(kMcBlock) void k_nl_edges(const uint8_t* __restrict__ flags, int64_t X, int64_t Y,
-                                                       int64_t Z, int64_t s0, int64_t p0, int64_t np,
-                                                       uint8_t* __restrict__ emask, uint32_t* __restrict__ cnt) {
-  __shared__ unsigned short s_em[256];
-  stage_emask(s_em);
-  const int64_t XY = X * Y, N = XY * np;
-  const int64_t j = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
-  if (j >= N) return;
-  const int64_t lz = j / XY, r = j - lz * XY, y = r / X, x = r - y * X;
-  const int64_t z = p0 + lz;
-  const int64_t f = (z - s0) * XY + y * X + x;  // slab-local index of the point
-  unsigned bits = 0;
-  if (x < X - 1) {
-    unsigned ref = 0;
-    for (int b = 0; b < 2; b++)
-      for (int a = 0; a < 2; a++)
-        if (y >= a && z - b >= s0) ref |= (s_em[flags[f - a * X - b * XY]] >> (a + 2 * b)) & 1u;
-    bits |= ref;
-  }
-  if (y < Y - 1) {
-    unsigned ref = 0;
-    for (int b = 0; b < 2; b++)
-      for (int a = 0; a < 2; a++)
-        if (x >= a && z - b >= s0) ref |= (s_em[flags[f - a - b * XY]] >> (4 + a + 2 * b)) & 1u;
-    bits |= ref << 1;
-  }
-  if (z < Z - 1) {
-    unsigned ref = 0;
-    for (int b = 0; b < 2; b++)
-      for (int a = 0; a < 2; a++)
-        if (x >= a && y >= b) ref |= (s_em[flags[f - a - b * X]] >> (8 + a + 2 * b)) & 1u;
-    bits |= ref << 2;
-  }
-  emask[j] = (uint8_t)bits;
-  cnt[j] = (bits & 1u) + ((bits >> 1) & 1u) + ((bits >> 2) & 1u);
 }
 
 // One vertex by bisection between grid points (x, y, z) and its +axis
@@ -1357,68 +1311,122 @@ __device__ __forceinline__ void place_vertex(const MapArgs& a, const RootRec64* 
   out[2] = m[2];
 }
 
-// The vertices of a range of points (off: the exclusive scan of the edge
-// counts, from the range's first point) in id order: the owning point
-// (relative to the range) and the edge's axis.
-__global__ __launch_bounds__(kMcBlock) void k_nl_vlist(const uint8_t* __restrict__ emask,
-                                                       const uint32_t* __restrict__ off, int64_t n,
-                                                       uint32_t* __restrict__ vpt, uint8_t* __restrict__ vax) {
-  const int64_t j = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
-  if (j >= n) return;
-  const unsigned bits = emask[j];
-  if (!bits) return;
-  uint32_t k = off[j] - off[0];
-  for (int axis = 0; axis < 3; axis++)
-    if (bits & (1u << axis)) {
-      vpt[k] = (uint32_t)j;
-      vax[k] = (uint8_t)axis;
-      k++;
+// Triangles and active cells of a slab, one word of cells per thread, as
+// k_mc_cells counts them. (One slab of 66 slices of 256^2: signs, edges and this
+// 19, 11 and 15 us; case bytes and edges from them 62 and 78, and five scans.) tword, aword: before word w in its group; groups: per
+// group, triangles from 0 on and active cells from `ngroups` on. kLost: the
+// triangles less those that k_nl_filter dropped.
+template <bool kLost>
+__global__ __launch_bounds__(kMcBlock) void k_nl_count(McGrid a, uint8_t* __restrict__ flags,
+                                                       const uint32_t* __restrict__ lost,
+                                                       uint32_t* __restrict__ tword, uint32_t* __restrict__ aword,
+                                                       uint32_t* __restrict__ groups, int64_t ngroups) {
+  const int64_t w = (int64_t)blockIdx.x * kMcGroupWords + threadIdx.x;
+  uint32_t count = 0, active = 0, total;
+  if (w < a.nw) {
+    active = (uint32_t)__popcll(word_cases(a, w, flags, &count));
+    if (kLost) count -= lost[w];
+    else a.drop[w] = 0;
+  }
+  const uint32_t t = block_prefix<kMcBlock>(count, &total);
+  if (threadIdx.x == 0) groups[blockIdx.x] = total;
+  const uint32_t c = block_prefix<kMcBlock>(active, &total);
+  if (threadIdx.x == 0) groups[ngroups + blockIdx.x] = total;
+  if (w >= a.nw) return;
+  tword[w] = t;
+  aword[w] = c;
+}
+
+// One block: groups holds n counts each of vertices, triangles and active
+// cells; all to exclusive offsets in place, and to pinned memory: the vertices of
+// points below p, all vertices, triangles, active cells. The block is small: one of
+// 1024 threads waited 0.3 ms for a CU with room for its 16 waves while the next
+// slab was evaluated on the other stream.
+constexpr int kTotalsBlock = 256;
+__global__ __launch_bounds__(kTotalsBlock) void k_nl_totals(uint32_t* __restrict__ groups, int64_t n,
+                                                          const uint2* __restrict__ ranks, int64_t p, int64_t owned,
+                                                          uint32_t* __restrict__ h_out) {
+  const int64_t per = (n + kTotalsBlock - 1) / kTotalsBlock, b = (int64_t)threadIdx.x * per;
+  uint32_t all = 0;
+  for (int which = 0; which < 3; which++, groups += n) {
+    uint32_t v = 0, total;
+    for (int64_t i = b; i < b + per && i < n; i++) v += groups[i];
+    uint32_t run = block_prefix<kTotalsBlock>(v, &total);
+    for (int64_t i = b; i < b + per && i < n; i++) {
+      const uint32_t c = groups[i];
+      // the thread that holds p's group
+      if (which == 0 && i == p / kMcGroupPoints && p < owned) {
+        const uint2 rk = ranks[p >> 3];
+        h_out[0] = run + rk.x + (uint32_t)__popc(rk.y & ((1u << (3 * (p & 7))) - 1u));
+      }
+      groups[i] = run;
+      run += c;
     }
+    if (which == 0) all = total;
+    if (threadIdx.x == 0) h_out[1 + which] = total;
+  }
+  if (threadIdx.x == 0 && p >= owned) h_out[0] = all;
+}
+
+// The slab's vertices from local id `from` on, in id order: the owning point
+// and the edge's axis. One wave per word of points.
+__global__ __launch_bounds__(kMcBlock) void k_nl_vlist(McGrid a, const uint64_t* __restrict__ ex,
+                                                       const uint64_t* __restrict__ ey,
+                                                       const uint64_t* __restrict__ ez,
+                                                       const uint2* __restrict__ ranks,
+                                                       const uint32_t* __restrict__ groups, uint32_t from,
+                                                       uint32_t* __restrict__ vpt, uint8_t* __restrict__ vax) {
+  const int64_t w0 = ((int64_t)blockIdx.x * kMcWaves + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) *
+                     kListWords;
+  const int lane = threadIdx.x & 63;
+#pragma unroll 1
+  for (int i = 0; i < kListWords; i++) {
+    const int64_t w = w0 + i;
+    if (w >= a.nw) break;
+    const uint64_t e[3] = {ex[w], ey[w], ez[w]};
+    if (!(e[0] | e[1] | e[2])) continue;
+    uint32_t k = groups[w / kMcGroupWords] + ranks[8 * w].x;
+#pragma unroll
+    for (int axis = 0; axis < 3; axis++)
+      k = __builtin_amdgcn_mbcnt_hi((uint32_t)(e[axis] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)e[axis], k));
+#pragma unroll
+    for (int axis = 0; axis < 3; axis++)
+      if (__builtin_amdgcn_inverse_ballot_w64(e[axis])) {
+        if (k >= from) {
+          vpt[k - from] = (uint32_t)(64 * w + lane);
+          vax[k - from] = (uint8_t)axis;
+        }
+        k++;
+      }
+  }
 }
 
 // Vertices by bisection, one per thread over the list: both end values
 // (evaluated, or read from the slab), then up to 6 midpoints (FP64 map
 // evaluations on full waves; about one point in ten owns an edge, so a thread
-// per point would leave most lanes idle). One launch takes two ranges of
-// points: the chunk's own points from slice p0a (list entries [0, nA), nA the
-// scan total minus the scan at the range's first point, off_a null when the
-// range is empty; vertex t gets id base + off_a[0] + t) and the next chunk's
-// first slice p0b (entries [b_start, b_start + nb), ids base + t), so the
-// slice's few vertices do not take a launch of their own. List entries hold
-// the point relative to their range's first point. ends_a / ends_b: null, or
-// the slab's values from the range's first point on, when they are the end
-// values' own (see slab_holds_end_values); the midpoints are always evaluated.
+// per point would leave most lanes idle). List entry t, a point of the slab
+// that starts at slice z0, gets id base + t. ends: null, or the slab's values,
+// when they are the end values' own (see slab_holds_end_values); the midpoints
+// are always evaluated.
+// FP64 VALU bound. For exponents 1 and 2 the registers are held to five waves
+// per SIMD (96, 136 B of a vertex's state spilled round the evaluation; 128 and
+// four before): meshes of 0.4 million vertices and more 3 to 7 % faster, smaller
+// ones as fast.
 template <int kPow, int kMap>
-__global__ __launch_bounds__(kMcBlock) void k_nl_vertices(MapArgs a, const RootRec64* __restrict__ roots,
-                                                          double iso, int64_t p0a, const double* __restrict__ ends_a,
-                                                          const uint32_t* __restrict__ off_a,
-                                                          const uint32_t* __restrict__ total_a, int64_t p0b,
-                                                          const double* __restrict__ ends_b, uint32_t b_start,
-                                                          uint32_t nb, const uint32_t* __restrict__ vpt,
+__global__ __launch_bounds__(kMcBlock, kPow == kExactOnly && kMap == kNlPlain ? 5 : 1) void k_nl_vertices(MapArgs a, const RootRec64* __restrict__ roots,
+                                                          double iso, int64_t z0, const double* __restrict__ ends,
+                                                          uint32_t n, const uint32_t* __restrict__ vpt,
                                                           const uint8_t* __restrict__ vax, uint32_t base,
                                                           double* __restrict__ verts, int32_t* __restrict__ edges,
                                                           unsigned int* __restrict__ bad) {
   const uint32_t t = blockIdx.x * kMcBlock + threadIdx.x;
-  int64_t p0, k;
-  const double* ends;
-  if (t >= b_start) {
-    if (t - b_start >= nb) return;
-    p0 = p0b;
-    ends = ends_b;
-    k = (int64_t)base + t;
-  } else {
-    if (!off_a) return;
-    const uint32_t first = off_a[0];
-    if (t >= *total_a - first) return;
-    p0 = p0a;
-    ends = ends_a;
-    k = (int64_t)base + first + t;
-  }
+  if (t >= n) return;
+  const int64_t k = (int64_t)base + t;
   const int64_t X = a.res[0], XY = X * a.res[1];
   const int64_t q = vpt[t];
   const int axis = vax[t];
   const int64_t lz = q / XY, r = q - lz * XY;
-  const int y = (int)(r / X), x = (int)(r - (int64_t)y * X), z = (int)(p0 + lz);
+  const int y = (int)(r / X), x = (int)(r - (int64_t)y * X), z = (int)(z0 + lz);
   const double* fa = ends ? ends + q : nullptr;
   const double* fb = ends ? ends + q + (axis == 0 ? 1 : axis == 1 ? X : XY) : nullptr;
   place_vertex<kPow, kMap>(a, roots, iso, x, y, z, axis, fa, fb, verts + 3 * k, bad);
@@ -1441,100 +1449,58 @@ static void launch_nl_vertices(const MapArgs& a, dim3 grid, hipStream_t s, Args.
                                           : k_nl_vertices<kExactOnly, kNlPlain>);
   hipLaunchKernelGGL(k, grid, dim3(kMcBlock), 0, s, a, args...);
 }
-// (x, y, z, flag) of the chunk's active cells, appended in cell order
-__global__ __launch_bounds__(kMcBlock) void k_nl_cells(const uint32_t* __restrict__ active, int64_t na,
-                                                       const uint8_t* __restrict__ flags, int64_t fo, int64_t X,
-                                                       int64_t XY, int64_t z0, int32_t* __restrict__ cells) {
-  const int64_t i = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
-  if (i >= na) return;
-  const int64_t c = active[i];
-  const int64_t lz = c / XY, r = c - lz * XY, y = r / X, x = r - y * X;
-  cells[4 * i + 0] = (int32_t)x;
-  cells[4 * i + 1] = (int32_t)y;
-  cells[4 * i + 2] = (int32_t)(z0 + lz);
-  cells[4 * i + 3] = flags[fo + c];
+// (x, y, z, flag) of the slab's active cells, in cell order; the slab starts at slice z0
+__global__ __launch_bounds__(kMcBlock) void k_nl_cells(McGrid a, const uint8_t* __restrict__ flags,
+                                                       const uint32_t* __restrict__ aword,
+                                                       const uint32_t* __restrict__ groups, int64_t z0,
+                                                       int32_t* __restrict__ cells) {
+  const int64_t p = (int64_t)blockIdx.x * kMcBlock + threadIdx.x, w = p >> 6;
+  const int lane = threadIdx.x & 63;
+  const unsigned flag = p < a.cells ? flags[p] : 0u;
+  const uint64_t act = __ballot(flag != 0u);
+  if (!flag) return;
+  const int64_t k = (int64_t)groups[w / kMcGroupWords] + aword[w] + __popcll(act & ((1ull << lane) - 1ull));
+  int64_t x, y, z;
+  point_xyz(a.g, p, x, y, z);
+  ((int4*)cells)[k] = int4{(int32_t)x, (int32_t)y, (int32_t)(z0 + z), (int32_t)flag};
 }
 
-// per-block active counts of cells in global slices [c0, c0 + nc) (slab-local flags from s0)
-__global__ __launch_bounds__(kMcBlock) void k_nl_active_count(const uint8_t* __restrict__ flags, int64_t XY,
-                                                              int64_t c0, int64_t s0, int64_t nc,
-                                                              uint32_t* __restrict__ blk) {
-  __shared__ uint32_t s_n[kMcBlock / 64];
-  const int64_t j = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
-  const bool act = j < XY * nc && kMc.ntri[flags[(c0 - s0) * XY + j]] > 0;
-  const unsigned long long m = __ballot(act);
-  if ((threadIdx.x & 63) == 0) s_n[threadIdx.x >> 6] = (uint32_t)__popcll(m);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t t = 0;
-    for (int i = 0; i < kMcBlock / 64; i++) t += s_n[i];
-    blk[blockIdx.x] = t;
-  }
-}
-
-__global__ __launch_bounds__(kMcBlock) void k_nl_active(const uint8_t* __restrict__ flags, int64_t XY, int64_t c0,
-                                                        int64_t s0, int64_t nc, const uint32_t* __restrict__ blk_off,
-                                                        uint32_t* __restrict__ active) {
-  __shared__ uint32_t s_n[kMcBlock / 64];
-  const int64_t j = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
-  const bool act = j < XY * nc && kMc.ntri[flags[(c0 - s0) * XY + j]] > 0;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const unsigned long long m = __ballot(act);
-  if (lane == 0) s_n[wave] = (uint32_t)__popcll(m);
-  __syncthreads();
-  uint32_t o = blk_off[blockIdx.x];
-  for (int i = 0; i < wave; i++) o += s_n[i];
-  if (act) active[o + __popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)j;  // chunk-local cell index
-}
-
-__global__ __launch_bounds__(kMcBlock) void k_nl_tricount(const uint32_t* __restrict__ active, int64_t na,
-                                                          const uint8_t* __restrict__ flags, int64_t fo,
-                                                          uint32_t* __restrict__ tcount) {
-  const int64_t i = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
-  if (i < na) tcount[i] = kMc.ntri[flags[fo + active[i]]];
-}
-
-// triangles of the chunk's active cells; owners at global z < z1 use base + off,
-// owners at z == z1 use base_next + slice_off
-__global__ __launch_bounds__(kMcBlock) void k_nl_triangles(
-    const uint32_t* __restrict__ active, int64_t na, const uint8_t* __restrict__ flags, int64_t fo, int64_t X,
-    int64_t XY, int64_t z0, int64_t z1, const uint8_t* __restrict__ emask, const uint32_t* __restrict__ off,
-    uint32_t base, const uint8_t* __restrict__ emask_next, const uint32_t* __restrict__ slice_off,
-    uint32_t base_next, const double* __restrict__ verts, const uint32_t* __restrict__ toff,
-    int32_t* __restrict__ tris_pre, uint32_t* __restrict__ keep) {
+// The degenerate filter (TRIANGLE_MESH.cpp:1088-1102) on every triangle of a
+// slab, one cell per thread: kmask holds what is left of a cell that lost any,
+// drop their bits and lost the triangles per word. Only for grids whose spacing
+// or map leaves the answer open (see nlmc_run).
+__global__ __launch_bounds__(kMcBlock) void k_nl_filter(McGrid a, const uint8_t* __restrict__ flags,
+                                                        const uint2* __restrict__ ranks,
+                                                        const uint32_t* __restrict__ groups, uint32_t id0,
+                                                        const double* __restrict__ verts, uint8_t* __restrict__ kmask,
+                                                        uint32_t* __restrict__ lost) {
   __shared__ uint32_t s_tri[1024];
   __shared__ uint8_t s_ntri[256];
   stage_tri(s_tri, s_ntri);
-  const int64_t i = (int64_t)blockIdx.x * kMcBlock + threadIdx.x;
-  if (i >= na) return;
-  const int64_t c = active[i];  // chunk-local cell index: (z - z0) * XY + y * X + x
-  const int flag = flags[fo + c];
-  const int n = s_ntri[flag];
-  uint32_t o = toff[i];
+  const int64_t p = (int64_t)blockIdx.x * kMcBlock + threadIdx.x, w = p >> 6;
+  const int64_t X = a.g.res[0];
+  const int flag = p < a.cells ? (int)flags[p] : 0;
+  const int n = flag ? s_ntri[flag] : 0;
+  unsigned dropped = 0;
   for (int t = 0; t < n; t++) {
-    int32_t v[3];
+    const double* v[3];
     for (int q = 0; q < 3; q++) {
       int dx, dy, dz, axis;
       edge_geom(tri_edge(s_tri, flag, 3 * t + q), dx, dy, dz, axis);
-      const int64_t owner = c + dx + dy * X + dz * XY;  // chunk-local point index
-      const unsigned lowbits = (1u << axis) - 1u;
-      if (z0 + owner / XY < z1) {
-        v[q] = (int32_t)(base + off[owner] + __popc(emask[owner] & lowbits));
-      } else {
-        const int64_t so = owner - (z1 - z0) * XY;
-        v[q] = (int32_t)(base_next + slice_off[so] + __popc(emask_next[so] & lowbits));
-      }
+      const int64_t o = p + dx + dy * X + dz * a.XY;
+      const uint2 rk = ranks[o >> 3];
+      v[q] = verts + 3 * ((int64_t)id0 + groups[o / kMcGroupPoints] + rk.x +
+                          __popc(rk.y & ((1u << (3 * (o & 7) + axis)) - 1u)));
     }
     const double eps = 1e-7;
-    const double* p0 = verts + 3 * (int64_t)v[0];
-    const double* p1 = verts + 3 * (int64_t)v[1];
-    const double* p2 = verts + 3 * (int64_t)v[2];
-    const bool degenerate = edge_len(p0, p1) < eps || edge_len(p0, p2) < eps || edge_len(p1, p2) < eps;
-    tris_pre[3 * (int64_t)o + 0] = v[0];
-    tris_pre[3 * (int64_t)o + 1] = v[1];
-    tris_pre[3 * (int64_t)o + 2] = v[2];
-    keep[o] = degenerate ? 0u : 1u;
-    o++;
+    if (edge_len(v[0], v[1]) < eps || edge_len(v[0], v[2]) < eps || edge_len(v[1], v[2]) < eps) dropped |= 1u << t;
+  }
+  if (dropped) kmask[p] = (uint8_t)(((1u << n) - 1u) & ~dropped);
+  const uint64_t m = __ballot(dropped != 0u);
+  const uint32_t sum = wave_last(wave_inclusive((uint32_t)__popc(dropped)));
+  if ((threadIdx.x & 63) == 0 && w < a.nw) {
+    a.drop[w] = m;
+    lost[w] = sum;
   }
 }
 
@@ -1563,12 +1529,20 @@ static qj_status grow_keep(T*& p, int64_t& cap, int64_t n, int64_t used, hipStre
 // tests; products of values of magnitude band or more do not underflow), so
 // the vertices are those of the evaluated end values. Not for the caller's
 // field (its values are not the map's), the Lagrange order (its value has
-// its own infinite case), the plain FP64 slabs (polar powers, where the
-// bisection evaluates exact ones), the AP flags or a band of 0.
+// its own infinite case), the plain FP64 slabs (the same values, but not worth
+// a case of their own), the AP flags or a band of 0.
 static bool slab_holds_end_values(const MapArgs& a, const double* src_field, double iso, qj_precision prec,
                                   double band) {
   return !src_field && prec == QJ_FP32_BAND && iso == 0.0 && band > 0.0 &&
          !(a.flags & (QJ_MAP_LAGRANGE | QJ_MAP_SKIP_ORIGIN | QJ_MAP_ADAPTIVE));
+}
+
+// what the word kernels need of a slab: its points' places in memory
+static void slab_geom(const MapArgs& a, GridGeom* g) {
+  *g = GridGeom{};
+  for (int i = 0; i < 3; i++) g->res[i] = a.res[i];
+  g->div_x = make_fastdiv((uint32_t)a.res[0]);
+  g->div_xy = make_fastdiv((uint32_t)((int64_t)a.res[0] * a.res[1]));
 }
 
 qj_status nlmc_run(qj_workspace* ws, const MapArgs& a0, const qj_rational* f, double iso, qj_precision prec,
@@ -1588,7 +1562,7 @@ qj_status nlmc_run(qj_workspace* ws, const MapArgs& a0, const qj_rational* f, do
     set_error("non-linear mesher: slab of %lld points exceeds 32-bit indices", (long long)(XY * (chunk + 3)));
     return QJ_ERR_CAPACITY;
   }
-  const int64_t slab_pts = XY * (chunk + 3), own_pts = XY * (chunk + 1);
+  const int64_t slab_pts = XY * (chunk + 2);
   qj_status st;
   // the slab stream is idle whenever the call returns, early error returns
   // included (its slab evaluations read the caller's roots)
@@ -1610,46 +1584,34 @@ qj_status nlmc_run(qj_workspace* ws, const MapArgs& a0, const qj_rational* f, do
     for (hipEvent_t* e : {&m.ev_start, &m.ev_field[0], &m.ev_field[1], &m.ev_free[0], &m.ev_free[1]})
       if (!*e) QJ_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
   }
-  if ((st = grow(m.flags, m.cap_flags, slab_pts, s)) ||
-      (st = grow(m.emask, m.cap_emask, own_pts, s)) || (st = grow(m.cnt, m.cap_cnt, own_pts, s)) ||
-      (st = grow(m.active, m.cap_active, own_pts, s)) || (st = grow(m.tri_off, m.cap_toff, own_pts, s)) ||
-      (st = grow(m.blk, m.cap_blk, (int64_t)nblocks(own_pts), s)) ||
-      (st = grow(m.slice_off, m.cap_slice, XY, s)))
+  MapArgs a = a0;
+  GridGeom geo;
+  slab_geom(a, &geo);
+  const int64_t wmax = (slab_pts + 63) / 64 + mc_pad_words(geo);
+  const int64_t gmax = (slab_pts + kMcGroupPoints - 1) / kMcGroupPoints;
+  // Bisection places a vertex at a multiple of 1/128 of its edge inside it (at
+  // most six halvings after the first middle), so vertices on edges that meet are
+  // at least sqrt(2) / 128 spacings apart, others a spacing: with spacings of
+  // 1e-4 no side is below 1e-7 and the filter has nothing to drop.
+  const bool sure = is_turned_grid(a, kSureSpacing, DBL_MAX) && grid_extent(a) <= kSureExtent;
+  if ((st = grow(m.words, m.cap_words, kMcArrays * wmax, s)) || (st = grow(m.ranks, m.cap_ranks, 8 * wmax, s)) ||
+      (st = grow(m.flags, m.cap_flags, 64 * ((slab_pts + 63) / 64), s)) ||
+      (st = grow(m.tword, m.cap_tword, wmax, s)) || (st = grow(m.aword, m.cap_aword, wmax, s)) ||
+      (st = grow(m.groups, m.cap_groups, 3 * gmax, s)) || (st = grow(m.d_base, m.cap_base, 4, s)) || (st = ensure_pinned(ws, 2, s)) ||
+      (!sure && ((st = grow(m.kmask, m.cap_kmask, slab_pts, s)) || (st = grow(m.lost, m.cap_lost, wmax, s)))))
     return st;
-  const size_t need_tmp = scan_tmp_bytes(5 * own_pts);
-  if (need_tmp > m.tmp_bytes) {
-    if (m.tmp) {
-      QJ_HIP(hipStreamSynchronize(s));
-      QJ_HIP(hipFree(m.tmp));
-    }
-    m.tmp = nullptr;
-    m.tmp_bytes = 0;
-    QJ_HIP(hipMalloc(&m.tmp, need_tmp));
-    m.tmp_bytes = need_tmp;
-  }
-  if (!m.totals) QJ_HIP(hipMalloc(&m.totals, 4 * sizeof(uint32_t)));
   if (!m.d_bad) QJ_HIP(hipMalloc(&m.d_bad, sizeof(unsigned int)));
   QJ_HIP(hipMemsetAsync(m.d_bad, 0, sizeof(unsigned int), s));
-  // the mesher's map: escape 2000 and the black-hole stop (TRIANGLE_MESH.cpp:97, 1789-1791)
-  MapArgs a = a0;
   const bool reuse_ends = slab_holds_end_values(a, src_field, iso, prec, band);
-  // slices [s0, s0 + ns) of the slab of the chunk that starts at slice zc: the
-  // chunk's points and one halo slice on each side
-  auto slab_range = [&](int64_t zc, int64_t& s0, int64_t& ns) {
-    const int64_t zc1 = zc + chunk < Z ? zc + chunk : Z;
-    s0 = zc > 0 ? zc - 1 : 0;
-    const int64_t s1 = zc1 + 1 < Z - 1 ? zc1 + 1 : Z - 1;
-    ns = s1 - s0 + 1;
-  };
+  // slices of the slab of the chunk that starts at slice zc: the chunk's and up to two above
+  auto slab_slices = [&](int64_t zc) { return std::min(zc + chunk + 2, Z) - zc; };
   // 1. slab of log|q| (or the caller's field, TRIANGLE_MESH.cpp:152-215): the
   // chunk at slice zc into slab[b] on stream s2 (the Lagrange order has no FP32
   // path: its slabs are FP64)
   auto eval_slab = [&](int64_t zc, int b) -> qj_status {
-    int64_t fs0, fns;
-    slab_range(zc, fs0, fns);
     MapArgs sa = a;
-    sa.res[2] = (int32_t)fns;
-    sa.zoff = (int32_t)fs0;
+    sa.res[2] = (int32_t)slab_slices(zc);
+    sa.zoff = (int32_t)zc;
     qj_status e = launch_field(ws, sa, f, (a.flags & QJ_MAP_LAGRANGE) ? QJ_FP64 : prec, band, m.slab[b], m.s2);
     if (e) return e;
     QJ_HIP(hipEventRecord(m.ev_field[b], m.s2));
@@ -1661,13 +1623,12 @@ qj_status nlmc_run(qj_workspace* ws, const MapArgs& a0, const qj_rational* f, do
     QJ_HIP(hipStreamWaitEvent(m.s2, m.ev_start, 0));
     if ((st = eval_slab(0, 0))) return st;
   }
-  uint64_t nv = 0, nt = 0, placed_next = 0;
+  uint64_t nv = 0, nt = 0, placed = 0;
+  volatile uint32_t* const h = (volatile uint32_t*)ws->h_pinned;
   for (int64_t z0 = 0, ci = 0; z0 < Z; z0 += chunk, ci++) {
     const int64_t z1 = z0 + chunk < Z ? z0 + chunk : Z;
-    int64_t s0, ns;
-    slab_range(z0, s0, ns);
     const int b = (int)(ci & 1);
-    const double* slab = src_field ? src_field + s0 * XY : m.slab[b];
+    const double* slab = src_field ? src_field + z0 * XY : m.slab[b];
     if (!src_field) {
       // the next chunk's slab goes into the other buffer once the previous
       // chunk's vertex kernel, its last reader, is done; this chunk's cases
@@ -1678,113 +1639,75 @@ qj_status nlmc_run(qj_workspace* ws, const MapArgs& a0, const qj_rational* f, do
       }
       QJ_HIP(hipStreamWaitEvent(s, m.ev_field[b], 0));
     }
-    const double* ends = reuse_ends ? slab : nullptr;
-    // 2. cases
-    hipLaunchKernelGGL(k_nl_flags, dim3(nblocks(XY * ns)), dim3(kMcBlock), 0, s, slab, X, Y, Z, s0, ns, m.flags);
+    // 2. signs, edges of the points in slices [z0, z1] and cells of [z0, z1)
+    geo.res[2] = (int32_t)slab_slices(z0);
+    McGrid mg = make_mc_grid(m, geo, wmax, 0.0, kMeasureAll);
+    mg.cells = XY * (std::min(z1, Z - 1) - z0);
+    mg.owned = XY * (std::min(z1 + 1, Z) - z0);
+    mg.floor = z0 == 0;
+    const int64_t ng = (mg.N + kMcGroupPoints - 1) / kMcGroupPoints;
+    uint32_t *gv = m.groups, *gt = gv + ng, *ga = gt + ng;
+    hipLaunchKernelGGL(k_mc_signs, blocks_of(mg.N, kSignPoints * kMcBlock), dim3(kMcBlock), 0, s, slab, mg.N, 0.0,
+                       mg.sgn);
     QJ_HIP(hipGetLastError());
-    // 3. edge masks of points [z0, z1] (z1 only when it exists)
-    const int64_t np = (z1 < Z ? z1 + 1 : Z) - z0;
-    hipLaunchKernelGGL(k_nl_edges, dim3(nblocks(XY * np)), dim3(kMcBlock), 0, s, m.flags, X, Y, Z, s0, z0, np,
-                       m.emask, m.cnt);
+    hipLaunchKernelGGL(k_mc_edges, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.ranks, gv);
     QJ_HIP(hipGetLastError());
-    // 4. vertex ids: owned points [z0, z1), and the next chunk's first slice separately
-    const int64_t nown = XY * (z1 - z0);
-    uint32_t h[4] = {0, 0, 0, 0};
-    if (z1 < Z) {
-      if ((st = scan_u32(m.cnt + nown, m.slice_off, XY, m.totals + 3, m.tmp, m.tmp_bytes, s))) return st;
-      QJ_HIP(hipMemcpyAsync(h + 3, m.totals + 3, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    }
-    if ((st = scan_u32(m.cnt, m.cnt, nown, m.totals + 1, m.tmp, m.tmp_bytes, s))) return st;
-    QJ_HIP(hipMemcpyAsync(h + 1, m.totals + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(k_nl_count<false>, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.flags,
+                       (const uint32_t*)nullptr, m.tword, m.aword, gt, ng);
+    QJ_HIP(hipGetLastError());
+    // 3. the counts: every buffer is sized from one read-back
+    hipLaunchKernelGGL(k_nl_totals, dim3(1), dim3(kTotalsBlock), 0, s, gv, ng, (const uint2*)m.ranks, XY * (z1 - z0),
+                       mg.owned, (uint32_t*)ws->h_pinned);
+    QJ_HIP(hipGetLastError());
     QJ_HIP(hipStreamSynchronize(s));
-    const uint64_t cnt_own = h[1], cnt_next = h[3];
-    if (nv + cnt_own + cnt_next > (uint64_t)INT32_MAX) return QJ_ERR_CAPACITY;
-    // The chunk's triangles reach the first slice of the next chunk, whose
-    // vertices the degenerate filter reads: place them now (ids base_next +
-    // slice_off, the ids the next chunk's numbering gives them) and skip the
-    // chunk's own first slice, placed by the previous chunk.
-    // keep what is already placed: ids < nv plus this chunk's first slice (placed by the previous chunk)
-    if ((st = grow_keep(m.verts, m.cap_v, 3 * (int64_t)(nv + cnt_own + cnt_next), 3 * (int64_t)(nv + placed_next),
-                        s)))
+    const uint64_t cnt_own = h[0], cnt_all = h[1], ntp = h[2], na = h[3];
+    if (nv + cnt_all > (uint64_t)INT32_MAX) return QJ_ERR_CAPACITY;
+    // 4. vertices: the chunk's triangles reach the first slice of the next
+    // chunk, so that slice's are placed now (with the ids that the next chunk's
+    // numbering gives them) and the chunk's own first slice was placed before
+    if ((st = grow_keep(m.verts, m.cap_v, 3 * (int64_t)(nv + cnt_all), 3 * (int64_t)(nv + placed), s)) ||
+        (st = grow_keep(m.c_edges, m.cap_ce, 4 * (int64_t)(nv + cnt_all), 4 * (int64_t)(nv + placed), s)) ||
+        (st = grow_keep(m.c_cells, m.cap_cc, 4 * (m.ncells + (int64_t)na), 4 * m.ncells, s)) ||
+        (st = grow_keep(m.tris, m.cap_t, 3 * (int64_t)(nt + ntp), 3 * (int64_t)nt, s)) ||
+        (st = grow(m.vpt, m.cap_vpt, (int64_t)cnt_all, s)) || (st = grow(m.vax, m.cap_vax, (int64_t)cnt_all, s)))
       return st;
-    if ((st = grow_keep(m.c_edges, m.cap_ce, 4 * (int64_t)(nv + cnt_own + cnt_next),
-                        4 * (int64_t)(nv + placed_next), s)))
-      return st;
-    const int64_t skip = z0 > 0 ? 1 : 0;
-    if ((st = grow(m.vpt, m.cap_vpt, (int64_t)(cnt_own + cnt_next), s))) return st;
-    if ((st = grow(m.vax, m.cap_vax, (int64_t)(cnt_own + cnt_next), s))) return st;
-    const bool own = cnt_own > 0 && z1 - z0 > skip;
-    if (own) {
-      const int64_t n = XY * (z1 - z0 - skip);
-      hipLaunchKernelGGL(k_nl_vlist, dim3(nblocks(n)), dim3(kMcBlock), 0, s, m.emask + skip * XY,
-                         m.cnt + skip * XY, n, m.vpt, m.vax);
+    if (cnt_all > placed) {
+      hipLaunchKernelGGL(k_nl_vlist, blocks_of(mg.nw, kListWords * kMcWaves), dim3(kMcBlock), 0, s, mg,
+                         (const uint64_t*)mg.edge[0], (const uint64_t*)mg.edge[1], (const uint64_t*)mg.edge[2],
+                         (const uint2*)m.ranks, (const uint32_t*)gv, (uint32_t)placed, m.vpt, m.vax);
       QJ_HIP(hipGetLastError());
-    }
-    if (cnt_next > 0) {
-      hipLaunchKernelGGL(k_nl_vlist, dim3(nblocks(XY)), dim3(kMcBlock), 0, s, m.emask + nown, m.slice_off, XY,
-                         m.vpt + cnt_own, m.vax + cnt_own);
-      QJ_HIP(hipGetLastError());
-    }
-    if (own || cnt_next > 0) {
-      launch_nl_vertices(a, dim3(nblocks((int64_t)(cnt_own + cnt_next))), s, f->d64, iso, z0 + skip,
-                         ends ? ends + (z0 + skip - s0) * XY : (const double*)nullptr,
-                         own ? (const uint32_t*)(m.cnt + skip * XY) : (const uint32_t*)nullptr,
-                         (const uint32_t*)(m.totals + 1), z1, ends ? ends + (z1 - s0) * XY : (const double*)nullptr,
-                         (uint32_t)cnt_own, (uint32_t)cnt_next, (const uint32_t*)m.vpt, (const uint8_t*)m.vax,
-                         (uint32_t)nv, m.verts, m.c_edges, m.d_bad);
+      launch_nl_vertices(a, dim3(nblocks((int64_t)(cnt_all - placed))), s, f->d64, iso, z0,
+                         reuse_ends ? slab : (const double*)nullptr, (uint32_t)(cnt_all - placed),
+                         (const uint32_t*)m.vpt, (const uint8_t*)m.vax, (uint32_t)(nv + placed), m.verts, m.c_edges,
+                         m.d_bad);
       QJ_HIP(hipGetLastError());
     }
     if (!src_field) QJ_HIP(hipEventRecord(m.ev_free[b], s));  // the last reader of slab[b] is queued
-    // 5. active cells of the chunk, in cell order
-    const int64_t cz1 = z1 < Z - 1 ? z1 : Z - 1;  // cells exist for z <= Z-2
-    const int64_t nc = cz1 > z0 ? cz1 - z0 : 0;
-    int64_t na = 0;
-    if (nc > 0) {
-      const int64_t nb = nblocks(XY * nc);
-      hipLaunchKernelGGL(k_nl_active_count, dim3((unsigned)nb), dim3(kMcBlock), 0, s, m.flags, XY, z0, s0, nc,
-                         m.blk);
-      QJ_HIP(hipGetLastError());
-      if ((st = scan_u32(m.blk, m.blk, nb, m.totals + 0, m.tmp, m.tmp_bytes, s))) return st;
-      hipLaunchKernelGGL(k_nl_active, dim3((unsigned)nb), dim3(kMcBlock), 0, s, m.flags, XY, z0, s0, nc, m.blk,
-                         m.active);
-      QJ_HIP(hipGetLastError());
-      QJ_HIP(hipMemcpyAsync(h, m.totals, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-      QJ_HIP(hipStreamSynchronize(s));
-      na = h[0];
-    }
+    // 5. active cells and triangles, in cell order
+    uint64_t kept = ntp;
     if (na > 0) {
-      const int64_t fo = (z0 - s0) * XY;
-      if ((st = grow_keep(m.c_cells, m.cap_cc, 4 * (m.ncells + na), 4 * m.ncells, s))) return st;
-      hipLaunchKernelGGL(k_nl_cells, dim3(nblocks(na)), dim3(kMcBlock), 0, s, m.active, na, m.flags, fo, X, XY, z0,
-                         m.c_cells + 4 * m.ncells);
+      hipLaunchKernelGGL(k_nl_cells, dim3(nblocks(mg.cells)), dim3(kMcBlock), 0, s, mg, (const uint8_t*)m.flags,
+                         (const uint32_t*)m.aword, (const uint32_t*)ga, z0, m.c_cells + 4 * m.ncells);
       QJ_HIP(hipGetLastError());
-      m.ncells += na;
-      hipLaunchKernelGGL(k_nl_tricount, dim3(nblocks(na)), dim3(kMcBlock), 0, s, m.active, na, m.flags, fo,
-                         m.tri_off);
-      QJ_HIP(hipGetLastError());
-      if ((st = scan_u32(m.tri_off, m.tri_off, na, m.totals + 2, m.tmp, m.tmp_bytes, s))) return st;
-      QJ_HIP(hipMemcpyAsync(h + 2, m.totals + 2, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-      QJ_HIP(hipStreamSynchronize(s));
-      const int64_t ntp = h[2];
-      if ((st = grow(m.tris_pre, m.cap_tp, 3 * ntp, s)) || (st = grow(m.keep, m.cap_keep, ntp, s))) return st;
-      hipLaunchKernelGGL(k_nl_triangles, dim3(nblocks(na)), dim3(kMcBlock), 0, s, m.active, na, m.flags, fo, X, XY,
-                         z0, z1, m.emask, m.cnt, (uint32_t)nv, m.emask + nown, m.slice_off,
-                         (uint32_t)(nv + cnt_own), m.verts, m.tri_off, m.tris_pre, m.keep);
-      QJ_HIP(hipGetLastError());
-      if ((st = scan_u32(m.keep, m.keep, ntp, m.totals + 3, m.tmp, m.tmp_bytes, s))) return st;
-      QJ_HIP(hipMemcpyAsync(h + 3, m.totals + 3, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-      QJ_HIP(hipStreamSynchronize(s));
-      const int64_t ntk = h[3];
-      if ((st = grow_keep(m.tris, m.cap_t, 3 * (int64_t)(nt + ntk), 3 * (int64_t)nt, s))) return st;
-      if (ntk > 0) {
-        hipLaunchKernelGGL(k_mc_squeeze, dim3(nblocks(ntp)), dim3(kMcBlock), 0, s, m.tris_pre, m.keep, ntp,
-                           m.totals + 3, m.tris + 3 * nt);
+      m.ncells += (int64_t)na;
+      if (!sure) {
+        hipLaunchKernelGGL(k_nl_filter, blocks_of(64 * mg.nw, kMcBlock), dim3(kMcBlock), 0, s, mg,
+                           (const uint8_t*)m.flags, (const uint2*)m.ranks, (const uint32_t*)gv, (uint32_t)nv,
+                           (const double*)m.verts, m.kmask, m.lost);
         QJ_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_nl_count<true>, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.flags,
+                           (const uint32_t*)m.lost, m.tword, m.aword, gt, ng);
+        QJ_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gt, ng, m.d_base, 0, 1);
+        QJ_HIP(hipGetLastError());
+        QJ_HIP(hipMemcpyAsync(&kept, m.d_base + 3, sizeof(kept), hipMemcpyDeviceToHost, s));
+        QJ_HIP(hipStreamSynchronize(s));
       }
-      nt += ntk;
+      if ((st = launch_tris(m, mg, gv, gt, nullptr, (uint32_t)nv, (int64_t)ntp, m.tris + 3 * nt, s))) return st;
     }
+    nt += kept;
     nv += cnt_own;
-    placed_next = cnt_next;
+    placed = cnt_all - cnt_own;
   }
   unsigned int bad = 0;
   QJ_HIP(hipMemcpyAsync(&bad, m.d_bad, sizeof(bad), hipMemcpyDeviceToHost, s));
