@@ -280,7 +280,6 @@ constexpr int kMcWaves = kMcBlock / 64;        // waves per workgroup
 constexpr int kMcGroupWords = kMcBlock;        // words per group: the unit of the two scans, one word per thread
 constexpr int kMcGroupPoints = 64 * kMcGroupWords;
 constexpr int kSignPoints = 8;                 // points per thread of k_mc_signs
-constexpr int kVertWords = 8;                  // words per wave of k_mc_vertices
 constexpr int kTriBlocks = 4;                  // blocks of 256 cells per wave of k_mc_tris, at most
 constexpr int kTriWaves = 256 * 16;            // waves that fill the chip before one takes a second block
 constexpr int kListWords = 4;                  // words per wave of k_nl_vlist
@@ -559,7 +558,9 @@ __global__ __launch_bounds__(kScanBlock) void k_mc_scan(uint32_t* __restrict__ g
 // Bound by the field's second read and the vertices' writes: a 256^3 torus tile
 // (4.5 million vertices, 109 MB) 69 us, 3.5 TB/s; neither two vertices per lane
 // in flight, nor stores made contiguous through LDS, nor leaving out the rotation
-// made it faster.
+// made it faster. Below 32 waves per CU a wave takes two words instead of eight
+// (97 x 101 x 89: 7.2 us, with eight 10.3).
+template <int kVertWords>
 __global__ __launch_bounds__(kMcBlock) void k_mc_vertices(const double* __restrict__ field, McGrid a,
                                                           const uint2* __restrict__ ranks,
                                                           const uint32_t* __restrict__ groups,
@@ -664,12 +665,20 @@ __device__ __forceinline__ unsigned mc_measure_cell(const double* __restrict__ f
         unsure |= d > kSureLong ? 0u : 1u << (3 * k + q);
       }
   }
-  unsigned dropped = 0;
-#pragma clang loop unroll(disable)
-  for (int t = 0; t < n; t++) {
-    const unsigned pairs = kMc.tpair[flag][t];
-    if (pairs & brief) dropped |= 1u << t;
-    if (a.prefilter && ((pairs & brief) || !(pairs & unsure))) continue;
+  *row = (1u << n) - 1u;
+  unsigned dropped = 0, measure = *row;
+  if (a.prefilter) {
+    measure = 0;
+#pragma unroll
+    for (int t = 0; t < 5; t++) {
+      const unsigned pairs = kMc.tpair[flag][t];  // none beyond the row's triangles
+      dropped |= pairs & brief ? 1u << t : 0u;
+      measure |= !(pairs & brief) && (pairs & unsure) ? 1u << t : 0u;
+    }
+  }
+  while (measure) {
+    const int t = __ffs(measure) - 1;
+    measure &= measure - 1;
     const unsigned nm = mc_near_edges(v, a.g, a.prefilter) & kMc.tmask[flag][t];
     const int m = __popc(nm);
     if (m < 2) continue;
@@ -698,7 +707,6 @@ __device__ __forceinline__ unsigned mc_measure_cell(const double* __restrict__ f
     }
     if (degenerate) dropped |= 1u << t;
   }
-  *row = (1u << n) - 1u;
   return dropped;
 }
 
@@ -743,17 +751,17 @@ __device__ __forceinline__ uint64_t word_cases(const McGrid& a, int64_t w, uint8
 // word operations on the corners' words. The degenerate filter measures the
 // cells with near vertices on two edges that meet at a corner, found the same
 // way (a border set by setBorders puts near vertices in every cell along it,
-// but on parallel edges), listed per wave and measured one per lane.
+// but on parallel edges), listed in LDS and measured one per thread.
 // flags: the case of every cell that has
-// triangles, else 0. Latency-bound: 256^3, 1024 blocks, 21 us, of which the
-// measurement's longest chain is 9. tword: the triangles before word w in its group; groups:
+// triangles, else 0. Latency-bound: 256^3, 1024 blocks, 17.5 us, of which the
+// measurement's longest chain is 6 (20 with every near pair measured). tword: the triangles before word w in its group; groups:
 // per group.
 __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict__ field, McGrid a,
                                                        uint8_t* __restrict__ flags, uint8_t* __restrict__ kmask,
                                                        uint32_t* __restrict__ tword,
                                                        uint32_t* __restrict__ groups) {
   __shared__ uint16_t s_list[kMcWaves][64 * 64];
-  __shared__ uint32_t s_drop[2 * kMcGroupWords], s_lost[kMcGroupWords];
+  __shared__ uint32_t s_drop[2 * kMcGroupWords], s_lost[kMcGroupWords], s_cells[kMcWaves];
   const int64_t w = (int64_t)blockIdx.x * kMcGroupWords + threadIdx.x;
   const int64_t X = a.g.res[0], XY = a.XY;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -782,25 +790,31 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict_
   }
   s_drop[2 * threadIdx.x] = s_drop[2 * threadIdx.x + 1] = 0u;
   s_lost[threadIdx.x] = 0u;
-  const uint32_t mine = (uint32_t)__popcll(candidates), incl = wave_inclusive(mine), cells = wave_last(incl);
-  if (cells) {
-    uint32_t k = incl - mine;
-    for (uint64_t m = candidates; m; m &= m - 1)
-      s_list[wave][k++] = (uint16_t)(lane << 6 | (__ffsll((unsigned long long)m) - 1));
-    wave_sync();
-    const int64_t p0 = 64 * (w - lane);
-    for (uint32_t j = lane; j < cells; j += 64) {
-      const unsigned i = s_list[wave][j];
-      unsigned row;
-      const unsigned d = mc_measure_cell(field, a, p0 + i, &row);
-      if (d) {
-        kmask[p0 + i] = (uint8_t)(row & ~d);
-        atomicOr(&s_drop[2 * 64 * wave + (i >> 5)], 1u << (i & 31u));
-        atomicAdd(&s_lost[64 * wave + (i >> 6)], (uint32_t)__popc(d));
-      }
+  const uint32_t mine = (uint32_t)__popcll(candidates), incl = wave_inclusive(mine);
+  uint32_t k = incl - mine;
+  for (uint64_t m = candidates; m; m &= m - 1)
+    s_list[wave][k++] = (uint16_t)(lane << 6 | (__ffsll((unsigned long long)m) - 1));
+  if (lane == 63) s_cells[wave] = incl;
+  __syncthreads();
+  // the four waves' lists one after another, over all threads
+  uint32_t from[kMcWaves + 1] = {0};
+#pragma unroll
+  for (int i = 0; i < kMcWaves; i++) from[i + 1] = from[i] + s_cells[i];
+  for (uint32_t j = threadIdx.x; j < from[kMcWaves]; j += kMcBlock) {
+    int v = 0;
+#pragma unroll
+    for (int i = 1; i < kMcWaves; i++) v += j >= from[i] ? 1 : 0;
+    const unsigned i = (unsigned)v << 12 | s_list[v][j - (v == 0 ? 0 : v == 1 ? from[1] : v == 2 ? from[2] : from[3])];
+    const int64_t p = (int64_t)blockIdx.x * kMcGroupPoints + i;
+    unsigned row;
+    const unsigned d = mc_measure_cell(field, a, p, &row);
+    if (d) {
+      kmask[p] = (uint8_t)(row & ~d);
+      atomicOr(&s_drop[i >> 5], 1u << (i & 31u));
+      atomicAdd(&s_lost[i >> 6], (uint32_t)__popc(d));
     }
-    wave_sync();
   }
+  __syncthreads();
   count -= s_lost[threadIdx.x];
   uint32_t total;
   const uint32_t before = block_prefix<kMcBlock>(count, &total);
@@ -1076,7 +1090,9 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
       hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gv, ng, m.d_base, k, 0);
       QJ_HIP(hipGetLastError());
       if (ng) {
-        hipLaunchKernelGGL(k_mc_vertices, blocks_of(mg.nw, kVertWords * kMcWaves), dim3(kMcBlock), 0, s, fields[k], mg,
+        const bool few = mg.nw < 2 * kTriWaves * 8;
+        hipLaunchKernelGGL(few ? k_mc_vertices<2> : k_mc_vertices<8>, blocks_of(mg.nw, (few ? 2 : 8) * kMcWaves),
+                           dim3(kMcBlock), 0, s, fields[k], mg,
                            (const uint2*)m.ranks, (const uint32_t*)gv, (const uint64_t*)(m.d_base + 2 * k), vcap,
                            verts);
         QJ_HIP(hipGetLastError());
