@@ -344,23 +344,74 @@ qj_status launch_check_one(const MapArgs& a, const RootRec64* roots, const doubl
 // ---------------------------------------------------------------- batched chunks (request loop)
 
 __global__ void k_zero_u32(uint32_t* p, int n) {
-  if ((int)threadIdx.x < n) p[threadIdx.x] = 0u;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0u;
 }
 
 __device__ __forceinline__ q64 chunk_start(const MapArgs& a, int64_t idx) { return GridSource::start(a, nullptr, idx); }
 
-// Work queue over (chunk, block-of-chunk) tiles: a resident grid takes tiles
+// Work queues over (chunk, block-of-chunk) tiles: a resident grid takes tiles
 // with one atomic per tile until every tile of its chunk range is taken, so a
 // launch costs what its used chunks cost (no empty blocks) and blocks that
-// draw cheap tiles take more of them. Every block leaves when the queue passes
-// the tile count.
-__device__ __forceinline__ int next_tile(uint32_t* queue) {
-  __shared__ int s_tile;
-  __syncthreads();  // the previous tile's readers are done with s_tile
-  if (threadIdx.x == 0) s_tile = (int)atomicAdd(queue, 1u);
-  __syncthreads();
-  return __builtin_amdgcn_readfirstlane(s_tile);  // uniform: descriptor reads become scalar loads
+// draw cheap tiles take more of them. The tiles are split over kQueues queues in
+// lines of their own, as are the band counts: atomics on one address come back
+// about one in 7 ns, so with one queue and one count a launch of requests with
+// 8 to 45 roots waited for them most of its time (k_batch32<1> 896 us a launch,
+// 360 with the split; <3>, more roots, 960 and 1000). A block starts at its own
+// queue and goes on to the next ones when that is empty. The next tile is
+// drawn while one is evaluated. Every block leaves when all queues are empty.
+constexpr int kQueues = 8, kQueueLine = 32;
+__host__ __device__ __forceinline__ int queue_start(int tiles, int q) { return (int)((int64_t)tiles * q / kQueues); }
+
+// Batch counters (uint32), a line each: per FP32 variant (0 for the FP64-only
+// kernel) and queue the tiles drawn and the band voxels listed.
+enum { BC_DRAWN = 0, BC_BAND = 1, BC_N = 4 * kQueues * 2 * kQueueLine };
+static_assert(BC_N == kBatchCounters, "");
+__device__ __forceinline__ int64_t batch_counter(int variant, int queue, int which) {
+  return (int64_t)((variant * kQueues + queue) * 2 + which) * kQueueLine;
 }
+
+struct Tile {
+  int tile, queue;  // tile < 0: none left
+};
+// The tiles of one variant; next() is called by every thread of the block and
+// gives them all the same tile. s: two LDS entries, used in turn, so that one
+// barrier per tile is enough.
+struct TileQueue {
+  uint32_t* counters;
+  int variant, tiles, queue, left, slot;
+  uint32_t drawn;
+  Tile* s;
+  __device__ __forceinline__ TileQueue(uint32_t* c, int v, int n, Tile* lds)
+      : counters(c), variant(v), tiles(n), queue((int)(blockIdx.x & (kQueues - 1))), left(kQueues), slot(0), s(lds) {
+    draw();
+  }
+  __device__ __forceinline__ void draw() {
+    drawn = 0;
+    if (threadIdx.x == 0 && left > 0) drawn = atomicAdd(counters + batch_counter(variant, queue, BC_DRAWN), 1u);
+  }
+  __device__ __forceinline__ Tile next() {
+    if (threadIdx.x == 0) {
+      Tile t{-1, 0};
+      while (left > 0) {
+        const int lo = queue_start(tiles, queue), n = queue_start(tiles, queue + 1) - lo;
+        if (drawn < (uint32_t)n) {
+          t = Tile{lo + (int)drawn, queue};
+          break;
+        }
+        queue = (queue + 1) & (kQueues - 1);
+        left--;
+        draw();
+      }
+      s[slot] = t;
+    }
+    __syncthreads();
+    // uniform: descriptor reads become scalar loads
+    const Tile t{__builtin_amdgcn_readfirstlane(s[slot].tile), __builtin_amdgcn_readfirstlane(s[slot].queue)};
+    slot ^= 1;
+    draw();
+    return t;
+  }
+};
 
 // A root block read through the constant address space: its loads are known
 // not to be clobbered by the kernel's stores, so a block-uniform address gives
@@ -377,27 +428,31 @@ __device__ __forceinline__ Roots32K roots32_const(const F4* blk, int n) {
                   (const __attribute__((address_space(4))) float*)r.e};
 }
 
-// Batch counters (uint32): [0] band count of integer-exponent chunks (list from
-// the front), [1] band count of general chunks (list from the back), [2..5]
-// FP32 queues per variant, [6] FP64 queue.
-enum { BC_BAND_INT = 0, BC_BAND_GEN = 1, BC_Q32 = 2, BC_Q64 = 6, BC_N = 8 };
-
 // Descriptors are grouped by FP32 variant: chunks [0, g1) have general
 // exponents, [g1, g2) integer exponents renormalised every 4 terms, [g2, g3)
 // every 2 and [g3, total) every 8.
+__device__ __forceinline__ int first_chunk(const ChunkDesc& d0, int variant) {
+  return variant == 0 ? 0 : (variant == 1 ? d0.g1 : (variant == 2 ? d0.g2 : (variant == 3 ? d0.g3 : d0.total)));
+}
+
+// A queue's band voxels go to the part of the list that its tiles would fill, in
+// the order of the tiles.
+__device__ __forceinline__ int64_t tile_entries(int64_t tiles, int chunk_voxels) {
+  return tiles * (chunk_voxels < kBlock ? chunk_voxels : kBlock);
+}
 template <int kVar>
 __global__ __launch_bounds__(kBlock) void k_batch32(const ChunkDesc* __restrict__ descs, int blocks_per_chunk,
-                                                    int chunk_voxels, uint32_t* __restrict__ blist, int64_t list_cap,
+                                                    int chunk_voxels, uint32_t* __restrict__ blist,
                                                     uint32_t* __restrict__ counters) {
   constexpr int kRN = kVar == 1 ? 4 : (kVar == 3 ? 8 : 2);
   constexpr bool kGen = kVar == 0;
-  const ChunkDesc& d0 = descs[0];
-  const int c0 = kVar == 0 ? 0 : (kVar == 1 ? d0.g1 : (kVar == 2 ? d0.g2 : d0.g3));
-  const int c1 = kVar == 0 ? d0.g1 : (kVar == 1 ? d0.g2 : (kVar == 2 ? d0.g3 : d0.total));
+  __shared__ Tile s_tile[2];
+  const int c0 = first_chunk(descs[0], kVar), c1 = first_chunk(descs[0], kVar + 1);
   const int tiles = (c1 - c0) * blocks_per_chunk;
-  for (int tile = next_tile(counters + BC_Q32 + kVar); tile < tiles; tile = next_tile(counters + BC_Q32 + kVar)) {
-    const int c = c0 + tile / blocks_per_chunk;
-    const int local = (tile % blocks_per_chunk) * kBlock + threadIdx.x;
+  TileQueue queue(counters, kVar, tiles, s_tile);
+  for (Tile t = queue.next(); t.tile >= 0; t = queue.next()) {
+    const int c = c0 + t.tile / blocks_per_chunk;
+    const int local = (t.tile % blocks_per_chunk) * kBlock + threadIdx.x;
     const ChunkDesc& d = descs[c];
     bool need = false;
     if (local < d.count) {
@@ -421,43 +476,43 @@ __global__ __launch_bounds__(kBlock) void k_batch32(const ChunkDesc* __restrict_
       }
     }
     const uint32_t e = (uint32_t)(c * chunk_voxels + local);
-    if (kGen) {
-      // general chunks fill the list from the back: entry k at list_cap - 1 - k
-      __shared__ uint32_t s_gbase;
-      const unsigned long long m = __ballot(need);
-      __shared__ uint32_t s_gcnt[kBlock / 64];
-      const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-      if (lane == 0) s_gcnt[wave] = (uint32_t)__popcll(m);
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        uint32_t t = 0;
-        for (int w = 0; w < kBlock / 64; w++) {
-          const uint32_t cw = s_gcnt[w];
-          s_gcnt[w] = t;
-          t += cw;
-        }
-        s_gbase = t ? atomicAdd(counters + BC_BAND_GEN, t) : 0u;
-      }
-      __syncthreads();
-      if (need) {
-        const uint32_t k = s_gbase + s_gcnt[wave] + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        blist[list_cap - 1 - (int64_t)k] = e;
-      }
-    } else {
-      block_append(need, e, blist, counters + BC_BAND_INT, (uint32_t)list_cap);
-    }
+    const int64_t lo = (int64_t)c0 * blocks_per_chunk + queue_start(tiles, t.queue);
+    const int own = queue_start(tiles, t.queue + 1) - queue_start(tiles, t.queue);
+    block_append(need, e, blist + tile_entries(lo, chunk_voxels), counters + batch_counter(kVar, t.queue, BC_BAND),
+                 (uint32_t)tile_entries(own, chunk_voxels));
   }
 }
 
-// FP64 for the band list of one exponent class (integer exponents as exact
-// products); kFromEnd reads the general chunks' list from the back.
-template <int kPow, bool kFromEnd>
-__global__ __launch_bounds__(kBlock) void k_batch64_list(const ChunkDesc* __restrict__ descs, int chunk_voxels,
-                                                         const uint32_t* __restrict__ list, int64_t list_cap,
-                                                         const uint32_t* __restrict__ count) {
-  const int64_t n = *count;
+// FP64 for the band lists of one exponent class: the general variant's
+// (kPow kExactInt) or the three integer variants' (exponents as exact products).
+template <int kPow>
+__global__ __launch_bounds__(kBlock) void k_batch64_list(const ChunkDesc* __restrict__ descs, int blocks_per_chunk,
+                                                         int chunk_voxels, const uint32_t* __restrict__ list,
+                                                         const uint32_t* __restrict__ counters) {
+  constexpr int kVar0 = kPow == kExactOnly ? 1 : 0, kLists = (kPow == kExactOnly ? 3 : 1) * kQueues;
+  __shared__ uint32_t s_end[kLists];
+  __shared__ int64_t s_at[kLists];  // the list's place less the entries before it
+  if (threadIdx.x < kLists) {
+    const int v = kVar0 + threadIdx.x / kQueues, q = threadIdx.x & (kQueues - 1);
+    const int c0 = first_chunk(descs[0], v), tiles = (first_chunk(descs[0], v + 1) - c0) * blocks_per_chunk;
+    s_end[threadIdx.x] = counters[batch_counter(v, q, BC_BAND)];
+    s_at[threadIdx.x] = tile_entries((int64_t)c0 * blocks_per_chunk + queue_start(tiles, q), chunk_voxels);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t sum = 0;
+    for (int i = 0; i < kLists; i++) {
+      s_at[i] -= sum;
+      sum += s_end[i];
+      s_end[i] = sum;
+    }
+  }
+  __syncthreads();
+  const int64_t n = s_end[kLists - 1];
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const uint32_t e = kFromEnd ? list[list_cap - 1 - i] : list[i];
+    int l = 0;
+    while (i >= (int64_t)s_end[l]) l++;
+    const uint32_t e = list[s_at[l] + i];
     const int c = (int)(e / (uint32_t)chunk_voxels);
     const int local = (int)(e - (uint32_t)c * (uint32_t)chunk_voxels);
     // the list interleaves the chunks that were in flight together, but a
@@ -485,10 +540,11 @@ __global__ __launch_bounds__(kBlock) void k_batch64_list(const ChunkDesc* __rest
 // FP64 for every voxel of every chunk, work-queue tiles
 __global__ __launch_bounds__(kBlock) void k_batch64(const ChunkDesc* __restrict__ descs, int blocks_per_chunk,
                                                     uint32_t* __restrict__ counters) {
-  const int tiles = descs[0].total * blocks_per_chunk;
-  for (int tile = next_tile(counters + BC_Q64); tile < tiles; tile = next_tile(counters + BC_Q64)) {
-    const int c = tile / blocks_per_chunk;
-    const int local = (tile - c * blocks_per_chunk) * kBlock + threadIdx.x;
+  __shared__ Tile s_tile[2];
+  TileQueue queue(counters, 0, descs[0].total * blocks_per_chunk, s_tile);
+  for (Tile t = queue.next(); t.tile >= 0; t = queue.next()) {
+    const int c = t.tile / blocks_per_chunk;
+    const int local = (t.tile - c * blocks_per_chunk) * kBlock + threadIdx.x;
     const ChunkDesc& d = descs[c];
     if (local < d.count) {
       const int64_t idx = d.start + local;
@@ -541,8 +597,7 @@ int batch_variant(const MapArgs& a) {
 qj_status launch_batch(const ChunkDesc* d_desc, int nchunks, int chunk_voxels, qj_precision prec, uint32_t* d_band,
                        uint32_t* d_counters, unsigned variants, hipStream_t s) {
   const int bpc = (chunk_voxels + kBlock - 1) / kBlock;
-  const int64_t cap = (int64_t)nchunks * chunk_voxels;
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, d_counters, (int)BC_N);
+  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(256), 0, s, d_counters, (int)BC_N);
   QJ_HIP(hipGetLastError());
   if (prec == QJ_FP64) {
     static const int g64 = resident_blocks((const void*)k_batch64);
@@ -557,29 +612,29 @@ qj_status launch_batch(const ChunkDesc* d_desc, int nchunks, int chunk_voxels, q
   // a variant with no chunks is not launched: an empty persistent grid still waits for free
   // compute units behind the other in-flight launch
   if (variants & 2u) {
-    hipLaunchKernelGGL(k_batch32<1>, dim3(g1), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels, d_band, cap, d_counters);
+    hipLaunchKernelGGL(k_batch32<1>, dim3(g1), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels, d_band, d_counters);
     QJ_HIP(hipGetLastError());
   }
   if (variants & 4u) {
-    hipLaunchKernelGGL(k_batch32<2>, dim3(g2), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels, d_band, cap, d_counters);
+    hipLaunchKernelGGL(k_batch32<2>, dim3(g2), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels, d_band, d_counters);
     QJ_HIP(hipGetLastError());
   }
   if (variants & 8u) {
-    hipLaunchKernelGGL(k_batch32<3>, dim3(g3), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels, d_band, cap, d_counters);
+    hipLaunchKernelGGL(k_batch32<3>, dim3(g3), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels, d_band, d_counters);
     QJ_HIP(hipGetLastError());
   }
   if (variants & 1u) {
-    hipLaunchKernelGGL(k_batch32<0>, dim3(g0), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels, d_band, cap, d_counters);
+    hipLaunchKernelGGL(k_batch32<0>, dim3(g0), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels, d_band, d_counters);
     QJ_HIP(hipGetLastError());
   }
   if (variants & 14u) {  // band voxels of the integer-exponent variants
-    hipLaunchKernelGGL((k_batch64_list<kExactOnly, false>), dim3(2048), dim3(kBlock), 0, s, d_desc, chunk_voxels,
-                       (const uint32_t*)d_band, cap, (const uint32_t*)(d_counters + BC_BAND_INT));
+    hipLaunchKernelGGL(k_batch64_list<kExactOnly>, dim3(2048), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels,
+                       (const uint32_t*)d_band, (const uint32_t*)d_counters);
     QJ_HIP(hipGetLastError());
   }
   if (variants & 1u) {  // band voxels of the general variant
-    hipLaunchKernelGGL((k_batch64_list<kExactInt, true>), dim3(1024), dim3(kBlock), 0, s, d_desc, chunk_voxels,
-                       (const uint32_t*)d_band, cap, (const uint32_t*)(d_counters + BC_BAND_GEN));
+    hipLaunchKernelGGL(k_batch64_list<kExactInt>, dim3(1024), dim3(kBlock), 0, s, d_desc, bpc, chunk_voxels,
+                       (const uint32_t*)d_band, (const uint32_t*)d_counters);
     QJ_HIP(hipGetLastError());
   }
   return QJ_OK;

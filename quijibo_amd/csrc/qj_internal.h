@@ -139,13 +139,17 @@ qj_status launch_check_one(const MapArgs& a, const RootRec64* roots, const doubl
 // renormalised every 4 terms (1), every 2 (2) or every 8 (3) (rn_of).
 int batch_variant(const MapArgs& a);
 // Enqueue one batch: FP32 bulk over every chunk then FP64 for the band (or
-// FP64 for all when prec == QJ_FP64). d_band/d_band_count: scratch of
-// nchunks * chunk_voxels entries; the count is cleared by a kernel, not a
-// memset, so the sequence can be captured in a graph and replayed.
-// d_counters: 8 uint32 (band counts and work queues), cleared at the start of
-// every batch; d_band: nchunks * chunk_voxels entries. variants: bit v set when
+// FP64 for all when prec == QJ_FP64). d_counters: kBatchCounters uint32 (band
+// counts and work queues), cleared at the start of every batch by a kernel, not
+// a memset, so the sequence can be captured in a graph and replayed. d_band:
+// nchunks * batch_band_entries(chunk_voxels) entries. variants: bit v set when
 // the batch holds chunks of FP32 variant v (kernels of absent variants are not
 // enqueued; ignored for QJ_FP64).
+constexpr int kBatchCounters = 2048;
+// band list entries per chunk: whole tiles of 256 voxels, or of a smaller chunk
+inline int64_t batch_band_entries(int chunk_voxels) {
+  return chunk_voxels < 256 ? chunk_voxels : ((int64_t)chunk_voxels + 255) / 256 * 256;
+}
 qj_status launch_batch(const ChunkDesc* d_desc, int nchunks, int chunk_voxels, qj_precision prec, uint32_t* d_band,
                        uint32_t* d_counters, unsigned variants, hipStream_t s);
 

@@ -128,7 +128,7 @@ struct Slot {
   ChunkDesc* h_desc = nullptr;
   ChunkDesc* d_desc = nullptr;
   uint32_t* d_band = nullptr;
-  uint32_t* d_band_count = nullptr;  // batch counters: band counts and work queues (8 x uint32)
+  uint32_t* d_band_count = nullptr;  // batch counters: band counts and work queues
   // one graph per set of FP32 variants present in a batch (bit v = variant v);
   // an FP64 server uses exec[0] only
   hipGraphExec_t exec[16] = {};
@@ -504,10 +504,10 @@ static qj_status capture_slot(qj_server* s, Slot& sl) {
   QJ_HIP(hipMalloc(&sl.d_desc, sizeof(ChunkDesc) * nch));
   QJ_HIP(hipMemset(sl.d_desc, 0, sizeof(ChunkDesc) * nch));
   if (s->cfg.precision == QJ_FP64) {
-    QJ_HIP(hipMalloc(&sl.d_band_count, 8 * sizeof(uint32_t)));  // work-queue counters
+    QJ_HIP(hipMalloc(&sl.d_band_count, kBatchCounters * sizeof(uint32_t)));  // work-queue counters
   } else {
-    QJ_HIP(hipMalloc(&sl.d_band, sizeof(uint32_t) * (size_t)nch * s->cfg.chunk_voxels));
-    QJ_HIP(hipMalloc(&sl.d_band_count, 8 * sizeof(uint32_t)));
+    QJ_HIP(hipMalloc(&sl.d_band, sizeof(uint32_t) * (size_t)nch * (size_t)batch_band_entries(s->cfg.chunk_voxels)));
+    QJ_HIP(hipMalloc(&sl.d_band_count, kBatchCounters * sizeof(uint32_t)));
   }
   QJ_HIP(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
   QJ_HIP(hipStreamCreateWithFlags(&sl.stream, hipStreamNonBlocking));
