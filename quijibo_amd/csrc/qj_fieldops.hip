@@ -227,16 +227,18 @@ __device__ __forceinline__ bool shell_cell(const double* __restrict__ d, int64_t
 // separable: one pass per axis, each the minimum over the line of value +
 // distance along it. (The sweeps took one launch, one counter read-back and
 // one wait each, about half the grid's edge of them: 50^3 25 sweeps, 1.5 ms.)
-// A block takes kLines lines of one axis; the minimum over a line of n cells by
+// A block takes 16 lines of one axis (4 rows for the
+// x pass, whose shells make most of the work: a cell per thread at 50^3); the minimum over a line of n cells by
 // doubling, v[i] = min(v[i], v[i - d] + d, v[i + d] + d) for d = 1, 2, 4, ... < n,
 // between two LDS copies. Lines of neighbouring x are taken together along y and
 // z, so that loads stay in runs of 64 B. The x pass starts from the shells; the
 // z pass writes the inverted, signed value (FIELD_3D.cpp:5286-5296: 1 / number,
 // negated inside and quartered outside) and the partial sums of its absolute
 // value; part's last entry counts the cells no shell reaches. Latency bound:
-// 50^3, 157 blocks a pass: 21.5 us along x (26 neighbours per cell for the
-// shells), 7.4 along y, 9.1 along z.
-constexpr int kLines = 16, kMaxLine = 512;
+// 50^3: 10 us along x (625 blocks; 21.5 with 16 rows each), 7 along y and 9 along z
+// (157 blocks).
+constexpr int kMaxLine = 512;
+constexpr int lines_of(int axis) { return axis == 0 ? 4 : 16; }
 constexpr uint32_t kFar = 0x3fffffffu;  // no shell cell on the lines so far
 enum LineAxis { kAxisX = 0, kAxisY = 1, kAxisZ = 2 };
 
@@ -251,6 +253,7 @@ template <int kAxis>
 __global__ __launch_bounds__(kOpsBlock) void k_layers(const double* __restrict__ d, int64_t X, int64_t Y, int64_t Z,
                                                       uint32_t* __restrict__ lay, double* __restrict__ out,
                                                       double* __restrict__ part) {
+  constexpr int kLines = lines_of(kAxis);
   extern __shared__ uint32_t s_v[];  // 2 x n x kLines
   const int64_t XY = X * Y;
   const int n = (int)(kAxis == kAxisX ? X : kAxis == kAxisY ? Y : Z);
@@ -394,12 +397,13 @@ __global__ __launch_bounds__(kOpsBlock) void k_normalize(double* __restrict__ v,
   }
 }
 
-// Block b: the total of partials [b nparts, (b + 1) nparts) to d_out[b] and,
-// with h_out, to pinned host memory; count0: the first one's count there too.
+// Block b: the total of partials [b nparts, (b + 1) nparts) (nlast of them in the
+// last block) to d_out[b] and, with h_out, to pinned host memory; count0: the first one's count there too.
 __global__ __launch_bounds__(kOpsBlock) void k_fold_sums(const double* __restrict__ part, int nparts,
-                                                         double* __restrict__ d_out, double* __restrict__ h_out,
+                                                         int nlast, double* __restrict__ d_out, double* __restrict__ h_out,
                                                          double* __restrict__ h_count) {
-  const Acc a = combine(part + 4 * (int64_t)blockIdx.x * nparts, nparts);
+  const Acc a = combine(part + 4 * (int64_t)blockIdx.x * nparts,
+                        blockIdx.x + 1 == gridDim.x ? nlast : nparts);
   if (threadIdx.x == 0) {
     const double t = total_of(a);
     if (d_out) d_out[blockIdx.x] = t;
@@ -445,7 +449,7 @@ __global__ __launch_bounds__(kOpsBlock) void k_cell_weights(GridGeom g, GridGeom
 // thresholds from blockIdx.y kScores on: the partial sums of
 // -tanh(alpha (F - threshold)) w(cell centre). FP64 VALU bound (the tanh); the
 // field and the cells' weights are read once per kScores thresholds. 50^3, 100
-// thresholds: 41 us; one threshold per block with the lookup and the library's
+// thresholds: 34 us; one threshold per block with the lookup and the library's
 // tanh 169 us, this split with the library's tanh 67 us.
 constexpr int kScores = 4;
 __global__ __launch_bounds__(kOpsBlock) void k_weight_score(const double* __restrict__ f,
@@ -620,6 +624,7 @@ static qj_status launch_layers(const double* d, int64_t X, int64_t Y, int64_t Z,
                                double* part, int64_t* blocks, hipStream_t s) {
   const int64_t n = kAxis == kAxisX ? X : kAxis == kAxisY ? Y : Z, lines = X * Y * Z / n;
   if (n <= kMaxLine) {
+    constexpr int kLines = lines_of(kAxis);
     const int64_t per = kAxis == kAxisY ? X : lines, outer = kAxis == kAxisY ? Z : 1;
     *blocks = outer * ((per + kLines - 1) / kLines);
     if (*blocks > INT32_MAX) return QJ_ERR_CAPACITY;
@@ -642,7 +647,7 @@ qj_status field_inverted_distance(qj_workspace* ws, const double* d_dist, const 
   const int64_t X = grid->res[0], Y = grid->res[1], Z = grid->res[2], n = X * Y * Z;
   if (n <= 0) return QJ_OK;
   const int64_t zlines = X * Y;
-  const int64_t zblocks = Z <= kMaxLine ? (zlines + kLines - 1) / kLines : (zlines + kOpsBlock - 1) / kOpsBlock;
+  const int64_t zblocks = Z <= kMaxLine ? (zlines + lines_of(kAxisZ) - 1) / lines_of(kAxisZ) : (zlines + kOpsBlock - 1) / kOpsBlock;
   const int64_t want = (n + kOpsBlock - 1) / kOpsBlock;
   const int grid_sum = (int)(want < kOpsGrid ? want : kOpsGrid);
   const int64_t nparts = std::max<int64_t>(zblocks, 2 * (int64_t)grid_sum);
@@ -664,20 +669,21 @@ qj_status field_inverted_distance(qj_workspace* ws, const double* d_dist, const 
     return st;
   // h_pinned: [0] the absolute sum of the result, [1] the cells without a number
   double* h = ws->h_pinned;
-  hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kOpsBlock), 0, s, (const double*)part, (int)nb, scal, h, h + 1);
+  hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kOpsBlock), 0, s, (const double*)part, (int)nb, (int)nb, scal, h,
+                     h + 1);
   QJ_HIP(hipGetLastError());
   if (normalized) {
     hipLaunchKernelGGL(k_normalize<0>, dim3(grid_sum), dim3(kOpsBlock), 0, s, d_out, d_dist, n, (const double*)scal,
                        part);
     QJ_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_fold_sums, dim3(2), dim3(kOpsBlock), 0, s, (const double*)part, grid_sum, scal,
+    hipLaunchKernelGGL(k_fold_sums, dim3(2), dim3(kOpsBlock), 0, s, (const double*)part, grid_sum, grid_sum, scal,
                        (double*)nullptr, (double*)nullptr);
     QJ_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_normalize<1>, dim3(grid_sum), dim3(kOpsBlock), 0, s, d_out, d_dist, n, (const double*)scal,
                        part);
     QJ_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kOpsBlock), 0, s, (const double*)part, grid_sum, (double*)nullptr, h,
-                       (double*)nullptr);
+    hipLaunchKernelGGL(k_fold_sums, dim3(1), dim3(kOpsBlock), 0, s, (const double*)part, grid_sum, grid_sum,
+                       (double*)nullptr, h, (double*)nullptr);
     QJ_HIP(hipGetLastError());
   }
   QJ_HIP(hipStreamSynchronize(s));
@@ -716,34 +722,39 @@ qj_status weight_scores(qj_workspace* ws, const double* d_field, const qj_grid* 
   make_geom(wgrid, &wg);
   const int64_t n = (int64_t)g.res[0] * g.res[1] * g.res[2];
   if (n <= 0 || nthr < 0) return QJ_ERR_INVALID;
-  const int64_t want = (n + kOpsBlock - 1) / kOpsBlock;
-  const int gx = (int)(want < 256 ? want : 256);
+  // up to 8 cells per thread where the thresholds fill the chip by themselves:
+  // the four block sums cost as much as some 10 cells (50^3, 100 thresholds: 1750
+  // blocks 34 us, 6400 of 2 cells 41)
+  const int64_t want = (n + kOpsBlock - 1) / kOpsBlock, ny = (nthr + kScores - 1) / kScores;
+  const int64_t per = std::min<int64_t>(8, std::max<int64_t>(1, want * ny / 1536));
+  const int gx = (int)std::min<int64_t>((want + per - 1) / per, 256);
+  const int gw = (int)std::min<int64_t>(want, 256);
   const int slots = nthr + 1;
   // the partials (the last slot's: the weights' absolute sum), the thresholds, the cells' weights
   const bool keep = n <= kKeepCells;
-  qj_status st = ensure_partials(ws, 4 * (int64_t)gx * slots + (int64_t)slots + (keep ? n : 0), s);
+  qj_status st = ensure_partials(ws, 4 * ((int64_t)gx * nthr + gw) + (int64_t)slots + (keep ? n : 0), s);
   if (st) return st;
   if ((st = ensure_pinned(ws, 2 * (int64_t)slots, s))) return st;
   double* part = ws->d_partials;
-  double* d_thr = part + 4 * (int64_t)gx * slots;
+  double* d_thr = part + 4 * ((int64_t)gx * nthr + gw);
   CellScratch cells;
   if (keep) cells.p = d_thr + slots;
   else QJ_HIP(hipMalloc(&cells.p, sizeof(double) * (size_t)n));
   cells.own = !keep;
   double* cw = (double*)cells.p;
-  hipLaunchKernelGGL(k_cell_weights, dim3(gx), dim3(kOpsBlock), 0, s, g, wg, d_weight, cw,
+  hipLaunchKernelGGL(k_cell_weights, dim3(gw), dim3(kOpsBlock), 0, s, g, wg, d_weight, cw,
                      part + 4 * (int64_t)gx * nthr);
   QJ_HIP(hipGetLastError());
   if (nthr) {
     double* h_thr = ws->h_pinned + slots;
     for (int t = 0; t < nthr; t++) h_thr[t] = thresholds[t];
     QJ_HIP(hipMemcpyAsync(d_thr, h_thr, sizeof(double) * (size_t)nthr, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_weight_score, dim3(gx, (nthr + kScores - 1) / kScores), dim3(kOpsBlock), 0, s, d_field,
+    hipLaunchKernelGGL(k_weight_score, dim3(gx, (unsigned)ny), dim3(kOpsBlock), 0, s, d_field,
                        (const double*)cw, n, (const double*)d_thr, nthr, alpha, part);
     QJ_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(k_fold_sums, dim3(slots), dim3(kOpsBlock), 0, s, (const double*)part, gx, (double*)nullptr,
-                     ws->h_pinned, (double*)nullptr);
+  hipLaunchKernelGGL(k_fold_sums, dim3(slots), dim3(kOpsBlock), 0, s, (const double*)part, gx, gw,
+                     (double*)nullptr, ws->h_pinned, (double*)nullptr);
   QJ_HIP(hipGetLastError());
   QJ_HIP(hipStreamSynchronize(s));
   for (int t = 0; t < nthr; t++) scores[t] = ws->h_pinned[t];
