@@ -127,8 +127,8 @@ __global__ __launch_bounds__(kBlock) void k_grid64(MapArgs a, const RootRec64* _
     cell_center(a, x, y, z + a.zoff, c);
     const q64 q0{c[0], c[1], c[2], a.slice};
     Res64 r;
-    if constexpr (kExt) r = eval64e<kPow>(a, roots, q0);
-    else r = eval64<kPow>(a, roots, q0);
+    if constexpr (kExt) r = eval64e<kPow>(a, (ConstRoots)roots, q0);
+    else r = eval64<kPow>(a, (ConstRoots)roots, q0);
     if (r.written) {
       out[idx] = r.F;
       nonfinite = !isfinite(r.F);
@@ -206,8 +206,8 @@ __global__ __launch_bounds__(kBlock) void k_list64(MapArgs a, const RootRec64* _
       const q64 q0 = Src::start(a, pts, idx);
       Res64 r;
       if constexpr (kEval == kRepass) r = eval64x(a, roots, q0);
-      else if constexpr (kEval == kExtRange) r = eval64e<kPow>(a, roots, q0);
-      else r = eval64<kPow>(a, roots, q0);
+      else if constexpr (kEval == kExtRange) r = eval64e<kPow>(a, (ConstRoots)roots, q0);
+      else r = eval64<kPow>(a, (ConstRoots)roots, q0);
       if (r.written) out[idx] = r.F;
       else if (pts) out[idx] = __builtin_nan("");
       vox++;
@@ -240,8 +240,8 @@ __global__ __launch_bounds__(kBlock) void k_band_sweep(MapArgs a, const RootRec6
     if (i < n_all && ((const unsigned long long*)out)[i] == kBandMark) {
       const q64 q0 = Src::start(a, pts, (uint32_t)i);
       Res64 r;
-      if constexpr (kEval == kExtRange) r = eval64e<kPow>(a, roots, q0);
-      else r = eval64<kPow>(a, roots, q0);
+      if constexpr (kEval == kExtRange) r = eval64e<kPow>(a, (ConstRoots)roots, q0);
+      else r = eval64<kPow>(a, (ConstRoots)roots, q0);
       if (r.written) out[i] = r.F;
       else if (pts) out[i] = __builtin_nan("");
       vox++;
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* 
   if (i < samples) {
     const int64_t idx = ((2 * i + 1) * nvox) / (2 * samples);
     const q64 q0 = GridSource::start(a, nullptr, idx);
-    Res64 r = eval64_any<kPow>(a, roots, q0);
+    Res64 r = eval64_any<kPow>(a, (ConstRoots)roots, q0);
     if ((a.flags & QJ_MAP_ADAPTIVE) && r.overflow) r = eval64x(a, roots, q0);
     if (r.written) {
       const double F = field[idx];
@@ -525,8 +525,7 @@ __global__ __launch_bounds__(kBlock) void k_batch64_list(const ChunkDesc* __rest
     const ChunkDesc& dl = descs[c];
     if (__ballot(dl.r64 != dw.r64) == 0ull) {
       const int64_t idx = dl.start + local;
-      typedef const __attribute__((address_space(4))) RootRec64 cR64;
-      const Res64 r = eval64_any<kPow>(dw.a, (cR64*)dw.r64, chunk_start(dw.a, idx));
+      const Res64 r = eval64_any<kPow>(dw.a, (ConstRoots)dw.r64, chunk_start(dw.a, idx));
       if (r.written) dw.out[idx] = r.F;
     } else {
       const ChunkDesc& d = descs[c];
@@ -548,8 +547,8 @@ __global__ __launch_bounds__(kBlock) void k_batch64(const ChunkDesc* __restrict_
     const ChunkDesc& d = descs[c];
     if (local < d.count) {
       const int64_t idx = d.start + local;
-      const Res64 r = (d.a.flags & QJ_MAP_LAGRANGE) ? eval64<kPolar>(d.a, d.r64, chunk_start(d.a, idx))
-                                                    : eval64_any<kExactInt>(d.a, d.r64, chunk_start(d.a, idx));
+      const Res64 r = (d.a.flags & QJ_MAP_LAGRANGE) ? eval64<kPolar>(d.a, (ConstRoots)d.r64, chunk_start(d.a, idx))
+                                                    : eval64_any<kExactInt>(d.a, (ConstRoots)d.r64, chunk_start(d.a, idx));
       if (r.written) d.out[idx] = r.F;
     }
   }

@@ -1234,7 +1234,7 @@ __device__ __forceinline__ double nonlinear_value(const MapArgs& a, const RootRe
     double magnitude = qmag(q), prev = magnitude;
     int it = 0;
     while (magnitude < a.escape && it < a.max_iter) {
-      q = qscale(lagrange64<kPow>(roots, a.nt, a.nb, q), a.exp_scaling);
+      q = qscale(lagrange64<kPow>((ConstRoots)roots, a.nt, a.nb, q), a.exp_scaling);
       magnitude = qmag(q);
       if (isinf(magnitude)) {
         magnitude = prev;
@@ -1249,7 +1249,7 @@ __device__ __forceinline__ double nonlinear_value(const MapArgs& a, const RootRe
     return isinf(v) ? (double)FLT_MAX : v;
   }
   const q64 q0{p[0], p[1], p[2], a.slice};
-  const Res64 r = kMap == kNlExt ? eval64e<kPow>(a, roots, q0) : eval64<kPow>(a, roots, q0);
+  const Res64 r = kMap == kNlExt ? eval64e<kPow>(a, (ConstRoots)roots, q0) : eval64<kPow>(a, (ConstRoots)roots, q0);
   return r.F - iso;
 }
 
