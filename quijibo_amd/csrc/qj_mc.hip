@@ -1424,12 +1424,11 @@ __global__ __launch_bounds__(kMcBlock) void k_nl_vlist(McGrid a, const uint64_t*
 // that starts at slice z0, gets id base + t. ends: null, or the slab's values,
 // when they are the end values' own (see slab_holds_end_values); the midpoints
 // are always evaluated.
-// FP64 VALU bound. For exponents 1 and 2 the registers are held to five waves
-// per SIMD (96, 136 B of a vertex's state spilled round the evaluation; 128 and
-// four before): meshes of 0.4 million vertices and more 3 to 7 % faster, smaller
-// ones as fast.
+// FP64 VALU bound beside the next slab's FP32 evaluation. No bound on the
+// registers (151 for exponents 1 and 2): held to five or four waves per SIMD
+// (136 to 224 B spilled) meshes take -1 to 4 % longer.
 template <int kPow, int kMap>
-__global__ __launch_bounds__(kMcBlock, kPow == kExactOnly && kMap == kNlPlain ? 5 : 1) void k_nl_vertices(MapArgs a, const RootRec64* __restrict__ roots,
+__global__ __launch_bounds__(kMcBlock) void k_nl_vertices(MapArgs a, const RootRec64* __restrict__ roots,
                                                           double iso, int64_t z0, const double* __restrict__ ends,
                                                           uint32_t n, const uint32_t* __restrict__ vpt,
                                                           const uint8_t* __restrict__ vax, uint32_t base,
