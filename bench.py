@@ -2,7 +2,7 @@
 
 One step = one evaluation of the whole 512^3 field (config-2 roots: 32 top + 32
 bottom Gaussian roots, powers in {1,2}, maxIter 4, escape 2000) with the FP32
-bulk + FP64 band kernel pair. The plain all-FP64 kernel is timed beside it.
+bulk + FP64 band kernel pair. The all-FP64 kernel is timed beside it.
 Inputs (roots) and the output field are resident in HBM during the timed region.
 
 Prints one JSON line on stdout; progress goes to stderr.
@@ -154,7 +154,7 @@ def main():
                                                                                  8 << 27)}))
         return
 
-    # plain FP64 kernel
+    # FP64 for every voxel
     log("fp64: warmup")
     api.field_eval(grid, r, params, FP64, out=out64, workspace=ws)
     torch.cuda.synchronize()
@@ -169,9 +169,8 @@ def main():
     k64 = _kernel_ms(api, ws)
     log("fp64: %.2f ms/step" % (t64 * 1e3))
 
-    # FP64 with exponents 1 and 2 as exact products: the same precision as the
-    # plain FP64 kernel, the algorithm of the FP32 path, so the two ratios
-    # below separate the algorithm's share of the speedup from precision's
+    # the same arithmetic under its other name (exponents 1 and 2 as exact
+    # products, as the FP32 path's band takes them)
     out64x = torch.empty(w.voxels, dtype=torch.float64, device="cuda")
     log("fp64 exact: warmup")
     api.field_eval(grid, r, params, FP64_EXACT, out=out64x, workspace=ws)
@@ -577,7 +576,7 @@ def c3_tiles(args, log):
                             "peak": 8000.0, "unit": "GB/s", "frac": round(mc_bytes / t_mc / 8e12, 4),
                             "note": "the fields read once (8 B per point) and the meshes written once (24 B per "
                                     "vertex, 12 B per triangle) over the call's time; the kernels are "
-                                    "latency-bound (profiles/marching_cubes_c3_tile.md)"},
+                                    "bound as profiles/case_kernels.md says"},
             "mc_note": "one qj_mc_run_tiles_into call over the 64 clamped tiles, the meshes written straight into "
                        "output tensors sized by an untimed call over the same tiles",
             "parity": parity}
