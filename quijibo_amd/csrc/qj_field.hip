@@ -10,7 +10,9 @@
 // sequences, or FP32 FMA plus native transcendentals).
 //
 // Kernels:
-//   k_grid64        FP64, reference expression order (the "plain FP64" method).
+//   k_grid64        FP64 for every voxel: exponents 1 and 2 as products, others
+//                   from the short functions of qj_math64.h, the last iteration
+//                   from norms (qj_eval.h); the Lagrange order in polar form.
 //   k_grid32        FP32 bulk with exact power-of-two range scaling (device
 //                   code in qj_fp32.h); marks the band |F| < band, non-finite
 //                   results and near-threshold escape / black-hole decisions
@@ -23,7 +25,7 @@
 //   k_batch32, k_batch64_list, k_batch64
 //                   the request loop's work-queue kernels over chunks of
 //                   many requests (FP32 bulk per exponent variant, FP64 band
-//                   lists, plain FP64).
+//                   lists, FP64 for every voxel).
 #include <float.h>
 
 #include "qj_geom.h"
@@ -108,7 +110,7 @@ __device__ __forceinline__ Res64 eval64x(const MapArgs& a, const RootRec64* __re
 // kPow: kExactOnly / kExactInt for QJ_FP64 and QJ_FP64_EXACT, kPolar for the
 // Lagrange order (QJ_MAP_LAGRANGE). kExt: the extended-range evaluator
 // (QJ_MAP_EXTENDED_RANGE). FP64 VALU bound: 32+32 roots with exponents 1 and 2,
-// 256^3, 4 iterations 43.7 to 3.4 ms, 64^3 with 8 roots 78 to 14 us against the
+// 256^3, 4 iterations 43.7 to 3.3 ms, 64^3 with 8 roots 78 to 12.6 us against the
 // device library's polar form for every power; with real exponents, 50^3 and one
 // iteration, 267 to 36 us. The extended range's band list of a 256^3 torus tile
 // (128+128 roots) 1.69 to 0.64 ms, the request loop's 1.40 to 0.80 ms a launch.

@@ -9,16 +9,17 @@
 // 64-bit words, and only vertices and triangles themselves take a lane each:
 //   k_mc_signs      one bit per point: the float sign test
 //   k_mc_edges      the +x, +y, +z edges that carry a vertex, and the vertices
-//                   before every 8 points within a group of 16384 points
-//   k_mc_scan       groups' vertex counts -> first vertex id per group (the
-//                   reference numbers vertices by std::map<pair<int,int>> order
-//                   = lower endpoint, then x<y<z)
+//                   before every 8 points within a group (16384 points);
+//                   its last block, or k_mc_scan: groups' vertex
+//                   counts -> first vertex id per group (the reference numbers
+//                   vertices by std::map<pair<int,int>> order = lower endpoint,
+//                   then x<y<z)
 //   k_mc_vertices   p0 + d0/(d0-d1) (p1-p0) at cell centres, no contraction,
 //                   and a bit per edge whose vertex lies near an end (an FP32
 //                   estimate)
 //   k_mc_cells      triangle counts, and the degenerate filter (edge < 1e-7
-//                   dropped) on the cells with two or more near vertices
-//   k_mc_scan       groups' triangle counts -> first triangle per group
+//                   dropped) on the cells whose near vertices lie on edges that
+//                   meet; its last block, or k_mc_scan: first triangle per group
 //   k_mc_tris       each kept triangle written once, in cell then table order
 #include <float.h>
 #include <math.h>
@@ -162,6 +163,7 @@ struct McState {
   // linear mesher over several fields: the vertices and triangles before each
   uint64_t* d_base = nullptr;
   int64_t cap_base = 0;
+  uint32_t* tickets = nullptr;  // blocks that have finished (see finish_scan)
 };
 
 // grid coordinates of a point index (the mesher runs on fields of < 2^32 points)
@@ -469,6 +471,91 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_signs(const double* __restrict_
   if (lane < kSignPoints && p0 + 64 * lane < N) sgn[p0 / 64 + lane] = mine;
 }
 
+// The groups' counts to exclusive offsets in place, by one block, and the running
+// total after this tile: base[2 tile + which] is what came before it; also in
+// h_base (pinned memory). kAtomic: the counts come from other blocks of the same
+// launch.
+template <int kThreads, bool kAtomic>
+__device__ __forceinline__ void scan_groups(uint32_t* __restrict__ groups, int64_t n, uint64_t* __restrict__ base,
+                                            uint64_t* __restrict__ h_base, int tile, int which) {
+  const auto count = [&](int64_t i) { return kAtomic ? atomicAdd(&groups[i], 0u) : groups[i]; };
+  const int64_t per = (n + kThreads - 1) / kThreads, b = (int64_t)threadIdx.x * per;
+  constexpr int kHeld = 4;  // counts in registers, so that up to 1024 groups are read once
+  uint32_t held[kHeld], v = 0;
+#pragma unroll
+  for (int k = 0; k < kHeld; k++) held[k] = k < per && b + k < n ? count(b + k) : 0u;
+#pragma unroll
+  for (int k = 0; k < kHeld; k++) v += held[k];
+  for (int64_t i = b + kHeld; i < b + per && i < n; i++) v += count(i);
+  uint32_t total;
+  uint32_t run = block_prefix<kThreads>(v, &total);
+  for (int64_t i = b; i < b + per && i < n; i++) {
+    uint32_t c = 0;
+    if (i - b < kHeld) {
+#pragma unroll
+      for (int k = 0; k < kHeld; k++) c = i - b == k ? held[k] : c;
+    } else {
+      c = count(i);
+    }
+    groups[i] = run;
+    run += c;
+  }
+  if (threadIdx.x == 0) {
+    if (tile == 0) base[which] = 0;
+    const uint64_t sum = (tile == 0 ? 0 : base[2 * tile + which]) + total;
+    base[2 * (tile + 1) + which] = sum;
+    if (h_base) h_base[2 * (tile + 1) + which] = sum;
+  }
+}
+
+__global__ __launch_bounds__(kScanBlock) void k_mc_scan(uint32_t* __restrict__ groups, int64_t n,
+                                                        uint64_t* __restrict__ base, uint64_t* __restrict__ h_base,
+                                                        int tile, int which) {
+  scan_groups<kScanBlock, false>(groups, n, base, h_base, tile, which);
+}
+
+// Where a kernel's last block to finish scans the counts, in place of a launch of
+// its own: counts, tickets and the scan's reads are read-modify-writes, which all
+// XCDs see in one order, and a ticket is drawn once the write before it has
+// returned. Beyond 64 blocks the tickets are drawn from kTickets lines first: on
+// one line they come back one in 7 ns (1024 blocks 9.8 us, 2 to 3 this way; the
+// launch 4.7 and the gap before it 2 to 5). Tickets are left at 0. Beyond
+// kFoldGroups a thread would read its counts one after another, twice, and the
+// launch is the better one (base null).
+constexpr int kTickets = 16, kTicketLine = 32, kFoldGroups = 4 * kMcBlock;
+struct ScanTail {
+  uint64_t *base, *h_base;
+  uint32_t* tickets;  // kTickets + 1 lines
+  int tile;
+};
+__device__ __forceinline__ bool draws_last(uint32_t* ticket, uint32_t after, uint32_t of) {
+  uint32_t one = 1;
+  asm volatile("" : "+v"(one) : "v"(after));  // not before `after` has come back
+  if (atomicAdd(ticket, one) != of - 1) return false;
+  atomicExch(ticket, 0u);
+  return true;
+}
+__device__ __forceinline__ void finish_scan(uint32_t* __restrict__ groups, uint32_t total, const ScanTail& t,
+                                            int which) {
+  __shared__ int s_last;
+  if (!t.base) {
+    if (threadIdx.x == 0) groups[blockIdx.x] = total;
+    return;
+  }
+  if (threadIdx.x == 0) {
+    const uint32_t blocks = gridDim.x, before = atomicExch(&groups[blockIdx.x], total);
+    if (blocks <= 64) {
+      s_last = draws_last(t.tickets, before, blocks);
+    } else {
+      const uint32_t sub = blockIdx.x % kTickets, of = (blocks - sub + kTickets - 1) / kTickets;
+      s_last = draws_last(t.tickets + (1 + sub) * kTicketLine, before, of) && draws_last(t.tickets, of, kTickets);
+    }
+  }
+  __syncthreads();
+  if (!s_last) return;
+  scan_groups<kMcBlock, true>(groups, gridDim.x, t.base, t.h_base, t.tile, which);
+}
+
 // every third bit of 24 from 8
 __device__ __forceinline__ uint32_t spread8(uint32_t x) {
   x = (x | x << 8) & 0x00f00fu;
@@ -482,10 +569,10 @@ __device__ __forceinline__ uint32_t spread8(uint32_t x) {
 // serves the triangle kernel's lookups: for points 64 w + 8 j.. the vertices
 // before them in the group and the 24 edge bits in id order (point, then axis),
 // so that a vertex's id is one masked bit count away. groups[]: vertices per
-// group. Latency-bound: 256^3, 1024 blocks, 10.7 us (from the case bytes of the
-// 12 cells around a point: 54 us).
+// group. Latency-bound: 256^3, 1024 blocks, 13 us with the scan (from the case
+// bytes of the 12 cells around a point: 54 us and 14 of scans).
 __global__ __launch_bounds__(kMcBlock) void k_mc_edges(McGrid a, uint2* __restrict__ ranks,
-                                                       uint32_t* __restrict__ groups) {
+                                                       uint32_t* __restrict__ groups, ScanTail tail) {
   const int64_t w = (int64_t)blockIdx.x * kMcGroupWords + threadIdx.x;
   const int64_t X = a.g.res[0];
   uint64_t e[3] = {0, 0, 0};
@@ -518,35 +605,15 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_edges(McGrid a, uint2* __restri
   }
   uint32_t total;
   uint32_t run = block_prefix<kMcBlock>((uint32_t)(__popcll(e[0]) + __popcll(e[1]) + __popcll(e[2])), &total);
-  if (threadIdx.x == 0) groups[blockIdx.x] = total;
-  if (w >= a.nw) return;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
+    if (w >= a.nw) break;
     const uint32_t bits = spread8((uint32_t)(e[0] >> (8 * j)) & 0xffu) | spread8((uint32_t)(e[1] >> (8 * j)) & 0xffu) << 1 |
                           spread8((uint32_t)(e[2] >> (8 * j)) & 0xffu) << 2;
     ranks[8 * w + j] = uint2{run, bits};
     run += (uint32_t)__popc(bits);
   }
-}
-
-// One block: the groups' counts to exclusive offsets in place, and the running
-// total after this tile: base[2 tile + which] is what came before it.
-__global__ __launch_bounds__(kScanBlock) void k_mc_scan(uint32_t* __restrict__ groups, int64_t n,
-                                                        uint64_t* __restrict__ base, int tile, int which) {
-  const int64_t per = (n + kScanBlock - 1) / kScanBlock, b = (int64_t)threadIdx.x * per;
-  uint32_t v = 0;
-  for (int64_t i = b; i < b + per && i < n; i++) v += groups[i];
-  uint32_t total;
-  uint32_t run = block_prefix<kScanBlock>(v, &total);
-  for (int64_t i = b; i < b + per && i < n; i++) {
-    const uint32_t c = groups[i];
-    groups[i] = run;
-    run += c;
-  }
-  if (threadIdx.x == 0) {
-    if (tile == 0) base[which] = 0;
-    base[2 * (tile + 1) + which] = (tile == 0 ? 0 : base[2 * tile + which]) + total;
-  }
+  finish_scan(groups, total, tail, 0);
 }
 
 // computeEdgeInterpolations (TRIANGLE_MESH.cpp:2373-2425). A wave lists the
@@ -753,13 +820,14 @@ __device__ __forceinline__ uint64_t word_cases(const McGrid& a, int64_t w, uint8
 // way (a border set by setBorders puts near vertices in every cell along it,
 // but on parallel edges), listed in LDS and measured one per thread.
 // flags: the case of every cell that has
-// triangles, else 0. Latency-bound: 256^3, 1024 blocks, 17.5 us, of which the
-// measurement's longest chain is 6 (20 with every near pair measured). tword: the triangles before word w in its group; groups:
+// triangles, else 0. Latency-bound: 256^3, 1024 blocks, 20.5 us with the
+// scan, of which the measurement's longest chain is 6 (20 with every near pair
+// measured). tword: the triangles before word w in its group; groups:
 // per group.
 __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict__ field, McGrid a,
                                                        uint8_t* __restrict__ flags, uint8_t* __restrict__ kmask,
                                                        uint32_t* __restrict__ tword,
-                                                       uint32_t* __restrict__ groups) {
+                                                       uint32_t* __restrict__ groups, ScanTail tail) {
   __shared__ uint16_t s_list[kMcWaves][64 * 64];
   __shared__ uint32_t s_drop[2 * kMcGroupWords], s_lost[kMcGroupWords], s_cells[kMcWaves];
   const int64_t w = (int64_t)blockIdx.x * kMcGroupWords + threadIdx.x;
@@ -818,11 +886,11 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict_
   count -= s_lost[threadIdx.x];
   uint32_t total;
   const uint32_t before = block_prefix<kMcBlock>(count, &total);
-  if (threadIdx.x == 0) groups[blockIdx.x] = total;
   if (w < a.nw) {
     a.drop[w] = (uint64_t)s_drop[2 * threadIdx.x + 1] << 32 | s_drop[2 * threadIdx.x];
     tword[w] = before;
   }
+  finish_scan(groups, total, tail, 1);
 }
 
 // addVertexPairTriangle (TRIANGLE_MESH.cpp:2490-2503) in cell order then table
@@ -1059,14 +1127,22 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
   const int64_t wmax = (nmax + 63) / 64 + pad_max;
   const int64_t gmax = (nmax + kMcGroupPoints - 1) / kMcGroupPoints;
   if ((st = grow(m.words, m.cap_words, kMcArrays * wmax, s)) || (st = grow(m.ranks, m.cap_ranks, 8 * wmax, s)) ||
-      (st = grow(m.flags, m.cap_flags, 64 * ((nmax + 63) / 64), s)) || (st = grow(m.kmask, m.cap_kmask, nmax, s)) || (st = grow(m.tword, m.cap_tword, wmax, s)) ||
+      (st = grow(m.flags, m.cap_flags, 64 * ((nmax + 63) / 64), s)) || (st = grow(m.kmask, m.cap_kmask, nmax, s)) ||
+      (st = grow(m.tword, m.cap_tword, wmax, s)) ||
       (st = grow(m.groups, m.cap_groups, 2 * gmax, s)) || (st = grow(m.d_base, m.cap_base, 2 * ((int64_t)n + 1), s)))
     return st;
+  if (!m.tickets) {
+    const size_t bytes = sizeof(uint32_t) * kTicketLine * (kTickets + 1);
+    QJ_HIP(hipMalloc(&m.tickets, bytes));
+    QJ_HIP(hipMemsetAsync(m.tickets, 0, bytes, s));
+  }
   // first sizes: a quarter of the points as vertices, half as triangles
   // (a 256^3 torus tile holds 0.42 and 0.73 of its points)
   if (!ext && m.cap_v == 0 && (st = grow(m.verts, m.cap_v, 3 * (total_pts / 4 + 1024), s))) return st;
   if (!ext && m.cap_t == 0 && (st = grow(m.tris, m.cap_t, 3 * (total_pts / 2 + 1024), s))) return st;
-  std::vector<uint64_t> base(2 * ((size_t)n + 1));
+  if ((st = ensure_pinned(ws, 2 * ((int64_t)n + 1), s))) return st;
+  uint64_t* const base = (uint64_t*)ws->h_pinned;
+  base[0] = base[1] = 0;
   std::vector<int64_t> counts(2 * (size_t)n);
   uint64_t totals[2] = {0, 0};
   for (int pass = 0; pass < 2; pass++) {
@@ -1080,15 +1156,21 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
       const McGrid mg = make_mc_grid(m, g, wmax, iso, prefilter[(size_t)k]);
       const int64_t ng = cells > 0 ? (N + kMcGroupPoints - 1) / kMcGroupPoints : 0;
       uint32_t *gv = m.groups, *gt = m.groups + gmax;
+      const ScanTail tail{ng <= kFoldGroups ? m.d_base : nullptr, base, m.tickets, k};
+      const auto scan = [&](uint32_t* groups, int which) -> qj_status {
+        if (ng > 0 && ng <= kFoldGroups) return QJ_OK;  // the kernel before it did
+        hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, groups, ng, m.d_base, base, k, which);
+        QJ_HIP(hipGetLastError());
+        return QJ_OK;
+      };
       if (ng) {
         hipLaunchKernelGGL(k_mc_signs, blocks_of(N, kSignPoints * kMcBlock), dim3(kMcBlock), 0, s, fields[k], N, iso,
                            mg.sgn);
         QJ_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_mc_edges, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.ranks, gv);
+        hipLaunchKernelGGL(k_mc_edges, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.ranks, gv, tail);
         QJ_HIP(hipGetLastError());
       }
-      hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gv, ng, m.d_base, k, 0);
-      QJ_HIP(hipGetLastError());
+      if ((st = scan(gv, 0))) return st;
       if (ng) {
         const bool few = mg.nw < 2 * kTriWaves * 8;
         hipLaunchKernelGGL(few ? k_mc_vertices<2> : k_mc_vertices<8>, blocks_of(mg.nw, (few ? 2 : 8) * kMcWaves),
@@ -1097,16 +1179,12 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
                            verts);
         QJ_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_mc_cells, dim3((unsigned)ng), dim3(kMcBlock), 0, s, fields[k], mg, m.flags, m.kmask,
-                           m.tword, gt);
+                           m.tword, gt, tail);
         QJ_HIP(hipGetLastError());
       }
-      hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gt, ng, m.d_base, k, 1);
-      QJ_HIP(hipGetLastError());
-      if (ng) {
-        if ((st = launch_tris(m, mg, gv, gt, (const uint64_t*)(m.d_base + 2 * k), 0, tcap, tris, s))) return st;
-      }
+      if ((st = scan(gt, 1))) return st;
+      if (ng && (st = launch_tris(m, mg, gv, gt, (const uint64_t*)(m.d_base + 2 * k), 0, tcap, tris, s))) return st;
     }
-    QJ_HIP(hipMemcpyAsync(base.data(), m.d_base, sizeof(uint64_t) * base.size(), hipMemcpyDeviceToHost, s));
     QJ_HIP(hipStreamSynchronize(s));
     for (int k = 0; k < n; k++)
       for (int i = 0; i < 2; i++)
@@ -1197,6 +1275,7 @@ void mc_free(qj_workspace* ws) {
   hipFree(m->c_edges);
   hipFree(m->c_cells);
   hipFree(m->d_base);
+  hipFree(m->tickets);
   delete m;
   ws->mc = nullptr;
 }
@@ -1665,7 +1744,7 @@ qj_status nlmc_run(qj_workspace* ws, const MapArgs& a0, const qj_rational* f, do
     hipLaunchKernelGGL(k_mc_signs, blocks_of(mg.N, kSignPoints * kMcBlock), dim3(kMcBlock), 0, s, slab, mg.N, 0.0,
                        mg.sgn);
     QJ_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_mc_edges, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.ranks, gv);
+    hipLaunchKernelGGL(k_mc_edges, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.ranks, gv, ScanTail{});
     QJ_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_nl_count<false>, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.flags,
                        (const uint32_t*)nullptr, m.tword, m.aword, gt, ng);
@@ -1713,7 +1792,7 @@ qj_status nlmc_run(qj_workspace* ws, const MapArgs& a0, const qj_rational* f, do
         hipLaunchKernelGGL(k_nl_count<true>, dim3((unsigned)ng), dim3(kMcBlock), 0, s, mg, m.flags,
                            (const uint32_t*)m.lost, m.tword, m.aword, gt, ng);
         QJ_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gt, ng, m.d_base, 0, 1);
+        hipLaunchKernelGGL(k_mc_scan, dim3(1), dim3(kScanBlock), 0, s, gt, ng, m.d_base, (uint64_t*)nullptr, 0, 1);
         QJ_HIP(hipGetLastError());
         QJ_HIP(hipMemcpyAsync(&kept, m.d_base + 3, sizeof(kept), hipMemcpyDeviceToHost, s));
         QJ_HIP(hipStreamSynchronize(s));

@@ -47,3 +47,16 @@ def test_words_match_the_oracle(gpu, res, kind):
         assert v.shape == ov.shape and t.shape == ot.shape
         assert np.array_equal(t, ot)
         assert ((v == ov) | (np.isnan(v) & np.isnan(ov))).all()
+
+
+@pytest.mark.parametrize("res", [(64, 64, 257), (128, 128, 1025)])
+def test_group_scans(gpu, res):
+    """65 groups (the tickets' second level) and 1025 (the scan of its own launch),
+    twice in one workspace: the tickets are left as they were found."""
+    n = res[0] * res[1] * res[2]
+    f = field_of("sparse", n, np.random.default_rng(n))
+    ov, ot = O.marching_cubes(O.make_grid(res, (0, 0, 0), (3, 3, 3), (1, 0, 0, 0)), f)
+    ws, d = api.Workspace(), torch.from_numpy(f).cuda()
+    for _ in range(2):
+        v, t = api.marching_cubes(d, api.make_grid(res, (0, 0, 0), (3, 3, 3)), workspace=ws)
+        assert np.array_equal(t, ot) and np.array_equal(v, ov)
