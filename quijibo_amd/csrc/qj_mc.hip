@@ -282,7 +282,7 @@ constexpr int kMcWaves = kMcBlock / 64;        // waves per workgroup
 constexpr int kMcGroupWords = kMcBlock;        // words per group: the unit of the two scans, one word per thread
 constexpr int kMcGroupPoints = 64 * kMcGroupWords;
 constexpr int kSignPoints = 8;                 // points per thread of k_mc_signs
-constexpr int kTriBlocks = 4;                  // blocks of 256 cells per wave of k_mc_tris, at most
+constexpr int kTriBlocks = 2;                  // blocks of 256 cells per wave of k_mc_tris, at most
 constexpr int kTriWaves = 256 * 16;            // waves that fill the chip before one takes a second block
 constexpr int kListWords = 4;                  // words per wave of k_nl_vlist
 constexpr int kScanBlock = 1024;
@@ -895,17 +895,18 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict_
 
 // addVertexPairTriangle (TRIANGLE_MESH.cpp:2490-2503) in cell order then table
 // order. A wave takes blocks of 256 cells, four consecutive ones per lane: it
-// lists a block's kept triangles (case row and triangle << 8 | cell) in LDS and
+// lists a block's kept triangles (5 case + triangle of the row; cell) in LDS and
 // writes them one per lane, so that consecutive lanes write consecutive
 // triangles. The owner of an edge of cell p is p + dx + dy X + dz XY: four rows
 // of points, whose ranks are staged in LDS with the groups' offsets added, so
 // that a corner's vertex id is one LDS read and a masked bit count; ids count
 // from id0, triangles from base[1] (null: 0). Triangles at or beyond tcap are not
-// written. Bound by vector instructions and LDS latency: a
-// 256^3 torus tile (9.1 million triangles, 109 MB) 62 us, 76 with a 16-bit rank
-// per point and case and kept bytes of every cell. `blocks` per wave: the
-// tables' staging is shared by up to kTriBlocks of them once the chip is full
-// (97 x 101 x 89, one block per wave: 6.5 us, four: 20.7).
+// written. Bound by LDS latency at 7 waves per SIMD: a 256^3 torus tile (9.1
+// million triangles, 109 MB) 54 us; 64 with 32-bit list entries (5 waves), 76 with a
+// 16-bit rank per point and case and kept bytes of every cell. `blocks` per wave:
+// the tables' staging is shared by up to kTriBlocks of them once the chip is full
+// (one, two, four: 70, 62, 64 us with 32-bit entries, two and four 54 and 57 now;
+// 97 x 101 x 89 with one 6.5, with four 20.7).
 constexpr int kRankRow = 34;  // 8-point ranks per row: 257 points from any phase
 __global__ __launch_bounds__(kMcBlock) void k_mc_tris(McGrid a, int blocks, const uint8_t* __restrict__ flags,
                                                       const uint64_t* __restrict__ drop,
@@ -919,7 +920,8 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_tris(McGrid a, int blocks, cons
   __shared__ uint32_t s_te32[256 * 5 / 2];
   __shared__ uint8_t s_n[256];
   __shared__ uint32_t s_edge[12];
-  __shared__ uint32_t s_list[kMcWaves][5 * 256];
+  __shared__ uint16_t s_row[kMcWaves][5 * 256];
+  __shared__ uint8_t s_cell[kMcWaves][5 * 256];
   __shared__ uint2 s_rank[kMcWaves][4 * kRankRow];
   const unsigned short* s_te = (const unsigned short*)s_te32;
   const int64_t X = a.g.res[0], XY = a.XY;
@@ -934,7 +936,8 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_tris(McGrid a, int blocks, cons
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t* const list = s_list[wave];
+  uint16_t* const list = s_row[wave];
+  uint8_t* const cell = s_cell[wave];
   uint2* const rank = s_rank[wave];
   const int64_t last_group = (a.nw - 1) / kMcGroupWords;
   const int64_t B0 = wave_index() * blocks;
@@ -976,14 +979,20 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_tris(McGrid a, int blocks, cons
     uint32_t at = incl - mine;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const uint32_t e0 = (((f4 >> (8 * i)) & 0xffu) * 5u) << 8 | (uint32_t)(4 * lane + i);
+      const uint32_t e0 = ((f4 >> (8 * i)) & 0xffu) * 5u, c = (uint32_t)(4 * lane + i);
       if (some_lost) {
         uint32_t k = at;
-        for (unsigned m = keep >> (5 * i) & 31u; m; m &= m - 1) list[k++] = e0 + ((uint32_t)(__ffs(m) - 1) << 8);
+        for (unsigned m = keep >> (5 * i) & 31u; m; m &= m - 1) {
+          cell[k] = (uint8_t)c;
+          list[k++] = (uint16_t)(e0 + (uint32_t)(__ffs(m) - 1));
+        }
       } else {
 #pragma unroll
         for (uint32_t t = 0; t < 5; t++)
-          if (t < n[i]) list[at + t] = e0 + (t << 8);
+          if (t < n[i]) {
+            list[at + t] = (uint16_t)(e0 + t);
+            cell[at + t] = (uint8_t)c;
+          }
       }
       at += n[i];
     }
@@ -994,8 +1003,7 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_tris(McGrid a, int blocks, cons
     wave_sync();
     const int64_t o = (int64_t)((base ? base[1] : 0) + tgroups[w0 / kMcGroupWords] + tword[w0]);
     for (uint32_t j = lane; j < total; j += 64) {
-      const uint32_t e = list[j];
-      const uint32_t te = s_te[e >> 8], c = e & 255u;
+      const uint32_t te = s_te[list[j]], c = cell[j];
       int32_t id[3];
 #pragma unroll
       for (int k = 0; k < 3; k++) {
