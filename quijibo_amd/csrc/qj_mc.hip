@@ -743,35 +743,30 @@ __device__ __forceinline__ unsigned mc_measure_cell(const double* __restrict__ f
       measure |= !(pairs & brief) && (pairs & unsure) ? 1u << t : 0u;
     }
   }
+  const unsigned near = measure ? mc_near_edges(v, a.g, a.prefilter) : 0u;
   while (measure) {
     const int t = __ffs(measure) - 1;
     measure &= measure - 1;
-    const unsigned nm = mc_near_edges(v, a.g, a.prefilter) & kMc.tmask[flag][t];
+    const unsigned nm = near & kMc.tmask[flag][t];
     const int m = __popc(nm);
     if (m < 2) continue;
-    // the near vertices in turn against the one before and the first (one
-    // inlined vertex: instruction fetches weigh on a kernel this short)
-    const double eps = 1e-7;
-    double first[3] = {}, before[3] = {};
-    bool degenerate = false;
+    double w[3][3] = {};
     unsigned r = nm;
-#pragma clang loop unroll(disable)
-    for (int j = 0; j < m; j++) {
-      const int e = __ffs(r) - 1;
-      r &= r - 1;
-      int dx, dy, dz, axis;
-      edge_geom(e, dx, dy, dz, axis);
-      const int64_t q0 = p + dx + dy * X + dz * XY;
-      const int64_t q1 = q0 + (axis == 0 ? 1 : (axis == 1 ? X : XY));
-      double v1[3];
-      mc_vertex(a.g, (int)x + dx, (int)y + dy, (int)z + dz, axis, field[q0], field[q1], a.iso, v1);
-      if (j > 0) degenerate |= edge_len(before, v1) < eps;
-      if (j == 2) degenerate |= edge_len(first, v1) < eps;
-      for (int i = 0; i < 3; i++) {
-        first[i] = j == 0 ? v1[i] : first[i];
-        before[i] = v1[i];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      if (j < m) {  // constant indices into w keep it in registers
+        const int e = __ffs(r) - 1;
+        r &= r - 1;
+        int dx, dy, dz, axis;
+        edge_geom(e, dx, dy, dz, axis);
+        const int64_t q0 = p + dx + dy * X + dz * XY;
+        const int64_t q1 = q0 + (axis == 0 ? 1 : (axis == 1 ? X : XY));
+        mc_vertex(a.g, (int)x + dx, (int)y + dy, (int)z + dz, axis, field[q0], field[q1], a.iso, w[j]);
       }
     }
+    const double eps = 1e-7;
+    bool degenerate = edge_len(w[0], w[1]) < eps;
+    if (m == 3) degenerate = degenerate || edge_len(w[0], w[2]) < eps || edge_len(w[1], w[2]) < eps;
     if (degenerate) dropped |= 1u << t;
   }
   return dropped;
