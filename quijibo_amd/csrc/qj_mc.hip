@@ -1289,7 +1289,8 @@ void mc_free(qj_workspace* ws) {
 // TRIANGLE_MESH::computeNonlinearMarchingCubesLowMemoryHuge (TRIANGLE_MESH.cpp:681-768)
 // streamed over z-chunks: for chunk [z0, z1) the map is evaluated on slices
 // [z0, z1 + 1] (two above for the edges of the points at z1, whose ids belong to
-// the next chunk; none below: an edge's ends say whether it carries a vertex),
+// the next chunk, which takes over their values; none below: an edge's ends say
+// whether it carries a vertex),
 // cases come from the raw slab values log|q| (TRIANGLE_MESH.cpp:379) as sign
 // words, as in the linear mesher, and every vertex is
 // placed by bisection on re-evaluated values log|q| - iso (nonlinearValue
@@ -1704,13 +1705,22 @@ qj_status nlmc_run(qj_workspace* ws, const MapArgs& a0, const qj_rational* f, do
   auto slab_slices = [&](int64_t zc) { return std::min(zc + chunk + 2, Z) - zc; };
   // 1. slab of log|q| (or the caller's field, TRIANGLE_MESH.cpp:152-215): the
   // chunk at slice zc into slab[b] on stream s2 (the Lagrange order has no FP32
-  // path: its slabs are FP64)
+  // path: its slabs are FP64). Its first two slices are the other slab's last two,
+  // evaluated on the same stream: they are copied (256^3 in chunks of 16 slices 4
+  // to 6 % faster, of 64 1 to 2).
   auto eval_slab = [&](int64_t zc, int b) -> qj_status {
-    MapArgs sa = a;
-    sa.res[2] = (int32_t)slab_slices(zc);
-    sa.zoff = (int32_t)zc;
-    qj_status e = launch_field(ws, sa, f, (a.flags & QJ_MAP_LAGRANGE) ? QJ_FP64 : prec, band, m.slab[b], m.s2);
-    if (e) return e;
+    const int64_t slices = slab_slices(zc), have = zc > 0 ? std::min<int64_t>(2, slices) : 0;
+    if (have)
+      QJ_HIP(hipMemcpyAsync(m.slab[b], m.slab[1 - b] + chunk * XY, sizeof(double) * (size_t)(have * XY),
+                            hipMemcpyDeviceToDevice, m.s2));
+    if (slices > have) {
+      MapArgs sa = a;
+      sa.res[2] = (int32_t)(slices - have);
+      sa.zoff = (int32_t)(zc + have);
+      qj_status e = launch_field(ws, sa, f, (a.flags & QJ_MAP_LAGRANGE) ? QJ_FP64 : prec, band, m.slab[b] + have * XY,
+                                 m.s2);
+      if (e) return e;
+    }
     QJ_HIP(hipEventRecord(m.ev_field[b], m.s2));
     return QJ_OK;
   };
