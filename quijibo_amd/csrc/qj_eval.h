@@ -23,8 +23,8 @@ __device__ __forceinline__ bool has_nan(const q64& q) { return isnan(q.w) || isn
 
 // How term64 takes (q - r)^e:
 //   kPolar      QUATERNION::pow's polar form as written, with the device library's
-//               functions, for every exponent (QUATERNION.cpp:375-393): the sampled
-//               cross-check and the Lagrange order
+//               functions, for every exponent (QUATERNION.cpp:375-393): the Lagrange
+//               order
 //   kExactInt   exponents exactly 1 and 2 as b and b*b, others by polar64
 //   kExactOnly  every exponent is 1 or 2 (the caller checked), no polar code
 // All agree to a few ulps per term and keep the polar form's special cases:
@@ -409,6 +409,25 @@ __device__ __forceinline__ q64 lagrange64(RP roots, int nt, int nb, const q64& q
   return r;
 }
 
+// One voxel of the map in Lagrange order (QJ_MAP_LAGRANGE), polar powers. The
+// API takes it with neither the AP flags nor the extended range; the mesher
+// evaluates it itself.
+template <class RP = const RootRec64*>
+__device__ __forceinline__ Res64 eval64_lagrange(const MapArgs& a, RP roots, q64 q) {
+  Res64 r{0.0, 0, true, false};
+  double magnitude = qmag(q);
+  int it = 0;
+  while (magnitude < a.escape && it < a.max_iter) {
+    q = qscale(lagrange64<kPolar>(roots, a.nt, a.nb, q), a.exp_scaling);
+    magnitude = qmag(q);
+    it++;
+    r.iters++;
+    if ((a.flags & QJ_MAP_BLACK_HOLE) && magnitude < kBlackHole) it = a.max_iter;
+  }
+  r.F = log(magnitude);
+  return r;
+}
+
 // One voxel of computeLogScaledPowerRationalMap (OPTIMIZE_3D.cpp:1317-1362) /
 // computeRationalMapAP's first pass (:1423-1475). Overflow detection replaces
 // fetestexcept(FE_OVERFLOW): any non-finite T, B, |B|^2, quotient or |q|.
@@ -430,17 +449,6 @@ __device__ __forceinline__ Res64 eval64(const MapArgs& a, RP roots, q64 q) {
         r.iters++;
         return r;
       }
-    }
-    // Lagrange order reaches eval64 only through QJ_FP64 (the API rejects it for
-    // the FP32 band, and the mesher evaluates it itself), as kPolar: the other
-    // instances carry no Lagrange code
-    if (kPow == kPolar && (a.flags & QJ_MAP_LAGRANGE)) {
-      q = qscale(lagrange64<kPow>(roots, a.nt, a.nb, q), a.exp_scaling);
-      magnitude = qmag(q);
-      it++;
-      r.iters++;
-      if ((a.flags & QJ_MAP_BLACK_HOLE) && magnitude < kBlackHole) it = a.max_iter;
-      continue;
     }
     q64 T, B;
     bool nan_top = false;
@@ -743,12 +751,10 @@ __device__ __forceinline__ Res64 eval64e(const MapArgs& a, RP roots, q64 q) {
 }
 
 // eval64 or, with QJ_MAP_EXTENDED_RANGE, eval64e (a uniform branch where a
-// wave's voxels share their map arguments). kPolar is the Lagrange order's,
-// which has no extended range.
-template <int kPow = kPolar, class RP = const RootRec64*>
+// wave's voxels share their map arguments).
+template <int kPow, class RP = const RootRec64*>
 __device__ __forceinline__ Res64 eval64_any(const MapArgs& a, RP roots, const q64& q) {
-  if constexpr (kPow != kPolar)
-    if (a.flags & QJ_MAP_EXTENDED_RANGE) return eval64e<kPow>(a, roots, q);
+  if (a.flags & QJ_MAP_EXTENDED_RANGE) return eval64e<kPow>(a, roots, q);
   return eval64<kPow>(a, roots, q);
 }
 

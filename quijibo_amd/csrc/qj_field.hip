@@ -107,14 +107,24 @@ __device__ __forceinline__ Res64 eval64x(const MapArgs& a, const RootRec64* __re
 // ---------------------------------------------------------------- kernels
 
 
-// kPow: kExactOnly / kExactInt for QJ_FP64 and QJ_FP64_EXACT, kPolar for the
-// Lagrange order (QJ_MAP_LAGRANGE). kExt: the extended-range evaluator
-// (QJ_MAP_EXTENDED_RANGE). FP64 VALU bound: 32+32 roots with exponents 1 and 2,
+// The FP64 evaluators: eval64, the extended range (QJ_MAP_EXTENDED_RANGE), the
+// Lagrange order (QJ_MAP_LAGRANGE; polar powers whatever kPow), the AP re-pass of
+// overflowed cells (polar powers).
+enum EvalKind { kPlainRange = 0, kExtRange = 1, kLagrange = 2, kRepass = 3 };
+template <int kEval, int kPow>
+__device__ __forceinline__ Res64 eval_kind(const MapArgs& a, const RootRec64* __restrict__ roots, const q64& q) {
+  if constexpr (kEval == kRepass) return eval64x(a, roots, q);
+  else if constexpr (kEval == kExtRange) return eval64e<kPow>(a, (ConstRoots)roots, q);
+  else if constexpr (kEval == kLagrange) return eval64_lagrange(a, (ConstRoots)roots, q);
+  else return eval64<kPow>(a, (ConstRoots)roots, q);
+}
+
+// kPow: kExactOnly or kExactInt. FP64 VALU bound: 32+32 roots with exponents 1 and 2,
 // 256^3, 4 iterations 43.7 to 3.3 ms, 64^3 with 8 roots 78 to 12.6 us against the
 // device library's polar form for every power; with real exponents, 50^3 and one
 // iteration, 267 to 36 us. The extended range's band list of a 256^3 torus tile
 // (128+128 roots) 1.69 to 0.64 ms, the request loop's 1.40 to 0.80 ms a launch.
-template <int kPow, bool kExt = false>
+template <int kEval, int kPow>
 __global__ __launch_bounds__(kBlock) void k_grid64(MapArgs a, const RootRec64* __restrict__ roots,
                                                    double* __restrict__ out, unsigned long long* __restrict__ cnt,
                                                    uint32_t* __restrict__ alist, uint32_t* __restrict__ acount,
@@ -127,10 +137,7 @@ __global__ __launch_bounds__(kBlock) void k_grid64(MapArgs a, const RootRec64* _
   if (valid) {
     double c[3];
     cell_center(a, x, y, z + a.zoff, c);
-    const q64 q0{c[0], c[1], c[2], a.slice};
-    Res64 r;
-    if constexpr (kExt) r = eval64e<kPow>(a, (ConstRoots)roots, q0);
-    else r = eval64<kPow>(a, (ConstRoots)roots, q0);
+    const Res64 r = eval_kind<kEval, kPow>(a, roots, q64{c[0], c[1], c[2], a.slice});
     if (r.written) {
       out[idx] = r.F;
       nonfinite = !isfinite(r.F);
@@ -187,7 +194,6 @@ __global__ __launch_bounds__(kBlock) void k_points32(MapArgs a, Consts32 k, cons
 // FP64 over a compacted list (count read on the device, at most cap entries
 // held), or over all n indices when list == nullptr. kPow: the PowMode
 // (kExactInt / kExactOnly for the FP32 path's band and range re-evaluation).
-enum EvalKind { kPlainRange = 0, kExtRange = 1, kRepass = 2 };
 template <class Src, int kEval, int kPow = kPolar>
 __global__ __launch_bounds__(kBlock) void k_list64(MapArgs a, const RootRec64* __restrict__ roots,
                                                    const double* __restrict__ pts,
@@ -205,11 +211,7 @@ __global__ __launch_bounds__(kBlock) void k_list64(MapArgs a, const RootRec64* _
     uint32_t idx = 0;
     if (i < n) {
       idx = list ? list[i] : (uint32_t)i;
-      const q64 q0 = Src::start(a, pts, idx);
-      Res64 r;
-      if constexpr (kEval == kRepass) r = eval64x(a, roots, q0);
-      else if constexpr (kEval == kExtRange) r = eval64e<kPow>(a, (ConstRoots)roots, q0);
-      else r = eval64<kPow>(a, (ConstRoots)roots, q0);
+      const Res64 r = eval_kind<kEval, kPow>(a, roots, Src::start(a, pts, idx));
       if (r.written) out[idx] = r.F;
       else if (pts) out[idx] = __builtin_nan("");
       vox++;
@@ -240,10 +242,7 @@ __global__ __launch_bounds__(kBlock) void k_band_sweep(MapArgs a, const RootRec6
     const int64_t i = base + threadIdx.x;
     bool ovf = false;
     if (i < n_all && ((const unsigned long long*)out)[i] == kBandMark) {
-      const q64 q0 = Src::start(a, pts, (uint32_t)i);
-      Res64 r;
-      if constexpr (kEval == kExtRange) r = eval64e<kPow>(a, (ConstRoots)roots, q0);
-      else r = eval64<kPow>(a, (ConstRoots)roots, q0);
+      const Res64 r = eval_kind<kEval, kPow>(a, roots, Src::start(a, pts, (uint32_t)i));
       if (r.written) out[i] = r.F;
       else if (pts) out[i] = __builtin_nan("");
       vox++;
@@ -287,7 +286,7 @@ __device__ __forceinline__ void block_max(double v, unsigned long long* cnt, int
 // (to max(1, |F64|)) differences over cells finite in both.
 // kSpread: copies per counter slot (a workspace's counters), or 1 for the
 // request loop's per-result block of CNT_N counters.
-template <int kPow, int kSpread = kCounterSpread>
+template <int kEval, int kPow, int kSpread = kCounterSpread>
 __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* __restrict__ roots,
                                                     const double* __restrict__ field, int64_t nvox, int64_t samples,
                                                     unsigned long long* __restrict__ cnt) {
@@ -297,7 +296,7 @@ __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* 
   if (i < samples) {
     const int64_t idx = ((2 * i + 1) * nvox) / (2 * samples);
     const q64 q0 = GridSource::start(a, nullptr, idx);
-    Res64 r = eval64_any<kPow>(a, (ConstRoots)roots, q0);
+    Res64 r = eval_kind<kEval, kPow>(a, roots, q0);
     if ((a.flags & QJ_MAP_ADAPTIVE) && r.overflow) r = eval64x(a, roots, q0);
     if (r.written) {
       const double F = field[idx];
@@ -321,9 +320,10 @@ __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* 
 
 template <int kSpread>
 static auto check_kernel(const MapArgs& a) {
-  return (a.flags & QJ_MAP_LAGRANGE) ? k_check64<kPolar, kSpread>
-         : a.gen                     ? k_check64<kExactInt, kSpread>
-                                     : k_check64<kExactOnly, kSpread>;
+  const bool ext = (a.flags & QJ_MAP_EXTENDED_RANGE) != 0;
+  return (a.flags & QJ_MAP_LAGRANGE) ? k_check64<kLagrange, kPolar, kSpread>
+         : a.gen ? (ext ? k_check64<kExtRange, kExactInt, kSpread> : k_check64<kPlainRange, kExactInt, kSpread>)
+                 : (ext ? k_check64<kExtRange, kExactOnly, kSpread> : k_check64<kPlainRange, kExactOnly, kSpread>);
 }
 
 __global__ void k_zero_u64(unsigned long long* p, int n) {
@@ -549,7 +549,7 @@ __global__ __launch_bounds__(kBlock) void k_batch64(const ChunkDesc* __restrict_
     const ChunkDesc& d = descs[c];
     if (local < d.count) {
       const int64_t idx = d.start + local;
-      const Res64 r = (d.a.flags & QJ_MAP_LAGRANGE) ? eval64<kPolar>(d.a, (ConstRoots)d.r64, chunk_start(d.a, idx))
+      const Res64 r = (d.a.flags & QJ_MAP_LAGRANGE) ? eval64_lagrange(d.a, (ConstRoots)d.r64, chunk_start(d.a, idx))
                                                     : eval64_any<kExactInt>(d.a, (ConstRoots)d.r64, chunk_start(d.a, idx));
       if (r.written) d.out[idx] = r.F;
     }
@@ -695,7 +695,7 @@ static qj_status launch_sweep(const FieldBufs& fb, const MapArgs& a, const qj_ra
 // The FP64 list kernel of the map's power mode and range.
 template <class Src>
 static auto list_kernel(const MapArgs& a) {
-  if (a.flags & QJ_MAP_LAGRANGE) return k_list64<Src, kPlainRange, kPolar>;
+  if (a.flags & QJ_MAP_LAGRANGE) return k_list64<Src, kLagrange>;
   if (a.flags & QJ_MAP_EXTENDED_RANGE)
     return a.gen ? k_list64<Src, kExtRange, kExactInt> : k_list64<Src, kExtRange, kExactOnly>;
   return a.gen ? k_list64<Src, kPlainRange, kExactInt> : k_list64<Src, kPlainRange, kExactOnly>;
@@ -736,15 +736,10 @@ static qj_status launch_field_bufs(const FieldBufs& fb, const MapArgs& a, const 
   mark(fb, s);
   const bool ext = (a.flags & QJ_MAP_EXTENDED_RANGE) != 0;
   const dim3 g64((unsigned)nblocks), b64(kBlock);
-  if (a.flags & QJ_MAP_LAGRANGE) {
-    hipLaunchKernelGGL(k_grid64<kPolar>, g64, b64, 0, s, a, f->d64, d_out, fb.counters, fb.alist, fb.list_count + 1,
-                       (uint32_t)fb.alist_cap);
-    QJ_HIP(hipGetLastError());
-    mark(fb, s);
-    mark(fb, s);
-  } else if (prec == QJ_FP64 || prec == QJ_FP64_EXACT) {
-    const auto k = a.gen ? (ext ? k_grid64<kExactInt, true> : k_grid64<kExactInt>)
-                         : (ext ? k_grid64<kExactOnly, true> : k_grid64<kExactOnly>);
+  if (prec == QJ_FP64 || prec == QJ_FP64_EXACT) {
+    const auto k = (a.flags & QJ_MAP_LAGRANGE) ? k_grid64<kLagrange, kPolar>
+                   : a.gen ? (ext ? k_grid64<kExtRange, kExactInt> : k_grid64<kPlainRange, kExactInt>)
+                           : (ext ? k_grid64<kExtRange, kExactOnly> : k_grid64<kPlainRange, kExactOnly>);
     hipLaunchKernelGGL(k, g64, b64, 0, s, a, f->d64, d_out, fb.counters, fb.alist, fb.list_count + 1,
                        (uint32_t)fb.alist_cap);
     QJ_HIP(hipGetLastError());
