@@ -120,10 +120,10 @@ typedef struct qj_eval_stats {
   int64_t adaptive_voxels;   /* cells flagged as overflowed (QJ_MAP_ADAPTIVE) */
   int64_t nonfinite;         /* non-finite results written */
   /* the sampled FP64 cross-check (qj_workspace_check), summed over fields */
-  int64_t checked;           /* cells re-evaluated in FP64 */
+  int64_t checked;           /* cells re-evaluated with the reference method in FP64 */
   int64_t check_sign_flips;  /* of those, cells where (float)F > 0 differs from FP64's */
   int64_t check_class_mismatch; /* cells whose class (finite, NaN, +inf, -inf) differs */
-  double check_max_abs_dF;   /* largest |F - F_fp64| over checked cells finite in both */
+  double check_max_abs_dF;   /* largest |F - F_fp64| (or |F_fp64 - F_reference|) over checked cells finite in both */
   double check_max_rel_dF;   /* largest |F - F_fp64| / max(1, |F_fp64|) */
 } qj_eval_stats;
 
@@ -154,11 +154,15 @@ qj_status qj_workspace_reset_stats(qj_workspace* ws, void* stream);
 /* The error statement of every field (no counterpart in the reference, which
  * has one precision): with samples > 0, each qj_field_eval on ws re-evaluates
  * `samples` evenly spaced cells (cell (2i+1) N / (2 samples), i < samples)
- * in FP64 as QJ_FP64 does (the extended-range re-pass for cells
- * QJ_MAP_ADAPTIVE flags) after
- * the field is written, and adds the comparison to the workspace statistics
- * (qj_eval_stats.checked ...). One extra kernel per field, about the latency
- * of one FP64 evaluation per cell.
+ * with the reference method in FP64 (polar powers, reference expression
+ * order; the extended-range re-pass for cells QJ_MAP_ADAPTIVE flags) and as
+ * QJ_FP64 does, after the field is written, and adds the comparison to the
+ * workspace statistics (qj_eval_stats.checked ...): signs and classes against
+ * the reference method, which writes no field itself (QJ_MAP_LAGRANGE maps
+ * apart); as the difference the larger of the field's from QJ_FP64's value and
+ * of that from the reference method's, so that a QJ_FP64 field shows its own
+ * error. One extra kernel per field, about the latency of one FP64 evaluation
+ * per cell (0.5 ms for 32+32 roots, maxIter 4).
  * 0 (the default) turns it off; at most 2^24. */
 qj_status qj_workspace_check(qj_workspace* ws, int64_t samples);
 
@@ -424,7 +428,7 @@ typedef struct qj_server_config {
                                  footprint or more wait behind it) and takes up to a quarter of each
                                  launch (0 = 0.25) */
   int32_t check_samples;      /* per-result error statement: cells of every finished field re-evaluated with
-                                 FP64 and compared (qj_completion.checked ...; 0 = off) */
+                                 the reference method in FP64 and compared (qj_completion.checked ...; 0 = off) */
   double escalate_abs_dF;     /* FP32_BAND servers with check_samples: a result whose sample shows a sign flip,
                                  a class mismatch or max |F - F_fp64| above this is computed again with every
                                  voxel in FP64 (exact integer powers) before it completes; its completion says

@@ -24,7 +24,8 @@ __device__ __forceinline__ bool has_nan(const q64& q) { return isnan(q.w) || isn
 // How term64 takes (q - r)^e:
 //   kPolar      QUATERNION::pow's polar form as written, with the device library's
 //               functions, for every exponent (QUATERNION.cpp:375-393): the Lagrange
-//               order
+//               order, and the sampled cross-check, whose evaluator shares nothing
+//               with the other two modes but the roots
 //   kExactInt   exponents exactly 1 and 2 as b and b*b, others by polar64
 //   kExactOnly  every exponent is 1 or 2 (the caller checked), no polar code
 // All agree to a few ulps per term and keep the polar form's special cases:
@@ -512,8 +513,10 @@ __device__ __forceinline__ void xnorm(xq& v) {
   }
 }
 // QUATERNION::pow (QUATERNION.cpp:375-393) with exps = exp(e log|q| + lnoff)
-// kept as mantissa * 2^k (the AP map's re-pass).
-__device__ __forceinline__ xq xpow(const q64& q, double e) {
+// kept as mantissa * 2^k (the AP map's re-pass and the cross-check); lnoff
+// carries the scale of a normalised base (e k ln 2 for a base m 2^k: the angle
+// does not depend on the scale).
+__device__ __forceinline__ xq xpow(const q64& q, double e, double lnoff = 0.0) {
   const double partial = q.x * q.x + q.y * q.y + q.z * q.z;
   const double qMagnitude = sqrt(partial + q.w * q.w);
   const double vMagnitude = sqrt(partial);
@@ -521,7 +524,7 @@ __device__ __forceinline__ xq xpow(const q64& q, double e) {
   const double scale = e * acos(q.w / qMagnitude) * vMagnitudeInv;
   const double magnitude = scale * vMagnitude;
   const double magnitudeInv = (magnitude > 0.0) ? 1.0 / magnitude : 0.0;
-  const double lnE = e * log(qMagnitude);
+  const double lnE = e * log(qMagnitude) + lnoff;
   int k = 0;
   double em;
   if (isfinite(lnE)) {
@@ -555,6 +558,7 @@ template <int kPow>
 __device__ __forceinline__ xq term_ext(const RootRec64& r, const q64& q) {
   xq n{qsub64x(q, r), 0};
   xnorm(n);
+  if (kPow == kPolar) return xpow(n.m, r.e, r.e * (double)n.e * 0.6931471805599453);
   if (kPow != kExactOnly && !is_one(r.e) && !is_two(r.e)) {
     double ln, slope;
     xq v{polar_unit(n.m, r.e, ln, slope), 0};
@@ -688,11 +692,13 @@ __device__ __forceinline__ bool last64e(const MapArgs& a, RP roots, const q64& q
 // escape and black-hole tests compare the FP64 value of |q| (exact whenever
 // it is representable; +inf or 0 beyond, which decides them the same way);
 // F = log|mantissa| + exponent ln 2. An iterate that continues below FP64's
-// range (no black-hole stop) continues from its FP64 value.
+// range (no black-hole stop) continues from its FP64 value. kPolar: every term
+// and product one by one, for the cross-check.
 template <int kPow, class RP = const RootRec64*>
 __device__ __forceinline__ Res64 eval64e(const MapArgs& a, RP roots, q64 q) {
   Res64 r{0.0, 0, true, false};
-  double magnitude = qmag64x(q);
+  auto mag = [](const q64& v) { return kPow == kPolar ? qmag(v) : qmag64x(v); };
+  double magnitude = mag(q);
   if ((a.flags & QJ_MAP_SKIP_ORIGIN) && magnitude < 1e-8) {
     r.written = false;
     return r;
@@ -700,15 +706,15 @@ __device__ __forceinline__ Res64 eval64e(const MapArgs& a, RP roots, q64 q) {
   double logmag = log(magnitude);
   int it = 0;
   while (magnitude < a.escape && it < a.max_iter) {
-    if (it + 1 == a.max_iter) {
-      if (last64e<kPow>(a, roots, q, r.F)) {
+    if constexpr (kPow != kPolar) {
+      if (it + 1 == a.max_iter && last64e<kPow>(a, roots, q, r.F)) {
         r.iters++;
         return r;
       }
     }
     xq v, B;
     double ln = 0.0;
-    bool grouped = a.term_bits <= kExtMaxTermBits;
+    bool grouped = kPow != kPolar && a.term_bits <= kExtMaxTermBits;
     if (grouped) {
 #pragma unroll 1
       for (int p = 0; p < 2; p++) {  // one copy of the loop's code
@@ -732,13 +738,13 @@ __device__ __forceinline__ Res64 eval64e(const MapArgs& a, RP roots, q64 q) {
       }
     }
     if (a.nb > 0) {
-      v.m = qdiv64x(v.m, B.m);
+      v.m = kPow == kPolar ? qdiv(v.m, B.m) : qdiv64x(v.m, B.m);
       v.e -= B.e;
     }
     v.m = qscale(v.m, a.exp_scaling);
     if (kPow == kExactInt && ln != 0.0) scale_ext(v, ln);  // the general terms' magnitude
     xnorm(v);
-    const double mm = qmag64x(v.m);
+    const double mm = mag(v.m);
     logmag = __builtin_fma((double)v.e, 0.6931471805599453, log(mm));
     magnitude = ldexp(mm, v.e);
     q = q64{ldexp(v.m.w, v.e), ldexp(v.m.x, v.e), ldexp(v.m.y, v.e), ldexp(v.m.z, v.e)};

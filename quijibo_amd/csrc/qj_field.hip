@@ -278,15 +278,29 @@ __device__ __forceinline__ void block_max(double v, unsigned long long* cnt, int
   __syncthreads();
 }
 
-// The error statement of a finished field: at `samples` evenly spaced cells
-// the map is evaluated again as QJ_FP64 does (the extended-range re-pass where
-// QJ_MAP_ADAPTIVE flags an overflow) and compared with the value written: counts of checked cells,
-// sign disagreements of (float)F > 0 (the mesher's predicate) and class
+// One cell evaluated for the cross-check: the extended-range re-pass where
+// QJ_MAP_ADAPTIVE flags an overflow.
+template <int kEval, int kPow>
+__device__ __forceinline__ Res64 eval_checked(const MapArgs& a, const RootRec64* __restrict__ roots, const q64& q) {
+  Res64 r = eval_kind<kEval, kPow>(a, roots, q);
+  if ((a.flags & QJ_MAP_ADAPTIVE) && r.overflow) r = eval64x(a, roots, q);
+  return r;
+}
+
+// The error statement of a finished field: `samples` evenly spaced cells are
+// evaluated again in FP64 with the reference method (polar powers of the device
+// library, reference expression order, every iteration in full) and as QJ_FP64
+// does. The reference method decides sign and class; it writes no field but the
+// Lagrange order's, so it checks the short functions, the norms of the last
+// iteration and the grouped products too. The difference is the larger of the
+// field's from QJ_FP64's value and of that from the reference method's: the
+// first alone is 0 for every cell that QJ_FP64's code wrote, the second alone
+// has its own rounding in it. Counts of checked cells, sign disagreements of (float)F > 0 (the mesher's predicate) and class
 // disagreements (finite / NaN / +-inf), and the largest absolute and relative
 // (to max(1, |F64|)) differences over cells finite in both.
 // kSpread: copies per counter slot (a workspace's counters), or 1 for the
 // request loop's per-result block of CNT_N counters.
-template <int kEval, int kPow, int kSpread = kCounterSpread>
+template <int kEval, int kSpread = kCounterSpread>
 __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* __restrict__ roots,
                                                     const double* __restrict__ field, int64_t nvox, int64_t samples,
                                                     unsigned long long* __restrict__ cnt) {
@@ -296,8 +310,9 @@ __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* 
   if (i < samples) {
     const int64_t idx = ((2 * i + 1) * nvox) / (2 * samples);
     const q64 q0 = GridSource::start(a, nullptr, idx);
-    Res64 r = eval_kind<kEval, kPow>(a, roots, q0);
-    if ((a.flags & QJ_MAP_ADAPTIVE) && r.overflow) r = eval64x(a, roots, q0);
+    const Res64 r = eval_checked<kEval, kPolar>(a, roots, q0);
+    double F64 = r.F;
+    if constexpr (kEval != kLagrange) F64 = eval_checked<kEval, kExactInt>(a, roots, q0).F;
     if (r.written) {
       const double F = field[idx];
       checked = 1;
@@ -305,7 +320,7 @@ __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* 
       if (fin != fin64 || isnan(F) != isnan(r.F) || (!fin && !isnan(F) && F != r.F)) {
         cls = 1;
       } else if (fin) {
-        dabs = fabs(F - r.F);
+        dabs = isfinite(F64) ? fmax(fabs(F - F64), fabs(F64 - r.F)) : fabs(F - r.F);
         drel = dabs / fmax(1.0, fabs(r.F));
       }
       flips = (((float)F > 0.0f) != ((float)r.F > 0.0f)) ? 1 : 0;
@@ -320,10 +335,9 @@ __global__ __launch_bounds__(kBlock) void k_check64(MapArgs a, const RootRec64* 
 
 template <int kSpread>
 static auto check_kernel(const MapArgs& a) {
-  const bool ext = (a.flags & QJ_MAP_EXTENDED_RANGE) != 0;
-  return (a.flags & QJ_MAP_LAGRANGE) ? k_check64<kLagrange, kPolar, kSpread>
-         : a.gen ? (ext ? k_check64<kExtRange, kExactInt, kSpread> : k_check64<kPlainRange, kExactInt, kSpread>)
-                 : (ext ? k_check64<kExtRange, kExactOnly, kSpread> : k_check64<kPlainRange, kExactOnly, kSpread>);
+  return (a.flags & QJ_MAP_LAGRANGE)         ? k_check64<kLagrange, kSpread>
+         : (a.flags & QJ_MAP_EXTENDED_RANGE) ? k_check64<kExtRange, kSpread>
+                                             : k_check64<kPlainRange, kSpread>;
 }
 
 __global__ void k_zero_u64(unsigned long long* p, int n) {
