@@ -218,9 +218,9 @@ __device__ __forceinline__ double edge_len(const double* a, const double* b) {
 // max |vi - c| (the edges are perpendicular). So with h >= kPrefilterSpacing
 // a triangle with at most one vertex within 2e-7 of an end of its edge has
 // every side longer than 1e-7. k_mc_vertices marks a vertex "near" from an FP32
-// estimate t' of its place t on the edge: near unless t' h >= kNearLimit and
-// (1 - t') h >= kNearLimit. |t' - t| stays below 2.5e-7 (corner values
-// rounded to float, one division and one subtraction), so with
+// estimate t' of its place t on the edge: near unless t' h > kNearLimit and
+// (1 - t') h > kNearLimit. |t' - t| stays below 2.5e-7 (corner values
+// rounded to float, one subtraction and the products), so with
 // h <= kPrefilterMaxSpacing every vertex within 2e-7 of an end is marked
 // (2e-7 + 2.5e-7 h < 1e-6); NaN or infinite corners mark it too. Triangles
 // with two or three marked vertices are measured with the FP64 vertices.
@@ -238,12 +238,15 @@ constexpr double kSureSpacing = 1e-4;
 enum McPrefilter { kMeasureAll = 0, kMeasureNear = 1, kMeasureUnsure = 2 };
 
 // Whether the vertex of an edge with end values v0, v1 and grid spacing h may
-// lie within 2e-7 of an end: near unless |v0| h >= 1e-6 |v0 - v1| and
-// |v1| h >= 1e-6 |v0 - v1| (a vertex at place t has t = |v0| / |v0 - v1| and
+// lie within 2e-7 of an end: near unless |v0| h > 1e-6 |v0 - v1| and
+// |v1| h > 1e-6 |v0 - v1| (a vertex at place t has t = |v0| / |v0 - v1| and
 // 1 - t = |v1| / |v0 - v1|, so no division); NaN and infinite ends make it near.
+// Strictly greater: between subnormal ends the right side can round to 0, and
+// an end of 0 is near then too (products rounded to n and n + 1 units of the
+// smallest float differ by their true values' order, so none is passed over).
 __device__ __forceinline__ bool mc_near(float v0, float v1, float h) {
   const float lim = kNearLimit * fabsf(v0 - v1);
-  return !(fabsf(v0) * h >= lim && fabsf(v1) * h >= lim);
+  return !(fabsf(v0) * h > lim && fabsf(v1) * h > lim);
 }
 
 // The 12-bit mask of a cell's near edges from its float corner values (corner
