@@ -13,8 +13,9 @@
 // sine 1.2 ulp, cosine 1.2e-16, square root and its reciprocal 0.5 and 1.7 ulp,
 // exponential 1.0 ulp.
 //
-// Callers keep arguments in range themselves (see the range tests beside each
-// use); outside it the results are finite garbage or NaN, never a trap.
+// Callers keep arguments in range themselves (see the range stated at each
+// function and polar_unit's tests); outside it the results are garbage or NaN,
+// never a trap.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -167,15 +168,18 @@ __device__ __forceinline__ double tanh64(double x) {
   return x != x ? x : (x == 0.0 ? x : q);
 }
 
-// sin(x) and cos(x) for |x| <= 2^30: x - k pi / 2 with pi / 2 in two parts,
-// then the two polynomials, swapped and signed by k.
+// sin(x) and cos(x) for |x| <= 2^52: x - k pi / 2 with pi / 2 in two parts (the
+// first difference is exact), then the two polynomials, swapped and signed by
+// the low bits of k, which are the last ones of k + 1.5 2^52. (Its callers'
+// x = e angle is rounded to half a radian and more beyond that, at exponents above
+// 10^15; those are not tested for.)
 template <bool kInLoop = false>
 __device__ __forceinline__ void sincos64(double x, double& sn, double& cs) {
 #pragma clang fp contract(off)
   const double dk = __builtin_rint(x * k64<kInLoop>(0.63661977236758138));
   double r = __builtin_fma(-dk, k64<kInLoop>(1.5707963267948966), x);
   r = __builtin_fma(-dk, k64<kInLoop>(6.123233995736766e-17), r);
-  const int k = (int)dk;
+  const int k = (int)(uint32_t)__builtin_bit_cast(uint64_t, dk + k64<kInLoop>(0x1.8p52));
   const double z = r * r;
   double p = k64<kInLoop>(1.5918129294866608e-10);
   p = __builtin_fma(p, z, k64<kInLoop>(-2.5051131845003624e-08));
