@@ -116,14 +116,23 @@ __device__ __forceinline__ bool is_two(double e) { return __builtin_bit_cast(uns
 // The angle comes from |v| and w directly where the reference takes
 // acos(w / |b|), which loses half its digits next to the real axis.
 // slope: m / |v|, the factor that the reference multiplies |b^e| by first.
+// kPlain: outside the extended range a base whose square is 0 or infinite in
+// FP64 gives what the reference's |b| of 0 or infinity gives: NaN or, where w^2
+// alone is infinite, an angle of pi / 2 and a magnitude of infinity or 0.
+template <bool kPlain>
 __device__ __forceinline__ q64 polar_unit(q64 b, double e, double& ln, double& slope) {
 #pragma clang fp contract(off)
   double partial = partial64(b);
   double n2 = __builtin_fma(b.w, b.w, partial);
   double lnoff = 0.0, vs = 1.0;
   slope = 0.0;
-  if (!(partial >= 0x1p-900 && n2 <= 0x1p900)) {
-    if (n2 < 0x1p-900 || n2 > 0x1p900) {
+  if (__builtin_expect(!(partial >= 0x1p-900 && n2 <= 0x1p900), 0)) {
+    if (kPlain && (n2 == 0.0 || n2 == __builtin_inf())) {
+      const bool real = partial > 0.0 && partial < __builtin_inf() && e != 0.0;
+      b.w = 0.0;
+      lnoff = __builtin_copysign(800.0, e);
+      n2 = real ? 1.0 : __builtin_nan("");
+    } else if (n2 < 0x1p-900 || n2 > 0x1p900) {
       const double s = n2 < 1.0 ? 0x1p500 : 0x1p-500;
       b = q64{b.w * s, b.x * s, b.y * s, b.z * s};
       lnoff = e * (n2 < 1.0 ? -346.57359027997264 : 346.57359027997264);  // -+500 ln 2
@@ -165,7 +174,7 @@ __device__ __forceinline__ q64 polar_unit(q64 b, double e, double& ln, double& s
 __device__ __forceinline__ q64 polar64(const q64& b, double e) {
 #pragma clang fp contract(off)
   double ln, slope;
-  const q64 u = polar_unit(b, e, ln, slope);
+  const q64 u = polar_unit<true>(b, e, ln, slope);
   const double ex = exp64<true>(ln);
   const double im = slope * ex < __builtin_inf() ? ex : __builtin_inf();
   return q64{u.w * ex, u.x * im, u.y * im, u.z * im};
@@ -561,7 +570,7 @@ __device__ __forceinline__ xq term_ext(const RootRec64& r, const q64& q) {
   if (kPow == kPolar) return xpow(n.m, r.e, r.e * (double)n.e * 0.6931471805599453);
   if (kPow != kExactOnly && !is_one(r.e) && !is_two(r.e)) {
     double ln, slope;
-    xq v{polar_unit(n.m, r.e, ln, slope), 0};
+    xq v{polar_unit<false>(n.m, r.e, ln, slope), 0};
     ln = __builtin_fma(r.e * (double)n.e, 0.6931471805599453, ln);
     scale_ext(v, ln);
     xnorm(v);
@@ -622,7 +631,7 @@ __device__ __forceinline__ bool poly_ext_grouped(RP r, int n, const q64& q, xq& 
       t = qmul64x(t, square64(b, partial64(b)));
     } else {
       double l, slope;
-      t = qmul64x(t, polar_unit(b, rt.e, l, slope));
+      t = qmul64x(t, polar_unit<false>(b, rt.e, l, slope));
       ln += l;
       ok = ok && rt.e > 0.0;  // cos m of a negative power can be 0 to any depth
     }

@@ -5,9 +5,10 @@ import numpy as np
 import pytest
 import torch
 
+import oracle as O
 import test_gpu_adjoint_paths as adjoint
 from quijibo_amd import api
-from quijibo_amd._lib import FP64, MAP_EXTENDED_RANGE
+from quijibo_amd._lib import FP64, FP64_EXACT, MAP_EXTENDED_RANGE
 
 pytestmark = pytest.mark.gpu
 LD = np.longdouble
@@ -131,3 +132,21 @@ def test_adjoint_of_large_exponents(gpu, e):
     eb = np.linalg.norm(b.cpu().numpy() - gp) / np.linalg.norm(gp)
     print("e %g: %.2e %.2e" % (e, ea, eb), flush=True)
     assert ea <= 1e-3 and eb <= 1e-3
+
+
+@pytest.mark.parametrize("iters", [1, 2])
+@pytest.mark.parametrize("prec", [FP64, FP64_EXACT])
+def test_bases_out_of_range(gpu, prec, iters):
+    """Real powers of bases whose square is 0 or infinite in FP64 are not finite,
+    as QUATERNION::pow's are (its |b| is 0 or infinite); the extended range takes
+    them. Beside them bases whose squares are just inside."""
+    s = np.array([1e-170, 3e-163, 1e-150, 1e-100, 1e-3, 0.5, 1e100, 1e150, 1e155, 1e200, 1e300])
+    pts = np.concatenate([s[:, None] * d for d in np.array([[1.0, 0.5, -0.25], [0.0, 1.0, 0.0], [-1.0, 1e-3, 0.0],
+                                                            [1.0, 1e-60, 0.0]])])
+    for e in (0.003, 0.4, 1.5):
+        gp = api.make_params(iters, np.inf, 1.0, 0.0, 0)
+        F = api.points_eval(torch.from_numpy(pts).cuda(), _poly([0, 0, 0, 0], e), gp, prec).cpu().numpy()
+        ref = O.points_eval(pts, O.poly([[0, 0, 0, 0]], [e]), O.poly(NONE, []), O.make_params(iters, np.inf, 1.0, 0.0, 0))
+        assert np.array_equal(np.isfinite(F), np.isfinite(ref)), (e, pts[np.isfinite(F) != np.isfinite(ref)])
+        fin = np.isfinite(ref)
+        assert np.max(np.abs(F[fin] - ref[fin]) / np.maximum(1.0, np.abs(ref[fin]))) <= 1e-9
