@@ -127,10 +127,13 @@ __device__ Acc combine(const double* __restrict__ part, int nparts) {
 __device__ __forceinline__ double total_of(const Acc& a) {
   return isfinite(a.special) ? a.s.hi + a.s.lo : a.special;
 }
-__device__ __forceinline__ void acc_value(Acc& a, double v) {
-  a.count += 1.0;
+__device__ __forceinline__ void acc_sum(Acc& a, double v) {
   if (isfinite(v)) a.s = dd_add1(a.s, v);
   else a.special += v;
+}
+__device__ __forceinline__ void acc_value(Acc& a, double v) {
+  a.count += 1.0;
+  acc_sum(a, v);
 }
 
 template <bool kNan>
@@ -449,8 +452,9 @@ __global__ __launch_bounds__(kOpsBlock) void k_cell_weights(GridGeom g, GridGeom
 // thresholds from blockIdx.y kScores on: the partial sums of
 // -tanh(alpha (F - threshold)) w(cell centre). FP64 VALU bound (the tanh); the
 // field and the cells' weights are read once per kScores thresholds. 50^3, 100
-// thresholds: 34 us; one threshold per block with the lookup and the library's
-// tanh 169 us, this split with the library's tanh 67 us.
+// thresholds: 39 us; one threshold per block with the lookup and the library's
+// tanh 169 us, this split with the library's tanh 67 us, with a tanh of 2.6
+// instead of 0.81 ulp 34 us.
 constexpr int kScores = 4;
 __global__ __launch_bounds__(kOpsBlock) void k_weight_score(const double* __restrict__ f,
                                                             const double* __restrict__ cw, int64_t n,
@@ -468,7 +472,7 @@ __global__ __launch_bounds__(kOpsBlock) void k_weight_score(const double* __rest
   for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
     const double F = f[i], w = cw[i];
 #pragma unroll
-    for (int k = 0; k < kScores; k++) acc_value(a[k], -tanh64(alpha * (F - thr[k])) * w);
+    for (int k = 0; k < kScores; k++) acc_sum(a[k], -tanh64(alpha * (F - thr[k])) * w);
   }
 #pragma unroll
   for (int k = 0; k < kScores; k++) {
@@ -723,8 +727,8 @@ qj_status weight_scores(qj_workspace* ws, const double* d_field, const qj_grid* 
   const int64_t n = (int64_t)g.res[0] * g.res[1] * g.res[2];
   if (n <= 0 || nthr < 0) return QJ_ERR_INVALID;
   // up to 8 cells per thread where the thresholds fill the chip by themselves:
-  // the four block sums cost as much as some 10 cells (50^3, 100 thresholds: 1750
-  // blocks 34 us, 6400 of 2 cells 41)
+  // the four block sums cost as much as some 10 cells (50^3, 100 thresholds: 6400
+  // blocks of 2 cells take a fifth longer than 1750)
   const int64_t want = (n + kOpsBlock - 1) / kOpsBlock, ny = (nthr + kScores - 1) / kScores;
   const int64_t per = std::min<int64_t>(8, std::max<int64_t>(1, want * ny / 1536));
   const int gx = (int)std::min<int64_t>((want + per - 1) / per, 256);

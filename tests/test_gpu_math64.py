@@ -42,6 +42,23 @@ def test_log(gpu):
     assert err.max() <= 1.0
 
 
+def test_tanh(gpu):
+    """A weight score over one cell of weight 1 is -tanh(alpha (F - threshold)).
+    At most 1 ulp, the bound of the library function it stands for."""
+    rng = np.random.default_rng(1)
+    x = np.concatenate([rng.uniform(-22, 22, 30000), rng.uniform(-1, 1, 30000), 2.0 ** rng.uniform(-60, 1, 20000),
+                        np.arange(-40, 41) * 0.34657359027997264 / 2, [0.0, -0.0, 30.0, -700.0, 1e300, np.inf, -np.inf, 5e-324]])
+    g = api.make_grid((1, 1, 1), lengths=(1.0, 1.0, 1.0))
+    one, zero = torch.ones(1, dtype=torch.float64, device="cuda"), torch.zeros(1, dtype=torch.float64, device="cuda")
+    parts = [api.weight_scores(zero, g, one, g, 1.0, p) for p in np.array_split(x, 2)]  # 1 (0 - x): -tanh(-x)
+    sc = np.concatenate([p[0] for p in parts])
+    assert all(p[1] == 1.0 for p in parts)
+    ref = np.tanh(x.astype(LD))
+    err = np.abs(sc - ref) / _ulp(ref)
+    print("tanh: %.3f ulp" % err.max(), flush=True)
+    assert err.max() <= 1.0
+
+
 def _polar(b, e):
     """b^e of QUATERNION::pow in long double: unit part's and magnitude's product, and the angle"""
     b = b.astype(LD)
