@@ -452,6 +452,14 @@ __global__ __launch_bounds__(kApBlock) void k_ap_fast(APArgs g, const RootRec64*
   }
   __syncthreads();
   const int nr = a.nt + a.nb, i0 = wave * nr / kWaves, i1 = (wave + 1) * nr / kWaves;
+  // the roots in turn from top and bottom, what is left of the longer one last: the
+  // running sums of logarithms stay small, and with them their roundings
+  const int pairs = 2 * (a.nt < a.nb ? a.nt : a.nb);
+  const int lo = (a.nt > a.nb ? 0 : a.nt) - (pairs >> 1);
+  auto root_at = [&](int j) {
+    const int two = (j >> 1) + (j & 1) * a.nt;
+    return j < pairs ? two : j + lo;
+  };
   double x[M], y[M], z[M], f[M] = {}, s[M] = {}, lm[M] = {}, l[R > 0 ? R : 1][M];
 #pragma unroll
   for (int u = 0; u < M; u++) {
@@ -476,14 +484,15 @@ __global__ __launch_bounds__(kApBlock) void k_ap_fast(APArgs g, const RootRec64*
 #pragma unroll
         for (int k = j; k < j + kGroup; k++) {
           const bool in = i0 + k < i1;
-          const int i = in ? i0 + k : i1 - 1;
+          const int i = root_at(in ? i0 + k : i1 - 1);
           const RootRec64 r = roots[i];
           add(r, in ? 0.5 * r.e : 0.0, i < a.nt, l[k]);
         }
       }
     }
   } else {
-    for (int i = i0; i < i1; i++) {
+    for (int j = i0; j < i1; j++) {
+      const int i = root_at(j);
       const RootRec64 r = roots[i];
       add(r, 0.5 * r.e, i < a.nt, l[0]);
     }
@@ -553,7 +562,7 @@ __global__ __launch_bounds__(kApBlock) void k_ap_fast(APArgs g, const RootRec64*
 #pragma unroll
         for (int u = 0; u < M; u++) v = __builtin_fma(dd[u], l[k][u], v);
         v = wave_sum63(v);
-        if (lane == 63) row[kApFastRows + i0 + k] = 0.5 * v;
+        if (lane == 63) row[kApFastRows + root_at(i0 + k)] = 0.5 * v;
       }
     }
     return;
@@ -581,7 +590,8 @@ __global__ __launch_bounds__(kApBlock) void k_ap_fast(APArgs g, const RootRec64*
     z[u] = in ? s_a[2][j] : 0.0;
     dd[u] = in ? s_a[3][j] : 0.0;
   }
-  for (int i = i0; i < i1; i++) {
+  for (int j = i0; j < i1; j++) {
+    const int i = root_at(j);
     const RootRec64 r = roots[i];
     const double dz = a.slice - r.z, dz2 = dz * dz;
     double v = 0.0;
