@@ -651,9 +651,10 @@ __global__ __launch_bounds__(kSumThreads) void k_ap_finish(const double* __restr
 // 256 cells a block keep four logarithms per lane in flight and share the block's
 // set-up; below 128 such blocks (half the CUs) 64 cells a block spread the work
 // further: 25^3 35.4 against 39.1 us a call, 40^3 43.5 against 39.8, 64^3 77.5
-// against 59.3 (64- against 256-cell blocks, 32+32 real exponents). A wave keeps up
-// to 8, 16 or 32 roots' logarithms in registers (128 to 192 VGPRs); beyond 256
-// roots they are computed twice (97^3 with 32+32 roots: 149 us that way, 128
+// against 59.3 (64- against 256-cell blocks, 32+32 real exponents). A wave keeps the
+// logarithms of up to 8 or 16 roots in registers (128 and 192 VGPRs), of up to 32
+// in 64-cell blocks; beyond 128 roots on grids of 256-cell blocks and 256 on
+// smaller ones they are computed twice (97^3 with 32+32 roots: 149 us that way, 128
 // kept). Against the product formulas for every cell: 97^3 2264 to 128 us a call,
 // 25^3 254 to 36 us; the kernel takes 113 us of the 128, its FP64 issue about 80.
 qj_status ap_grads(qj_workspace* ws, const MapArgs& a, const qj_rational* f, const qj_grid* wg, const double* d_weight,
