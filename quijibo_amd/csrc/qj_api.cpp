@@ -21,6 +21,8 @@ void set_error(const char* fmt, ...) {
 }
 
 qj_status hip_fail(hipError_t e, const char* what) {
+  // reported here: left in the runtime it would be the next launch's error as well
+  (void)hipGetLastError();
   set_error("%s failed: %s", what, hipGetErrorString(e));
   return e == hipErrorOutOfMemory ? QJ_ERR_NOMEM : QJ_ERR_HIP;
 }
