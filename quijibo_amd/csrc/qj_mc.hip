@@ -1138,9 +1138,18 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
       (st = grow(m.groups, m.cap_groups, 2 * gmax, s)) || (st = grow(m.d_base, m.cap_base, 2 * ((int64_t)n + 1), s)))
     return st;
   if (!m.tickets) {
+    // cleared before anything else can count on them: an error return below does not
+    // wait for s, and the next call may come on another stream
     const size_t bytes = sizeof(uint32_t) * kTicketLine * (kTickets + 1);
-    QJ_HIP(hipMalloc(&m.tickets, bytes));
-    QJ_HIP(hipMemsetAsync(m.tickets, 0, bytes, s));
+    uint32_t* t = nullptr;
+    QJ_HIP(hipMalloc(&t, bytes));
+    hipError_t e = hipMemsetAsync(t, 0, bytes, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+      hipFree(t);
+      return hip_fail(e, "clearing the tickets");
+    }
+    m.tickets = t;
   }
   // first sizes: a quarter of the points as vertices, half as triangles
   // (a 256^3 torus tile holds 0.42 and 0.73 of its points)
