@@ -17,9 +17,10 @@
 //   k_mc_vertices   p0 + d0/(d0-d1) (p1-p0) at cell centres, no contraction,
 //                   and a bit per edge whose vertex lies near an end (an FP32
 //                   estimate)
-//   k_mc_cells      triangle counts, and the degenerate filter (edge < 1e-7
-//                   dropped) on the cells whose near vertices lie on edges that
-//                   meet; its last block, or k_mc_scan: first triangle per group
+//   k_mc_measure    the degenerate filter (edge < 1e-7 dropped) on the cells whose
+//                   near vertices lie on edges that meet, where estimates do not
+//                   decide it (kMeasureAll, kMeasureNear) and groups are few
+//   k_mc_cells      triangle counts, and elsewhere the degenerate filter; its last block, or k_mc_scan: first triangle per group
 //   k_mc_tris       each kept triangle written once, in cell then table order
 #include <float.h>
 #include <math.h>
@@ -812,11 +813,89 @@ __device__ __forceinline__ uint64_t word_cases(const McGrid& a, int64_t w, uint8
   return act;
 }
 
+// The cells of word w that may hold a triangle with two near vertices on edges that
+// meet at a corner, among those of act (a border set by setBorders puts near
+// vertices in every cell along it, but on parallel edges).
+__device__ __forceinline__ uint64_t meeting_near_edges(const McGrid& a, int64_t w, uint64_t act) {
+  const int64_t X = a.g.res[0], XY = a.XY;
+  uint64_t near[12], cells = 0;
+#pragma unroll
+  for (int e = 0; e < 12; e++) {
+    int dx = 0, dy = 0, dz = 0, axis = 0;
+    edge_parts(e, dx, dy, dz, axis);
+    near[e] = shifted_word(a.near[axis], w, dx + dy * X + dz * XY);
+  }
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const int dx = k >> 2, dy = (k >> 1) & 1, dz = k & 1;
+    const uint64_t nx = near[dy + 2 * dz], ny = near[4 + dx + 2 * dz], nz = near[8 + dx + 2 * dy];
+    cells |= (nx & (ny | nz)) | (ny & nz);
+  }
+  return cells & act;
+}
+
+// The degenerate filter where estimates do not decide it (kMeasureAll,
+// kMeasureNear): the first wave finds the candidates of `words` words, one per
+// thread, and lists them in LDS, where all four take them one per thread. drop: the
+// cells that lost triangles, kmask what they keep, lost the triangles lost per
+// word. k_mc_cells does the same for its groups of 16384 cells; where those are fewer
+// than the CUs and noise or values of 0 and 1 make every second cell a candidate,
+// its blocks take 400 us one after another, and this kernel's spread over the chip.
+// FP64 VALU bound. Times beside measure_words.
+constexpr int kMeasureWords = 64;
+__global__ __launch_bounds__(kMcBlock) void k_mc_measure(const double* __restrict__ field, McGrid a, int words,
+                                                         uint8_t* __restrict__ kmask, uint32_t* __restrict__ lost) {
+  __shared__ uint16_t s_list[64 * kMeasureWords];
+  __shared__ uint32_t s_drop[2 * kMeasureWords], s_lost[kMeasureWords], s_cells;
+  const int tid = threadIdx.x;
+  const int64_t w0 = xcd_block(gridDim.x) * words, w = w0 + tid;
+  const bool own = tid < words && w < a.nw;
+  if (tid < kMeasureWords) {
+    uint64_t cells = 0;
+    if (own) {
+      const EndMasks end = end_masks(a, w);
+      uint64_t any = 0, all = ~0ull;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const uint64_t c = shifted_word(a.sgn, w, (k >> 2) + ((k >> 1) & 1) * (int64_t)a.g.res[0] + (k & 1) * a.XY);
+        any |= c;
+        all &= c;
+      }
+      cells = any & ~all & ~(end.x | end.y | end.z | bits_from(a.cells - 64 * w));
+      if (cells && a.prefilter) cells = meeting_near_edges(a, w, cells);
+    }
+    s_drop[2 * tid] = s_drop[2 * tid + 1] = 0u;
+    s_lost[tid] = 0u;
+    const uint32_t mine = (uint32_t)__popcll(cells), incl = wave_inclusive(mine);
+    uint32_t k = incl - mine;
+    for (uint64_t m = cells; m; m &= m - 1)
+      s_list[k++] = (uint16_t)(tid << 6 | (__ffsll((unsigned long long)m) - 1));
+    if (tid == 63) s_cells = incl;
+  }
+  __syncthreads();
+  for (uint32_t j = tid; j < s_cells; j += kMcBlock) {
+    const unsigned i = s_list[j];
+    const int64_t p = 64 * w0 + i;
+    unsigned row;
+    const unsigned d = mc_measure_cell(field, a, p, &row);
+    if (d) {
+      kmask[p] = (uint8_t)(row & ~d);
+      atomicOr(&s_drop[i >> 5], 1u << (i & 31u));
+      atomicAdd(&s_lost[i >> 6], (uint32_t)__popc(d));
+    }
+  }
+  __syncthreads();
+  if (own) {
+    a.drop[w] = (uint64_t)s_drop[2 * tid + 1] << 32 | s_drop[2 * tid];
+    lost[w] = s_lost[tid];
+  }
+}
+
 // Triangle counts, one word of cells per thread: the counts' three bits as
 // word operations on the corners' words. The degenerate filter measures the
 // cells with near vertices on two edges that meet at a corner, found the same
-// way (a border set by setBorders puts near vertices in every cell along it,
-// but on parallel edges), listed in LDS and measured one per thread.
+// way, listed in LDS and measured one per thread, unless lost says what
+// k_mc_measure dropped.
 // flags: the case of every cell that has
 // triangles, else 0. Latency-bound: 256^3, 1024 blocks, 20.5 us with the
 // scan, of which the measurement's longest chain is 6 (20 with every near pair
@@ -824,35 +903,19 @@ __device__ __forceinline__ uint64_t word_cases(const McGrid& a, int64_t w, uint8
 // per group.
 __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict__ field, McGrid a,
                                                        uint8_t* __restrict__ flags, uint8_t* __restrict__ kmask,
+                                                       const uint32_t* __restrict__ lost,
                                                        uint32_t* __restrict__ tword,
                                                        uint32_t* __restrict__ groups, ScanTail tail) {
   __shared__ uint16_t s_list[kMcWaves][64 * 64];
   __shared__ uint32_t s_drop[2 * kMcGroupWords], s_lost[kMcGroupWords], s_cells[kMcWaves];
   const int64_t w = (int64_t)blockIdx.x * kMcGroupWords + threadIdx.x;
-  const int64_t X = a.g.res[0], XY = a.XY;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint64_t act = 0, candidates = 0;
+  uint64_t candidates = 0;
   uint32_t count = 0;
   if (w < a.nw) {
-    act = word_cases(a, w, flags, &count);
-    if (act && a.prefilter) {
-      uint64_t near[12];
-#pragma unroll
-      for (int e = 0; e < 12; e++) {
-        int dx = 0, dy = 0, dz = 0, axis = 0;
-        edge_parts(e, dx, dy, dz, axis);
-        near[e] = shifted_word(a.near[axis], w, dx + dy * X + dz * XY);
-      }
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const int dx = k >> 2, dy = (k >> 1) & 1, dz = k & 1;
-        const uint64_t nx = near[dy + 2 * dz], ny = near[4 + dx + 2 * dz], nz = near[8 + dx + 2 * dy];
-        candidates |= (nx & (ny | nz)) | (ny & nz);
-      }
-    } else {
-      candidates = ~0ull;
-    }
-    candidates &= act;
+    const uint64_t act = word_cases(a, w, flags, &count);
+    if (lost) count -= lost[w];
+    else if (act) candidates = a.prefilter ? meeting_near_edges(a, w, act) : act;
   }
   s_drop[2 * threadIdx.x] = s_drop[2 * threadIdx.x + 1] = 0u;
   s_lost[threadIdx.x] = 0u;
@@ -885,7 +948,7 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_cells(const double* __restrict_
   uint32_t total;
   const uint32_t before = block_prefix<kMcBlock>(count, &total);
   if (w < a.nw) {
-    a.drop[w] = (uint64_t)s_drop[2 * threadIdx.x + 1] << 32 | s_drop[2 * threadIdx.x];
+    if (!lost) a.drop[w] = (uint64_t)s_drop[2 * threadIdx.x + 1] << 32 | s_drop[2 * threadIdx.x];
     tword[w] = before;
   }
   finish_scan(groups, total, tail, 1);
@@ -1091,6 +1154,18 @@ static qj_status launch_tris(const McState& m, const McGrid& mg, const uint32_t*
   return QJ_OK;
 }
 
+// Words per block of k_mc_measure, or 0 where k_mc_cells measures: where estimates
+// decide nearly all (kMeasureUnsure), and beyond one group per CU. 256 cells a block,
+// one per thread, until 2048 blocks fill the chip, then more. Calls in us, in
+// k_mc_cells and in a kernel of its own (a case byte per cell and a kernel over all
+// cells, before): kMeasureAll, noise, 24^3 409 / 66 (123), 64^3 545 / 87 (139), 97^3
+// 578 / 147 (216), 160^3 601 / 439 (584), 256^3 1811 / 1706 (2231); a sphere's surface
+// 77 / 55 (110), 73 / 56 (114), 69 / 65 (122), 87 / 90 (171), 142 / 160 (311).
+static int measure_words(const McGrid& a, int64_t groups) {
+  if (a.prefilter == kMeasureUnsure || groups > 256) return 0;
+  return (int)std::min<int64_t>(kMeasureWords, std::max<int64_t>(4, (a.nw + 2047) / 2048));
+}
+
 // Meshes n fields one after another on the stream without waiting on the
 // host: every count stays on the device (running vertex and triangle totals,
 // per-tile counts) and is read back once at the end. The vertex and triangle
@@ -1111,6 +1186,7 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
   std::vector<GridGeom> geo((size_t)n);
   std::vector<int> prefilter((size_t)n);
   int64_t nmax = 0, total_pts = 0, pad_max = 0;
+  bool measured = false;
   for (int k = 0; k < n; k++) {
     GridGeom& g = geo[(size_t)k];
     make_geom(&grids[k], &g);
@@ -1127,6 +1203,7 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
     prefilter[(size_t)k] = !is_turned_grid(g, kPrefilterSpacing, kPrefilterMaxSpacing) ? kMeasureAll
                            : grid_extent(g) <= kSureExtent                            ? kMeasureUnsure
                                                                                       : kMeasureNear;
+    measured |= prefilter[(size_t)k] != kMeasureUnsure;
   }
   qj_status st;
   // words of 64 points, plus what the reads of a word's +y and +z rows run past the end
@@ -1134,7 +1211,7 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
   const int64_t gmax = (nmax + kMcGroupPoints - 1) / kMcGroupPoints;
   if ((st = grow(m.words, m.cap_words, kMcArrays * wmax, s)) || (st = grow(m.ranks, m.cap_ranks, 8 * wmax, s)) ||
       (st = grow(m.flags, m.cap_flags, 64 * ((nmax + 63) / 64), s)) || (st = grow(m.kmask, m.cap_kmask, nmax, s)) ||
-      (st = grow(m.tword, m.cap_tword, wmax, s)) ||
+      (st = grow(m.tword, m.cap_tword, wmax, s)) || (measured && (st = grow(m.lost, m.cap_lost, wmax, s))) ||
       (st = grow(m.groups, m.cap_groups, 2 * gmax, s)) || (st = grow(m.d_base, m.cap_base, 2 * ((int64_t)n + 1), s)))
     return st;
   if (!m.tickets) {
@@ -1193,7 +1270,14 @@ qj_status mc_run_tiles(qj_workspace* ws, int n, const double* const* fields, con
                            (const uint2*)m.ranks, (const uint32_t*)gv, (const uint64_t*)(m.d_base + 2 * k), vcap,
                            verts);
         QJ_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_mc_cells, dim3((unsigned)ng), dim3(kMcBlock), 0, s, fields[k], mg, m.flags, m.kmask,
+        const uint32_t* lost = nullptr;
+        if (const int words = measure_words(mg, ng)) {
+          hipLaunchKernelGGL(k_mc_measure, blocks_of(mg.nw, words), dim3(kMcBlock), 0, s, fields[k], mg, words,
+                             m.kmask, m.lost);
+          QJ_HIP(hipGetLastError());
+          lost = m.lost;
+        }
+        hipLaunchKernelGGL(k_mc_cells, dim3((unsigned)ng), dim3(kMcBlock), 0, s, fields[k], mg, m.flags, m.kmask, lost,
                            m.tword, gt, tail);
         QJ_HIP(hipGetLastError());
       }
