@@ -1155,14 +1155,15 @@ static qj_status launch_tris(const McState& m, const McGrid& mg, const uint32_t*
 }
 
 // Words per block of k_mc_measure, or 0 where k_mc_cells measures: where estimates
-// decide nearly all (kMeasureUnsure), and beyond one group per CU. 256 cells a block,
+// decide nearly all (kMeasureUnsure), and beyond two groups per CU. 256 cells a block,
 // one per thread, until 2048 blocks fill the chip, then more. Calls in us, in
 // k_mc_cells and in a kernel of its own (a case byte per cell and a kernel over all
 // cells, before): kMeasureAll, noise, 24^3 409 / 66 (123), 64^3 545 / 87 (139), 97^3
-// 578 / 147 (216), 160^3 601 / 439 (584), 256^3 1811 / 1706 (2231); a sphere's surface
-// 77 / 55 (110), 73 / 56 (114), 69 / 65 (122), 87 / 90 (171), 142 / 160 (311).
+// 578 / 147 (216), 160^3 601 / 439 (584), 168^3 858 / 503 (677), 200^3 957 / 824 (1057),
+// 256^3 1811 / 1706 (2231); a sphere's surface 77 / 55 (110), 73 / 56 (114), 69 / 65
+// (122), 87 / 90 (171), 87 / 90 (174), 100 / 105 (206), 142 / 160 (311).
 static int measure_words(const McGrid& a, int64_t groups) {
-  if (a.prefilter == kMeasureUnsure || groups > 256) return 0;
+  if (a.prefilter == kMeasureUnsure || groups > 512) return 0;
   return (int)std::min<int64_t>(kMeasureWords, std::max<int64_t>(4, (a.nw + 2047) / 2048));
 }
 

@@ -1,6 +1,6 @@
 """Marching cubes where the degenerate filter measures vertices (spacings beyond the
 prefilter's, coordinates beyond the estimates'): dense and sparse candidates, blocks
-of 4 to 32 words with ragged ends, and fields beyond 256 groups, which measure in
+of 4 to 32 words with ragged ends, and fields beyond 512 groups, which measure in
 the counting kernel. Bit for bit against the oracle mesher."""
 import numpy as np
 import pytest
@@ -25,7 +25,7 @@ def _field(kind, n, rng):
 @pytest.mark.parametrize("res, kind", [
     ((2, 2, 2), "binary"), ((5, 9, 3), "noise"), ((24, 23, 25), "binary"), ((65, 64, 63), "noise"),
     ((65, 64, 63), "sparse"), ((97, 101, 89), "binary"), ((129, 127, 130), "sparse"), ((163, 162, 161), "sparse"),
-    ((163, 162, 161), "binary"),
+    ((163, 162, 161), "binary"), ((209, 203, 202), "sparse"),
 ])
 def test_measured_cells(gpu, res, kind):
     n = res[0] * res[1] * res[2]
