@@ -32,19 +32,6 @@ __device__ __forceinline__ bool has_nan(const q64& q) { return isnan(q.w) || isn
 // b = 0 gives NaN, v = 0 gives (|w|^e, +0 * v).
 enum PowMode { kPolar = 0, kExactInt = 1, kExactOnly = 2 };
 
-// One root record by value through any pointer type (generic, or the constant
-// address space where a kernel wants scalar loads of a pointer it read from
-// memory).
-// Roots read through the constant address space: known not to be clobbered by
-// the kernel's stores and atomics, so a uniform address gives scalar loads in
-// every loop (without it the kernels that store or count inside their loop took
-// three vector loads per root, with one wave per SIMD a cache latency each).
-typedef const __attribute__((address_space(4))) RootRec64* ConstRoots;
-template <class RP>
-__device__ __forceinline__ RootRec64 load_root64(RP p) {
-  return RootRec64{p->w, p->x, p->y, p->z, p->e, p->p};
-}
-
 // f on roots r[i], r[i + 1], ... r[end - 1] in order, the loads of four at once:
 // the terms branch on the exponent, which keeps the compiler from hoisting the
 // next root's load, which then costs its latency where few waves share a SIMD

@@ -15,7 +15,8 @@
 //   as they stand and redoes overflowed cells with a shared binary exponent per
 //   quaternion (the reference redoes them in long double, :9011-9103); so is
 //   every cell when some exponent is negative (QUATERNION::pow then drops the
-//   imaginary part, and |b^e| is not |b|^e).
+//   imaginary part, and |b^e| is not |b|^e) or the exponents are so large that few
+//   cells would be spared (ap_from_logs).
 //   Sums are over fixed trees, so results do not depend on scheduling.
 //
 // k_adjoint: reverse mode through max_iter iterations of the map at points.
@@ -171,7 +172,7 @@ __device__ __forceinline__ double bottom_term_x(const q64& left, const q64& powe
 // and bulk) into acc. Every lane of the wave calls this (the reductions are
 // wave-wide); lanes with active == false add zeros.
 template <class Q>
-__device__ __forceinline__ void cell_terms(const APArgs& g, const RootRec64* __restrict__ roots, const q64& q0,
+__device__ __forceinline__ void cell_terms(const APArgs& g, ConstRoots roots, const q64& q0,
                                            const Q& T, const Q& B, double w, bool active, double* acc, int K) {
   const MapArgs& a = g.a;
   Q R = T;
@@ -193,7 +194,7 @@ __device__ __forceinline__ void cell_terms(const APArgs& g, const RootRec64* __r
     for (int i = a.nt - 1; i >= 0; i--) {
       double vt = 0.0, vb = 0.0;
       if (valid) {
-        const RootRec64 r = roots[i];
+        const RootRec64 r = load_root64(roots + i);
         const q64 base = qsub(q0, q64{r.w, r.x, r.y, r.z});
         const Q power = pw<Q>(base, r.e);
         const Q right = S;  // S_{i+1}
@@ -216,12 +217,12 @@ __device__ __forceinline__ void cell_terms(const APArgs& g, const RootRec64* __r
     }
   }
   if (a.nb > 0) {
-    const RootRec64* rb = roots + a.nt;
+    const ConstRoots rb = roots + a.nt;
     Q S = one;
     for (int i = a.nb - 1; i >= 0; i--) {
       double vt = 0.0, vb = 0.0;
       if (valid) {
-        const RootRec64 r = rb[i];
+        const RootRec64 r = load_root64(rb + i);
         const q64 base = qsub(q0, q64{r.w, r.x, r.y, r.z});
         const Q power = pw<Q>(base, r.e);
         const Q right = S;
@@ -255,7 +256,7 @@ __device__ __forceinline__ void cell_terms(const APArgs& g, const RootRec64* __r
 }
 
 template <class Q>
-__device__ __forceinline__ Q poly_fwd(const RootRec64* __restrict__ r, int n, const q64& q) {
+__device__ __forceinline__ Q poly_fwd(ConstRoots r, int n, const q64& q) {
   Q res = pw<Q>(qsub(q, q64{r[0].w, r[0].x, r[0].y, r[0].z}), r[0].e);
   for (int i = 1; i < n; i++) res = mul(res, pw<Q>(qsub(q, q64{r[i].w, r[i].x, r[i].y, r[i].z}), r[i].e));
   return res;
@@ -293,10 +294,71 @@ __device__ __forceinline__ bool ap_cell(const APArgs& g, const double* __restric
   return true;
 }
 
-// the formulas as they stand, for the cells of `left` (one bit per cell, 64
-// cells a word), or for every cell when left is null. Each block takes a
-// contiguous run of groups of 256 cells and writes one row of partial sums.
-__global__ __launch_bounds__(kGBlock) void k_ap_grads(APArgs g, const RootRec64* __restrict__ roots,
+// log(|q - r|^2) for a point (x, y, z, .) with (q.z - r.z)^2 given
+__device__ __forceinline__ double log_norm2(double x, double y, double z, const RootRec64& r, double dz2) {
+  const double dw = x - r.w, dx = y - r.x, dy = z - r.y;
+  return log64(__builtin_fma(dw, dw, __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz2))));
+}
+__device__ __forceinline__ double log_norm2(const q64& q, const RootRec64& r) {
+  const double dz = q.z - r.z;
+  return log_norm2(q.w, q.x, q.y, r, dz * dz);
+}
+
+// Bounds of the cells that k_ap_grads takes from logarithms: the sums of e |log|b||
+// of each polynomial, and |log|R|| + |log c|. Then T, B, their prefixes and
+// suffixes and R are within e^+-330, their squares within e^+-660, and a product of
+// a top and a bottom factor within e^660 times scalar and logarithm: no step of the
+// formulas leaves FP64's range but those that bottom_term_x takes up.
+constexpr double kApEach = 330.0;
+
+// One cell from logarithms, as k_ap_fast takes it, for the lanes of cell; clears
+// those that are out of bounds.
+__device__ __forceinline__ void log_cell(const APArgs& g, ConstRoots roots, const q64& q0, bool& cell, double& F) {
+  const MapArgs& a = g.a;
+  double f = 0.0, st = 0.0, sb = 0.0, lm = 0.0;
+  for (int i = 0; i < a.nt + a.nb; i++) {
+    const RootRec64 r = load_root64(roots + i);
+    const double l = log_norm2(q0, r), h = 0.5 * r.e;
+    f = __builtin_fma(i < a.nt ? h : -h, l, f);
+    if (i < a.nt) st = __builtin_fma(h, fabs(l), st);
+    else sb = __builtin_fma(h, fabs(l), sb);
+    lm = fmax(lm, fabs(l));
+  }
+  cell = cell && lm < 600.0 && st < kApEach && sb < kApEach && fabs(f) + fabs(g.log_c) < kApEach;
+  if (cell) F = f + g.log_c;
+}
+__device__ __forceinline__ void log_terms(const APArgs& g, ConstRoots roots, const q64& q0, double F, double w,
+                                          bool cell, double* acc, int K) {
+  const MapArgs& a = g.a;
+  double d = 0.0, gts = 0.0, gbs = 0.0;
+  if (cell) {
+    const double t = tanh(g.alpha * (F - g.thr));
+    d = -g.alpha * w * (1 - t * t);
+    if (!isfinite(d)) d = 0.0;  // a non-finite weight leaves the root terms out
+  }
+  for (int i = 0; i < a.nt + a.nb; i++) {
+    const RootRec64 r = load_root64(roots + i);
+    const double v = d != 0.0 ? 0.5 * d * log_norm2(q0, r) : 0.0;
+    const bool top = i < a.nt;
+    const double s = top ? a.sc_top : (a.sc_bottom > 0.0 ? -a.sc_bottom : 0.0);  // OPTIMIZE_3D.cpp:10084
+    if (top) gts = __builtin_fma(r.p, v, gts);
+    else if (!(r.p < 1e-8)) gbs = __builtin_fma(-r.p, v, gbs);  // :10404-10405
+    wave_acc(acc, K, SL_ROOTS + i, s * v);
+  }
+  wave_acc(acc, K, SL_GTS, gts);
+  wave_acc(acc, K, SL_GBS, gbs);
+}
+
+// The formulas as they stand, for the cells of `left` (kLeft; one bit per cell, 64
+// cells a word) or for every cell. Each block takes a
+// contiguous run of groups of 256 cells and writes one row of partial sums. The
+// cells of `left` whose polynomials are each in range (k_ap_fast tests their sum)
+// are taken from logarithms here as well: 64^3 with 200+200 real exponents, 1 %
+// of the cells left, 6.3 ms a call without that, 0.90 with it (4.6 by the formulas for
+// every cell). Held to two blocks per CU (284 registers otherwise): 64^3 with a
+// negative exponent 5.5 to 4.7 ms.
+template <bool kLeft>
+__global__ __launch_bounds__(kGBlock, 2) void k_ap_grads(APArgs g, const RootRec64* __restrict__ roots,
                                                       const double* __restrict__ weight, double* __restrict__ field,
                                                       const unsigned long long* __restrict__ left, int64_t per,
                                                       double* __restrict__ partials, int K,
@@ -306,9 +368,10 @@ __global__ __launch_bounds__(kGBlock) void k_ap_grads(APArgs g, const RootRec64*
   for (int i = threadIdx.x; i < (kGBlock / 64) * K; i += kGBlock) acc[i] = 0.0;
   __syncthreads();
   const int64_t N = (int64_t)a.res[0] * a.res[1] * a.res[2];
-  const int64_t groups = (N + kGBlock - 1) / kGBlock, g1 = min((int64_t)(blockIdx.x + 1) * per, groups);
-  int64_t g0 = (int64_t)blockIdx.x * per;
-  if (left) {
+  int64_t g0 = blockIdx.x, g1 = g0 + 1;  // every cell: a group per block
+  if constexpr (kLeft) {
+    g0 = blockIdx.x * per;
+    g1 = min(g0 + per, (N + kGBlock - 1) / kGBlock);
     // a run without a flagged cell is passed over with one load per thread
     const int64_t nw = (N + 63) / 64, w1 = min(g1 * (kGBlock / 64), nw);
     bool any = false;
@@ -318,21 +381,27 @@ __global__ __launch_bounds__(kGBlock) void k_ap_grads(APArgs g, const RootRec64*
   for (int64_t gi = g0; gi < g1; gi++) {
     const int64_t idx = gi * kGBlock + threadIdx.x;
     bool active = idx < N;
-    if (left) active = active && ((left[idx >> 6] >> (idx & 63)) & 1ull);
+    if constexpr (kLeft) active = active && ((left[idx >> 6] >> (idx & 63)) & 1ull);
     if (!__ballot(active)) continue;
     double w = 0.0;
     q64 q0{0, 0, 0, 0};
     double Ffield = 0.0;
     bool iterate = false;
     if (active) iterate = ap_cell(g, weight, field, idx, q0, w, Ffield);
+    bool logs = kLeft && iterate;
+    if (kLeft && __ballot(logs)) {
+      log_cell(g, (ConstRoots)roots, q0, logs, Ffield);
+      if (__ballot(logs)) log_terms(g, (ConstRoots)roots, q0, Ffield, w, logs, acc, K);
+    }
     // forward sweep (computeRationalMapAP with one iteration)
+    const bool formulas = iterate && !logs;
     q64 T{1, 0, 0, 0}, B{1, 0, 0, 0};
     bool ovf = false;
-    if (iterate) {
-      T = poly_fwd<q64>(roots, a.nt, q0);
+    if (formulas) {
+      T = poly_fwd<q64>((ConstRoots)roots, a.nt, q0);
       q64 qn;
       if (a.nb > 0) {
-        B = poly_fwd<q64>(roots + a.nt, a.nb, q0);
+        B = poly_fwd<q64>((ConstRoots)roots + a.nt, a.nb, q0);
         qn = qdiv(T, B);
         const double m2 = B.w * B.w + B.x * B.x + B.y * B.y + B.z * B.z;
         ovf = !(ok(T) && ok(B) && isfinite(m2) && ok(qn));
@@ -346,19 +415,19 @@ __global__ __launch_bounds__(kGBlock) void k_ap_grads(APArgs g, const RootRec64*
       Ffield = log(mag);
     }
     // gradients in FP64 for the cells that stayed finite
-    cell_terms<q64>(g, roots, q0, T, B, w, iterate && !ovf, acc, K);
+    if (__ballot(formulas)) cell_terms<q64>(g, (ConstRoots)roots, q0, T, B, w, formulas && !ovf, acc, K);
     // overflowed cells: the whole cell with explicit binary exponents
-    const bool redo = iterate && ovf;
+    const bool redo = formulas && ovf;
     if (__ballot(redo)) {
       xq TX = xfrom(q64{1, 0, 0, 0}), BX = TX;
       if (redo) {
-        TX = poly_fwd<xq>(roots, a.nt, q0);
-        if (a.nb > 0) BX = poly_fwd<xq>(roots + a.nt, a.nb, q0);
+        TX = poly_fwd<xq>((ConstRoots)roots, a.nt, q0);
+        if (a.nb > 0) BX = poly_fwd<xq>((ConstRoots)roots + a.nt, a.nb, q0);
         const xq R = scaled(mul(TX, inv(BX)), a.exp_scaling);
         const double l = logmag(R);
         Ffield = isnan(l) ? 0.0 : l;  // OPTIMIZE_3D.cpp:1557-1561
       }
-      cell_terms<xq>(g, roots, q0, TX, BX, w, redo, acc, K);
+      cell_terms<xq>(g, (ConstRoots)roots, q0, TX, BX, w, redo, acc, K);
     }
     if (iterate) field[idx] = Ffield;
     double sc = 0.0, ge = 0.0;
@@ -404,12 +473,6 @@ __device__ __forceinline__ double wave_sum63(double v) {
 constexpr double kApRange = 340.0;
 constexpr int kApWaves = 8, kApBlock = 64 * kApWaves;
 constexpr int kApFastRows = 2;  // score, grad_exp, then sum of dSdF log|b_i| per root
-
-// log(|q - r|^2) for a point (x, y, z, .) with (q.z - r.z)^2 given
-__device__ __forceinline__ double log_norm2(double x, double y, double z, const RootRec64& r, double dz2) {
-  const double dw = x - r.w, dx = y - r.x, dy = z - r.y;
-  return log64(__builtin_fma(dw, dw, __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz2))));
-}
 
 // The AP pass of the cells that stay in range: 64 M cells per block, lane l of
 // every wave holding cells l, l + 64, ... Each of the eight waves takes an eighth
@@ -648,6 +711,35 @@ __global__ __launch_bounds__(kSumThreads) void k_ap_finish(const double* __restr
   }
 }
 
+// Whether the cells are worth k_ap_fast. |b^e| = |b|^e needs exponents that are not
+// negative. And where a polynomial's sum of e |log|b|| is out of bounds (kApEach) in
+// many cells, most waves of k_ap_grads hold one and run the formulas after all.
+// Roots 0.6 about the centre of a box of edge 3, calls in us by the formulas alone and
+// with k_ap_fast, by that sum at the box's far corner (each logarithm at least 1): 8+8
+// roots, 64^3, at 250 / 360 / 460 / 610 226 / 239 / 387 / 457 and 81 / 87 / 352 / 518;
+// 32+32 roots, 97^3, at 325 / 450 / 610 2264 / 2408 / 3779 and 467 / 2102 / 5129, 16^3
+// at 450 253 and 307; 200+200 roots, 64^3, at 380 4134 and 874. So up to 400.
+static bool ap_from_logs(const MapArgs& a, const std::vector<RootRec64>& roots) {
+  const double most = 400.0;
+  double half = 0.0, away = 0.0, e[2] = {0.0, 0.0};
+  for (int i = 0; i < 3; i++) half += 0.25 * a.dx[i] * a.dx[i] * (double)a.res[i] * (double)a.res[i];
+  half = sqrt(half);
+  auto distance2 = [&](const RootRec64& r) {
+    const double d[4] = {r.w - a.center[0], r.x - a.center[1], r.y - a.center[2], r.z - a.slice};
+    return d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + d[3] * d[3];
+  };
+  for (size_t i = 0; i < roots.size(); i++) {
+    if (!(roots[i].e >= 0.0 && roots[i].e <= DBL_MAX)) return false;
+    e[(int)i >= a.nt] += roots[i].e;
+    away = fmax(away, distance2(roots[i]));
+  }
+  if (fmax(e[0], e[1]) * fmax(1.0, ::log(half + sqrt(away))) <= most) return true;
+  double s[2] = {0.0, 0.0};
+  for (size_t i = 0; i < roots.size(); i++)
+    s[(int)i >= a.nt] += roots[i].e * fmax(1.0, ::log(half + sqrt(distance2(roots[i]))));
+  return s[0] <= most && s[1] <= most;
+}
+
 // 256 cells a block keep four logarithms per lane in flight and share the block's
 // set-up; below 128 such blocks (half the CUs) 64 cells a block spread the work
 // further: 25^3 35.4 against 39.1 us a call, 40^3 43.5 against 39.8, 64^3 77.5
@@ -667,15 +759,14 @@ qj_status ap_grads(qj_workspace* ws, const MapArgs& a, const qj_rational* f, con
     set_error("too many roots for the gradient kernel (%d)", nr);
     return QJ_ERR_CAPACITY;
   }
-  bool fast = true;  // |b^e| = |b|^e needs exponents that are not negative
-  for (const RootRec64& r : f->h64) fast &= r.e >= 0.0 && r.e <= DBL_MAX;
+  const bool fast = ap_from_logs(a, f->h64);
   const int64_t groups = (N + kGBlock - 1) / kGBlock;
   const bool wide = groups >= 128;
   const int per_wave = (nr + kApWaves - 1) / kApWaves;  // roots of the busiest wave
   const int64_t cells = wide || per_wave > 32 ? 256 : 64;
   const int64_t rows_f = fast ? (N + cells - 1) / cells : 0;
   // rows of the general kernel: one per group when it does all the work
-  const int64_t per = fast ? (groups + 255) / 256 : 1, rows_g = (groups + per - 1) / per;
+  const int64_t per = fast ? (groups + 511) / 512 : 1, rows_g = (groups + per - 1) / per;
   const int64_t nwords = (N + 63) / 64;
   qj_status st = ensure_partials(ws, rows_f * KF + rows_g * K + nwords + 1, s);
   if (st) return st;
@@ -701,8 +792,8 @@ qj_status ap_grads(qj_workspace* ws, const MapArgs& a, const qj_rational* f, con
     hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(64), 0, s, nad);
   }
   QJ_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_ap_grads, dim3((unsigned)rows_g), dim3(kGBlock), lds, s, g, f->d64, d_weight, d_field,
-                     fast ? (const unsigned long long*)left : (const unsigned long long*)nullptr, per, pg, K, nad);
+  hipLaunchKernelGGL(fast ? k_ap_grads<true> : k_ap_grads<false>, dim3((unsigned)rows_g), dim3(kGBlock), lds, s, g,
+                     f->d64, d_weight, d_field, (const unsigned long long*)left, per, pg, K, nad);
   QJ_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_ap_finish, dim3((K + kApCols - 1) / kApCols, 2), dim3(kSumThreads), 0, s, (const double*)pf,
                      rows_f, KF, (const double*)pg, rows_g, K, (const unsigned long long*)nad, ws->h_pinned);

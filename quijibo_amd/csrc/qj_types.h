@@ -13,6 +13,16 @@ struct RootRec64 {
   double e;   // power_scalar * powers[i], rounded as the reference does (POLYNOMIAL_4D.cpp:914,919)
   double p;   // powers[i]
 };
+// Roots read through the constant address space: known not to be clobbered by
+// the kernel's stores and atomics, so a uniform address gives scalar loads in
+// every loop (without it the kernels that store or count inside their loop took
+// three vector loads per root, with one wave per SIMD a cache latency each).
+typedef const __attribute__((address_space(4))) RootRec64* ConstRoots;
+// One root record by value through any pointer type.
+template <class RP>
+__device__ __forceinline__ RootRec64 load_root64(RP p) {
+  return RootRec64{p->w, p->x, p->y, p->z, p->e, p->p};
+}
 // FP32 view of one root (host side; kernels read the packed block below).
 struct RootRec32 {
   float w, x, y, z;
