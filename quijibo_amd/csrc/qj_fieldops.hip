@@ -415,34 +415,40 @@ __global__ __launch_bounds__(kOpsBlock) void k_fold_sums(const double* __restric
   }
 }
 
-// The weight at every cell centre (the trilinear lookup) and the partial sums of
-// its absolute value: once per call, where the score kernel repeated both for
-// every threshold.
+// The weight at the centre of cell i (the trilinear lookup). small: fewer than 2^32 cells.
+__device__ __forceinline__ double cell_weight(const GridGeom& g, const GridGeom& wg, const double* __restrict__ w,
+                                              int64_t i, bool small) {
+  const int64_t X = g.res[0], XY = X * g.res[1];
+  int64_t x, y, z;
+  if (small) {
+    const uint32_t p = (uint32_t)i, zu = fast_div(p, g.div_xy), r = p - zu * (uint32_t)XY;
+    const uint32_t yu = fast_div(r, g.div_x);
+    z = zu;
+    y = yu;
+    x = r - yu * (uint32_t)X;
+  } else {
+    z = i / XY;
+    const int64_t r = i - z * XY;
+    y = r / X;
+    x = r - y * X;
+  }
+  double c[3];
+  cell_center(g, (int)x, (int)y, (int)z, c);
+  return field_lookup(wg, w, c);
+}
+
+// The weight at every cell and the partial sums of its absolute value: once per
+// call, where the score kernel repeated both for every threshold.
 __global__ __launch_bounds__(kOpsBlock) void k_cell_weights(GridGeom g, GridGeom wg, const double* __restrict__ w,
                                                             double* __restrict__ out, double* __restrict__ part) {
-  const int64_t n = (int64_t)g.res[0] * g.res[1] * g.res[2], X = g.res[0], XY = X * g.res[1];
+  const int64_t n = (int64_t)g.res[0] * g.res[1] * g.res[2];
   const bool small = n <= (int64_t)0xffffffffll;
   Acc a{{0.0, 0.0}, 0.0, 0.0};
   const int64_t stride = (int64_t)gridDim.x * kOpsBlock;
   for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
-    int64_t x, y, z;
-    if (small) {
-      const uint32_t p = (uint32_t)i, zu = fast_div(p, g.div_xy), r = p - zu * (uint32_t)XY;
-      const uint32_t yu = fast_div(r, g.div_x);
-      z = zu;
-      y = yu;
-      x = r - yu * (uint32_t)X;
-    } else {
-      z = i / XY;
-      const int64_t r = i - z * XY;
-      y = r / X;
-      x = r - y * X;
-    }
-    double c[3];
-    cell_center(g, (int)x, (int)y, (int)z, c);
-    const double wt = field_lookup(wg, w, c);
+    const double wt = cell_weight(g, wg, w, i, small);
     out[i] = wt;
-    acc_value(a, fabs(wt));
+    acc_sum(a, fabs(wt));
   }
   a = block_reduce(a);
   if (threadIdx.x == 0) store_part(part, blockIdx.x, a);
@@ -478,6 +484,41 @@ __global__ __launch_bounds__(kOpsBlock) void k_weight_score(const double* __rest
   for (int k = 0; k < kScores; k++) {
     const Acc s = block_reduce(a[k]);
     if (threadIdx.x == 0 && t0 + k < nthr) store_part(part, (int64_t)(t0 + k) * gridDim.x + blockIdx.x, s);
+    __syncthreads();
+  }
+}
+
+// The same for at most kScores thresholds (kN of them) in one pass: lookup, scores and
+// the weights' absolute sum (slot kN) together, with no array of cell weights between.
+// Up to 1024 blocks. FP64 VALU bound. One threshold, 128^3, 256^3 and 300^3: 47, 156 and 232 us; by
+// the two kernels, which take four thresholds for one and 8 bytes a cell, 84, 388 and
+// 962; a lookup per threshold and the library's tanh 76, 332 and 511.
+struct FewThresholds {
+  double t[kScores];
+};
+template <int kN>
+__global__ __launch_bounds__(kOpsBlock) void k_few_scores(const double* __restrict__ f, GridGeom g, GridGeom wg,
+                                                          const double* __restrict__ w, FewThresholds thr,
+                                                          double alpha, double* __restrict__ part) {
+  const int64_t n = (int64_t)g.res[0] * g.res[1] * g.res[2];
+  const bool small = n <= (int64_t)0xffffffffll;
+  Acc a[kN + 1];
+#pragma unroll
+  for (int k = 0; k <= kN; k++) a[k] = Acc{{0.0, 0.0}, 0.0, 0.0};
+  const int64_t stride = (int64_t)gridDim.x * kOpsBlock;
+  for (int64_t i = (int64_t)blockIdx.x * kOpsBlock + threadIdx.x; i < n; i += stride) {
+    const double wt = cell_weight(g, wg, w, i, small);
+    if (kN) {
+      const double F = f[i];
+#pragma unroll
+      for (int k = 0; k < kN; k++) acc_sum(a[k], -tanh64(alpha * (F - thr.t[k])) * wt);
+    }
+    acc_sum(a[kN], fabs(wt));
+  }
+#pragma unroll
+  for (int k = 0; k <= kN; k++) {
+    const Acc s = block_reduce(a[k]);
+    if (threadIdx.x == 0) store_part(part, (int64_t)k * gridDim.x + blockIdx.x, s);
     __syncthreads();
   }
 }
@@ -726,6 +767,29 @@ qj_status weight_scores(qj_workspace* ws, const double* d_field, const qj_grid* 
   make_geom(wgrid, &wg);
   const int64_t n = (int64_t)g.res[0] * g.res[1] * g.res[2];
   if (n <= 0 || nthr < 0) return QJ_ERR_INVALID;
+  const int slots = nthr + 1;
+  qj_status st;
+  if (nthr <= kScores) {
+    const int gx = (int)std::min<int64_t>((n + kOpsBlock - 1) / kOpsBlock, 1024);
+    if ((st = ensure_partials(ws, 4 * (int64_t)gx * slots, s))) return st;
+    if ((st = ensure_pinned(ws, slots, s))) return st;
+    FewThresholds few{};
+    for (int t = 0; t < nthr; t++) few.t[t] = thresholds[t];
+    const auto k = nthr == 0   ? k_few_scores<0>
+                   : nthr == 1 ? k_few_scores<1>
+                   : nthr == 2 ? k_few_scores<2>
+                   : nthr == 3 ? k_few_scores<3>
+                               : k_few_scores<4>;
+    hipLaunchKernelGGL(k, dim3(gx), dim3(kOpsBlock), 0, s, d_field, g, wg, d_weight, few, alpha, ws->d_partials);
+    QJ_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_fold_sums, dim3(slots), dim3(kOpsBlock), 0, s, (const double*)ws->d_partials, gx, gx,
+                       (double*)nullptr, ws->h_pinned, (double*)nullptr);
+    QJ_HIP(hipGetLastError());
+    QJ_HIP(hipStreamSynchronize(s));
+    for (int t = 0; t < nthr; t++) scores[t] = ws->h_pinned[t];
+    if (max_score) *max_score = ws->h_pinned[nthr];
+    return QJ_OK;
+  }
   // up to 8 cells per thread where the thresholds fill the chip by themselves:
   // the four block sums cost as much as some 10 cells (50^3, 100 thresholds: 6400
   // blocks of 2 cells take a fifth longer than 1750)
@@ -733,11 +797,9 @@ qj_status weight_scores(qj_workspace* ws, const double* d_field, const qj_grid* 
   const int64_t per = std::min<int64_t>(8, std::max<int64_t>(1, want * ny / 1536));
   const int gx = (int)std::min<int64_t>((want + per - 1) / per, 256);
   const int gw = (int)std::min<int64_t>(want, 256);
-  const int slots = nthr + 1;
   // the partials (the last slot's: the weights' absolute sum), the thresholds, the cells' weights
   const bool keep = n <= kKeepCells;
-  qj_status st = ensure_partials(ws, 4 * ((int64_t)gx * nthr + gw) + (int64_t)slots + (keep ? n : 0), s);
-  if (st) return st;
+  if ((st = ensure_partials(ws, 4 * ((int64_t)gx * nthr + gw) + (int64_t)slots + (keep ? n : 0), s))) return st;
   if ((st = ensure_pinned(ws, 2 * (int64_t)slots, s))) return st;
   double* part = ws->d_partials;
   double* d_thr = part + 4 * ((int64_t)gx * nthr + gw);
@@ -749,14 +811,12 @@ qj_status weight_scores(qj_workspace* ws, const double* d_field, const qj_grid* 
   hipLaunchKernelGGL(k_cell_weights, dim3(gw), dim3(kOpsBlock), 0, s, g, wg, d_weight, cw,
                      part + 4 * (int64_t)gx * nthr);
   QJ_HIP(hipGetLastError());
-  if (nthr) {
-    double* h_thr = ws->h_pinned + slots;
-    for (int t = 0; t < nthr; t++) h_thr[t] = thresholds[t];
-    QJ_HIP(hipMemcpyAsync(d_thr, h_thr, sizeof(double) * (size_t)nthr, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_weight_score, dim3(gx, (unsigned)ny), dim3(kOpsBlock), 0, s, d_field,
-                       (const double*)cw, n, (const double*)d_thr, nthr, alpha, part);
-    QJ_HIP(hipGetLastError());
-  }
+  double* h_thr = ws->h_pinned + slots;
+  for (int t = 0; t < nthr; t++) h_thr[t] = thresholds[t];
+  QJ_HIP(hipMemcpyAsync(d_thr, h_thr, sizeof(double) * (size_t)nthr, hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_weight_score, dim3(gx, (unsigned)ny), dim3(kOpsBlock), 0, s, d_field,
+                     (const double*)cw, n, (const double*)d_thr, nthr, alpha, part);
+  QJ_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_fold_sums, dim3(slots), dim3(kOpsBlock), 0, s, (const double*)part, gx, gw,
                      (double*)nullptr, ws->h_pinned, (double*)nullptr);
   QJ_HIP(hipGetLastError());
