@@ -48,7 +48,8 @@ class JuliaField(torch.autograd.Function):
             both = torch.cat([gr.view(-1), gp]).cpu()
             gr, gp = both[:gr.numel()].view(-1, 4), both[gr.numel():]
         outs = [gr[:nt], gp[:nt], gr[nt:], gp[nt:]]
-        outs = [o.to(device=d, dtype=t) for o, d, t in zip(outs, ctx.devices, ctx.dtypes)]
+        own = not gr.is_cuda  # a gradient on the host owns its memory
+        outs = [o.to(device=d, dtype=t, copy=own) for o, d, t in zip(outs, ctx.devices, ctx.dtypes)]
         return (None, outs[0], outs[1], outs[2], outs[3], None, None, None, None, None)
 
 
