@@ -45,8 +45,11 @@ __device__ __forceinline__ double div64(double n, double d) {
 
 // log(x) for normal positive x. x = 2^k m with m in [sqrt(1/2), sqrt(2)),
 // f = m - 1 (exact), s = f / (2 + f): log m = 2 atanh(s) = 2 s + s R(s^2) =
-// f - s (f - R), since 2 s = f - s f. Zero, denormal, infinite and NaN x give
-// a finite result beyond +-700.
+// f - s (f - R), since 2 s = f - s f. This reduction, with the offset to the
+// high word that splits at sqrt(1/2), and this form of the sum are the published
+// method of fdlibm's e_log.c (K. C. Ng, Sun Microsystems, 1993); the polynomial
+// is fit_math64.py's. Zero, denormal, infinite and NaN x give a finite result
+// beyond +-700.
 template <bool kInLoop = false>
 __device__ __forceinline__ double log64(double x) {
 #pragma clang fp contract(off)
