@@ -169,23 +169,10 @@ def main():
     k64 = _kernel_ms(api, ws)
     log("fp64: %.2f ms/step" % (t64 * 1e3))
 
-    # the same arithmetic under its other name (exponents 1 and 2 as exact
-    # products, as the FP32 path's band takes them)
+    # QJ_FP64_EXACT is the same kernel under its other name: compared, not timed again
     out64x = torch.empty(w.voxels, dtype=torch.float64, device="cuda")
-    log("fp64 exact: warmup")
     api.field_eval(grid, r, params, FP64_EXACT, out=out64x, workspace=ws)
-    torch.cuda.synchronize()
-    ws.reset_stats()
-    api._lib.load().qj_workspace_timing(ws.handle, 1)
-    t0 = time.perf_counter()
-    for _ in range(args.fp64_steps):
-        api.field_eval(grid, r, params, FP64_EXACT, out=out64x, workspace=ws)
-    torch.cuda.synchronize()
-    t64x = (time.perf_counter() - t0) / args.fp64_steps
-    k64x = _kernel_ms(api, ws)
-    api._lib.load().qj_workspace_timing(ws.handle, 0)
-    log("fp64 exact: %.2f ms/step" % (t64x * 1e3))
-    f64x = out64x.cpu().numpy()
+    exact_same = bool(torch.equal(out64x.view(torch.int64), out64.view(torch.int64)))
     del out64x
 
     # FP32 bulk + FP64 band
@@ -204,6 +191,18 @@ def main():
     k32 = _kernel_ms(api, ws)
     api._lib.load().qj_workspace_timing(ws.handle, 0)
     log("fp32+band: %.2f ms/step" % (t32 * 1e3))
+
+    # the band's cells and the FP64 field share an evaluator; the sampled check's
+    # reference method (polar powers, reference order) is neither's
+    sample = {}
+    for name, prec, out in (("fp64", FP64, out64), ("fp32band", FP32_BAND, out32)):
+        ws.check(65536)
+        ws.reset_stats()
+        api.field_eval(grid, r, params, prec, args.band, out=out, workspace=ws)
+        st = ws.stats()
+        sample[name] = {"cells": st["checked"], "sign_flips": st["check_sign_flips"],
+                        "class_mismatches": st["check_class_mismatch"], "max_rel_dF": st["check_max_rel_dF"]}
+    ws.check(0)
 
     f64 = out64.cpu().numpy()
     f32 = out32.cpu().numpy()
@@ -271,15 +270,12 @@ def main():
                        "achieved_tflops": round(fp64_flops / (fp64_ms * 1e-3) / 1e12, 3),
                        "peak": PEAK_FP64_TFLOPS},
         "speedup_vs_fp64": round(value / value64, 3),
-        "fp64_exact": {"value": round(nominal / t64x / 1e9, 4), "ms_per_step": round(t64x * 1e3, 3),
-                       "kernel_ms": round(k64x["bulk_ms"] / max(1, k64x["launches"]), 3),
-                       "what": "all voxels in FP64, exponents 1 and 2 as exact products (QJ_FP64_EXACT)",
-                       "sign_flips_vs_fp64_gpu": int(np.count_nonzero((f64.astype(np.float32) > 0) !=
-                                                                      (f64x.astype(np.float32) > 0)))},
-        "speedup_vs_fp64_exact": round(value / (nominal / t64x / 1e9), 3),
+        "fp64_exact": {"same_bytes_as_fp64": exact_same,
+                       "what": "QJ_FP64_EXACT, the same kernel as fp64_plain's under its other name: not timed again"},
         "band": {"voxels": st32["band_voxels"] // args.steps, "fraction": st32["band_voxels"] / args.steps / w.voxels,
                  "band_kernel_ms": round(band_ms, 4)},
-        "parity": {"sign_flips_vs_fp64_gpu": flips_vs_fp64, "max_abs_dF_vs_fp64_gpu": maxdf},
+        "parity": {"sign_flips_vs_fp64_gpu": flips_vs_fp64, "max_abs_dF_vs_fp64_gpu": maxdf,
+                   "reference_method_sample": sample},
         "roofline": roofline,
         "cpu_baseline": cpu,
         "c3_1024_tiles": c3,

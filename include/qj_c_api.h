@@ -162,7 +162,7 @@ qj_status qj_workspace_reset_stats(qj_workspace* ws, void* stream);
  * apart); as the difference the larger of the field's from QJ_FP64's value and
  * of that from the reference method's, so that a QJ_FP64 field shows its own
  * error. One extra kernel per field, about the latency of one FP64 evaluation
- * per cell (0.5 ms for 32+32 roots, maxIter 4).
+ * per cell by each of the two methods (0.26 ms for 32+32 roots, maxIter 4).
  * 0 (the default) turns it off; at most 2^24. */
 qj_status qj_workspace_check(qj_workspace* ws, int64_t samples);
 
