@@ -120,9 +120,12 @@ __device__ __forceinline__ Res64 eval_kind(const MapArgs& a, const RootRec64* __
 }
 
 // kPow: kExactOnly or kExactInt. FP64 VALU bound: 32+32 roots with exponents 1 and 2,
-// 256^3, 4 iterations 43.7 to 3.3 ms, 64^3 with 8 roots 78 to 12.6 us against the
+// 256^3, 4 iterations 43.7 to 3.2 ms, 64^3 with 8 roots 78 to 11.5 us against the
 // device library's polar form for every power; with real exponents, 50^3 and one
-// iteration, 267 to 36 us. The extended range's band list of a 256^3 torus tile
+// iteration, 267 to 35 us. Dearer than that form: grids below about 40^3 whose last
+// iteration's norms could leave FP64's range, so that the products follow them (24^3,
+// 32+32 real exponents, three iterations 193 to 232 us, two 132 to 133, four 253 to
+// 238). The extended range's band list of a 256^3 torus tile
 // (128+128 roots) 1.69 to 0.64 ms, the request loop's 1.40 to 0.80 ms a launch.
 template <int kEval, int kPow>
 __global__ __launch_bounds__(kBlock) void k_grid64(MapArgs a, const RootRec64* __restrict__ roots,
@@ -295,9 +298,11 @@ __device__ __forceinline__ Res64 eval_checked(const MapArgs& a, const RootRec64*
 // iteration and the grouped products too. The difference is the larger of the
 // field's from QJ_FP64's value and of that from the reference method's: the
 // first alone is 0 for every cell that QJ_FP64's code wrote, the second alone
-// has its own rounding in it. Counts of checked cells, sign disagreements of (float)F > 0 (the mesher's predicate) and class
-// disagreements (finite / NaN / +-inf), and the largest absolute and relative
-// (to max(1, |F64|)) differences over cells finite in both.
+// has its own rounding in it. Counts of checked cells, sign disagreements of
+// (float)F > 0 (the mesher's predicate) and class disagreements (finite / NaN /
+// +-inf), and the largest absolute and relative (to max(1, |F|)) differences over
+// cells finite in both. Bound by one cell's latency: 4096 to 65,536 cells, 32+32
+// roots, four iterations 0.26 ms a field (the reference method alone 0.22 to 0.25).
 // kSpread: copies per counter slot (a workspace's counters), or 1 for the
 // request loop's per-result block of CNT_N counters.
 template <int kEval, int kSpread = kCounterSpread>

@@ -490,9 +490,9 @@ __global__ __launch_bounds__(kOpsBlock) void k_weight_score(const double* __rest
 
 // The same for at most kScores thresholds (kN of them) in one pass: lookup, scores and
 // the weights' absolute sum (slot kN) together, with no array of cell weights between.
-// Up to 1024 blocks. FP64 VALU bound. One threshold, 128^3, 256^3 and 300^3: 47, 156 and 232 us; by
-// the two kernels, which take four thresholds for one and 8 bytes a cell, 84, 388 and
-// 962; a lookup per threshold and the library's tanh 76, 332 and 511.
+// Up to 1024 blocks. FP64 VALU bound. One threshold, 128^3, 256^3 and 300^3: 47, 156
+// and 232 us; by the two kernels, which take four thresholds for one and 8 bytes a
+// cell, 84, 388 and 962; a lookup per threshold and the library's tanh 76, 332 and 511.
 struct FewThresholds {
   double t[kScores];
 };

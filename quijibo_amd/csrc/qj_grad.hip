@@ -747,8 +747,8 @@ static bool ap_from_logs(const MapArgs& a, const std::vector<RootRec64>& roots) 
 // logarithms of up to 8 or 16 roots in registers (128 and 192 VGPRs), of up to 32
 // in 64-cell blocks; beyond 128 roots on grids of 256-cell blocks and 256 on
 // smaller ones they are computed twice (97^3 with 32+32 roots: 149 us that way, 128
-// kept). Against the product formulas for every cell: 97^3 2264 to 128 us a call,
-// 25^3 254 to 36 us; the kernel takes 113 us of the 128, its FP64 issue about 80.
+// kept). Against the product formulas for every cell: 97^3 2280 to 126 us a call,
+// 25^3 257 to 36 us; the kernel takes 108 us of the 126, its FP64 issue about 80.
 qj_status ap_grads(qj_workspace* ws, const MapArgs& a, const qj_rational* f, const qj_grid* wg, const double* d_weight,
                    double alpha, double thr, double* d_field, double* gt, double* gb, qj_ap_grads* out,
                    hipStream_t s) {

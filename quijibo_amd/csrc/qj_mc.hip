@@ -897,7 +897,7 @@ __global__ __launch_bounds__(kMcBlock) void k_mc_measure(const double* __restric
 // way, listed in LDS and measured one per thread, unless lost says what
 // k_mc_measure dropped.
 // flags: the case of every cell that has
-// triangles, else 0. Latency-bound: 256^3, 1024 blocks, 20.5 us with the
+// triangles, else 0. Latency-bound: 256^3, 1024 blocks, 19.2 us with the
 // scan, of which the measurement's longest chain is 6 (20 with every near pair
 // measured). tword: the triangles before word w in its group; groups:
 // per group.
