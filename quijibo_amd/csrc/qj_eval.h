@@ -403,8 +403,9 @@ __device__ __forceinline__ q64 lagrange64(RP roots, int nt, int nb, const q64& q
   q64 r{1.0, 0.0, 0.0, 0.0};
   const int same = nt < nb ? nt : nb;
   for (int i = 0; i < same; i++) {
-    r = qmul(r, term64<kPow>(load_root64(roots + i), q));
-    r = qdiv(r, term64<kPow>(load_root64(bot + i), q));
+    const RootRec64 t = load_root64(roots + i), d = load_root64(bot + i);  // d's load behind t's term
+    r = qmul(r, term64<kPow>(t, q));
+    r = qdiv(r, term64<kPow>(d, q));
   }
   for (int i = same; i < nt; i++) r = qmul(r, term64<kPow>(load_root64(roots + i), q));
   for (int i = same; i < nb; i++) r = qdiv(r, term64<kPow>(load_root64(bot + i), q));
