@@ -123,9 +123,9 @@ __device__ __forceinline__ Res64 eval_kind(const MapArgs& a, const RootRec64* __
 // 256^3, 4 iterations 43.7 to 3.2 ms, 64^3 with 8 roots 78 to 11.5 us against the
 // device library's polar form for every power; with real exponents, 50^3 and one
 // iteration, 267 to 35 us. Dearer than that form: grids below about 40^3 whose last
-// iteration's norms could leave FP64's range, so that the products follow them (24^3,
-// 32+32 real exponents, three iterations 193 to 232 us, two 132 to 133, four 253 to
-// 238). The extended range's band list of a 256^3 torus tile
+// iteration's norms could leave FP64's range, so that the products follow them (33^3,
+// 100+100 real exponents, three iterations 590 to 710 us; 24^3 with 32+32, whose norms
+// stay in it, 193 to 119). The extended range's band list of a 256^3 torus tile
 // (128+128 roots) 1.69 to 0.64 ms, the request loop's 1.40 to 0.80 ms a launch.
 template <int kEval, int kPow>
 __global__ __launch_bounds__(kBlock) void k_grid64(MapArgs a, const RootRec64* __restrict__ roots,
