@@ -44,12 +44,14 @@ class JuliaField(torch.autograd.Function):
         gr, gp = api.points_adjoint(points, ctx.rational, ctx.params, g, ctx.precision)
         nt = ctx.nt
         if gr.is_cuda and all(d.type == "cpu" for d in ctx.devices):
-            # one copy to the host (each waits for the stream) instead of one per gradient
-            both = torch.cat([gr.view(-1), gp]).cpu()
-            gr, gp = both[:gr.numel()].view(-1, 4), both[gr.numel():]
-        outs = [gr[:nt], gp[:nt], gr[nt:], gp[nt:]]
-        own = not gr.is_cuda  # a gradient on the host owns its memory
-        outs = [o.to(device=d, dtype=t, copy=own) for o, d, t in zip(outs, ctx.devices, ctx.dtypes)]
+            # one copy to the host (each waits for the stream) instead of one per gradient;
+            # then each of them in memory of its own
+            nb = gp.numel() - nt
+            host = torch.split_with_sizes_copy(torch.cat([gr.view(-1), gp]).cpu(), [4 * nt, 4 * nb, nt, nb])
+            outs = [host[0].view(nt, 4), host[2], host[1].view(nb, 4), host[3]]
+        else:
+            outs = [gr[:nt], gp[:nt], gr[nt:], gp[nt:]]
+        outs = [o.to(device=d, dtype=t) for o, d, t in zip(outs, ctx.devices, ctx.dtypes)]
         return (None, outs[0], outs[1], outs[2], outs[3], None, None, None, None, None)
 
 
