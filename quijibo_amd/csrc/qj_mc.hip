@@ -20,7 +20,8 @@
 //   k_mc_measure    the degenerate filter (edge < 1e-7 dropped) on the cells whose
 //                   near vertices lie on edges that meet, where estimates do not
 //                   decide it (kMeasureAll, kMeasureNear) and groups are few
-//   k_mc_cells      triangle counts, and elsewhere the degenerate filter; its last block, or k_mc_scan: first triangle per group
+//   k_mc_cells      triangle counts, and elsewhere the degenerate filter; its last
+//                   block, or k_mc_scan: first triangle per group
 //   k_mc_tris       each kept triangle written once, in cell then table order
 #include <float.h>
 #include <math.h>
